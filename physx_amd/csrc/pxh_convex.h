@@ -994,11 +994,7 @@ PXH_D int capsulePoly(float r, float hh, const xf& x0, const Poly& B, const xf& 
 		const PC& c = mc[i == 0 ? i0 : i1];
 		const float sep = c.pen - r;
 		if (cd >= sep)
-		{
-			o.p[o.count] = xtrans(x0, c.la) - wn * r;
-			o.sep[o.count] = sep;
-			o.count++;
-		}
+			pushContact(o, xtrans(x0, c.la) - wn * r, sep);
 	}
 	return o.count;
 }

