@@ -82,8 +82,8 @@ int broadphase(Ctx* s, int n, int nWorlds, const int* d_scene, const int* d_grou
 	const int nblocks = (n + radix_tile() - 1) / radix_tile();
 	PXH_CHECK(s->hist.ensure(size_t(256) * std::max(nblocks, 1)));
 	bool alt = false;
-	const int bitEnd = 32 + ((bitsFor(totalRows) + 7) / 8) * 8;
-	launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, n, 0, bitEnd, s->hist.p, s->scanTmp.p, st, alt);
+	launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, n, 32, bitsFor(totalRows - 1u), s->hist.p, st,
+	                  alt);
 	s->sortedKeys = alt ? s->keys2.p : s->keys.p;
 	const uint32_t* sv = alt ? s->vals2.p : s->vals.p;
 
@@ -168,14 +168,10 @@ int bp_update(Ctx* bp, const float* bounds, const uint32_t* groups, const float*
 	launch_pair_keys(P, bp->pairs.p, ids, bp->pkCur.p, bp->vals.p, st);
 	const int nblocks = (P + radix_tile() - 1) / radix_tile();
 	PXH_CHECK(bp->hist.ensure(size_t(256) * std::max(nblocks, 1)));
-	PXH_CHECK(bp->scanTmp.ensure(
-	    scan_tmp_size(std::max<int64_t>(std::max<int64_t>(int64_t(256) * std::max(nblocks, 1), P + 1),
-	                                    int64_t(bp->nCur) + 1)) +
-	    1024));
+	PXH_CHECK(bp->scanTmp.ensure(scan_tmp_size(std::max<int64_t>(P + 1, int64_t(bp->nCur) + 1)) + 1024));
 	bool alt = false;
-	const int bits = 32 + ((bitsFor(uint64_t(ids ? std::max<uint32_t>(idBound, 1u) : uint32_t(std::max(n, 1)))) + 7) / 8) * 8;
-	launch_radix_sort(bp->pkCur.p, bp->vals.p, bp->pkTmp.p, bp->vals2.p, P, 0, bits, bp->hist.p, bp->scanTmp.p, st,
-	                  alt);
+	const int bits = bitsFor(uint64_t(ids ? std::max<uint32_t>(idBound, 1u) : uint32_t(std::max(n, 1))) - 1);
+	launch_radix_sort(bp->pkCur.p, bp->vals.p, bp->pkTmp.p, bp->vals2.p, P, bits, bits, bp->hist.p, st, alt);
 	if (alt)
 		std::swap(bp->pkCur, bp->pkTmp);
 	bp->nCur = P;

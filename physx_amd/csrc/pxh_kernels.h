@@ -128,8 +128,10 @@ int64_t scan_tmp_size(int64_t n);
 void launch_scan(uint32_t* data, int64_t n, uint32_t* tmp, hipStream_t st);
 // keys per radix-sort workgroup (its histogram holds 256 counts per workgroup)
 int radix_tile();
-void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t* vals2, int n, int bitBegin,
-                       int bitEnd, uint32_t* hist, uint32_t* scanTmp, hipStream_t st, bool& resultInAlt);
+// stable sort by the key's high word, below 2^highBits, then by the low
+// lowBits bits of its low word (0: the low word is not compared)
+void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t* vals2, int n, int lowBits,
+                       int highBits, uint32_t* hist, hipStream_t st, bool& resultInAlt);
 
 void launch_bounds(int n, const float4* pos, const float4* rot, const float4* geom, const HullSet& hs, float co,
                    float4* bmin, float4* bmax, hipStream_t st);

@@ -64,148 +64,345 @@ PXH_D uint32_t blockExclScan(uint32_t v, uint32_t* sh, uint32_t& total)
 	return r;
 }
 
-constexpr int SCAN_THREADS = 256, SCAN_ITEMS = 8, SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
+// Exclusive scan in two launches: the sums of 4,096-element tiles, then every
+// tile adds up the sums before it and scans its own elements; an array of one
+// tile needs the second launch alone. Bound by launches and their latency at
+// the step's sizes: 11 us on average at 262k bodies, where three launches and a
+// second pass over the data took 13. A tile of 4,096 keeps the sums to add up
+// below 1,500 for the largest arrays here (six pair classes of a million
+// bodies).
+constexpr int SCAN_THREADS = 256, SCAN_ITEMS = 16, SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
 
-// in-place exclusive scan of each 2048-element tile; tile sums to blockSums
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(uint32_t* data, int64_t n, uint32_t* blockSums)
+// sum over the block; every thread gets it (sh: 8 entries)
+PXH_D uint32_t blockSum(uint32_t v, uint32_t* sh)
 {
-	__shared__ uint32_t sh[33];
-	__shared__ uint32_t tile[SCAN_TILE];
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1)
+		v += __shfl_xor(v, o, 64);
+	if ((threadIdx.x & 63) == 0)
+		sh[threadIdx.x >> 6] = v;
+	__syncthreads();
+	uint32_t t = 0;
+	for (int w = 0; w < int(blockDim.x >> 6); w++)
+		t += sh[w];
+	__syncthreads();
+	return t;
+}
+
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_sums(const uint32_t* data, int64_t n, uint32_t* sums)
+{
+	__shared__ uint32_t sh[8];
 	const int64_t base = int64_t(blockIdx.x) * SCAN_TILE;
+	uint32_t v = 0;
+#pragma unroll
 	for (int k = 0; k < SCAN_ITEMS; k++)
 	{
 		const int64_t g = base + k * SCAN_THREADS + threadIdx.x;
-		tile[k * SCAN_THREADS + threadIdx.x] = g < n ? data[g] : 0u;
+		v += g < n ? data[g] : 0u;
 	}
-	__syncthreads();
-	uint32_t loc[SCAN_ITEMS];
-	uint32_t sum = 0;
+	v = blockSum(v, sh);
+	if (threadIdx.x == 0)
+		sums[blockIdx.x] = v;
+}
+
+// in-place exclusive scan of each tile, offset by the sums of the tiles before it
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(uint32_t* data, int64_t n, const uint32_t* sums)
+{
+	__shared__ uint32_t sh[33];
+	__shared__ uint32_t tile[SCAN_TILE + SCAN_TILE / 32];   // a word of padding every 32: no bank conflicts
+	auto at = [](int i) { return i + (i >> 5); };
+	const int64_t base = int64_t(blockIdx.x) * SCAN_TILE;
+#pragma unroll
 	for (int k = 0; k < SCAN_ITEMS; k++)
 	{
-		loc[k] = tile[threadIdx.x * SCAN_ITEMS + k];
+		const int i = k * SCAN_THREADS + threadIdx.x;
+		tile[at(i)] = base + i < n ? data[base + i] : 0u;
+	}
+	uint32_t before = 0;
+	for (int t = threadIdx.x; t < int(blockIdx.x); t += SCAN_THREADS)
+		before += sums[t];
+	before = blockSum(before, sh);   // its barriers also publish the tile
+	uint32_t loc[SCAN_ITEMS];
+	uint32_t sum = 0;
+#pragma unroll
+	for (int k = 0; k < SCAN_ITEMS; k++)
+	{
+		loc[k] = tile[at(threadIdx.x * SCAN_ITEMS + k)];
 		sum += loc[k];
 	}
 	uint32_t total;
-	uint32_t pre = blockExclScan(sum, sh, total);
+	uint32_t pre = before + blockExclScan(sum, sh, total);
+#pragma unroll
 	for (int k = 0; k < SCAN_ITEMS; k++)
 	{
-		tile[threadIdx.x * SCAN_ITEMS + k] = pre;
+		tile[at(threadIdx.x * SCAN_ITEMS + k)] = pre;
 		pre += loc[k];
 	}
 	__syncthreads();
+#pragma unroll
 	for (int k = 0; k < SCAN_ITEMS; k++)
 	{
-		const int64_t g = base + k * SCAN_THREADS + threadIdx.x;
-		if (g < n)
-			data[g] = tile[k * SCAN_THREADS + threadIdx.x];
+		const int i = k * SCAN_THREADS + threadIdx.x;
+		if (base + i < n)
+			data[base + i] = tile[at(i)];
 	}
-	if (threadIdx.x == 0 && blockSums)
-		blockSums[blockIdx.x] = total;
-}
-
-__global__ void k_scan_add(uint32_t* data, int64_t n, const uint32_t* blockOffsets)
-{
-	const int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (g < n)
-		data[g] += blockOffsets[g / SCAN_TILE];
 }
 
 // ---------------------------------------------------------------------------
 // LSD radix sort of (u64 key, u32 value), 8-bit digits, stable
 // ---------------------------------------------------------------------------
-// 512-key tiles: a 262k-key sort spreads over 512 workgroups, two per CU
-constexpr int RS_THREADS = 256, RS_ITEMS = 2, RS_TILE = RS_THREADS * RS_ITEMS;
+// A key is two fields, the low lowBits bits of its low word below its high
+// word; the digits run over the two fields joined, so the unused bits between
+// them cost no pass.
+//
+// Up to RS_SMALL keys: one launch, one workgroup keeps the keys in registers
+// through every pass. More: two launches a pass, the digit counts of 4,096-key
+// tiles and the scatter, in which each tile adds up the counts of the tiles
+// before it itself (a 262,144-key sort has 64 tiles), so no scan runs between.
+// A key's rank in its wave comes from eight ballots (the lanes with its digit).
+// Bound by launches and latency. 262,144 broadphase keys (51 bits, seven
+// passes): 107 us, where a count, a scan of three launches and a bit-by-bit
+// split a pass took 219; 4,096 keys (six passes): 30 us in one launch against
+// 117 in thirty; a million keys: 18 us a scatter against 22.
+constexpr int RS_THREADS = 1024, RS_ITEMS = 4, RS_TILE = RS_THREADS * RS_ITEMS;
+constexpr int RS_SMALL_THREADS = 1024, RS_SMALL_ITEMS = 8, RS_SMALL = RS_SMALL_THREADS * RS_SMALL_ITEMS;
 int radix_tile() { return RS_TILE; }
 
-__global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const uint64_t* keys, int n, int shift, uint32_t* hist, int nblocks)
+PXH_D uint32_t rsDigit(uint64_t key, int lowBits, int shift)
+{
+	const uint64_t low = lowBits >= 32 ? (key & 0xFFFFFFFFull) : (key & ((1ull << lowBits) - 1ull));
+	return uint32_t((((key >> 32) << lowBits) | low) >> shift) & 0xFFu;
+}
+
+// the lanes of the wave that are valid and hold digit d
+PXH_D uint64_t rsPeers(uint32_t d, bool valid)
+{
+	uint64_t m = __ballot(valid);
+#pragma unroll
+	for (int b = 0; b < 8; b++)
+	{
+		const bool one = d >> b & 1u;
+		const uint64_t v = __ballot(one);
+		m &= one ? v : ~v;
+	}
+	return m;
+}
+
+__global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const uint64_t* keys, int n, int lowBits, int shift,
+                                                        uint32_t* hist)
 {
 	__shared__ uint32_t cnt[256];
-	cnt[threadIdx.x] = 0;
+	if (threadIdx.x < 256)
+		cnt[threadIdx.x] = 0;
 	__syncthreads();
 	const int base = blockIdx.x * RS_TILE;
+#pragma unroll
 	for (int k = 0; k < RS_ITEMS; k++)
 	{
 		const int g = base + k * RS_THREADS + threadIdx.x;
 		if (g < n)
-			atomicAdd(&cnt[uint32_t(keys[g] >> shift) & 0xFFu], 1u);
+			atomicAdd(&cnt[rsDigit(keys[g], lowBits, shift)], 1u);
 	}
 	__syncthreads();
-	hist[threadIdx.x * nblocks + blockIdx.x] = cnt[threadIdx.x];
+	if (threadIdx.x < 256)
+		hist[int64_t(blockIdx.x) * 256 + threadIdx.x] = cnt[threadIdx.x];
 }
 
 __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const uint64_t* kin, const uint32_t* vin, uint64_t* kout,
-                                                            uint32_t* vout, int n, int shift, const uint32_t* hist,
-                                                            int nblocks)
+                                                           uint32_t* vout, int n, int lowBits, int shift,
+                                                           const uint32_t* hist, int nblocks)
 {
-	__shared__ uint64_t sk[RS_TILE];
-	__shared__ uint32_t sv[RS_TILE];
+	constexpr int WAVES = RS_THREADS / 64, PARTS = RS_THREADS / 256;
+	__shared__ uint32_t cnt[WAVES][256];
+	__shared__ uint32_t part[PARTS][2][256];
+	__shared__ uint32_t start[256], shift0[256];
 	__shared__ uint32_t sh[33];
-	__shared__ uint32_t dstart[256];
-	const int base = blockIdx.x * RS_TILE;
-	const int nvalid = min(RS_TILE, n - base);
+	__shared__ uint64_t xk[RS_TILE];
+	__shared__ uint32_t xv[RS_TILE];
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	// item k of the wave: 64 keys in order, the wave's items one after the other
+	const int base = blockIdx.x * RS_TILE + w * (64 * RS_ITEMS) + lane;
+	uint64_t key[RS_ITEMS];
+	uint32_t val[RS_ITEMS];
+#pragma unroll
 	for (int k = 0; k < RS_ITEMS; k++)
 	{
-		const int l = k * RS_THREADS + threadIdx.x;
-		const int g = base + l;
-		sk[l] = g < n ? kin[g] : ~0ull;
-		sv[l] = g < n ? vin[g] : 0u;
+		const int g = base + 64 * k;
+		key[k] = g < n ? kin[g] : 0ull;
+		val[k] = g < n ? vin[g] : 0u;
+	}
+	for (int i = lane; i < 256; i += 64)
+		cnt[w][i] = 0u;
+	// this digit's count over all tiles and over the tiles before this one,
+	// every PARTS-th tile to each part of the block
+	{
+		const int d = threadIdx.x & 255, p = threadIdx.x >> 8;
+		uint32_t all = 0, before = 0;
+#pragma unroll 8
+		for (int b = p; b < nblocks; b += PARTS)
+		{
+			const uint32_t c = hist[int64_t(b) * 256 + d];
+			all += c;
+			before += b < int(blockIdx.x) ? c : 0u;
+		}
+		part[p][0][d] = all;
+		part[p][1][d] = before;
+	}
+	// ranks among the wave's earlier keys of the same digit; a wave's LDS
+	// accesses keep their order, and only it uses its counters here
+	uint32_t rank[RS_ITEMS];
+	volatile uint32_t* mine = cnt[w];
+#pragma unroll
+	for (int k = 0; k < RS_ITEMS; k++)
+	{
+		const uint32_t d = rsDigit(key[k], lowBits, shift);
+		const bool valid = base + 64 * k < n;
+		const uint64_t m = rsPeers(d, valid);
+		const uint32_t lower = uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+		const uint32_t had = mine[d];
+		rank[k] = had + lower;
+		if (valid && lower == 0)
+			mine[d] = had + uint32_t(__popcll(m));
 	}
 	__syncthreads();
-	// stable split of the tile by each of the 8 bits, least significant first
-	uint64_t k8[RS_ITEMS];
-	uint32_t v8[RS_ITEMS];
-	for (int k = 0; k < RS_ITEMS; k++)
+	// the digit's first place in the output and in this tile's sorted order
 	{
-		k8[k] = sk[threadIdx.x * RS_ITEMS + k];
-		v8[k] = sv[threadIdx.x * RS_ITEMS + k];
-	}
-	for (int b = 0; b < 8; b++)
-	{
-		const int bit = shift + b;
-		uint32_t zeros = 0;
-		for (int k = 0; k < RS_ITEMS; k++)
-			zeros += ((k8[k] >> bit) & 1ull) ? 0u : 1u;
-		uint32_t totalZeros;
-		const uint32_t zb = blockExclScan(zeros, sh, totalZeros);
-		uint32_t z = zb, o = totalZeros + threadIdx.x * RS_ITEMS - zb;
-		__syncthreads();
-		for (int k = 0; k < RS_ITEMS; k++)
+		const int d = threadIdx.x & 255;
+		uint32_t own = 0, total = 0, before = 0;
+		if (threadIdx.x < 256)
 		{
-			const bool one = (k8[k] >> bit) & 1ull;
-			const uint32_t dst = one ? o++ : z++;
-			sk[dst] = k8[k];
-			sv[dst] = v8[k];
+#pragma unroll
+			for (int i = 0; i < WAVES; i++)
+			{
+				const uint32_t c = cnt[i][d];
+				cnt[i][d] = own;
+				own += c;
+			}
+#pragma unroll
+			for (int p = 0; p < PARTS; p++)
+			{
+				total += part[p][0][d];
+				before += part[p][1][d];
+			}
 		}
-		__syncthreads();
-		for (int k = 0; k < RS_ITEMS; k++)
+		uint32_t sum;
+		const uint32_t local = blockExclScan(own, sh, sum);
+		const uint32_t pre = blockExclScan(total, sh, sum);
+		if (threadIdx.x < 256)
 		{
-			k8[k] = sk[threadIdx.x * RS_ITEMS + k];
-			v8[k] = sv[threadIdx.x * RS_ITEMS + k];
+			start[d] = local;
+			shift0[d] = pre + before - local;
 		}
-		__syncthreads();
-	}
-	// digit starts inside the sorted tile
-	for (int k = 0; k < RS_ITEMS; k++)
-	{
-		const int p = threadIdx.x * RS_ITEMS + k;
-		const uint32_t d = uint32_t(k8[k] >> shift) & 0xFFu;
-		const uint32_t dp = p == 0 ? 0xFFFFFFFFu : (uint32_t(sk[p - 1] >> shift) & 0xFFu);
-		if (p < nvalid && d != dp)
-			dstart[d] = p;
 	}
 	__syncthreads();
+	// through LDS in sorted order, so the keys of a digit leave side by side
+#pragma unroll
+	for (int k = 0; k < RS_ITEMS; k++)
+		if (base + 64 * k < n)
+		{
+			const uint32_t d = rsDigit(key[k], lowBits, shift);
+			const uint32_t at = start[d] + cnt[w][d] + rank[k];
+			xk[at] = key[k];
+			xv[at] = val[k];
+		}
+	__syncthreads();
+	const int live = min(RS_TILE, n - int(blockIdx.x) * RS_TILE);
+#pragma unroll
 	for (int k = 0; k < RS_ITEMS; k++)
 	{
-		const int p = k * RS_THREADS + threadIdx.x;
-		if (p < nvalid)
+		const int at = k * RS_THREADS + threadIdx.x;
+		if (at < live)
 		{
-			const uint64_t key = sk[p];
-			const uint32_t d = uint32_t(key >> shift) & 0xFFu;
-			const uint32_t dst = hist[d * nblocks + blockIdx.x] + (p - dstart[d]);
-			kout[dst] = key;
-			vout[dst] = sv[p];
+			const uint64_t x = xk[at];
+			const uint32_t dst = shift0[rsDigit(x, lowBits, shift)] + uint32_t(at);
+			kout[dst] = x;
+			vout[dst] = xv[at];
 		}
 	}
+}
+
+// every pass of up to 1,024 * ITEMS keys in one workgroup
+template <int ITEMS>
+__global__ void __launch_bounds__(RS_SMALL_THREADS) k_rs_small(uint64_t* keys, uint32_t* vals, int n, int lowBits,
+                                                               int bits)
+{
+	constexpr int WAVES = RS_SMALL_THREADS / 64;
+	__shared__ uint32_t cnt[WAVES][256];
+	__shared__ uint32_t start[256];
+	__shared__ uint32_t sh[33];
+	__shared__ uint64_t xk[RS_SMALL_THREADS * ITEMS];
+	__shared__ uint32_t xv[RS_SMALL_THREADS * ITEMS];
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	const int base = w * (64 * ITEMS) + lane;
+	uint64_t key[ITEMS];
+	uint32_t val[ITEMS];
+#pragma unroll
+	for (int k = 0; k < ITEMS; k++)
+	{
+		const int g = base + 64 * k;
+		key[k] = g < n ? keys[g] : 0ull;
+		val[k] = g < n ? vals[g] : 0u;
+	}
+	for (int shift = 0; shift < bits; shift += 8)
+	{
+		for (int i = lane; i < 256; i += 64)
+			cnt[w][i] = 0u;
+		uint32_t rank[ITEMS];
+		volatile uint32_t* mine = cnt[w];
+#pragma unroll
+		for (int k = 0; k < ITEMS; k++)
+		{
+			const uint32_t d = rsDigit(key[k], lowBits, shift);
+			const bool valid = base + 64 * k < n;
+			const uint64_t m = rsPeers(d, valid);
+			const uint32_t lower = uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+			const uint32_t had = mine[d];
+			rank[k] = had + lower;
+			if (valid && lower == 0)
+				mine[d] = had + uint32_t(__popcll(m));
+		}
+		__syncthreads();
+		uint32_t total = 0;
+		if (threadIdx.x < 256)
+		{
+#pragma unroll
+			for (int i = 0; i < WAVES; i++)
+			{
+				const uint32_t c = cnt[i][threadIdx.x];
+				cnt[i][threadIdx.x] = total;
+				total += c;
+			}
+		}
+		uint32_t sum;
+		const uint32_t pre = blockExclScan(total, sh, sum);
+		if (threadIdx.x < 256)
+			start[threadIdx.x] = pre;
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < ITEMS; k++)
+			if (base + 64 * k < n)
+			{
+				const uint32_t d = rsDigit(key[k], lowBits, shift);
+				const uint32_t at = start[d] + cnt[w][d] + rank[k];
+				xk[at] = key[k];
+				xv[at] = val[k];
+			}
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < ITEMS; k++)
+			if (base + 64 * k < n)
+			{
+				key[k] = xk[base + 64 * k];
+				val[k] = xv[base + 64 * k];
+			}
+	}
+#pragma unroll
+	for (int k = 0; k < ITEMS; k++)
+		if (base + 64 * k < n)
+		{
+			keys[base + 64 * k] = key[k];
+			vals[base + 64 * k] = val[k];
+		}
 }
 
 // ---------------------------------------------------------------------------
@@ -2975,45 +3172,45 @@ static inline int nblk(int64_t n, int t) { return int((n + t - 1) / t); }
 
 void launch_scan(uint32_t* data, int64_t n, uint32_t* tmp, hipStream_t st)
 {
-	// tmp must hold ceil(n/2048) + ceil(n/2048^2) + ... entries
+	// tmp must hold scan_tmp_size(n) entries
 	if (n <= 0)
 		return;
-	const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-	k_scan_tiles<<<int(nb), SCAN_THREADS, 0, st>>>(data, n, nb > 1 ? tmp : nullptr);
+	const int nb = nblk(n, SCAN_TILE);
 	if (nb > 1)
-	{
-		launch_scan(tmp, nb, tmp + nb, st);
-		k_scan_add<<<nblk(n, 256), 256, 0, st>>>(data, n, tmp);
-	}
+		k_scan_sums<<<nb, SCAN_THREADS, 0, st>>>(data, n, tmp);
+	k_scan_tiles<<<nb, SCAN_THREADS, 0, st>>>(data, n, tmp);
 }
 
-int64_t scan_tmp_size(int64_t n)
-{
-	int64_t total = 0;
-	while (n > 1)
-	{
-		n = (n + SCAN_TILE - 1) / SCAN_TILE;
-		total += n;
-	}
-	return total + 1;
-}
+int64_t scan_tmp_size(int64_t n) { return (std::max<int64_t>(n, 0) + SCAN_TILE - 1) / SCAN_TILE + 1; }
 
-void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t* vals2, int n, int bitBegin,
-                       int bitEnd, uint32_t* hist, uint32_t* scanTmp, hipStream_t st, bool& resultInAlt)
+void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t* vals2, int n, int lowBits,
+                       int highBits, uint32_t* hist, hipStream_t st, bool& resultInAlt)
 {
 	resultInAlt = false;
-	if (n <= 0)
+	const int bits = lowBits + highBits;
+	if (n <= 0 || bits <= 0)
 		return;
+	if (n <= RS_SMALL)
+	{
+		if (n <= RS_SMALL_THREADS)
+			k_rs_small<1><<<1, RS_SMALL_THREADS, 0, st>>>(keys, vals, n, lowBits, bits);
+		else if (n <= 2 * RS_SMALL_THREADS)
+			k_rs_small<2><<<1, RS_SMALL_THREADS, 0, st>>>(keys, vals, n, lowBits, bits);
+		else if (n <= 4 * RS_SMALL_THREADS)
+			k_rs_small<4><<<1, RS_SMALL_THREADS, 0, st>>>(keys, vals, n, lowBits, bits);
+		else
+			k_rs_small<8><<<1, RS_SMALL_THREADS, 0, st>>>(keys, vals, n, lowBits, bits);
+		return;
+	}
 	const int nb = nblk(n, RS_TILE);
 	uint64_t* ka = keys;
 	uint32_t* va = vals;
 	uint64_t* kb = keys2;
 	uint32_t* vb = vals2;
-	for (int shift = bitBegin; shift < bitEnd; shift += 8)
+	for (int shift = 0; shift < bits; shift += 8)
 	{
-		k_rs_hist<<<nb, RS_THREADS, 0, st>>>(ka, n, shift, hist, nb);
-		launch_scan(hist, int64_t(256) * nb, scanTmp, st);
-		k_rs_scatter<<<nb, RS_THREADS, 0, st>>>(ka, va, kb, vb, n, shift, hist, nb);
+		k_rs_hist<<<nb, RS_THREADS, 0, st>>>(ka, n, lowBits, shift, hist);
+		k_rs_scatter<<<nb, RS_THREADS, 0, st>>>(ka, va, kb, vb, n, lowBits, shift, hist, nb);
 		uint64_t* tk = ka; ka = kb; kb = tk;
 		uint32_t* tv = va; va = vb; vb = tv;
 		resultInAlt = !resultInAlt;

@@ -78,7 +78,7 @@ size_t carve(unsigned char* base, NoAllocBP& c)
 	const size_t N = kMaxBoxes, P = kMaxPairs;
 	const size_t NP = std::max(N, P);
 	const size_t tiles = (NP + size_t(pxh::radix_tile()) - 1) / size_t(pxh::radix_tile());
-	const size_t scanN = std::max({size_t(pxh::PAIR_CLASSES) * N + 1, size_t(256) * 1024, 256 * tiles, P + 1});
+	const size_t scanN = std::max({size_t(pxh::PAIR_CLASSES) * N + 1, size_t(256) * 1024, P + 1});
 	Carver k{base};
 	k.take(c.bmin, N); k.take(c.bmax, N); k.take(c.smin, N); k.take(c.smax, N);
 	k.take(c.gridF, 1); k.take(c.gridI, 1); k.take(c.gridAcc, 5);

@@ -1887,8 +1887,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	{
 		const int nb = (C + pxh::radix_tile() - 1) / pxh::radix_tile();
 		PXH_CHECK(s->hist.ensure(size_t(256) * std::max(nb, 1)));
-		PXH_CHECK(s->scanTmp.ensure(pxh::scan_tmp_size(std::max<int64_t>(int64_t(256) * std::max(nb, 1), C + 1)) +
-		                            1024));
+		PXH_CHECK(s->scanTmp.ensure(pxh::scan_tmp_size(int64_t(C) + 1) + 1024));
 	}
 	int rounds = 0;
 	const int kMaxRounds = 960;
@@ -1940,8 +1939,8 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		pxh::launch_color_keys_world(C, s->conColor.p, s->conA.p, s->scene.p, uint32_t(colorBound), s->keys.p,
 		                             s->vals.p, st);
 		bool alt = false;
-		pxh::launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, C, 32,
-		                       32 + ((bitsFor(slots) + 7) / 8) * 8, s->hist.p, s->scanTmp.p, st, alt);
+		pxh::launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, C, 0, bitsFor(slots - 1), s->hist.p, st,
+		                       alt);
 		const uint64_t* ck = alt ? s->keys2.p : s->keys.p;
 		const uint32_t* cv = alt ? s->vals2.p : s->vals.p;
 		pxh::launch_row_start(C, ck, s->segStart.p, uint32_t(slots), st);
@@ -1983,8 +1982,8 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		PXH_CHECK(s->colorCount.ensure(size_t(colorBound) + 2));
 		pxh::launch_color_keys(C, s->conColor.p, uint32_t(colorBound), s->keys.p, s->vals.p, st);
 		bool alt = false;
-		pxh::launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, C, 32,
-		                       32 + ((bitsFor(uint64_t(colorBound)) + 7) / 8) * 8, s->hist.p, s->scanTmp.p, st, alt);
+		pxh::launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, C, 0, bitsFor(uint64_t(colorBound)),
+		                       s->hist.p, st, alt);
 		const uint64_t* ck = alt ? s->keys2.p : s->keys.p;
 		const uint32_t* cv = alt ? s->vals2.p : s->vals.p;
 		pxh::launch_row_start(C, ck, s->colorCount.p, uint32_t(colorBound), st);
