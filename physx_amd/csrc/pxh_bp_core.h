@@ -50,11 +50,11 @@ inline int readCounts(hipStream_t st, uint32_t* host, const uint32_t* const* src
 
 // the write pass of the sweep (again after the pair buffer has grown)
 template <typename Ctx>
-int bp_write_pairs(Ctx* s, int n, const int* d_scene, const int* d_group, const uint32_t* d_rowOff, hipStream_t st,
-                   size_t pairCap, uint64_t groupLut = GROUP_LUT_ALL)
+int bp_write_pairs(Ctx* s, int classes, int n, const int* d_scene, const int* d_group, const uint32_t* d_rowOff,
+                   hipStream_t st, size_t pairCap, uint64_t groupLut = GROUP_LUT_ALL)
 {
 	PXH_CHECK(s->pairs.ensure(std::max<size_t>(pairCap, 1)));
-	launch_sweep(true, n, s->sortedKeys, s->smin.p, s->smax.p, d_scene, d_group, groupLut, s->gridI.p, d_rowOff,
+	launch_sweep(true, classes, n, s->sortedKeys, s->smin.p, s->smax.p, d_scene, d_group, groupLut, s->gridI.p, d_rowOff,
 	             s->rowStart.p, nullptr, s->counts.p, s->pairs.p, uint32_t(pairCap), st);
 	return PXH_OK;
 }
@@ -63,22 +63,23 @@ int bp_write_pairs(Ctx* s, int n, const int* d_scene, const int* d_group, const 
 // nWorlds worlds whose row table d_rowOff (nWorlds + 1 entries, totalRows in
 // all) is already on the device, produce the class-ordered pair list without a
 // host round trip: the pair count stays on the device at
-// counts[PAIR_CLASSES * n] (class c ends at counts[(c + 1) * n]) and at most
+// counts[classes * n] (class c ends at counts[(c + 1) * n]) and at most
 // pairCap pairs are written.
 template <typename Ctx>
-int broadphase(Ctx* s, int n, int nWorlds, const int* d_scene, const int* d_group, const uint32_t* d_rowOff,
-               uint32_t totalRows, hipStream_t st, size_t pairCap, uint64_t groupLut = GROUP_LUT_ALL)
+int broadphase(Ctx* s, int classes, int n, int nWorlds, int maxWorldBodies, const int* d_scene, const int* d_group,
+               const uint32_t* d_rowOff, uint32_t totalRows, hipStream_t st, size_t pairCap,
+               uint64_t groupLut = GROUP_LUT_ALL)
 {
 	PXH_CHECK(s->gridF.ensure(nWorlds));
 	PXH_CHECK(s->gridI.ensure(nWorlds));
-	PXH_CHECK(s->scanTmp.ensure(scan_tmp_size(std::max<int64_t>(int64_t(PAIR_CLASSES) * n + 1, 256 * 1024)) + 1024));
+	PXH_CHECK(s->scanTmp.ensure(scan_tmp_size(std::max<int64_t>(int64_t(classes) * n + 1, 256 * 1024)) + 1024));
 	PXH_CHECK(s->gridAcc.ensure(size_t(5) * nWorlds));
-	launch_scene_grid(n, nWorlds, d_scene, s->bmin.p, s->bmax.p, s->gridAcc.p, s->gridF.p, s->gridI.p, d_rowOff, st);
 	PXH_CHECK(s->keys.ensure(n));
 	PXH_CHECK(s->keys2.ensure(n));
 	PXH_CHECK(s->vals.ensure(n));
 	PXH_CHECK(s->vals2.ensure(n));
-	launch_keys(n, s->bmin.p, s->bmax.p, d_scene, s->gridF.p, s->gridI.p, d_rowOff, s->keys.p, s->vals.p, st);
+	launch_scene_grid(n, nWorlds, maxWorldBodies, s->bodyStart.p, d_scene, s->bmin.p, s->bmax.p, s->gridAcc.p,
+	                  s->gridF.p, s->gridI.p, d_rowOff, s->keys.p, s->vals.p, st);
 	const int nblocks = (n + radix_tile() - 1) / radix_tile();
 	PXH_CHECK(s->hist.ensure(size_t(256) * std::max(nblocks, 1)));
 	bool alt = false;
@@ -93,13 +94,12 @@ int broadphase(Ctx* s, int n, int nWorlds, const int* d_scene, const int* d_grou
 	launch_gather_sorted(n, sv, s->bmin.p, s->bmax.p, s->smin.p, s->smax.p, st);
 	launch_row_start(n, s->sortedKeys, s->rowStart.p, totalRows, st);
 
-	const int64_t nc = int64_t(PAIR_CLASSES) * n + 1;
+	const int64_t nc = int64_t(classes) * n + 1;
 	PXH_CHECK(s->counts.ensure(nc));
-	PXH_CHECK(hipMemsetAsync(s->counts.p + PAIR_CLASSES * int64_t(n), 0, sizeof(uint32_t), st));
-	launch_sweep(false, n, s->sortedKeys, s->smin.p, s->smax.p, d_scene, d_group, groupLut, s->gridI.p, d_rowOff,
+	launch_sweep(false, classes, n, s->sortedKeys, s->smin.p, s->smax.p, d_scene, d_group, groupLut, s->gridI.p, d_rowOff,
 	             s->rowStart.p, s->counts.p, nullptr, nullptr, 0u, st);
 	launch_scan(s->counts.p, nc, s->scanTmp.p, st);
-	return bp_write_pairs(s, n, d_scene, d_group, d_rowOff, st, pairCap, groupLut);
+	return bp_write_pairs(s, classes, n, d_scene, d_group, d_rowOff, st, pairCap, groupLut);
 }
 
 // Standalone broadphase update (PxBroadPhase::update, PxBroadPhase.h:576) on a
@@ -134,10 +134,10 @@ int bp_update(Ctx* bp, const float* bounds, const uint32_t* groups, const float*
 		launch_row_off_single(bp->rowOff.p, rows, st);
 		if (growPairs)
 			bp->pairCap = std::max(bp->pairCap, size_t(4) * n);
-		int r = broadphase(bp, n, 1, bp->scene.p, bp->group.p, bp->rowOff.p, rows, st, bp->pairCap, groupLut);
+		int r = broadphase(bp, 1, n, 1, n, bp->scene.p, bp->group.p, bp->rowOff.p, rows, st, bp->pairCap, groupLut);
 		if (r)
 			return r;
-		const uint32_t* src[1] = {bp->counts.p + PAIR_CLASSES * int64_t(n)};
+		const uint32_t* src[1] = {bp->counts.p + n};
 		r = readCounts(st, hostCounts, src, 1);
 		if (r)
 			return r;
@@ -153,7 +153,7 @@ int bp_update(Ctx* bp, const float* bounds, const uint32_t* groups, const float*
 				return PXH_ERR_CAPACITY;
 			}
 			bp->pairCap = size_t(P) + size_t(P) / 4;
-			r = bp_write_pairs(bp, n, bp->scene.p, bp->group.p, bp->rowOff.p, st, bp->pairCap, groupLut);
+			r = bp_write_pairs(bp, 1, n, bp->scene.p, bp->group.p, bp->rowOff.p, st, bp->pairCap, groupLut);
 			if (r)
 				return r;
 		}

@@ -135,12 +135,12 @@ void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t
 
 void launch_bounds(int n, const float4* pos, const float4* rot, const float4* geom, const HullSet& hs, float co,
                    float4* bmin, float4* bmax, hipStream_t st);
-// rowOff: per-world row table (nScenes + 1), each world's slice capping its rows
-void launch_scene_grid(int n, int nScenes, const int* scene, const float4* bmin, const float4* bmax, uint32_t* acc,
-                       float4* gridF, int2* gridI, const uint32_t* rowOff, hipStream_t st);
+// each world's row grid and each body's (row, minX) sweep key; rowOff:
+// per-world row table (nScenes + 1), each world's slice capping its rows
+void launch_scene_grid(int n, int nScenes, int maxWorldBodies, const int* bodyStart, const int* scene,
+                       const float4* bmin, const float4* bmax, uint32_t* acc, float4* gridF, int2* gridI,
+                       const uint32_t* rowOff, uint64_t* keys, uint32_t* vals, hipStream_t st);
 void launch_row_off_single(uint32_t* rowOff, uint32_t cap, hipStream_t st);
-void launch_keys(int n, const float4* bmin, const float4* bmax, const int* scene, const float4* gridF,
-                 const int2* gridI, const uint32_t* rowOff, uint64_t* keys, uint32_t* vals, hipStream_t st);
 void launch_gather_sorted(int n, const uint32_t* sv, const float4* bmin, const float4* bmax, float4* smin,
                           float4* smax, hipStream_t st);
 void launch_row_start(int n, const uint64_t* sk, uint32_t* rowStart, uint32_t totalRows, hipStream_t st);
@@ -148,7 +148,9 @@ void launch_row_start(int n, const uint64_t* sk, uint32_t* rowStart, uint32_t to
 // null: no filter) with groupLut, the filter table of BpFilter as a bit mask
 // (bit type0 * 8 + type1, type = group & 7), equal groups never pairing
 constexpr uint64_t GROUP_LUT_ALL = ~0ull;
-void launch_sweep(bool write, int n, const uint64_t* sk, const float4* smin, const float4* smax, const int* scene,
+// classes: pair classes that can occur, 1 (one geometry type), PAIR_CLASS_FIRST_CONVEX
+// (no convex meshes) or PAIR_CLASSES
+void launch_sweep(bool write, int classes, int n, const uint64_t* sk, const float4* smin, const float4* smax, const int* scene,
                   const int* group, uint64_t groupLut, const int2* gridI, const uint32_t* rowOff,
                   const uint32_t* rowStart, uint32_t* counts, const uint32_t* offsets, uint2* pairs, uint32_t pairCap,
                   hipStream_t st);

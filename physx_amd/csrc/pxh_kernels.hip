@@ -20,6 +20,7 @@
 #include "pxh_mesh.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace pxh {
 
@@ -465,64 +466,103 @@ __global__ void k_bounds(int n, const float4* pos, const float4* rot, const floa
 // preserving integer atomics (one per wave when the wave holds one world).
 PXH_D float decode_float(uint32_t u) { return __uint_as_float((u & 0x80000000u) ? (u ^ 0x80000000u) : ~u); }
 
+// Bodies are read side by side, sixteen to a lane; a block of one world reduces
+// in LDS and makes one set of atomics, a wave over several worlds one set for
+// each of them. Bound by the atomics on one world's five words: 262,144 bodies
+// take 12 us in 64 blocks, 19 us in 256.
 constexpr int GRID_ITEMS = 16;
+
+struct GridRange
+{
+	uint32_t v[5];   // lowest / highest centre y, lowest / highest centre z, widest box
+};
+PXH_D void gridMerge(GridRange& a, const GridRange& b)
+{
+	a.v[0] = min(a.v[0], b.v[0]); a.v[1] = max(a.v[1], b.v[1]);
+	a.v[2] = min(a.v[2], b.v[2]); a.v[3] = max(a.v[3], b.v[3]);
+	a.v[4] = max(a.v[4], b.v[4]);
+}
+// every lane gets the wave's range
+PXH_D GridRange gridWave(GridRange a)
+{
+#pragma unroll
+	for (int o = 1; o < 64; o <<= 1)
+	{
+		GridRange b;
+#pragma unroll
+		for (int k = 0; k < 5; k++)
+			b.v[k] = __shfl_xor(a.v[k], o, 64);
+		gridMerge(a, b);
+	}
+	return a;
+}
+PXH_D void gridAtomic(uint32_t* w, const GridRange& a)
+{
+	atomicMin(&w[0], a.v[0]); atomicMax(&w[1], a.v[1]); atomicMin(&w[2], a.v[2]); atomicMax(&w[3], a.v[3]);
+	atomicMax(&w[4], a.v[4]);
+}
+
 __global__ void __launch_bounds__(256) k_grid_reduce(int n, const float4* bmin, const float4* bmax, const int* scene,
                                                       uint32_t* acc)
 {
-	__shared__ uint32_t red[5][256];
+	__shared__ GridRange red[4];
 	const int base = blockIdx.x * 256 * GRID_ITEMS;
-	const int first = base + threadIdx.x * GRID_ITEMS;
 	const int blockLast = min(n, base + 256 * GRID_ITEMS) - 1;
-	// one world in the whole block: reduce in LDS, one atomic set per block
-	const bool blockUniform = scene[base] == scene[blockLast];
-	uint32_t v[5] = {0xFFFFFFFFu, 0u, 0xFFFFFFFFu, 0u, 0u};
-	int cur = -1;
-	for (int i = first; i < min(n, first + GRID_ITEMS); i++)
-	{
-		const int s = scene[i];
-		if (s != cur && cur >= 0 && !blockUniform)
-		{
-			uint32_t* w = acc + 5 * int64_t(cur);
-			atomicMin(&w[0], v[0]); atomicMax(&w[1], v[1]); atomicMin(&w[2], v[2]); atomicMax(&w[3], v[3]);
-			atomicMax(&w[4], v[4]);
-			v[0] = 0xFFFFFFFFu; v[1] = 0u; v[2] = 0xFFFFFFFFu; v[3] = 0u; v[4] = 0u;
-		}
-		cur = s;
+	const int lane = threadIdx.x & 63;
+	const GridRange none = {{0xFFFFFFFFu, 0u, 0xFFFFFFFFu, 0u, 0u}};
+	auto load = [&](int i, GridRange& r) {
 		const float4 a = bmin[i], b = bmax[i];
 		const uint32_t cy = encode_float(0.5f * (a.y + b.y)), cz = encode_float(0.5f * (a.z + b.z));
-		v[0] = min(v[0], cy); v[1] = max(v[1], cy); v[2] = min(v[2], cz); v[3] = max(v[3], cz);
-		v[4] = max(v[4], encode_float(fmaxf(b.y - a.y, b.z - a.z)));
-	}
-	if (!blockUniform)
+		r = {{cy, cy, cz, cz, encode_float(fmaxf(b.y - a.y, b.z - a.z))}};
+	};
+	if (scene[base] == scene[blockLast])
 	{
-		if (cur >= 0)
+		// one world in the whole block (bodies are ordered by world)
+		GridRange t = none;
+#pragma unroll 4
+		for (int k = 0; k < GRID_ITEMS; k++)
 		{
-			uint32_t* w = acc + 5 * int64_t(cur);
-			atomicMin(&w[0], v[0]); atomicMax(&w[1], v[1]); atomicMin(&w[2], v[2]); atomicMax(&w[3], v[3]);
-			atomicMax(&w[4], v[4]);
+			const int i = base + k * 256 + threadIdx.x;
+			if (i < n)
+			{
+				GridRange r;
+				load(i, r);
+				gridMerge(t, r);
+			}
+		}
+		t = gridWave(t);
+		if (lane == 0)
+			red[threadIdx.x >> 6] = t;
+		__syncthreads();
+		if (threadIdx.x == 0)
+		{
+			for (int k = 1; k < 4; k++)
+				gridMerge(t, red[k]);
+			gridAtomic(acc + 5 * int64_t(scene[base]), t);
 		}
 		return;
 	}
-	for (int k = 0; k < 5; k++)
-		red[k][threadIdx.x] = v[k];
-	__syncthreads();
-	for (int o = 128; o > 0; o >>= 1)
+	for (int k = 0; k < GRID_ITEMS; k++)
 	{
-		if (threadIdx.x < o)
+		const int i = base + k * 256 + threadIdx.x;
+		GridRange own = none;
+		int world = -1;
+		if (i < n)
 		{
-			red[0][threadIdx.x] = min(red[0][threadIdx.x], red[0][threadIdx.x + o]);
-			red[1][threadIdx.x] = max(red[1][threadIdx.x], red[1][threadIdx.x + o]);
-			red[2][threadIdx.x] = min(red[2][threadIdx.x], red[2][threadIdx.x + o]);
-			red[3][threadIdx.x] = max(red[3][threadIdx.x], red[3][threadIdx.x + o]);
-			red[4][threadIdx.x] = max(red[4][threadIdx.x], red[4][threadIdx.x + o]);
+			load(i, own);
+			world = scene[i];
 		}
-		__syncthreads();
-	}
-	if (threadIdx.x == 0)
-	{
-		uint32_t* w = acc + 5 * int64_t(scene[base]);
-		atomicMin(&w[0], red[0][0]); atomicMax(&w[1], red[1][0]); atomicMin(&w[2], red[2][0]);
-		atomicMax(&w[3], red[3][0]); atomicMax(&w[4], red[4][0]);
+		uint64_t todo = __ballot(world >= 0);
+		while (todo)
+		{
+			const int lead = __ffsll((unsigned long long)todo) - 1;
+			const int w = __shfl(world, lead);
+			const bool mine = world == w;
+			todo &= ~__ballot(mine);
+			const GridRange r = gridWave(mine ? own : none);
+			if (lane == lead)
+				gridAtomic(acc + 5 * int64_t(w), r);
+		}
 	}
 }
 
@@ -541,19 +581,14 @@ __global__ void k_grid_init(int nScenes, uint32_t* acc)
 // table up front, so no count comes back before the sort): the cell grows
 // until ny * nz fits. Cells only need to be at least as wide as the widest
 // box; wider cells give the same pairs with longer sweeps.
-__global__ void k_grid_finish(int nScenes, const uint32_t* acc, float4* gridF, int2* gridI, const uint32_t* rowOff)
+PXH_D void gridCells(const GridRange& w, int64_t cap, float4& gf, int2& gi)
 {
-	const int s = blockIdx.x * blockDim.x + threadIdx.x;
-	if (s >= nScenes)
-		return;
-	const uint32_t* w = acc + 5 * int64_t(s);
-	const bool empty = w[0] == 0xFFFFFFFFu && w[1] == 0u;
-	const float ly = empty ? 0.0f : decode_float(w[0]), hy = empty ? 0.0f : decode_float(w[1]);
-	const float lz = empty ? 0.0f : decode_float(w[2]), hz = empty ? 0.0f : decode_float(w[3]);
-	const float wm = empty ? 0.0f : decode_float(w[4]);
+	const bool empty = w.v[0] == 0xFFFFFFFFu && w.v[1] == 0u;
+	const float ly = empty ? 0.0f : decode_float(w.v[0]), hy = empty ? 0.0f : decode_float(w.v[1]);
+	const float lz = empty ? 0.0f : decode_float(w.v[2]), hz = empty ? 0.0f : decode_float(w.v[3]);
+	const float wm = empty ? 0.0f : decode_float(w.v[4]);
 	float cell = wm * 1.01f + 1e-6f;
 	cell = fmaxf(cell, fmaxf(hy - ly, hz - lz) * (1.0f / 1000.0f));
-	const int64_t cap = int64_t(rowOff[s + 1] - rowOff[s]);
 	int ny = 1, nz = 1;
 	for (int it = 0; it < 96; it++)
 	{
@@ -569,8 +604,19 @@ __global__ void k_grid_finish(int nScenes, const uint32_t* acc, float4* gridF, i
 		nz = 1;
 		cell = fmaxf(cell, fmaxf(hy - ly, hz - lz) + 1.0f);
 	}
-	gridF[s] = make_float4(ly, lz, 1.0f / cell, cell);
-	gridI[s] = make_int2(ny, nz);
+	gf = make_float4(ly, lz, 1.0f / cell, cell);
+	gi = make_int2(ny, nz);
+}
+
+__global__ void k_grid_finish(int nScenes, const uint32_t* acc, float4* gridF, int2* gridI, const uint32_t* rowOff)
+{
+	const int s = blockIdx.x * blockDim.x + threadIdx.x;
+	if (s >= nScenes)
+		return;
+	GridRange w;
+	for (int k = 0; k < 5; k++)
+		w.v[k] = acc[5 * int64_t(s) + k];
+	gridCells(w, int64_t(rowOff[s + 1] - rowOff[s]), gridF[s], gridI[s]);
 }
 
 // row table of a single world with cap rows
@@ -583,22 +629,73 @@ __global__ void k_row_off_single(uint32_t* rowOff, uint32_t cap)
 	}
 }
 
+PXH_D uint64_t sweepKey(float4 a, float4 b, float4 gf, int2 gi, uint32_t rowOff)
+{
+	const float cy = 0.5f * (a.y + b.y), cz = 0.5f * (a.z + b.z);
+	const int iy = min(max(int(floorf((cy - gf.x) * gf.z)), 0), gi.x - 1);
+	const int iz = min(max(int(floorf((cz - gf.y) * gf.z)), 0), gi.y - 1);
+	const uint32_t row = rowOff + uint32_t(iz * gi.x + iy);
+	return (uint64_t(row) << 32) | encode_float(a.x);
+}
+
 __global__ void k_keys(int n, const float4* bmin, const float4* bmax, const int* scene, const float4* gridF,
                        const int2* gridI, const uint32_t* rowOff, uint64_t* keys, uint32_t* vals)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= n)
 		return;
-	const float4 a = bmin[i], b = bmax[i];
 	const int s = scene[i];
-	const float4 gf = gridF[s];
-	const int2 gi = gridI[s];
-	const float cy = 0.5f * (a.y + b.y), cz = 0.5f * (a.z + b.z);
-	const int iy = min(max(int(floorf((cy - gf.x) * gf.z)), 0), gi.x - 1);
-	const int iz = min(max(int(floorf((cz - gf.y) * gf.z)), 0), gi.y - 1);
-	const uint32_t row = rowOff[s] + uint32_t(iz * gi.x + iy);
-	keys[i] = (uint64_t(row) << 32) | encode_float(a.x);
+	keys[i] = sweepKey(bmin[i], bmax[i], gridF[s], gridI[s], rowOff[s]);
 	vals[i] = uint32_t(i);
+}
+
+// Grid and sweep keys of worlds that one workgroup each can take (the launch
+// has a workgroup a world): the range, the cells and the keys in one launch
+// without atomics, for k_grid_init, k_grid_reduce, k_grid_finish and k_keys.
+__global__ void __launch_bounds__(1024) k_world_grid(const int* bodyStart, const float4* bmin, const float4* bmax,
+                                                     float4* gridF, int2* gridI, const uint32_t* rowOff,
+                                                     uint64_t* keys, uint32_t* vals)
+{
+	__shared__ GridRange red[16];
+	__shared__ float4 sF;
+	__shared__ int2 sI;
+	const int w = blockIdx.x;
+	const int b0 = bodyStart[w], b1 = bodyStart[w + 1];
+	GridRange t = {{0xFFFFFFFFu, 0u, 0xFFFFFFFFu, 0u, 0u}};
+#pragma unroll 4
+	for (int i = b0 + int(threadIdx.x); i < b1; i += int(blockDim.x))
+	{
+		const float4 a = bmin[i], b = bmax[i];
+		const uint32_t cy = encode_float(0.5f * (a.y + b.y)), cz = encode_float(0.5f * (a.z + b.z));
+		const GridRange r = {{cy, cy, cz, cz, encode_float(fmaxf(b.y - a.y, b.z - a.z))}};
+		gridMerge(t, r);
+	}
+	t = gridWave(t);
+	if ((threadIdx.x & 63) == 0)
+		red[threadIdx.x >> 6] = t;
+	__syncthreads();
+	const uint32_t ro = rowOff[w];
+	if (threadIdx.x == 0)
+	{
+		for (int k = 1; k < int(blockDim.x >> 6); k++)
+			gridMerge(t, red[k]);
+		float4 gf;
+		int2 gi;
+		gridCells(t, int64_t(rowOff[w + 1] - ro), gf, gi);
+		sF = gf;
+		sI = gi;
+		gridF[w] = gf;
+		gridI[w] = gi;
+	}
+	__syncthreads();
+	const float4 gf = sF;
+	const int2 gi = sI;
+#pragma unroll 4
+	for (int i = b0 + int(threadIdx.x); i < b1; i += int(blockDim.x))
+	{
+		keys[i] = sweepKey(bmin[i], bmax[i], gf, gi, ro);
+		vals[i] = uint32_t(i);
+	}
 }
 
 __global__ void k_gather_sorted(int n, const uint32_t* sortedVals, const float4* bmin, const float4* bmax,
@@ -616,27 +713,37 @@ __global__ void k_gather_sorted(int n, const uint32_t* sortedVals, const float4*
 
 // rowStart[r] = first sorted position of row r; rowStart[totalRows] = n.
 // Keys past totalRows count as totalRows (rowStart has totalRows + 2 entries).
-// Lane s fills the rows from the previous key's row (exclusive) to its own;
-// the rows after the last key are filled by k_row_tail, one lane per row.
-__global__ void k_row_start(int n, const uint64_t* sortedKeys, uint32_t* rowStart, uint32_t totalRows)
+// Lane s fills the rows from the previous key's row (exclusive) to its own, a
+// long run of empty rows with its whole wave (one lane alone took 38 us where
+// worlds leave hundreds of rows empty); the rows after the last key have a lane
+// each.
+__global__ void __launch_bounds__(256) k_row_start(int n, const uint64_t* sortedKeys, uint32_t* rowStart,
+                                                   uint32_t totalRows)
 {
-	const int s = blockIdx.x * blockDim.x + threadIdx.x;
-	if (s >= n)
-		return;
-	const uint32_t r = min(uint32_t(sortedKeys[s] >> 32), totalRows);
-	const int64_t rp = s == 0 ? -1 : int64_t(min(uint32_t(sortedKeys[s - 1] >> 32), totalRows));
-	for (int64_t rr = rp + 1; rr <= int64_t(r); rr++)
-		rowStart[rr] = uint32_t(s);
-}
-
-__global__ void k_row_tail(int n, const uint64_t* sortedKeys, uint32_t* rowStart, uint32_t totalRows)
-{
-	const int64_t rr = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (rr > int64_t(totalRows) || n <= 0)
-		return;
-	const uint32_t last = min(uint32_t(sortedKeys[n - 1] >> 32), totalRows);
-	if (rr > int64_t(last))
-		rowStart[rr] = uint32_t(n);
+	const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	const int64_t last = int64_t(min(uint32_t(sortedKeys[n - 1] >> 32), totalRows));
+	if (t > last && t <= int64_t(totalRows))
+		rowStart[t] = uint32_t(n);
+	int64_t r = 0, from = 1;   // rows [from, r] start at t
+	if (t < n)
+	{
+		r = int64_t(min(uint32_t(sortedKeys[t] >> 32), totalRows));
+		from = t == 0 ? 0 : int64_t(min(uint32_t(sortedKeys[t - 1] >> 32), totalRows)) + 1;
+	}
+	const int lane = threadIdx.x & 63;
+	const bool longRun = r - from >= 4;
+	uint64_t todo = __ballot(longRun);
+	while (todo)
+	{
+		const int lead = __ffsll((unsigned long long)todo) - 1;
+		todo &= todo - 1;
+		const int64_t f = __shfl(from, lead), e = __shfl(r, lead), v = __shfl(t, lead);
+		for (int64_t k = f + lane; k <= e; k += 64)
+			rowStart[k] = uint32_t(v);
+	}
+	if (!longRun)
+		for (int64_t k = from; k <= r; k++)
+			rowStart[k] = uint32_t(t);
 }
 
 __global__ void k_fill_u32(uint32_t* p, int64_t n, uint32_t v)
@@ -662,6 +769,7 @@ PXH_D int pairClass(int t0, int t1)
 // inclusive test on inflated bounds (BpBroadPhaseABP.cpp:2246-2262, :2474).
 // WRITE=false counts pairs per class into counts[cls*n + s]; WRITE=true writes
 // them at the scanned offsets.
+//
 // Broadphase group filter (Bp::groupFiltering, lowlevelaabb/include/BpFiltering.h:99-109):
 // boxes of equal groups never pair; otherwise bit (type0 * 8 + type1) of lut,
 // type = group & 7 (BpFilter's 7 x 7 table, lowlevelaabb/src/BpFiltering.cpp,
@@ -671,17 +779,28 @@ PXH_D bool groupsPair(int g0, int g1, uint64_t lut)
 	return g0 != g1 && ((lut >> ((g0 & 7) * 8 + (g1 & 7))) & 1ull);
 }
 
-template <bool WRITE>
-__global__ void k_sweep(int n, const uint64_t* sortedKeys, const float4* smin, const float4* smax, const int* scene,
-                        const int* group, uint64_t groupLut, const int2* gridI, const uint32_t* rowOff,
-                        const uint32_t* rowStart, uint32_t* counts, const uint32_t* offsets, uint2* pairs,
-                        uint32_t pairCap)
+// G lanes share a body, each taking 9 / G of the nine rows in order, so a body's
+// pairs keep their places: one lane for all nine rows is a chain of nine binary
+// searches and scans. launch_sweep has the rule and its figures. With G > 1 the
+// write pass first counts its lanes' pairs again to place them.
+// CLASSES: pair classes that can occur (1: the standalone broadphase's boxes, 3:
+// no convex hulls, 6).
+constexpr int SWEEP_THREADS = 256;
+template <bool WRITE, int G, int CLASSES>
+__global__ void __launch_bounds__(SWEEP_THREADS) k_sweep(int n, const uint64_t* sortedKeys, const float4* smin,
+                                                         const float4* smax, const int* scene, const int* group,
+                                                         uint64_t groupLut, const int2* gridI, const uint32_t* rowOff,
+                                                         const uint32_t* rowStart, uint32_t* counts,
+                                                         const uint32_t* offsets, uint2* pairs, uint32_t pairCap)
 {
-	const int s = blockIdx.x * blockDim.x + threadIdx.x;
-	if (s >= n)
-		return;
-	const uint64_t key = sortedKeys[s];
-	const float4 a0 = smin[s], a1 = smax[s];
+	constexpr int PER = 63 / G, ROWS = 9 / G;   // bodies of a wave (its last lane idles), rows of a lane
+	const int lane = threadIdx.x & 63;
+	const int slot = lane / G, sub = lane - slot * G;
+	const int s = (blockIdx.x * (SWEEP_THREADS / 64) + (threadIdx.x >> 6)) * PER + slot;
+	const bool live = slot < PER && s < n;
+	const int at = live ? s : n - 1;
+	const uint64_t key = sortedKeys[at];
+	const float4 a0 = smin[at], a1 = smax[at];
 	const uint32_t i = __float_as_uint(a1.w);
 	const int ti = int(a0.w);
 	const int sc = scene[i];
@@ -691,44 +810,45 @@ __global__ void k_sweep(int n, const uint64_t* sortedKeys, const float4* smin, c
 	const uint32_t ro = rowOff[sc];
 	const int lr = int(r - ro);
 	const int cy = lr % gi.x, cz = lr / gi.x;
-	uint32_t cnt[PAIR_CLASSES];
-	uint32_t off[PAIR_CLASSES];
-	for (int c = 0; c < PAIR_CLASSES; c++)
+	uint32_t lo[ROWS], hi[ROWS];
+#pragma unroll
+	for (int q = 0; q < ROWS; q++)
 	{
-		cnt[c] = 0u;
-		off[c] = WRITE ? offsets[int64_t(c) * n + s] : 0u;
-	}
-	for (int dz = -1; dz <= 1; dz++)
-	{
-		const int z = cz + dz;
-		if (z < 0 || z >= gi.y)
+		const int row = sub * ROWS + q;
+		const int z = cz + row / 3 - 1, y = cy + row % 3 - 1;
+		lo[q] = hi[q] = 0u;
+		if (!live || z < 0 || z >= gi.y || y < 0 || y >= gi.x)
 			continue;
-		for (int dy = -1; dy <= 1; dy++)
+		const uint32_t rr = ro + uint32_t(z * gi.x + y);
+		uint32_t l = rowStart[rr];
+		hi[q] = rowStart[rr + 1];
+		if (rr == r)
+			l = uint32_t(s) + 1u;
+		else
 		{
-			const int y = cy + dy;
-			if (y < 0 || y >= gi.x)
-				continue;
-			const uint32_t rr = ro + uint32_t(z * gi.x + y);
-			uint32_t lo = rowStart[rr];
-			const uint32_t hi = rowStart[rr + 1];
-			if (rr == r)
-				lo = uint32_t(s) + 1u;
-			else
+			// first position whose (minX key, body index) follows ours
+			uint32_t h = hi[q];
+			while (l < h)
 			{
-				// first position whose (minX key, body index) follows ours
-				uint32_t l = lo, h = hi;
-				while (l < h)
-				{
-					const uint32_t m = (l + h) >> 1;
-					const uint64_t km = sortedKeys[m];
-					const bool after = (uint32_t(km) > uint32_t(key)) ||
-					                   (uint32_t(km) == uint32_t(key) && __float_as_uint(smax[m].w) > i);
-					if (after) h = m;
-					else l = m + 1;
-				}
-				lo = l;
+				const uint32_t m = (l + h) >> 1;
+				const uint64_t km = sortedKeys[m];
+				const bool after = (uint32_t(km) > uint32_t(key)) ||
+				                   (uint32_t(km) == uint32_t(key) && __float_as_uint(smax[m].w) > i);
+				if (after) h = m;
+				else l = m + 1;
 			}
-			for (uint32_t j = lo; j < hi; j++)
+		}
+		lo[q] = l;
+	}
+	uint32_t cnt[CLASSES];
+#pragma unroll
+	for (int c = 0; c < CLASSES; c++)
+		cnt[c] = 0u;
+	// the candidates of this lane's rows: found(class, body index, its type)
+	auto visit = [&](auto found) {
+#pragma unroll
+		for (int q = 0; q < ROWS; q++)
+			for (uint32_t j = lo[q]; j < hi[q]; j++)
 			{
 				const float4 b0 = smin[j];
 				if (b0.x > a1.x)
@@ -740,29 +860,64 @@ __global__ void k_sweep(int n, const uint64_t* sortedKeys, const float4* smin, c
 				if (group && !groupsPair(gi_, group[jj], groupLut))
 					continue;
 				const int tj = int(b0.w);
-				const int c = pairClass(ti, tj);
-				if (WRITE)
-				{
-					// shape order of the reference's contact managers: the lower
-					// geometry type first (contact-method table order); two
-					// shapes of one type put the later-added body first
-					// (shouldSwapBodies, simulationcontroller/src/ScNPhaseCore.cpp:182-249)
-					uint32_t pa, pb;
-					if (ti != tj) { pa = ti < tj ? i : jj; pb = ti < tj ? jj : i; }
-					else { pa = max(i, jj); pb = min(i, jj); }
-					// pairs past the buffer's capacity are counted, not written
-					if (off[c] < pairCap)
-						pairs[off[c]] = make_uint2(pa, pb);
-					off[c]++;
-				}
-				else
-					cnt[c]++;
+				found(CLASSES == 1 ? 0 : pairClass(ti, tj), jj, tj);
 			}
-		}
-	}
+	};
+	visit([&](int cls, uint32_t, int) {
+#pragma unroll
+		for (int c = 0; c < CLASSES; c++)
+			cnt[c] += cls == c ? 1u : 0u;
+	});
 	if (!WRITE)
-		for (int c = 0; c < PAIR_CLASSES; c++)
-			counts[int64_t(c) * n + s] = cnt[c];
+	{
+		// the scan's last entry (its total) starts as zero
+		if (live && sub == 0 && s == 0)
+			counts[int64_t(CLASSES) * n] = 0u;
+#pragma unroll
+		for (int c = 0; c < CLASSES; c++)
+		{
+			uint32_t sum = 0;
+#pragma unroll
+			for (int k = 0; k < G; k++)
+				sum += __shfl(cnt[c], min(slot * G + k, 63));
+			if (live && sub == 0)
+				counts[int64_t(c) * n + s] = sum;
+		}
+		return;
+	}
+	// the lane's first place in each class: the body's, and its earlier rows' pairs
+	uint32_t off[CLASSES];
+#pragma unroll
+	for (int c = 0; c < CLASSES; c++)
+	{
+		uint32_t inc = cnt[c];
+#pragma unroll
+		for (int d = 1; d < G; d <<= 1)
+		{
+			const uint32_t t = __shfl_up(inc, d);
+			if (sub >= d)
+				inc += t;
+		}
+		off[c] = (live ? offsets[int64_t(c) * n + s] : 0u) + inc - cnt[c];
+	}
+	visit([&](int cls, uint32_t jj, int tj) {
+		// shape order of the reference's contact managers: the lower
+		// geometry type first (contact-method table order); two
+		// shapes of one type put the later-added body first
+		// (shouldSwapBodies, simulationcontroller/src/ScNPhaseCore.cpp:182-249)
+		uint32_t pa, pb;
+		if (ti != tj) { pa = ti < tj ? i : jj; pb = ti < tj ? jj : i; }
+		else { pa = max(i, jj); pb = min(i, jj); }
+		// pairs past the buffer's capacity are counted, not written
+#pragma unroll
+		for (int c = 0; c < CLASSES; c++)
+			if (cls == c)
+			{
+				if (off[c] < pairCap)
+					pairs[off[c]] = make_uint2(pa, pb);
+				off[c]++;
+			}
+	});
 }
 
 // ---------------------------------------------------------------------------
@@ -3225,22 +3380,32 @@ void launch_bounds(int n, const float4* pos, const float4* rot, const float4* ge
 {
 	PXH_LAUNCH(k_bounds, n, n, pos, rot, geom, hs, co, bmin, bmax);
 }
-void launch_scene_grid(int n, int nScenes, const int* scene, const float4* bmin, const float4* bmax, uint32_t* acc,
-                       float4* gridF, int2* gridI, const uint32_t* rowOff, hipStream_t st)
+// Worlds of up to 8,192 bodies take a workgroup each (4,096 bodies in one world:
+// 7 us against 11 in four launches); a larger world takes the launches over
+// all bodies, whose blocks spread over the chip.
+constexpr int WORLD_GRID_MAX = 8192;
+void launch_scene_grid(int n, int nScenes, int maxWorldBodies, const int* bodyStart, const int* scene,
+                       const float4* bmin, const float4* bmax, uint32_t* acc, float4* gridF, int2* gridI,
+                       const uint32_t* rowOff, uint64_t* keys, uint32_t* vals, hipStream_t st)
 {
+	if (maxWorldBodies <= WORLD_GRID_MAX)
+	{
+		int threads = 64;
+		while (threads < 1024 && 2 * threads < maxWorldBodies)
+			threads *= 2;
+		if (nScenes > 0)
+			k_world_grid<<<nScenes, threads, 0, st>>>(bodyStart, bmin, bmax, gridF, gridI, rowOff, keys, vals);
+		return;
+	}
 	PXH_LAUNCH(k_grid_init, nScenes, nScenes, acc);
 	if (n > 0)
 		k_grid_reduce<<<nblk(n, 256 * GRID_ITEMS), 256, 0, st>>>(n, bmin, bmax, scene, acc);
 	PXH_LAUNCH(k_grid_finish, nScenes, nScenes, acc, gridF, gridI, rowOff);
+	PXH_LAUNCH(k_keys, n, n, bmin, bmax, scene, gridF, gridI, rowOff, keys, vals);
 }
 void launch_row_off_single(uint32_t* rowOff, uint32_t cap, hipStream_t st)
 {
 	k_row_off_single<<<1, 64, 0, st>>>(rowOff, cap);
-}
-void launch_keys(int n, const float4* bmin, const float4* bmax, const int* scene, const float4* gridF,
-                 const int2* gridI, const uint32_t* rowOff, uint64_t* keys, uint32_t* vals, hipStream_t st)
-{
-	PXH_LAUNCH(k_keys, n, n, bmin, bmax, scene, gridF, gridI, rowOff, keys, vals);
 }
 void launch_gather_sorted(int n, const uint32_t* sv, const float4* bmin, const float4* bmax, float4* smin,
                           float4* smax, hipStream_t st)
@@ -3249,25 +3414,53 @@ void launch_gather_sorted(int n, const uint32_t* sv, const float4* bmin, const f
 }
 void launch_row_start(int n, const uint64_t* sk, uint32_t* rowStart, uint32_t totalRows, hipStream_t st)
 {
+	const int64_t rows = int64_t(totalRows) + 1;
 	if (n == 0)
-	{
-		PXH_LAUNCH(k_fill_u32, int64_t(totalRows) + 1, rowStart, int64_t(totalRows) + 1, 0u);
-		return;
-	}
-	PXH_LAUNCH(k_row_start, n, n, sk, rowStart, totalRows);
-	PXH_LAUNCH(k_row_tail, int64_t(totalRows) + 1, n, sk, rowStart, totalRows);
+		PXH_LAUNCH(k_fill_u32, rows, rowStart, rows, 0u);
+	else
+		PXH_LAUNCH(k_row_start, std::max<int64_t>(n, rows), n, sk, rowStart, totalRows);
 }
-void launch_sweep(bool write, int n, const uint64_t* sk, const float4* smin, const float4* smax, const int* scene,
-                  const int* group, uint64_t groupLut, const int2* gridI, const uint32_t* rowOff,
+template <int G, int CLASSES>
+static void sweepPass(bool write, int n, const uint64_t* sk, const float4* smin, const float4* smax, const int* scene,
+                      const int* group, uint64_t groupLut, const int2* gridI, const uint32_t* rowOff,
+                      const uint32_t* rowStart, uint32_t* counts, const uint32_t* offsets, uint2* pairs,
+                      uint32_t pairCap, hipStream_t st)
+{
+	const int blocks = nblk(n, (SWEEP_THREADS / 64) * (63 / G));
+	if (write)
+		k_sweep<true, G, CLASSES><<<blocks, SWEEP_THREADS, 0, st>>>(n, sk, smin, smax, scene, group, groupLut, gridI,
+		                                                          rowOff, rowStart, counts, offsets, pairs, pairCap);
+	else
+		k_sweep<false, G, CLASSES><<<blocks, SWEEP_THREADS, 0, st>>>(n, sk, smin, smax, scene, group, groupLut, gridI,
+		                                                           rowOff, rowStart, counts, offsets, pairs, pairCap);
+}
+void launch_sweep(bool write, int classes, int n, const uint64_t* sk, const float4* smin, const float4* smax,
+                  const int* scene, const int* group, uint64_t groupLut, const int2* gridI, const uint32_t* rowOff,
                   const uint32_t* rowStart, uint32_t* counts, const uint32_t* offsets, uint2* pairs, uint32_t pairCap,
                   hipStream_t st)
 {
-	if (write)
-		PXH_LAUNCH(k_sweep<true>, n, n, sk, smin, smax, scene, group, groupLut, gridI, rowOff, rowStart, counts,
-		           offsets, pairs, pairCap);
+	if (n <= 0)
+		return;
+	auto pass = [&](auto lanes) {
+		constexpr int G = decltype(lanes)::value;
+		if (classes == 1)
+			sweepPass<G, 1>(write, n, sk, smin, smax, scene, group, groupLut, gridI, rowOff, rowStart, counts, offsets,
+			                pairs, pairCap, st);
+		else if (classes == PAIR_CLASS_FIRST_CONVEX)
+			sweepPass<G, PAIR_CLASS_FIRST_CONVEX>(write, n, sk, smin, smax, scene, group, groupLut, gridI, rowOff,
+			                                      rowStart, counts, offsets, pairs, pairCap, st);
+		else
+			sweepPass<G, PAIR_CLASSES>(write, n, sk, smin, smax, scene, group, groupLut, gridI, rowOff, rowStart, counts,
+			                           offsets, pairs, pairCap, st);
+	};
+	// nine lanes a body while the chip has room for them; beyond, the loads of
+	// the write pass's second look at each row cost more than the shorter chains
+	// save (both passes, nine lanes against one: 4,096 boxes 22 / 83 us, 20,011
+	// bodies 44 / 150, 100,003 boxes 80 / 126, 262,144 bodies 339 / 269)
+	if (n <= 131072)
+		pass(std::integral_constant<int, 9>());
 	else
-		PXH_LAUNCH(k_sweep<false>, n, n, sk, smin, smax, scene, group, groupLut, gridI, rowOff, rowStart, counts,
-		           offsets, pairs, pairCap);
+		pass(std::integral_constant<int, 1>());
 }
 void launch_np_pairs(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotBase, const uint2* pairs,
                      const float4* pos, const float4* rot, const float4* geom, float cd, float tol, float4* ctN,

@@ -1672,10 +1672,12 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		s->aggDirty = false;
 	}
 	const int* bpGroup = s->hAggSelf.empty() ? nullptr : s->bpGroup.p;
-	int r = broadphase(s, n, nWorlds, s->scene.p, bpGroup, s->rowOff.p, s->totalRows, st, s->pairCap);
+	const int classes = s->nConvexBodies > 0 ? pxh::PAIR_CLASSES : pxh::PAIR_CLASS_FIRST_CONVEX;
+	int r = broadphase(s, classes, n, nWorlds, s->maxWorldBodies, s->scene.p, bpGroup, s->rowOff.p, s->totalRows, st,
+	                   s->pairCap);
 	if (r)
 		return r;
-	const uint32_t* dP = s->counts.p + pxh::PAIR_CLASSES * int64_t(n);
+	const uint32_t* dP = s->counts.p + classes * int64_t(n);
 	const int Q = s->Q;
 	s->statPlanePairs = Q;
 
@@ -1714,7 +1716,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		const int S = pairEnd + nMB * pxh::MESH_MAXP;   // slots: planes, body pairs, mesh patches
 		if (attempt > 0)
 		{
-			r = bp_write_pairs(s, n, s->scene.p, bpGroup, s->rowOff.p, st, s->pairCap);
+			r = bp_write_pairs(s, classes, n, s->scene.p, bpGroup, s->rowOff.p, st, s->pairCap);
 			if (r)
 				return r;
 		}
