@@ -69,9 +69,8 @@ struct Rows
 // by pair key through an open-addressing table (keys ~0 = empty).
 struct PatchIO
 {
-	const uint64_t* htKey;     // previous step's table (null: no previous step)
-	const int* htVal;          // row of the previous step holding the key
-	uint32_t htMask;           // table size - 1 (power of two)
+	const ulonglong2* table;   // previous step's table, (pair key, row) (null: no previous step)
+	uint32_t tableMask;        // table size - 1 (power of two)
 	const float4* prev;        // previous step's patches
 	const uint32_t* prevBroken;
 	const int* prevColor;      // previous step's colour of each row
@@ -124,6 +123,22 @@ struct SleepState
 	float threshold;     // PxRigidDynamic::setSleepThreshold
 };
 
+// what the colouring keeps of each body in a step, and the step's device words:
+// constraints without a carried colour, those left after the rounds (two words,
+// used in turn), rounds made, largest colour
+struct ColorState
+{
+	unsigned long long* mask;  // colours below 64 in use at the body
+	uint32_t* need;            // the body's mask is read: it has an open or a body-plane constraint
+	uint32_t* next;            // first colour past those of 64 and more
+	uint32_t* words;           // STEP_WORDS
+};
+enum { STEP_OPEN = 0, STEP_LEFT = 1, STEP_RAN = 2, STEP_TOP = 3, STEP_LEFT2 = 4, STEP_WORDS = 8 };
+// longest list whose rounds run in one workgroup; the lists of a 262,144-body bin
+// and of 8,192 worlds, some thousands, took 117 and 247 us in one and 60 and 67
+// in launches over the whole chip
+constexpr int COLOR_SHORT_LIST = 2048;
+
 int64_t scan_tmp_size(int64_t n);
 void launch_scan(uint32_t* data, int64_t n, uint32_t* tmp, hipStream_t st);
 // keys per radix-sort workgroup (its histogram holds 256 counts per workgroup)
@@ -132,9 +147,11 @@ int radix_tile();
 // lowBits bits of its low word (0: the low word is not compared)
 void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t* vals2, int n, int lowBits,
                        int highBits, uint32_t* hist, hipStream_t st, bool& resultInAlt);
+// whether a sort of n keys of `bits` bits leaves its result in keys2 / vals2
+bool radix_result_in_alt(int n, int bits);
 
 void launch_bounds(int n, const float4* pos, const float4* rot, const float4* geom, const HullSet& hs, float co,
-                   float4* bmin, float4* bmax, hipStream_t st);
+                   float4* bmin, float4* bmax, ColorState cs, hipStream_t st);
 // each world's row grid and each body's (row, minX) sweep key; rowOff:
 // per-world row table (nScenes + 1), each world's slice capping its rows
 void launch_scene_grid(int n, int nScenes, int maxWorldBodies, const int* bodyStart, const int* scene,
@@ -143,7 +160,9 @@ void launch_scene_grid(int n, int nScenes, int maxWorldBodies, const int* bodySt
 void launch_row_off_single(uint32_t* rowOff, uint32_t cap, hipStream_t st);
 void launch_gather_sorted(int n, const uint32_t* sv, const float4* bmin, const float4* bmax, float4* smin,
                           float4* smax, hipStream_t st);
-void launch_row_start(int n, const uint64_t* sk, uint32_t* rowStart, uint32_t totalRows, hipStream_t st);
+// words (may be null): STEP_WORDS device words copied to hostWords (host memory)
+void launch_row_start(int n, const uint64_t* sk, uint32_t* rowStart, uint32_t totalRows, hipStream_t st,
+                      const uint32_t* words = nullptr, uint32_t* hostWords = nullptr);
 // write pass: pairs beyond pairCap are counted but not written; group (may be
 // null: no filter) with groupLut, the filter table of BpFilter as a bit mask
 // (bit type0 * 8 + type1, type = group & 7), equal groups never pairing
@@ -175,36 +194,37 @@ void launch_np_planes_convex(int Q, int slotBase, const int* qBody, const int* q
 void launch_copy_contacts(int C, int maxPairs, const int* order, const int* conA, const int* conB, const int* conSlot,
                           const float4* ctN, const float4* ctP, const float* nF, float4* out, uint32_t* nbPairs,
                           hipStream_t st);
-// slots [0, Q) are body-plane pairs, body pairs follow up to the device count *dP
-void launch_touch_flags(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, uint32_t* flags,
-                        hipStream_t st);
-// constraint list; conPKey: world-relative pair identity (world tag 16 | local a
-// 24 | local b or 0x800000 | plane 24)
-void launch_con_build(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, const uint32_t* scanned,
-                      const uint2* pairs, const int* qBody, const int* qPlane, const int* meshBody, int nPlanes,
-                      const int* local, const int* planeLocal, const int* world, const int* worldTag, int* conA,
-                      int* conB, int* conSlot, uint64_t* conKey, uint64_t* conPKey, int* conColor, hipStream_t st);
+// constraint list of the touching slots: slots [0, Q) are body-plane pairs, body
+// pairs follow up to the device count *dP; conPKey: world-relative pair identity
+// (world tag 16 | local a 24 | local b or 0x800000 | plane 24). flags: S entries,
+// tileSums: one per con_tile() slots; hostCounts (host memory) receives *dP, the constraint
+// count and *overflow (0 when null)
+int con_tile();
+void launch_con_build(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, uint32_t* flags,
+                      uint32_t* tileSums, const uint2* pairs, const int* qBody, const int* qPlane, const int* meshBody,
+                      int nPlanes, const int* local, const int* planeLocal, const int* world, const int* worldTag,
+                      const uint32_t* overflow, int* conA, int* conB, int* conSlot, uint64_t* conKey,
+                      uint64_t* conPKey, int* conColor, uint32_t* hostCounts, hipStream_t st);
 // out[i] = in[idx[i]], elements of 4 or 16 bytes
 void launch_gather(int n, const int* idx, const void* in, void* out, int bytes, hipStream_t st);
-// colouring over list[i] (identity when null) for i below *mDev (or m when
-// mDev is null); m bounds the count
-void launch_color_round(int m, const uint32_t* mDev, const int* list, int round, const int* conA, const int* conB,
-                        const uint64_t* conKey, int* conColor, uint64_t* best, uint64_t* mask, hipStream_t st);
-void launch_color_uncolored(int m, const uint32_t* mDev, const int* list, const int* conColor, uint32_t* flags,
-                            hipStream_t st);
-void launch_color_compact(int m, const int* list, const uint32_t* flags, const uint32_t* scanned, int* out,
-                          hipStream_t st);
-void launch_fill_u64(uint64_t* p, int n, uint64_t v, hipStream_t st);
+// colouring rounds over list[i] for i below *mDev (m bounds it): the constraints
+// left go to out, their count to *left, the rounds made to *ran. oneBlock: one
+// launch, for lists of at most COLOR_SHORT_LIST (a longer one is left as it is
+// with *ran = 0); best: 2 n entries
+void launch_color_rounds(int m, const uint32_t* mDev, const int* list, int firstRound, int rounds, int n,
+                         const int* conA, const int* conB, const uint64_t* conKey, int* conColor, uint64_t* best,
+                         ColorState cs, int* out, uint32_t* left, uint32_t* ran, bool oneBlock, hipStream_t st);
 void launch_fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t st);
-void launch_color_keys(int C, const int* conColor, uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st);
-void launch_static_colors(int n, int C, const int* conA, const int* conB, int* conColor, uint32_t* bodyNext,
-                          hipStream_t st);
-void launch_patch_table(int m, const uint64_t* keys, uint64_t* htKey, int* htVal, uint32_t htMask, hipStream_t st);
+// body-plane colours, then the (colour, index) sort keys
+void launch_color_keys(int C, const int* conA, const int* conB, int* conColor, ColorState cs, uint32_t limit,
+                       uint64_t* keys, uint32_t* vals, hipStream_t st);
+void launch_patch_table(int m, const uint64_t* keys, ulonglong2* table, uint32_t mask, hipStream_t st);
 // finds each constraint's row of the previous step; body-body constraints keep
-// their previous colour (marked in the per-body colour masks)
+// their previous colour, the others go to list (count in cs.words[STEP_OPEN])
 void launch_con_prev(int C, const int* conA, const int* conB, const int* conSlot, PatchIO io, int* conColor,
-                     uint64_t* mask, hipStream_t st);
-void launch_max_color(int C, const int* conColor, uint32_t* maxColor, hipStream_t st);
+                     ColorState cs, int* list, hipStream_t st);
+// colour masks, from the carried colours, of the bodies marked in cs.need
+void launch_color_mask(int C, const int* conA, const int* conB, const int* conColor, ColorState cs, hipStream_t st);
 // extLin / extAng (may be null: none set): accelerations set through the
 // Direct GPU API, applied for this step and cleared; prevLin / prevAng (may be
 // null) receive the velocities before the step
@@ -212,18 +232,20 @@ void launch_preintegrate(int n, const float4* pos, const float4* rot, const floa
                          const float4* invI, float3 gdt, float linDampDt, float angDampDt, float maxLinSq,
                          float maxAngSq, bool pgs, SolverBodies sb, float dt, float4* extLin, float4* extAng,
                          float4* prevLin, float4* prevAng, const uint32_t* sleepFlags, hipStream_t st);
+// counters: 4 per 256 constraints (partial sums); hostCounters (host memory): contact points, friction
+// rows, body-body constraints and their friction rows
 void launch_prep(int C, const int* order, const int* conA, const int* conB, const int* conSlot, const float4* ctN,
                  const float4* ctP, const float4* pos, const float4* rot, SolverBodies sb, float invStepDt,
                  float scale, float restDist, float fot, Rows rows, PatchIO patches, unsigned long long* counters,
-                 hipStream_t st);
+                 unsigned long long* hostCounters, hipStream_t st);
 // broken: when not null, each row's friction-clamp flag of this pass is stored there
 // evStart/evStop (optional): recorded by the dispatch itself at the kernel's start and end
 void launch_solve(int begin, int end, int C, Rows rows, SolverBodies sb, float minPen, float muS, float muD,
                   float invStepDt, float biasScale, float scale, uint32_t* broken, hipStream_t st,
                   hipEvent_t evStart = nullptr, hipEvent_t evStop = nullptr);
 // rows in (world, colour) order for the per-world solve
-void launch_color_keys_world(int C, const int* conColor, const int* conA, const int* bodyWorld, uint32_t limit,
-                             uint64_t* keys, uint32_t* vals, hipStream_t st);
+void launch_color_keys_world(int C, const int* conA, const int* conB, int* conColor, ColorState cs,
+                             const int* bodyWorld, uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st);
 int solve_world_threads();
 // every TGS iteration of every world in one launch of `grid` persistent
 // workgroups; queueHead: one device counter (zeroed by the launch);
@@ -240,7 +262,7 @@ void launch_solve_worlds(int grid, int nWorlds, const int* worldOrder, uint32_t*
 void launch_prep_pgs(int C, const int* order, const int* conA, const int* conB, const int* conSlot,
                      const float4* ctN, const float4* ctP, const float4* pos, const float4* rot, SolverBodies sb,
                      float invDt, float muS, float muD, float restDist, float fot, Rows rows, float* rowsU,
-                     PatchIO patches, unsigned long long* counters, hipStream_t st);
+                     PatchIO patches, unsigned long long* counters, unsigned long long* hostCounters, hipStream_t st);
 void launch_solve_pgs(int begin, int end, int C, Rows rows, const float* rowsU, SolverBodies sb, bool doFriction,
                       bool velocityPass, uint32_t* broken, hipStream_t st, hipEvent_t evStart = nullptr,
                       hipEvent_t evStop = nullptr);

@@ -448,12 +448,19 @@ PXH_D void shapeBounds(int i, const float4* pos, const float4* rot, const float4
 
 // shape bounds plus the broadphase's contact-distance inflation
 // (lowlevelaabb/src/BpBroadPhaseABP.cpp:1187-1192)
+// The step's first launch over the bodies also clears what its colouring keeps
+// per body and its few device words.
 __global__ void k_bounds(int n, const float4* pos, const float4* rot, const float4* geom, HullSet hs, float co,
-                         float4* bmin, float4* bmax)
+                         float4* bmin, float4* bmax, ColorState cs)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < STEP_WORDS)
+		cs.words[i] = 0u;
 	if (i >= n)
 		return;
+	cs.mask[i] = 0ull;
+	cs.need[i] = 0u;
+	cs.next[i] = 0u;
 	f3 mn, mx;
 	shapeBounds(i, pos, rot, geom, hs, mn, mx);
 	bmin[i] = make_float4(mn.x - co, mn.y - co, mn.z - co, geom[i].w);
@@ -717,10 +724,14 @@ __global__ void k_gather_sorted(int n, const uint32_t* sortedVals, const float4*
 // long run of empty rows with its whole wave (one lane alone took 38 us where
 // worlds leave hundreds of rows empty); the rows after the last key have a lane
 // each.
+// Where the host reads the starts, rowStart is host memory, and the step's words
+// go along; copies of a few words cost 3 us each on the stream.
 __global__ void __launch_bounds__(256) k_row_start(int n, const uint64_t* sortedKeys, uint32_t* rowStart,
-                                                   uint32_t totalRows)
+                                                   uint32_t totalRows, const uint32_t* words, uint32_t* hostWords)
 {
 	const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (words && t < STEP_WORDS)
+		hostWords[t] = words[t];
 	const int64_t last = int64_t(min(uint32_t(sortedKeys[n - 1] >> 32), totalRows));
 	if (t > last && t <= int64_t(totalRows))
 		rowStart[t] = uint32_t(n);
@@ -1246,13 +1257,32 @@ PXH_D bool liveSlot(int s, int Q, int pairEnd, const uint32_t* dP)
 	return s < Q || s >= pairEnd || uint32_t(s - Q) < *dP;
 }
 
-__global__ void k_touch_flags(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, uint32_t* flags)
+// flags of the touching slots and their sums over CON_TILE-slot tiles (smaller
+// than the scan's: a thread that built up to sixteen constraints one after the
+// other took 20 us at 20,011 bodies)
+constexpr int CON_THREADS = 256, CON_ITEMS = 4, CON_TILE = CON_THREADS * CON_ITEMS;
+int con_tile() { return CON_TILE; }
+__global__ void __launch_bounds__(CON_THREADS) k_touch_flags(int S, int Q, int pairEnd, const uint32_t* dP,
+                                                             const float4* ctN, uint32_t* flags, uint32_t* sums)
 {
-	const int s = blockIdx.x * blockDim.x + threadIdx.x;
-	if (s < S)
-		flags[s] = liveSlot(s, Q, pairEnd, dP) && __float_as_int(ctN[s].w) > 0 ? 1u : 0u;
+	__shared__ uint32_t sh[8];
+	const int base = blockIdx.x * CON_TILE;
+	uint32_t v = 0;
+#pragma unroll
+	for (int k = 0; k < CON_ITEMS; k++)
+	{
+		const int s = base + k * CON_THREADS + threadIdx.x;
+		if (s < S)
+		{
+			const uint32_t f = liveSlot(s, Q, pairEnd, dP) && __float_as_int(ctN[s].w) > 0 ? 1u : 0u;
+			flags[s] = f;
+			v += f;
+		}
+	}
+	v = blockSum(v, sh);
+	if (threadIdx.x == 0)
+		sums[blockIdx.x] = v;
 }
-
 // Pair identity across steps, world-relative so it survives changes to other
 // worlds: world (16 bits) | local index of a (24 bits) | local index of b or
 // 0x800000 | plane index (24 bits).
@@ -1264,15 +1294,14 @@ PXH_D uint64_t worldPairKey(int w, uint32_t la, uint32_t lb)
 
 // constraint list: touching pair slots in slot order, with the scene-local
 // ordering key used by the colouring
-__global__ void k_con_build(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, const uint32_t* scanned,
-                            const uint2* pairs, const int* qBody, const int* qPlane, const int* meshBody, int nPlanes,
-                            const int* local, const int* planeLocal, const int* world, const int* worldTag, int* conA,
-                            int* conB, int* conSlot, uint64_t* conKey, uint64_t* conPKey, int* conColor)
+// Each tile of slots adds up the counts of the tiles before it and scans its
+// own flags; the last one leaves the pair and constraint counts (and whether
+// the mesh candidates overflowed) in the host's words, which saves the copies.
+PXH_D void buildConstraint(int s, int c, int Q, int pairEnd, const uint2* pairs, const int* qBody, const int* qPlane,
+                           const int* meshBody, int nPlanes, const int* local, const int* planeLocal, const int* world,
+                           const int* worldTag, int* conA, int* conB, int* conSlot, uint64_t* conKey,
+                           uint64_t* conPKey, int* conColor)
 {
-	const int s = blockIdx.x * blockDim.x + threadIdx.x;
-	if (s >= S || !(liveSlot(s, Q, pairEnd, dP) && __float_as_int(ctN[s].w) > 0))
-		return;
-	const int c = int(scanned[s]);
 	int a, b;
 	uint32_t la, lb;
 	if (s >= pairEnd)
@@ -1306,25 +1335,78 @@ __global__ void k_con_build(int S, int Q, int pairEnd, const uint32_t* dP, const
 	conColor[c] = b >= 0 ? -1 : -2;  // -2: body-plane, placed after the body-body rounds
 }
 
+__global__ void __launch_bounds__(CON_THREADS) k_con_build(
+    int S, int Q, int pairEnd, const uint32_t* dP, const uint32_t* flags, const uint32_t* sums, const uint2* pairs,
+    const int* qBody, const int* qPlane, const int* meshBody, int nPlanes, const int* local, const int* planeLocal,
+    const int* world, const int* worldTag, const uint32_t* overflow, int* conA, int* conB, int* conSlot,
+    uint64_t* conKey, uint64_t* conPKey, int* conColor, uint32_t* hostCounts)
+{
+	__shared__ uint32_t sh[33];
+	__shared__ uint32_t waveSum[CON_ITEMS][CON_THREADS / 64];
+	const int base = blockIdx.x * CON_TILE;
+	uint32_t before = 0;
+	for (int t = threadIdx.x; t < int(blockIdx.x); t += CON_THREADS)
+		before += sums[t];
+	before = blockSum(before, sh);
+	// slot k * CON_THREADS + thread of the tile: its place among the wave's flags
+	// of row k, then the waves before it
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	uint32_t mine = 0;   // bit k: slot k of this thread touches
+	uint32_t rank[CON_ITEMS];
+#pragma unroll
+	for (int k = 0; k < CON_ITEMS; k++)
+	{
+		const int s = base + k * CON_THREADS + threadIdx.x;
+		const bool f = s < S && flags[s] != 0u;
+		const uint64_t m = __ballot(f);
+		rank[k] = uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+		mine |= f ? 1u << k : 0u;
+		if (lane == 0)
+			waveSum[k][w] = uint32_t(__popcll(m));
+	}
+	__syncthreads();
+	uint32_t run = before;
+#pragma unroll
+	for (int k = 0; k < CON_ITEMS; k++)
+	{
+		uint32_t at = run;
+#pragma unroll
+		for (int i = 0; i < CON_THREADS / 64; i++)
+		{
+			at += i < w ? waveSum[k][i] : 0u;
+			run += waveSum[k][i];
+		}
+		if (mine >> k & 1u)
+			buildConstraint(base + k * CON_THREADS + threadIdx.x, int(at + rank[k]), Q, pairEnd, pairs, qBody, qPlane,
+			                meshBody, nPlanes, local, planeLocal, world, worldTag, conA, conB, conSlot, conKey, conPKey,
+			                conColor);
+	}
+	if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+	{
+		hostCounts[0] = *dP;
+		hostCounts[1] = run;
+		hostCounts[2] = overflow ? *overflow : 0u;
+	}
+}
+
 // ---------------------------------------------------------------------------
 // colouring: a body-body constraint joins colour r when its key is the minimum
 // over the uncoloured constraints of both its bodies (deterministic, and a
 // function of each world's own content); body-plane constraints then follow
 // every colour of their body's body-body constraints
 // ---------------------------------------------------------------------------
-__global__ void k_fill_u64(uint64_t* p, int n, uint64_t v)
+__global__ void k_fill_u64(uint64_t* p, int64_t n, uint64_t v)
 {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
 	if (i < n)
 		p[i] = v;
 }
 
-// Colouring kernels run over the still-uncoloured constraints: list[i] when a
-// compacted list is given, else i, for i below the count *mDev on the device
-// (or the host bound m when mDev is null). They loop grid-stride so the grid
-// can be sized for the bound while few constraints remain.
-PXH_D int listed(const int* list, int i) { return list ? list[i] : i; }
-PXH_D int listCount(int m, const uint32_t* mDev) { return mDev ? min(m, int(*mDev)) : m; }
+// Colouring kernels run over the list of the still-uncoloured (body-body)
+// constraints, list[i] for i below the count *mDev on the device, which m
+// bounds. They loop grid-stride so the grid can be sized for the bound while few
+// constraints remain.
+PXH_D int listCount(int m, const uint32_t* mDev) { return min(m, int(*mDev)); }
 #define PXH_GRID_STRIDE(i, count) \
 	for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < (count); i += gridDim.x * blockDim.x)
 
@@ -1334,11 +1416,9 @@ __global__ void k_color_reset(int m, const uint32_t* mDev, const int* list, cons
 	const int mm = listCount(m, mDev);
 	PXH_GRID_STRIDE(i, mm)
 	{
-		const int c = listed(list, i);
+		const int c = list[i];
 		best[conA[c]] = ~0ull;
-		const int b = conB[c];
-		if (b >= 0)
-			best[b] = ~0ull;
+		best[conB[c]] = ~0ull;
 	}
 }
 
@@ -1348,96 +1428,249 @@ __global__ void k_color_min(int m, const uint32_t* mDev, const int* list, const 
 	const int mm = listCount(m, mDev);
 	PXH_GRID_STRIDE(i, mm)
 	{
-		const int c = listed(list, i);
+		const int c = list[i];
 		if (conColor[c] != -1)
 			continue;
 		const unsigned long long k = conKey[c];
 		atomicMin(&best[conA[c]], k);
-		const int b = conB[c];
-		if (b >= 0)
-			atomicMin(&best[b], k);
+		atomicMin(&best[conB[c]], k);
 	}
 }
 
 // A local minimum takes the smallest colour used by neither of its bodies
 // (first fit on 64-bit per-body colour masks; colours past 63 fall back to
-// one colour per round, 64 + round). Minima of one round share no body, so
-// their mask updates never race with each other's reads.
+// one colour per round, 64 + round, and raise the bodies' `next`, the first
+// colour past them). Minima of one round share no body, so their mask updates
+// never race with each other's reads.
 __global__ void k_color_pick(int m, const uint32_t* mDev, const int* list, int round, const int* conA,
                              const int* conB, const uint64_t* conKey, int* conColor, const unsigned long long* best,
-                             unsigned long long* mask)
+                             unsigned long long* nextBest, ColorState cs)
 {
+	unsigned long long* mask = cs.mask;
 	const int mm = listCount(m, mDev);
 	PXH_GRID_STRIDE(i, mm)
 	{
-		const int c = listed(list, i);
+		const int c = list[i];
 		if (conColor[c] != -1)
 			continue;
 		const unsigned long long k = conKey[c];
 		const int a = conA[c], b = conB[c];
-		if (best[a] == k && (b < 0 || best[b] == k))
+		nextBest[a] = ~0ull;
+		nextBest[b] = ~0ull;
+		if (best[a] == k && best[b] == k)
 		{
-			const unsigned long long used = mask[a] | (b >= 0 ? mask[b] : 0ull);
+			const unsigned long long used = mask[a] | mask[b];
 			const int col = used == ~0ull ? 64 + round : __ffsll((long long)~used) - 1;
 			conColor[c] = col;
 			if (col < 64)
 			{
 				atomicOr(&mask[a], 1ull << col);
-				if (b >= 0)
-					atomicOr(&mask[b], 1ull << col);
+				atomicOr(&mask[b], 1ull << col);
+			}
+			else
+			{
+				atomicMax(&cs.next[a], uint32_t(col + 1));
+				atomicMax(&cs.next[b], uint32_t(col + 1));
 			}
 		}
 	}
 }
 
-// flags[i] for i <= m (flags[m] = 0 ends the scan)
-__global__ void k_color_uncolored(int m, const uint32_t* mDev, const int* list, const int* conColor, uint32_t* flags)
+// appends value to out where take, at the count *total (one atomic a block;
+// the order is left to chance, which nothing that reads the lists depends on)
+PXH_D void blockAppend(bool take, int value, int* out, uint32_t* total)
 {
-	const int mm = listCount(m, mDev);
-	PXH_GRID_STRIDE(i, m + 1)
-		flags[i] = i < mm && conColor[listed(list, i)] == -1 ? 1u : 0u;
+	__shared__ uint32_t waveCnt[16], blockBase;
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+	const uint64_t m = __ballot(take);
+	if (lane == 0)
+		waveCnt[w] = uint32_t(__popcll(m));
+	__syncthreads();
+	if (threadIdx.x == 0)
+	{
+		uint32_t sum = 0;
+		for (int i = 0; i < nw; i++)
+		{
+			const uint32_t c = waveCnt[i];
+			waveCnt[i] = sum;
+			sum += c;
+		}
+		blockBase = sum ? atomicAdd(total, sum) : 0u;
+	}
+	__syncthreads();
+	if (take)
+		out[blockBase + waveCnt[w] + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = value;
+	__syncthreads();
 }
 
-__global__ void k_color_compact(int m, const int* list, const uint32_t* flags, const uint32_t* scanned, int* out)
+// the constraints of the list that the rounds left uncoloured, as the next list
+__global__ void __launch_bounds__(256) k_color_left(int m, const uint32_t* mDev, const int* list, const int* conColor,
+                                                    int* out, uint32_t* left, uint32_t* ran, uint32_t rounds)
 {
-	PXH_GRID_STRIDE(i, m)
-		if (flags[i])
-			out[scanned[i]] = listed(list, i);
+	const int mm = listCount(m, mDev);
+	if (blockIdx.x == 0 && threadIdx.x == 0)
+		*ran = rounds;
+	for (int base = blockIdx.x * 256; base < mm; base += gridDim.x * 256)
+	{
+		const int i = base + threadIdx.x;
+		const int c = i < mm ? list[i] : 0;
+		blockAppend(i < mm && conColor[c] == -1, c, out, left);
+	}
+}
+
+// Up to `rounds` colouring rounds of a short list (at most `limit`; else it only
+// says so, *ran = 0) in one workgroup, ending when nothing is left; the same
+// rounds as k_color_reset / min / pick. A settled step leaves a few hundred new
+// constraints, for which eight rounds were 24 launches and 55 us; this takes 9 us
+// on a 20,011-body bin. best holds two arrays of n: a round's picks clear the next round's
+// minima. The minima and masks change in L2 by atomics and are read there
+// (agent-scope loads), since the first-level cache may hold older lines.
+PXH_D unsigned long long loadAgent(const unsigned long long* p)
+{
+	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+PXH_D void storeAgent(unsigned long long* p, unsigned long long v)
+{
+	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// every memory operation of the wave done, then the block's barrier
+PXH_D void blockPhase()
+{
+	__atomic_signal_fence(__ATOMIC_SEQ_CST);
+	__builtin_amdgcn_s_waitcnt(0);
+	__syncthreads();
+}
+constexpr int ROUND_THREADS = 1024;
+__global__ void __launch_bounds__(ROUND_THREADS) k_color_rounds(const uint32_t* mDev, int limit, const int* list,
+                                                                int firstRound, int rounds, int n, const int* conA,
+                                                                const int* conB, const uint64_t* conKey, int* conColor,
+                                                                unsigned long long* best, ColorState cs, int* out,
+                                                                uint32_t* left, uint32_t* ran)
+{
+	const int m = int(*mDev);
+	if (m > limit)
+	{
+		if (threadIdx.x == 0)
+		{
+			*left = uint32_t(m);
+			*ran = 0u;
+		}
+		return;
+	}
+	for (int i = threadIdx.x; i < m; i += ROUND_THREADS)
+	{
+		const int c = list[i];
+		storeAgent(&best[conA[c]], ~0ull);
+		storeAgent(&best[conB[c]], ~0ull);
+	}
+	blockPhase();
+	bool open = m > 0;
+	for (int r = 0; r < rounds && open; r++)
+	{
+		unsigned long long* cur = best + (r & 1) * int64_t(n);
+		unsigned long long* nxt = best + ((r + 1) & 1) * int64_t(n);
+		for (int i = threadIdx.x; i < m; i += ROUND_THREADS)
+		{
+			const int c = list[i];
+			if (conColor[c] != -1)
+				continue;
+			const unsigned long long k = conKey[c];
+			atomicMin(&cur[conA[c]], k);
+			atomicMin(&cur[conB[c]], k);
+		}
+		blockPhase();
+		int more = 0;
+		for (int i = threadIdx.x; i < m; i += ROUND_THREADS)
+		{
+			const int c = list[i];
+			if (conColor[c] != -1)
+				continue;
+			const unsigned long long k = conKey[c];
+			const int a = conA[c], b = conB[c];
+			if (loadAgent(&cur[a]) == k && loadAgent(&cur[b]) == k)
+			{
+				const unsigned long long used = loadAgent(&cs.mask[a]) | loadAgent(&cs.mask[b]);
+				const int col = used == ~0ull ? 64 + firstRound + r : __ffsll((long long)~used) - 1;
+				conColor[c] = col;
+				if (col < 64)
+				{
+					atomicOr(&cs.mask[a], 1ull << col);
+					atomicOr(&cs.mask[b], 1ull << col);
+				}
+				else
+				{
+					atomicMax(&cs.next[a], uint32_t(col + 1));
+					atomicMax(&cs.next[b], uint32_t(col + 1));
+				}
+			}
+			else
+				more = 1;
+			storeAgent(&nxt[a], ~0ull);
+			storeAgent(&nxt[b], ~0ull);
+		}
+		blockPhase();
+		open = __syncthreads_or(more) != 0;
+	}
+	if (threadIdx.x == 0)
+	{
+		*left = 0u;
+		*ran = uint32_t(rounds);
+	}
+	blockPhase();
+	for (int base = 0; open && base < m; base += ROUND_THREADS)
+	{
+		const int i = base + threadIdx.x;
+		const int c = i < m ? list[i] : 0;
+		blockAppend(i < m && conColor[c] == -1, c, out, left);
+	}
+}
+
+// Colour masks of the bodies that need theirs: those of a constraint still to be
+// coloured and those with a body-plane constraint (k_con_prev marks them). Most
+// constraints of a settled pile touch neither and make no atomic.
+__global__ void k_color_mask(int C, const int* conA, const int* conB, const int* conColor, ColorState cs)
+{
+	const int c = blockIdx.x * blockDim.x + threadIdx.x;
+	if (c >= C)
+		return;
+	const int col = conColor[c];
+	if (col < 0)
+		return;   // body-plane or not coloured yet; a carried colour is below 64
+	const int a = conA[c], b = conB[c];
+	if (cs.need[a])
+		atomicOr(&cs.mask[a], 1ull << col);
+	if (cs.need[b])
+		atomicOr(&cs.mask[b], 1ull << col);
 }
 
 // Body-plane constraints go after every colour of their body's body-body
 // constraints, one colour each in constraint order (the reference places
 // static constraints at maxSolverNormalProgress + k:
-// lowleveldynamics/src/DyConstraintPartition.cpp:168-179, 604-616).
-__global__ void k_body_next(int C, const int* conA, const int* conB, const int* conColor, uint32_t* bodyNext)
+// lowleveldynamics/src/DyConstraintPartition.cpp:168-179, 604-616). The last
+// colour of a body is the top bit of its mask, or past 63 its `next`. A body's
+// body-plane constraints are consecutive in the constraint list (slots are
+// body-major); k counts the ones before c.
+PXH_D int constraintColor(int c, const int* conA, const int* conB, const ColorState& cs, int* conColor)
 {
-	const int c = blockIdx.x * blockDim.x + threadIdx.x;
-	if (c >= C || conB[c] < 0)
-		return;
-	const uint32_t nx = uint32_t(conColor[c] + 1);
-	atomicMax(&bodyNext[conA[c]], nx);
-	atomicMax(&bodyNext[conB[c]], nx);
-}
-
-// A body's body-plane constraints are consecutive in the constraint list
-// (slots are body-major); k counts the ones before c.
-__global__ void k_static_color(int C, const int* conA, const int* conB, const uint32_t* bodyNext, int* conColor)
-{
-	const int c = blockIdx.x * blockDim.x + threadIdx.x;
-	if (c >= C || conB[c] >= 0)
-		return;
+	if (conB[c] >= 0)
+		return conColor[c];
 	const int a = conA[c];
 	int k = 0;
 	for (int e = c - 1; e >= 0 && conA[e] == a && conB[e] < 0; e--)
 		k++;
-	conColor[c] = int(bodyNext[a]) + k;
+	const unsigned long long m = cs.mask[a];
+	const int next = max(int(cs.next[a]), m ? 64 - __clzll((long long)m) : 0);
+	conColor[c] = next + k;
+	return next + k;
 }
 
 // open-addressing table of the previous step's pair keys -> row (keys are
 // unique; the table has at least twice as many slots as keys)
 PXH_D uint32_t patchSlot(uint64_t key, uint32_t mask) { return uint32_t(mix64(key)) & mask; }
 
-__global__ void k_patch_insert(int m, const uint64_t* keys, unsigned long long* htKey, int* htVal, uint32_t mask)
+// an entry is the key and its row side by side, so a probe touches one line;
+// the whole table starts at ~0 (no key has that value)
+__global__ void k_patch_insert(int m, const uint64_t* keys, unsigned long long* table, uint32_t mask)
 {
 	const int o = blockIdx.x * blockDim.x + threadIdx.x;
 	if (o >= m)
@@ -1446,9 +1679,9 @@ __global__ void k_patch_insert(int m, const uint64_t* keys, unsigned long long* 
 	uint32_t slot = patchSlot(key, mask);
 	for (uint32_t probe = 0; probe <= mask; probe++)
 	{
-		if (atomicCAS(&htKey[slot], ~0ull, key) == ~0ull)
+		if (atomicCAS(&table[2 * int64_t(slot)], ~0ull, key) == ~0ull)
 		{
-			htVal[slot] = o;
+			table[2 * int64_t(slot) + 1] = (unsigned long long)(o);
 			return;
 		}
 		slot = (slot + 1) & mask;
@@ -1457,17 +1690,17 @@ __global__ void k_patch_insert(int m, const uint64_t* keys, unsigned long long* 
 
 PXH_D int patchFind(const PatchIO& io, uint64_t key)
 {
-	if (!io.htKey)
+	if (!io.table)
 		return -1;
-	uint32_t slot = patchSlot(key, io.htMask);
-	for (uint32_t probe = 0; probe <= io.htMask; probe++)
+	uint32_t slot = patchSlot(key, io.tableMask);
+	for (uint32_t probe = 0; probe <= io.tableMask; probe++)
 	{
-		const uint64_t k = io.htKey[slot];
-		if (k == key)
-			return io.htVal[slot];
-		if (k == ~0ull)
+		const ulonglong2 e = io.table[slot];
+		if (e.x == key)
+			return int(e.y);
+		if (e.x == ~0ull)
 			return -1;
-		slot = (slot + 1) & io.htMask;
+		slot = (slot + 1) & io.tableMask;
 	}
 	return -1;
 }
@@ -1477,76 +1710,84 @@ PXH_D int patchFind(const PatchIO& io, uint64_t key)
 // (below 64): those constraints were coloured together then, so they never
 // share a colour at a body now. The reference GPU solver keeps its partitions
 // from step to step the same way (gpusolver/src/PxgConstraintPartition.cpp:1940).
-__global__ void k_con_prev(int C, const int* conA, const int* conB, const int* conSlot, PatchIO io, int* conColor,
-                           unsigned long long* mask)
+// Lists the others and marks the bodies whose masks the colouring reads.
+__global__ void __launch_bounds__(256) k_con_prev(int C, const int* conA, const int* conB, const int* conSlot,
+                                                  PatchIO io, int* conColor, ColorState cs, int* list)
 {
 	const int c = blockIdx.x * blockDim.x + threadIdx.x;
-	if (c >= C)
-		return;
-	const int a = conA[c], b = conB[c];
-	const uint64_t pkey = io.conPKey[c];
-	const int po = patchFind(io, pkey);
-	if (io.prevRow)
-		io.prevRow[c] = po;
-	io.conRec[2 * int64_t(c)] = make_int4(a, b, conSlot[c], po);
-	io.conRec[2 * int64_t(c) + 1] = make_int4(int(uint32_t(pkey)), int(uint32_t(pkey >> 32)), 0, 0);
-	if (b >= 0 && po >= 0)
+	bool open = false;
+	if (c < C)
 	{
-		const int pc = io.prevColor[po];
-		if (pc >= 0 && pc < 64)
+		const int a = conA[c], b = conB[c];
+		const uint64_t pkey = io.conPKey[c];
+		const int po = patchFind(io, pkey);
+		if (io.prevRow)
+			io.prevRow[c] = po;
+		io.conRec[2 * int64_t(c)] = make_int4(a, b, conSlot[c], po);
+		io.conRec[2 * int64_t(c) + 1] = make_int4(int(uint32_t(pkey)), int(uint32_t(pkey >> 32)), 0, 0);
+		if (b < 0)
+			cs.need[a] = 1u;
+		else
 		{
-			conColor[c] = pc;
-			atomicOr(&mask[a], 1ull << pc);
-			atomicOr(&mask[b], 1ull << pc);
+			const int pc = po >= 0 ? io.prevColor[po] : -1;
+			if (pc >= 0 && pc < 64)
+				conColor[c] = pc;
+			else
+			{
+				open = true;
+				cs.need[a] = 1u;
+				cs.need[b] = 1u;
+			}
 		}
 	}
-}
-
-// block-level maximum then one atomic per block (grid-stride)
-__global__ void __launch_bounds__(256) k_max_color(int C, const int* conColor, uint32_t* maxColor)
-{
-	__shared__ int red[256];
-	int v = 0;
-	for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < C; c += gridDim.x * blockDim.x)
-		v = max(v, conColor[c]);
-	red[threadIdx.x] = v;
-	__syncthreads();
-	for (int o = 128; o > 0; o >>= 1)
-	{
-		if (threadIdx.x < o)
-			red[threadIdx.x] = max(red[threadIdx.x], red[threadIdx.x + o]);
-		__syncthreads();
-	}
-	if (threadIdx.x == 0)
-		atomicMax(maxColor, uint32_t(red[0]));
+	blockAppend(open, c, list, cs.words + STEP_OPEN);
 }
 
 // colour-ordered constraint list by a stable radix sort of (colour, index)
 // A constraint not coloured yet (-1, when the rounds have not finished) sorts
 // to colour `limit`, past every real colour.
-__global__ void k_color_keys(int C, const int* conColor, uint32_t limit, uint64_t* keys, uint32_t* vals)
+__global__ void k_color_keys(int C, const int* conA, const int* conB, int* conColor, ColorState cs, uint32_t limit,
+                             uint64_t* keys, uint32_t* vals)
 {
 	const int c = blockIdx.x * blockDim.x + threadIdx.x;
 	if (c < C)
 	{
-		const int col = conColor[c];
+		const int col = constraintColor(c, conA, conB, cs, conColor);
 		const uint32_t k = col < 0 ? limit : min(uint32_t(col), limit);
 		keys[c] = (uint64_t(k) << 32) | uint32_t(c);
 		vals[c] = uint32_t(c);
 	}
 }
-// rows ordered by (world, colour): key world * CB + colour, CB = limit + 1
-__global__ void k_color_keys_world(int C, const int* conColor, const int* conA, const int* bodyWorld,
-                                   uint32_t limit, uint64_t* keys, uint32_t* vals)
+// rows ordered by (world, colour): key world * CB + colour, CB = limit + 1; the
+// largest colour in the step's words (one atomic a block)
+__global__ void __launch_bounds__(256) k_color_keys_world(int C, const int* conA, const int* conB, int* conColor,
+                                                          ColorState cs, const int* bodyWorld, uint32_t limit,
+                                                          uint64_t* keys, uint32_t* vals)
 {
+	__shared__ int red[4];
 	const int c = blockIdx.x * blockDim.x + threadIdx.x;
+	int top = 0;
 	if (c < C)
 	{
-		const int col = conColor[c];
+		const int col = constraintColor(c, conA, conB, cs, conColor);
 		const uint32_t k = col < 0 ? limit : min(uint32_t(col), limit);
 		const uint64_t w = uint64_t(bodyWorld[conA[c]]);
 		keys[c] = ((w * (limit + 1) + k) << 32) | uint32_t(c);
 		vals[c] = uint32_t(c);
+		top = max(col, 0);
+	}
+#pragma unroll
+	for (int o = 1; o < 64; o <<= 1)
+		top = max(top, __shfl_xor(top, o));
+	if ((threadIdx.x & 63) == 0)
+		red[threadIdx.x >> 6] = top;
+	__syncthreads();
+	if (threadIdx.x == 0)
+	{
+		top = max(max(red[0], red[1]), max(red[2], red[3]));
+		// most blocks stay below the maximum that others have left
+		if (uint32_t(top) > __hip_atomic_load(&cs.words[STEP_TOP], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+			atomicMax(&cs.words[STEP_TOP], uint32_t(top));
 	}
 }
 
@@ -3338,6 +3579,8 @@ void launch_scan(uint32_t* data, int64_t n, uint32_t* tmp, hipStream_t st)
 
 int64_t scan_tmp_size(int64_t n) { return (std::max<int64_t>(n, 0) + SCAN_TILE - 1) / SCAN_TILE + 1; }
 
+bool radix_result_in_alt(int n, int bits) { return n > RS_SMALL && ((bits + 7) / 8) % 2 == 1; }
+
 void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t* vals2, int n, int lowBits,
                        int highBits, uint32_t* hist, hipStream_t st, bool& resultInAlt)
 {
@@ -3357,7 +3600,7 @@ void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t
 			k_rs_small<8><<<1, RS_SMALL_THREADS, 0, st>>>(keys, vals, n, lowBits, bits);
 		return;
 	}
-	const int nb = nblk(n, RS_TILE);
+	const int nb = nblk(n, RS_TILE);   // radix_result_in_alt says where the result lands
 	uint64_t* ka = keys;
 	uint32_t* va = vals;
 	uint64_t* kb = keys2;
@@ -3376,9 +3619,9 @@ void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t
 	do { if ((n) > 0) kernel<<<nblk((n), 256), 256, 0, st>>>(__VA_ARGS__); } while (0)
 
 void launch_bounds(int n, const float4* pos, const float4* rot, const float4* geom, const HullSet& hs, float co,
-                   float4* bmin, float4* bmax, hipStream_t st)
+                   float4* bmin, float4* bmax, ColorState cs, hipStream_t st)
 {
-	PXH_LAUNCH(k_bounds, n, n, pos, rot, geom, hs, co, bmin, bmax);
+	PXH_LAUNCH(k_bounds, n, n, pos, rot, geom, hs, co, bmin, bmax, cs);
 }
 // Worlds of up to 8,192 bodies take a workgroup each (4,096 bodies in one world:
 // 7 us against 11 in four launches); a larger world takes the launches over
@@ -3412,13 +3655,14 @@ void launch_gather_sorted(int n, const uint32_t* sv, const float4* bmin, const f
 {
 	PXH_LAUNCH(k_gather_sorted, n, n, sv, bmin, bmax, smin, smax);
 }
-void launch_row_start(int n, const uint64_t* sk, uint32_t* rowStart, uint32_t totalRows, hipStream_t st)
+void launch_row_start(int n, const uint64_t* sk, uint32_t* rowStart, uint32_t totalRows, hipStream_t st,
+                      const uint32_t* words, uint32_t* hostWords)
 {
 	const int64_t rows = int64_t(totalRows) + 1;
 	if (n == 0)
 		PXH_LAUNCH(k_fill_u32, rows, rowStart, rows, 0u);
 	else
-		PXH_LAUNCH(k_row_start, std::max<int64_t>(n, rows), n, sk, rowStart, totalRows);
+		PXH_LAUNCH(k_row_start, std::max<int64_t>(n, rows), n, sk, rowStart, totalRows, words, hostWords);
 }
 template <int G, int CLASSES>
 static void sweepPass(bool write, int n, const uint64_t* sk, const float4* smin, const float4* smax, const int* scene,
@@ -3568,20 +3812,19 @@ void launch_joint_solve(int begin, int end, const int4* info, const float4* head
 	k_joint_solve<<<nblk(end - begin, 64), 64, 0, st>>>(begin, end, info, head, rows, sb.vel, sb.dq, sb.i0, sb.i1,
 	                                                     elapsed, conclude ? 1 : 0, sleepFlags);
 }
-void launch_touch_flags(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, uint32_t* flags,
-                        hipStream_t st)
+void launch_con_build(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, uint32_t* flags,
+                      uint32_t* scanTmp, const uint2* pairs, const int* qBody, const int* qPlane, const int* meshBody,
+                      int nPlanes, const int* local, const int* planeLocal, const int* world, const int* worldTag,
+                      const uint32_t* overflow, int* conA, int* conB, int* conSlot, uint64_t* conKey,
+                      uint64_t* conPKey, int* conColor, uint32_t* hostCounts, hipStream_t st)
 {
-	PXH_LAUNCH(k_touch_flags, S, S, Q, pairEnd, dP, ctN, flags);
+	const int nb = std::max(nblk(S, CON_TILE), 1);
+	k_touch_flags<<<nb, CON_THREADS, 0, st>>>(S, Q, pairEnd, dP, ctN, flags, scanTmp);
+	k_con_build<<<nb, CON_THREADS, 0, st>>>(S, Q, pairEnd, dP, flags, scanTmp, pairs, qBody, qPlane, meshBody, nPlanes,
+	                                         local, planeLocal, world, worldTag, overflow, conA, conB, conSlot, conKey,
+	                                         conPKey, conColor, hostCounts);
 }
-void launch_con_build(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, const uint32_t* scanned,
-                      const uint2* pairs, const int* qBody, const int* qPlane, const int* meshBody, int nPlanes,
-                      const int* local, const int* planeLocal, const int* world, const int* worldTag, int* conA,
-                      int* conB, int* conSlot, uint64_t* conKey, uint64_t* conPKey, int* conColor, hipStream_t st)
-{
-	PXH_LAUNCH(k_con_build, S, S, Q, pairEnd, dP, ctN, scanned, pairs, qBody, qPlane, meshBody, nPlanes, local,
-	           planeLocal, world, worldTag, conA, conB, conSlot, conKey, conPKey, conColor);
-}
-// out[i] = in[idx[i]] for elements of `bytes` (4 or 16) bytes
+
 __global__ void k_gather4(int n, const int* idx, const uint32_t* in, uint32_t* out)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -3603,55 +3846,47 @@ void launch_gather(int n, const int* idx, const void* in, void* out, int bytes, 
 }
 // colouring launches are grid-stride over at most 1024 blocks
 static int colorBlocks(int m) { return std::max(1, std::min(nblk(m, 256), 1024)); }
-void launch_color_round(int m, const uint32_t* mDev, const int* list, int round, const int* conA, const int* conB,
-                        const uint64_t* conKey, int* conColor, uint64_t* best, uint64_t* mask, hipStream_t st)
+void launch_color_rounds(int m, const uint32_t* mDev, const int* list, int firstRound, int rounds, int n,
+                         const int* conA, const int* conB, const uint64_t* conKey, int* conColor, uint64_t* best,
+                         ColorState cs, int* out, uint32_t* left, uint32_t* ran, bool oneBlock, hipStream_t st)
 {
-	if (m <= 0)
-		return;
 	unsigned long long* bst = reinterpret_cast<unsigned long long*>(best);
+	if (oneBlock)
+	{
+		k_color_rounds<<<1, ROUND_THREADS, 0, st>>>(mDev, COLOR_SHORT_LIST, list, firstRound, rounds, n, conA, conB,
+		                                            conKey, conColor, bst, cs, out, left, ran);
+		return;
+	}
 	const int g = colorBlocks(m);
 	k_color_reset<<<g, 256, 0, st>>>(m, mDev, list, conA, conB, bst);
-	k_color_min<<<g, 256, 0, st>>>(m, mDev, list, conA, conB, conKey, conColor, bst);
-	k_color_pick<<<g, 256, 0, st>>>(m, mDev, list, round, conA, conB, conKey, conColor, bst,
-	                                reinterpret_cast<unsigned long long*>(mask));
+	for (int r = 0; r < rounds; r++)
+	{
+		unsigned long long* cur = bst + (r & 1) * int64_t(n);
+		unsigned long long* nxt = bst + ((r + 1) & 1) * int64_t(n);
+		k_color_min<<<g, 256, 0, st>>>(m, mDev, list, conA, conB, conKey, conColor, cur);
+		k_color_pick<<<g, 256, 0, st>>>(m, mDev, list, firstRound + r, conA, conB, conKey, conColor, cur, nxt, cs);
+	}
+	k_fill_u32<<<1, 64, 0, st>>>(left, 1, 0u);
+	k_color_left<<<g, 256, 0, st>>>(m, mDev, list, conColor, out, left, ran, uint32_t(rounds));
 }
-void launch_color_uncolored(int m, const uint32_t* mDev, const int* list, const int* conColor, uint32_t* flags,
-                            hipStream_t st)
+void launch_color_mask(int C, const int* conA, const int* conB, const int* conColor, ColorState cs, hipStream_t st)
 {
-	k_color_uncolored<<<colorBlocks(m + 1), 256, 0, st>>>(m, mDev, list, conColor, flags);
+	PXH_LAUNCH(k_color_mask, C, C, conA, conB, conColor, cs);
 }
-void launch_color_compact(int m, const int* list, const uint32_t* flags, const uint32_t* scanned, int* out,
-                          hipStream_t st)
+void launch_patch_table(int m, const uint64_t* keys, ulonglong2* table, uint32_t mask, hipStream_t st)
 {
-	if (m > 0)
-		k_color_compact<<<colorBlocks(m), 256, 0, st>>>(m, list, flags, scanned, out);
-}
-void launch_fill_u64(uint64_t* p, int n, uint64_t v, hipStream_t st) { PXH_LAUNCH(k_fill_u64, n, p, n, v); }
-void launch_static_colors(int n, int C, const int* conA, const int* conB, int* conColor, uint32_t* bodyNext,
-                          hipStream_t st)
-{
-	PXH_LAUNCH(k_fill_u32, n, bodyNext, int64_t(n), 0u);
-	PXH_LAUNCH(k_body_next, C, C, conA, conB, conColor, bodyNext);
-	PXH_LAUNCH(k_static_color, C, C, conA, conB, bodyNext, conColor);
-}
-void launch_patch_table(int m, const uint64_t* keys, uint64_t* htKey, int* htVal, uint32_t htMask, hipStream_t st)
-{
-	PXH_LAUNCH(k_fill_u64, int(htMask) + 1, htKey, int(htMask) + 1, ~0ull);
-	PXH_LAUNCH(k_patch_insert, m, m, keys, reinterpret_cast<unsigned long long*>(htKey), htVal, htMask);
+	PXH_LAUNCH(k_fill_u64, 2 * int64_t(mask) + 2, reinterpret_cast<uint64_t*>(table), 2 * int64_t(mask) + 2, ~0ull);
+	PXH_LAUNCH(k_patch_insert, m, m, keys, reinterpret_cast<unsigned long long*>(table), mask);
 }
 void launch_con_prev(int C, const int* conA, const int* conB, const int* conSlot, PatchIO io, int* conColor,
-                     uint64_t* mask, hipStream_t st)
+                     ColorState cs, int* list, hipStream_t st)
 {
-	PXH_LAUNCH(k_con_prev, C, C, conA, conB, conSlot, io, conColor, reinterpret_cast<unsigned long long*>(mask));
+	PXH_LAUNCH(k_con_prev, C, C, conA, conB, conSlot, io, conColor, cs, list);
 }
-void launch_color_keys(int C, const int* conColor, uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st)
+void launch_color_keys(int C, const int* conA, const int* conB, int* conColor, ColorState cs, uint32_t limit,
+                       uint64_t* keys, uint32_t* vals, hipStream_t st)
 {
-	PXH_LAUNCH(k_color_keys, C, C, conColor, limit, keys, vals);
-}
-void launch_max_color(int C, const int* conColor, uint32_t* maxColor, hipStream_t st)
-{
-	if (C > 0)
-		k_max_color<<<std::min(nblk(C, 256), 256), 256, 0, st>>>(C, conColor, maxColor);
+	PXH_LAUNCH(k_color_keys, C, C, conA, conB, conColor, cs, limit, keys, vals);
 }
 void launch_preintegrate(int n, const float4* pos, const float4* rot, const float4* lin, const float4* ang,
                          const float4* invI, float3 gdt, float linDampDt, float angDampDt, float maxLinSq,
@@ -3664,15 +3899,15 @@ void launch_preintegrate(int n, const float4* pos, const float4* rot, const floa
 void launch_prep(int C, const int* order, const int* conA, const int* conB, const int* conSlot, const float4* ctN,
                  const float4* ctP, const float4* pos, const float4* rot, SolverBodies sb, float invStepDt,
                  float scale, float restDist, float fot, Rows rows, PatchIO patches, unsigned long long* counters,
-                 hipStream_t st)
+                 unsigned long long* hostCounters, hipStream_t st)
 {
 	(void)pos;
 	(void)rot;
 	(void)conA;
 	(void)conB;
 	(void)conSlot;
-	PXH_LAUNCH(k_prep, C, C, order, ctN, ctP, sb.rec, invStepDt, scale, restDist, fot, rows, patches, counters + 4);
-	k_sum_counters<<<1, 256, 0, st>>>(nblk(C, 256), counters + 4, counters);
+	PXH_LAUNCH(k_prep, C, C, order, ctN, ctP, sb.rec, invStepDt, scale, restDist, fot, rows, patches, counters);
+	k_sum_counters<<<1, 256, 0, st>>>(nblk(C, 256), counters, hostCounters);
 }
 void launch_solve(int begin, int end, int C, Rows rows, SolverBodies sb, float minPen, float muS, float muD,
                   float invStepDt, float biasScale, float scale, uint32_t* broken, hipStream_t st, hipEvent_t evStart,
@@ -3688,10 +3923,10 @@ void launch_solve(int begin, int end, int C, Rows rows, SolverBodies sb, float m
 		k_solve<<<grid, block, 0, st>>>(begin, end, C, rows, sb.vel, minPen, muS, muD, invStepDt, biasScale, scale,
 		                                broken);
 }
-void launch_color_keys_world(int C, const int* conColor, const int* conA, const int* bodyWorld, uint32_t limit,
-                             uint64_t* keys, uint32_t* vals, hipStream_t st)
+void launch_color_keys_world(int C, const int* conA, const int* conB, int* conColor, ColorState cs,
+                             const int* bodyWorld, uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st)
 {
-	PXH_LAUNCH(k_color_keys_world, C, C, conColor, conA, bodyWorld, limit, keys, vals);
+	PXH_LAUNCH(k_color_keys_world, C, C, conA, conB, conColor, cs, bodyWorld, limit, keys, vals);
 }
 int solve_world_threads() { return SOLVE_WORLD_THREADS; }
 void launch_fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t st)
@@ -3723,7 +3958,7 @@ void launch_solve_worlds(int grid, int nWorlds, const int* worldOrder, uint32_t*
 void launch_prep_pgs(int C, const int* order, const int* conA, const int* conB, const int* conSlot,
                      const float4* ctN, const float4* ctP, const float4* pos, const float4* rot, SolverBodies sb,
                      float invDt, float muS, float muD, float restDist, float fot, Rows rows, float* rowsU,
-                     PatchIO patches, unsigned long long* counters, hipStream_t st)
+                     PatchIO patches, unsigned long long* counters, unsigned long long* hostCounters, hipStream_t st)
 {
 	(void)pos;
 	(void)rot;
@@ -3731,8 +3966,8 @@ void launch_prep_pgs(int C, const int* order, const int* conA, const int* conB, 
 	(void)conB;
 	(void)conSlot;
 	PXH_LAUNCH(k_prep_pgs, C, C, order, ctN, ctP, sb.rec, invDt, muS, muD, restDist, fot, rows, rowsU, patches,
-	           counters + 4);
-	k_sum_counters<<<1, 256, 0, st>>>(nblk(C, 256), counters + 4, counters);
+	           counters);
+	k_sum_counters<<<1, 256, 0, st>>>(nblk(C, 256), counters, hostCounters);
 }
 void launch_solve_pgs(int begin, int end, int C, Rows rows, const float* rowsU, SolverBodies sb, bool doFriction,
                       bool velocityPass, uint32_t* broken, hipStream_t st, hipEvent_t evStart, hipEvent_t evStop)

@@ -177,10 +177,10 @@ struct pxh_scene_t
 	DBuf<uint2> pairs;
 	DBuf<float4> ctN, ctP;
 	DBuf<int> conA, conB, conSlot, conColor, order;
-	DBuf<uint64_t> conKey, conPKey, best, mask;
+	DBuf<uint64_t> conKey, conPKey, best;
+	DBuf<unsigned long long> mask;
 	DBuf<int> colList, colList2;
-	DBuf<uint32_t> colFlags;
-	DBuf<uint32_t> colorCount, scratch;
+	DBuf<uint32_t> scratch;
 	DBuf<unsigned long long> counters;    // contact points, friction rows, dynamic-dynamic constraints
 	int64_t statFriction = 0, statDynCon = 0, statRounds = 0, statDynFriction = 0, statSolveLaunches = 0;
 	pxh::SolverBodies sb{};
@@ -196,9 +196,9 @@ struct pxh_scene_t
 	DBuf<int> patchColor[2];
 	DBuf<int> prevRow;
 	DBuf<int4> conRec;   // packed per-constraint record the preparation gathers
-	DBuf<uint64_t> htKey;
-	DBuf<int> htVal;
-	DBuf<uint32_t> bodyNext;
+	DBuf<ulonglong2> patchTable;
+	DBuf<uint32_t> bodyNext, bodyNeed, stepWords;
+	uint32_t lastOpen = 0;                // constraints the last step coloured anew
 	int patchCur = 0;
 	int nPrevRows = 0;
 	// capacities and tables sized on the host so a step needs few host round trips
@@ -206,7 +206,6 @@ struct pxh_scene_t
 	size_t pairCap = 0;                   // pair buffer capacity (grown when exceeded)
 	uint32_t totalRows = 0;               // broadphase row table size (rowOff on the device)
 	int maxPlanes = 0;                    // most planes in one world
-	DBuf<uint32_t> colCounts;             // colouring compaction offsets
 	// Direct GPU API forces and torques as accelerations for the next step
 	// (allocated, zeroed, on the first one) and the velocities before the
 	// last step (with enable_body_accelerations)
@@ -400,14 +399,14 @@ struct pxh_scene_t
 		f(rows); f(rowOff); f(rowStart); f(vals); f(vals2); f(hist); f(scanTmp); f(counts); f(flags); f(gridAcc);
 		f(keys); f(keys2); f(pairs); f(ctN); f(ctP);
 		f(conA); f(conB); f(conSlot); f(conColor); f(order); f(conKey); f(conPKey); f(best); f(mask);
-		f(colList); f(colList2); f(colFlags); f(colorCount); f(scratch); f(counters);
+		f(colList); f(colList2); f(scratch); f(counters);
 		f(sbVel); f(sbP); f(sbDQ); f(sbI0); f(sbI1); f(sbOrig); f(sbRec);
 		f(rhI); f(rhF); f(rnA); f(rnB); f(rfT); f(rfA); f(rfB); f(rnF); f(rfF); f(rnU);
 		for (int k = 0; k < 2; k++)
 		{
 			f(patch[k]); f(patchKey[k]); f(patchBroken[k]); f(patchColor[k]);
 		}
-		f(prevRow); f(conRec); f(htKey); f(htVal); f(bodyNext); f(colCounts); f(gatherTmp); f(gatherIdx);
+		f(prevRow); f(conRec); f(patchTable); f(bodyNext); f(bodyNeed); f(stepWords); f(gatherTmp); f(gatherIdx);
 		f(worldOrder); f(segStart); f(solveQueue); f(extLin); f(extAng); f(prevLin); f(prevAng);
 		f(evFound); f(evFoundScan); f(evMatched); f(evLost); f(evLostScan); f(evFoundKeys); f(evLostKeys);
 		f(jInfo); f(jFrame); f(jParam); f(jHead); f(jRows); f(jKeys); f(bpGroup);
@@ -642,11 +641,13 @@ int rebuild_topology(pxh_scene_t* s)
 	return PXH_OK;
 }
 
-// pinned host staging of a scene: colour ranges in [0, kHostColorSlots), the
-// step's device counters (u64) at kHostCounterSlot
+// pinned host words of a scene, written by the kernels: colour ranges (and
+// before them the pair and constraint counts) in [0, kHostColorSlots), the
+// step's counters (u64) at kHostCounterSlot, its device words at kHostWordSlot
 constexpr size_t kHostCountsBytes = 65536;
 constexpr int kHostColorSlots = 15000;
 constexpr int kHostCounterSlot = 15000;
+constexpr int kHostWordSlot = 15016;
 
 // b[i] = b[idx[i]] for i < n, through a scratch buffer that stays with the scene
 template <typename T>
@@ -1653,8 +1654,13 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	// 1. bounds + broadphase; the pair count stays on the device (dP)
 	PXH_CHECK(s->bmin.ensure(n));
 	PXH_CHECK(s->bmax.ensure(n));
+	PXH_CHECK(s->mask.ensure(n));
+	PXH_CHECK(s->bodyNeed.ensure(n));
+	PXH_CHECK(s->bodyNext.ensure(n));
+	PXH_CHECK(s->stepWords.ensure(pxh::STEP_WORDS));
+	const pxh::ColorState colors{s->mask.p, s->bodyNeed.p, s->bodyNext.p, s->stepWords.p};
 	int pk = s->profBegin(0);
-	pxh::launch_bounds(n, s->pos.p, s->rot.p, s->geom.p, s->hullSet(), co, s->bmin.p, s->bmax.p, st);
+	pxh::launch_bounds(n, s->pos.p, s->rot.p, s->geom.p, s->hullSet(), co, s->bmin.p, s->bmax.p, colors, st);
 	s->profEnd(pk);
 	s->pairCap = std::max(s->pairCap, size_t(s->desc.max_pairs_per_body) * n);
 	if (s->aggDirty)
@@ -1773,10 +1779,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 			                          int(s->hJType.size()), s->jInfo.p, s->lin.p, s->ang.p, ss, st);
 		}
 		PXH_CHECK(s->flags.ensure(size_t(S) + 1));
-		PXH_CHECK(s->scanTmp.ensure(pxh::scan_tmp_size(int64_t(S) + 1) + 1024));
-		pxh::launch_touch_flags(S, Q, pairEnd, dP, s->ctN.p, s->flags.p, st);
-		PXH_CHECK(hipMemsetAsync(s->flags.p + S, 0, sizeof(uint32_t), st));
-		pxh::launch_scan(s->flags.p, int64_t(S) + 1, s->scanTmp.p, st);
+		PXH_CHECK(s->scanTmp.ensure(size_t(S) / size_t(pxh::con_tile()) + 1));
 		const size_t Sc = std::max(S, 1);
 		PXH_CHECK(s->conA.ensure(Sc));
 		PXH_CHECK(s->conB.ensure(Sc));
@@ -1784,13 +1787,11 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		PXH_CHECK(s->conColor.ensure(Sc));
 		PXH_CHECK(s->conKey.ensure(Sc));
 		PXH_CHECK(s->conPKey.ensure(Sc));
-		pxh::launch_con_build(S, Q, pairEnd, dP, s->ctN.p, s->flags.p, s->pairs.p, s->qBody.p, s->qPlane.p,
-		                      s->meshBody.p, s->m, s->local.p, s->planeLocal.p, s->scene.p, s->worldTag.p, s->conA.p,
-		                      s->conB.p, s->conSlot.p, s->conKey.p, s->conPKey.p, s->conColor.p, st);
-		const uint32_t* src[3] = {dP, s->flags.p + S, nMB > 0 ? s->meshOverflow.p : dP};
-		r = readCounts(st, s->hostCounts, src, 3);
-		if (r)
-			return r;
+		pxh::launch_con_build(S, Q, pairEnd, dP, s->ctN.p, s->flags.p, s->scanTmp.p, s->pairs.p, s->qBody.p,
+		                      s->qPlane.p, s->meshBody.p, s->m, s->local.p, s->planeLocal.p, s->scene.p, s->worldTag.p,
+		                      nMB > 0 ? s->meshOverflow.p : nullptr, s->conA.p, s->conB.p, s->conSlot.p, s->conKey.p,
+		                      s->conPKey.p, s->conColor.p, s->hostCounts, st);
+		PXH_CHECK(hipStreamSynchronize(st));
 		P = int(s->hostCounts[0]);
 		C = int(s->hostCounts[1]);
 		if (nMB > 0 && s->hostCounts[2])
@@ -1813,26 +1814,27 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	//    constraints, its previous colour
 	const size_t Cc = std::max(C, 1);
 	const int cur = s->patchCur, prv = cur ^ 1;
-	PXH_CHECK(s->best.ensure(n));
-	PXH_CHECK(s->mask.ensure(n));
+	PXH_CHECK(s->best.ensure(2 * size_t(n)));
 	PXH_CHECK(s->prevRow.ensure(Cc));
 	PXH_CHECK(s->conRec.ensure(2 * Cc));
-	pxh::launch_fill_u64(s->mask.p, n, 0ull, st);
+	PXH_CHECK(s->colList.ensure(Cc));
+	PXH_CHECK(s->colList2.ensure(Cc));
 	pxh::PatchIO pio{};
 	pio.corrDist = d.friction_correlation_distance;
 	pio.conPKey = s->conPKey.p;
 	pio.conRec = s->conRec.p;
 	if (s->nPrevRows > 0)
 	{
+		// at most half full, and at most a quarter while the table is small: the
+		// probes of one lane are a chain of atomics, the clearing streams
+		const uint32_t load = s->nPrevRows < 65536 ? 4u : 2u;
 		uint32_t size = 64;
-		while (size < 2u * uint32_t(s->nPrevRows))
+		while (size < load * uint32_t(s->nPrevRows))
 			size <<= 1;
-		PXH_CHECK(s->htKey.ensure(size));
-		PXH_CHECK(s->htVal.ensure(size));
-		pxh::launch_patch_table(s->nPrevRows, s->patchKey[prv].p, s->htKey.p, s->htVal.p, size - 1, st);
-		pio.htKey = s->htKey.p;
-		pio.htVal = s->htVal.p;
-		pio.htMask = size - 1;
+		PXH_CHECK(s->patchTable.ensure(size));
+		pxh::launch_patch_table(s->nPrevRows, s->patchKey[prv].p, s->patchTable.p, size - 1, st);
+		pio.table = s->patchTable.p;
+		pio.tableMask = size - 1;
 		pio.prev = s->patch[prv].p;
 		pio.prevBroken = s->patchBroken[prv].p;
 		pio.prevColor = s->patchColor[prv].p;
@@ -1840,7 +1842,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	}
 	// every step: the packed constraint records (and, after a previous step,
 	// each constraint's previous row and colour)
-	pxh::launch_con_prev(C, s->conA.p, s->conB.p, s->conSlot.p, pio, s->conColor.p, s->mask.p, st);
+	pxh::launch_con_prev(C, s->conA.p, s->conB.p, s->conSlot.p, pio, s->conColor.p, colors, s->colList.p, st);
 
 	// touch found / lost events: constraints without a previous row, and
 	// previous rows that no constraint found, as pair keys
@@ -1872,16 +1874,11 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	}
 
 	// 5. colouring of the remaining body-body constraints: rounds of local key
-	//    minima, each taking its first free colour, over a compacted list of the
+	//    minima, each taking its first free colour, over the list of the
 	//    uncoloured constraints whose count stays on the device; then the
 	//    body-plane colours and the colour order. One host round trip reads the
 	//    colour ranges and what is left uncoloured (a first step, with nothing
 	//    carried over, may need further rounds).
-	PXH_CHECK(s->colList.ensure(Cc));
-	PXH_CHECK(s->colList2.ensure(Cc));
-	PXH_CHECK(s->colFlags.ensure(Cc + 1));
-	PXH_CHECK(s->colCounts.ensure(Cc + 1));
-	PXH_CHECK(s->bodyNext.ensure(n));
 	PXH_CHECK(s->keys.ensure(Cc));
 	PXH_CHECK(s->keys2.ensure(Cc));
 	PXH_CHECK(s->vals.ensure(Cc));
@@ -1889,28 +1886,13 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	{
 		const int nb = (C + pxh::radix_tile() - 1) / pxh::radix_tile();
 		PXH_CHECK(s->hist.ensure(size_t(256) * std::max(nb, 1)));
-		PXH_CHECK(s->scanTmp.ensure(pxh::scan_tmp_size(int64_t(C) + 1) + 1024));
 	}
 	int rounds = 0;
 	const int kMaxRounds = 960;
-	const int* list = nullptr;         // null: every constraint
-	const uint32_t* mDev = nullptr;    // null: count C
-	int bound = C;                     // host bound on the list length
 	if (64 + kMaxRounds + s->maxPlanes + 2 > kHostColorSlots)
 		return fail(PXH_ERR_CAPACITY, "pxh_scene_simulate: too many planes in one world");
-	auto compact = [&]() {
-		int* out = list == s->colList.p ? s->colList2.p : s->colList.p;
-		pxh::launch_color_uncolored(bound, mDev, list, s->conColor.p, s->colFlags.p, st);
-		(void)hipMemcpyAsync(s->colCounts.p, s->colFlags.p, sizeof(uint32_t) * (size_t(bound) + 1),
-		                     hipMemcpyDeviceToDevice, st);
-		pxh::launch_scan(s->colCounts.p, int64_t(bound) + 1, s->scanTmp.p, st);
-		pxh::launch_color_compact(bound, list, s->colFlags.p, s->colCounts.p, out, st);
-		list = out;
-		mDev = s->colCounts.p + bound;
-	};
 	int nColors = 0;
 	std::vector<uint32_t> colorStart(1, 0);
-	int remaining = C;
 	// the per-world solve: TGS, and every world small enough for one workgroup
 	// (layout auto), or as the tuning asks
 	const int layout = s->tuning[0];
@@ -1920,46 +1902,83 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	s->lastWorldSolve = worldSolve;
 	int CB = 0;   // per-world solve: colour slots per world
 	if (worldSolve)
-		PXH_CHECK(s->solveQueue.ensure(2));
-	while (C > 0 && worldSolve)
+		PXH_CHECK(s->solveQueue.ensure(1));
+	if (C > 0)
+		pxh::launch_color_mask(C, s->conA.p, s->conB.p, s->conColor.p, colors, st);
+	// a short list (by the last step's, or on a first step the whole list) runs
+	// its rounds in one launch, which leaves a list that turns out longer to the
+	// launches of the next turn
+	bool oneBlock = (s->nPrevRows > 0 ? int64_t(s->lastOpen) : int64_t(C)) <= pxh::COLOR_SHORT_LIST;
+	int* list = s->colList.p;
+	int* out = s->colList2.p;
+	int listWord = pxh::STEP_OPEN, leftWord = pxh::STEP_LEFT;
+	int bound = C;   // host bound on the list length
+	const uint32_t* hostWords = s->hostCounts + kHostWordSlot;
+	while (C > 0)
 	{
-		compact();
-		const int batch = s->nPrevRows > 0 && rounds == 0 ? 8 : 48;
-		for (int k = 0; k < batch && rounds < kMaxRounds; k++, rounds++)
-			pxh::launch_color_round(bound, mDev, list, rounds, s->conA.p, s->conB.p, s->conKey.p, s->conColor.p,
-			                        s->best.p, s->mask.p, st);
-		compact();
-		pxh::launch_static_colors(n, C, s->conA.p, s->conB.p, s->conColor.p, s->bodyNext.p, st);
-		// row order: stable radix sort of (world, colour, index); the row
-		// starts of every (world, colour) come from the sorted keys
+		const int batch = std::min(s->nPrevRows > 0 && rounds == 0 ? 8 : 48, kMaxRounds - rounds);
+		pxh::launch_color_rounds(bound, s->stepWords.p + listWord, list, rounds, batch, n, s->conA.p, s->conB.p,
+		                         s->conKey.p, s->conColor.p, s->best.p, colors, out, s->stepWords.p + leftWord,
+		                         s->stepWords.p + pxh::STEP_RAN, oneBlock, st);
+		rounds += batch;
+		// row order: stable radix sort of (colour, index), colours staying below
+		// 64 + rounds + planes per world; for the per-world solve of (world,
+		// colour, index), the row starts of every (world, colour) from the keys
 		const int colorBound = 64 + rounds + s->maxPlanes + 1;
-		CB = colorBound + 1;
-		const uint64_t slots = uint64_t(nWorlds) * uint64_t(CB);
-		if (slots >= (1ull << 31))
-			return fail(PXH_ERR_CAPACITY, "pxh_scene_simulate: too many (world, colour) slots for the per-world solve");
-		PXH_CHECK(s->segStart.ensure(size_t(slots) + 2));
-		pxh::launch_color_keys_world(C, s->conColor.p, s->conA.p, s->scene.p, uint32_t(colorBound), s->keys.p,
-		                             s->vals.p, st);
-		bool alt = false;
-		pxh::launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, C, 0, bitsFor(slots - 1), s->hist.p, st,
-		                       alt);
+		uint64_t slots = uint64_t(colorBound) + 1;
+		if (worldSolve)
+		{
+			CB = colorBound + 1;
+			slots = uint64_t(nWorlds) * uint64_t(CB);
+			if (slots >= (1ull << 31))
+				return fail(PXH_ERR_CAPACITY,
+				            "pxh_scene_simulate: too many (world, colour) slots for the per-world solve");
+			PXH_CHECK(s->segStart.ensure(size_t(slots) + 2));
+		}
+		const int bits = bitsFor(slots - 1);
+		bool alt = pxh::radix_result_in_alt(C, bits);
+		uint32_t* va = alt ? s->vals.p : reinterpret_cast<uint32_t*>(s->order.p);
+		uint32_t* vb = alt ? reinterpret_cast<uint32_t*>(s->order.p) : s->vals2.p;
+		if (worldSolve)
+			pxh::launch_color_keys_world(C, s->conA.p, s->conB.p, s->conColor.p, colors, s->scene.p,
+			                             uint32_t(colorBound), s->keys.p, va, st);
+		else
+			pxh::launch_color_keys(C, s->conA.p, s->conB.p, s->conColor.p, colors, uint32_t(colorBound), s->keys.p, va,
+			                       st);
+		pxh::launch_radix_sort(s->keys.p, va, s->keys2.p, vb, C, 0, bits, s->hist.p, st, alt);
 		const uint64_t* ck = alt ? s->keys2.p : s->keys.p;
-		const uint32_t* cv = alt ? s->vals2.p : s->vals.p;
-		pxh::launch_row_start(C, ck, s->segStart.p, uint32_t(slots), st);
-		PXH_CHECK(hipMemcpyAsync(s->order.p, cv, sizeof(int) * C, hipMemcpyDeviceToDevice, st));
-		pxh::launch_fill_u32(s->solveQueue.p + 1, 1, 0u, st);
-		pxh::launch_max_color(C, s->conColor.p, s->solveQueue.p + 1, st);
-		PXH_CHECK(hipMemcpyAsync(s->hostCounts, mDev, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-		PXH_CHECK(hipMemcpyAsync(s->hostCounts + 1, s->solveQueue.p + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+		pxh::launch_row_start(C, ck, worldSolve ? s->segStart.p : s->hostCounts,
+		                      worldSolve ? uint32_t(slots) : uint32_t(colorBound), st, s->stepWords.p,
+		                      s->hostCounts + kHostWordSlot);
 		PXH_CHECK(hipStreamSynchronize(st));
-		remaining = int(s->hostCounts[0]);
+		s->lastOpen = hostWords[pxh::STEP_OPEN];
+		const int remaining = int(hostWords[leftWord]);
+		if (hostWords[pxh::STEP_RAN] == 0 && oneBlock && remaining > 0)
+		{
+			// the list was too long for one workgroup: nothing was coloured yet
+			oneBlock = false;
+			rounds -= batch;
+			continue;
+		}
 		if (remaining == 0)
 		{
-			nColors = int(s->hostCounts[1]) + 1;
+			if (worldSolve)
+				nColors = int(hostWords[pxh::STEP_TOP]) + 1;
+			else
+			{
+				colorStart.assign(s->hostCounts, s->hostCounts + colorBound + 1);
+				nColors = colorBound;
+				while (nColors > 0 && colorStart[nColors] == colorStart[nColors - 1])
+					nColors--;
+				colorStart.resize(size_t(nColors) + 1);
+			}
 			break;
 		}
 		if (rounds >= kMaxRounds)
 			return fail(PXH_ERR_CAPACITY, "pxh_scene_simulate: colouring did not finish in 960 rounds");
+		std::swap(list, out);
+		listWord = leftWord;
+		leftWord = leftWord == pxh::STEP_LEFT ? pxh::STEP_LEFT2 : pxh::STEP_LEFT;
 		bound = remaining;
 	}
 	if (worldSolve && C == 0)
@@ -1968,45 +1987,6 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		CB = 1;
 		PXH_CHECK(s->segStart.ensure(size_t(nWorlds) + 2));
 		pxh::launch_fill_u32(s->segStart.p, int64_t(nWorlds) + 1, 0u, st);
-	}
-	while (C > 0 && !worldSolve)
-	{
-		compact();
-		const int batch = s->nPrevRows > 0 && rounds == 0 ? 8 : 48;
-		for (int k = 0; k < batch && rounds < kMaxRounds; k++, rounds++)
-			pxh::launch_color_round(bound, mDev, list, rounds, s->conA.p, s->conB.p, s->conKey.p, s->conColor.p,
-			                        s->best.p, s->mask.p, st);
-		compact();
-		pxh::launch_static_colors(n, C, s->conA.p, s->conB.p, s->conColor.p, s->bodyNext.p, st);
-		// colour order: stable radix sort of (colour, index); colours stay below
-		// 64 + rounds + planes per world
-		const int colorBound = 64 + rounds + s->maxPlanes + 1;
-		PXH_CHECK(s->colorCount.ensure(size_t(colorBound) + 2));
-		pxh::launch_color_keys(C, s->conColor.p, uint32_t(colorBound), s->keys.p, s->vals.p, st);
-		bool alt = false;
-		pxh::launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, C, 0, bitsFor(uint64_t(colorBound)),
-		                       s->hist.p, st, alt);
-		const uint64_t* ck = alt ? s->keys2.p : s->keys.p;
-		const uint32_t* cv = alt ? s->vals2.p : s->vals.p;
-		pxh::launch_row_start(C, ck, s->colorCount.p, uint32_t(colorBound), st);
-		PXH_CHECK(hipMemcpyAsync(s->order.p, cv, sizeof(int) * C, hipMemcpyDeviceToDevice, st));
-		PXH_CHECK(hipMemcpyAsync(s->hostCounts, s->colorCount.p, sizeof(uint32_t) * (size_t(colorBound) + 1),
-		                         hipMemcpyDeviceToHost, st));
-		PXH_CHECK(hipMemcpyAsync(s->hostCounts + colorBound + 1, mDev, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-		PXH_CHECK(hipStreamSynchronize(st));
-		remaining = int(s->hostCounts[colorBound + 1]);
-		if (remaining == 0)
-		{
-			colorStart.assign(s->hostCounts, s->hostCounts + colorBound + 1);
-			nColors = colorBound;
-			while (nColors > 0 && colorStart[nColors] == colorStart[nColors - 1])
-				nColors--;
-			colorStart.resize(size_t(nColors) + 1);
-			break;
-		}
-		if (rounds >= kMaxRounds)
-			return fail(PXH_ERR_CAPACITY, "pxh_scene_simulate: colouring did not finish in 960 rounds");
-		bound = remaining;
 	}
 	s->statColors = nColors;
 	s->statRounds = rounds;
@@ -2049,8 +2029,9 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		                       1.0f / dt,
 		                       0.5f * biasCoefficient, d.tolerance_length, s->jHead.p, s->jRows.p,
 		                       sleeping ? s->slFlags.p : nullptr, st);
-	// four step counters, then four per-block partial sums of the preparation
-	PXH_CHECK(s->counters.ensure(4 + 4 * ((Cc + 255) / 256)));
+	// four partial sums per block of the preparation; their totals go to the host
+	PXH_CHECK(s->counters.ensure(4 * ((Cc + 255) / 256)));
+	unsigned long long* hostCounters = reinterpret_cast<unsigned long long*>(s->hostCounts + kHostCounterSlot);
 	// friction patches and colours of this step's rows go to the [cur] buffers
 	PXH_CHECK(s->patch[cur].ensure(6 * Cc));
 	PXH_CHECK(s->patchKey[cur].ensure(Cc));
@@ -2066,14 +2047,12 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		PXH_CHECK(s->rnU.ensure(4 * Cc));
 		pxh::launch_prep_pgs(C, s->order.p, s->conA.p, s->conB.p, s->conSlot.p, s->ctN.p, s->ctP.p, s->pos.p,
 		                     s->rot.p, sb, 1.0f / dt, d.static_friction, d.dynamic_friction, 2.0f * d.rest_offset,
-		                     d.friction_offset_threshold, rows, s->rnU.p, pio, s->counters.p, st);
+		                     d.friction_offset_threshold, rows, s->rnU.p, pio, s->counters.p, hostCounters, st);
 	}
 	else
 		pxh::launch_prep(C, s->order.p, s->conA.p, s->conB.p, s->conSlot.p, s->ctN.p, s->ctP.p, s->pos.p, s->rot.p,
 		                 sb, invStepDt, scale, 2.0f * d.rest_offset, d.friction_offset_threshold, rows, pio,
-		                 s->counters.p, st);
-	PXH_CHECK(hipMemcpyAsync(s->hostCounts + kHostCounterSlot, s->counters.p, 4 * sizeof(unsigned long long),
-	                         hipMemcpyDeviceToHost, st));
+		                 s->counters.p, hostCounters, st);
 	s->profEnd(pk);
 
 	// 7. solve. PGS (solveV_Blocks, lowleveldynamics/src/DySolverControl.cpp:163-380):
