@@ -2200,50 +2200,100 @@ PXH_D void prepBody(int o, int C, const int* order, const float4* ctN, const flo
 }
 
 // one colour: each lane solves one constraint (solveContact /
-// solveDynamicContactsStep, lowleveldynamics/src/DyTGSContactPrep.cpp:1490-1843).
-// All rows of the lane are loaded before any arithmetic so a wave keeps every
-// gather in flight at once; 64-lane blocks spread a colour over all CUs.
+// solveDynamicContactsStep, lowleveldynamics/src/DyTGSContactPrep.cpp:1490-1843);
+// 64-lane blocks spread a colour over all CUs. A short colour is bound by its
+// chain: arguments, row header, rows and bodies together, some 700 instructions
+// of one wave, stores. So all arguments come before anything depends on them,
+// and the rows' loads are issued ahead of the bodies': a colour of 4,400 rows
+// took 5.9 us with the bodies first and an early exit, and takes 4.7 (the step
+// of a 20,011-body bin 1.43 -> 1.22 ms; 262,144 bodies 3.60 -> 3.49).
 constexpr int SOLVE_THREADS = 64;
 constexpr int SOLVE_WORLD_THREADS = 64;
 
-// One TGS contact row o. Body velocity records are at vel[4 * (index -
-// bodyBase)] (bodyBase 0: the scene-wide array; a world's first body: that
-// world's records staged in LDS); the arithmetic is the same either way.
-__device__ __forceinline__ void solveContactRowTGS(int o, int C, const Rows& rows, float4* vel, int bodyBase,
-                                                   float minPen, float muS, float muD, float invStepDt,
-                                                   float biasScale, float scale, uint32_t* broken)
+// Body velocity records: the scene's array, or a world's records
+// in LDS, whose first body is `base`).
+struct VelPlain
 {
-	const int4 hi = rows.hI[o];
-	const float4 hf = rows.hF[o];
-	const int a = hi.x - bodyBase, b = hi.y < 0 ? hi.y : hi.y - bodyBase;
-	const int cnt = hi.z & 0xFF, nF = hi.z >> 8;
-	const bool dynB = hi.y >= 0;
-	// gathers: both bodies
-	const float4* va = vel + 4 * int64_t(a);
-	const float4 la4 = va[0], aa4 = va[1], dla4 = va[2], am04 = va[3];
-	float4 lb4 = make_float4(0, 0, 0, 0), ab4 = lb4, am14 = lb4, dlb4 = lb4;
-	if (dynB)
+	float4* v;
+	int base;
+	PXH_D void load(int body, float4 (&r)[4]) const
 	{
-		const float4* vb = vel + 4 * int64_t(b);
-		lb4 = vb[0]; ab4 = vb[1]; dlb4 = vb[2]; am14 = vb[3];
+		const float4* p = v + 4 * int64_t(body - base);
+		r[0] = p[0]; r[1] = p[1]; r[2] = p[2]; r[3] = p[3];
 	}
-	// rows
+	PXH_D void store(int body, float4 lin, float4 ang) const
+	{
+		float4* p = v + 4 * int64_t(body - base);
+		p[0] = lin;
+		p[1] = ang;
+	}
+	// the substeps' summed linear and angular motion
+	PXH_D void storeMoved(int body, float4 lin, float4 ang) const
+	{
+		float4* p = v + 4 * int64_t(body - base);
+		p[2] = lin;
+		p[3] = ang;
+	}
+};
+
+// with the bodies' turn over the substeps, which the joint rows read
+struct VelTurn : VelPlain
+{
+	const float4* dq;
+	PXH_D float4 turn(int body) const { return dq[body]; }
+};
+
+// one TGS contact row's data but for its bodies
+struct TgsRow
+{
+	int4 hi;
+	float4 hf;
 	float4 nA[4], nB[4], fT[4], fA[4], fB[4];
 	float nFc[4], fFc[4];
+};
+PXH_D void loadTgsRow(int o, int C, const Rows& rows, TgsRow& r)
+{
+	r.hi = rows.hI[o];
+	r.hf = rows.hF[o];
+	const int cnt = r.hi.z & 0xFF, nF = r.hi.z >> 8;
+	const bool dynB = r.hi.y >= 0;
 #pragma unroll
 	for (int k = 0; k < 4; k++)
 	{
 		const int64_t ri = k * int64_t(C) + o;
 		if (k < cnt)
 		{
-			nA[k] = rows.nA[ri]; nB[k] = rows.nB[ri]; nFc[k] = rows.nF[ri];
+			r.nA[k] = rows.nA[ri]; r.nB[k] = rows.nB[ri]; r.nFc[k] = rows.nF[ri];
 		}
 		if (k < nF)
 		{
-			fT[k] = rows.fT[ri]; fA[k] = rows.fA[ri]; fFc[k] = rows.fF[ri];
-			fB[k] = dynB ? rows.fB[ri] : make_float4(0, 0, 0, 0);
+			r.fT[k] = rows.fT[ri]; r.fA[k] = rows.fA[ri]; r.fFc[k] = rows.fF[ri];
+			r.fB[k] = dynB ? rows.fB[ri] : make_float4(0, 0, 0, 0);
 		}
 	}
+}
+
+// One TGS contact row o; the arithmetic is the same wherever the velocity
+// records are.
+template <class Vel>
+__device__ __forceinline__ void solveTgsRow(int o, int C, const Rows& rows, TgsRow& row, const Vel& vel, float minPen,
+                                            float muS, float muD, float invStepDt, float biasScale, float scale,
+                                            uint32_t* broken)
+{
+	const int4 hi = row.hi;
+	const float4 hf = row.hf;
+	const int cnt = hi.z & 0xFF, nF = hi.z >> 8;
+	const bool dynB = hi.y >= 0;
+	float4 va[4], vb[4];
+	vel.load(hi.x, va);
+	if (dynB)
+		vel.load(hi.y, vb);
+	else
+		vb[0] = vb[1] = vb[2] = vb[3] = make_float4(0, 0, 0, 0);
+	const float4 la4 = va[0], aa4 = va[1], dla4 = va[2], am04 = va[3];
+	const float4 lb4 = vb[0], ab4 = vb[1], dlb4 = vb[2], am14 = vb[3];
+	const float4(&nA)[4] = row.nA, (&nB)[4] = row.nB, (&fT)[4] = row.fT, (&fA)[4] = row.fA, (&fB)[4] = row.fB;
+	float(&nFc)[4] = row.nFc, (&fFc)[4] = row.fFc;
 	const f3 n = mk(hf);
 	const float invMassA = la4.w, invMassB = lb4.w;
 	f3 l0 = mk(la4), a0 = mk(aa4), l1 = mk(lb4), a1 = mk(ab4);
@@ -2333,23 +2383,34 @@ __device__ __forceinline__ void solveContactRowTGS(int o, int C, const Rows& row
 		if (k < nF)
 			rows.fF[ri] = fFc[k];
 	}
-	vel[4 * int64_t(a)] = f4(l0, invMassA);
-	vel[4 * int64_t(a) + 1] = f4(a0, 0.0f);
+	vel.store(hi.x, f4(l0, invMassA), f4(a0, 0.0f));
 	if (dynB)
-	{
-		vel[4 * int64_t(b)] = f4(l1, invMassB);
-		vel[4 * int64_t(b) + 1] = f4(a1, 0.0f);
-	}
+		vel.store(hi.y, f4(l1, invMassB), f4(a1, 0.0f));
+}
+
+template <class Vel>
+__device__ __forceinline__ void solveContactRowTGS(int o, int C, const Rows& rows, const Vel& vel, float minPen,
+                                                   float muS, float muD, float invStepDt, float biasScale,
+                                                   float scale, uint32_t* broken)
+{
+	TgsRow row;
+	loadTgsRow(o, C, rows, row);
+	solveTgsRow(o, C, rows, row, vel, minPen, muS, muD, invStepDt, biasScale, scale, broken);
 }
 
 __global__ void __launch_bounds__(SOLVE_THREADS) k_solve(int begin, int end, int C, Rows rows, float4* vel,
                                                           float minPen, float muS, float muD, float invStepDt,
                                                           float biasScale, float scale, uint32_t* broken)
 {
-	const int o = begin + blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= end)
+	// lanes past the colour's end load its last row and leave after the loads, so
+	// the kernel's arguments come in one scalar load before the first row's
+	const int own = begin + blockIdx.x * SOLVE_THREADS + threadIdx.x;
+	const int o = min(own, end - 1);
+	TgsRow row;
+	loadTgsRow(o, C, rows, row);
+	if (own >= end)
 		return;
-	solveContactRowTGS(o, C, rows, vel, 0, minPen, muS, muD, invStepDt, biasScale, scale, broken);
+	solveTgsRow(o, C, rows, row, VelPlain{vel, 0}, minPen, muS, muD, invStepDt, biasScale, scale, broken);
 }
 
 // ---------------------------------------------------------------------------
@@ -2485,42 +2546,53 @@ __global__ void k_prep_pgs(int C, const int* order, const float4* ctN, const flo
 // velocity changes in vel[4i], vel[4i+1]. velocityPass: rows concluded after the
 // last position pass use their unbiased error and friction without bias
 // (concludeContact, DySolverConstraints.cpp:508-549).
-__global__ void __launch_bounds__(SOLVE_THREADS) k_solve_pgs(int begin, int end, int C, Rows rows,
-                                                              const float* rowsU, float4* vel, int doFriction,
-                                                              int velocityPass, uint32_t* broken)
+struct PgsRow
 {
-	const int o = begin + blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= end)
-		return;
-	const int4 hi = rows.hI[o];
-	const float4 hf = rows.hF[o];
-	const int a = hi.x, b = hi.y;
-	const int cnt = hi.z & 0xFF, nF = doFriction ? hi.z >> 8 : 0;
-	const bool dynB = b >= 0;
-	const float4* va = vel + 4 * int64_t(a);
-	const float4 la4 = va[0], aa4 = va[1];
-	float4 lb4 = make_float4(0, 0, 0, 0), ab4 = lb4;
-	if (dynB)
-	{
-		const float4* vb = vel + 4 * int64_t(b);
-		lb4 = vb[0]; ab4 = vb[1];
-	}
+	int4 hi;
+	float4 hf;
 	float4 nA[4], nB[4], fT[4], fA[4], fB[4];
 	float nFc[4], fFc[4], err[4];
+};
+PXH_D void loadPgsRow(int o, int C, const Rows& rows, const float* rowsU, bool doFriction, bool velocityPass, PgsRow& r)
+{
+	r.hi = rows.hI[o];
+	r.hf = rows.hF[o];
+	const int cnt = r.hi.z & 0xFF, nF = doFriction ? r.hi.z >> 8 : 0;
 #pragma unroll
 	for (int k = 0; k < 4; k++)
 	{
 		const int64_t ri = k * int64_t(C) + o;
 		if (k < cnt)
 		{
-			nA[k] = rows.nA[ri]; nB[k] = rows.nB[ri]; nFc[k] = rows.nF[ri];
-			err[k] = velocityPass ? rowsU[ri] : nA[k].w;
+			r.nA[k] = rows.nA[ri]; r.nB[k] = rows.nB[ri]; r.nFc[k] = rows.nF[ri];
+			r.err[k] = velocityPass ? rowsU[ri] : r.nA[k].w;
 		}
 		if (k < nF)
 		{
-			fT[k] = rows.fT[ri]; fA[k] = rows.fA[ri]; fB[k] = rows.fB[ri]; fFc[k] = rows.fF[ri];
+			r.fT[k] = rows.fT[ri]; r.fA[k] = rows.fA[ri]; r.fB[k] = rows.fB[ri]; r.fFc[k] = rows.fF[ri];
 		}
 	}
+}
+
+// (only the first half of a record is used: the compiler drops the other loads)
+template <class Vel>
+__device__ __forceinline__ void solvePgsRow(int o, int C, const Rows& rows, PgsRow& row, const Vel& vel,
+                                            bool doFriction, bool velocityPass, uint32_t* broken)
+{
+	const int4 hi = row.hi;
+	const float4 hf = row.hf;
+	const int cnt = hi.z & 0xFF, nF = doFriction ? hi.z >> 8 : 0;
+	const bool dynB = hi.y >= 0;
+	float4 va[4], vb[4];
+	vel.load(hi.x, va);
+	if (dynB)
+		vel.load(hi.y, vb);
+	else
+		vb[0] = vb[1] = make_float4(0, 0, 0, 0);
+	const float4 la4 = va[0], aa4 = va[1], lb4 = vb[0], ab4 = vb[1];
+	const float4(&nA)[4] = row.nA, (&nB)[4] = row.nB, (&fT)[4] = row.fT, (&fA)[4] = row.fA, (&fB)[4] = row.fB;
+	float(&nFc)[4] = row.nFc, (&fFc)[4] = row.fFc;
+	const float(&err)[4] = row.err;
 	const f3 n = mk(hf);
 	const float invMassA = la4.w, invMassB = lb4.w;
 	f3 l0 = mk(la4), a0 = mk(aa4), l1 = mk(lb4), a1 = mk(ab4);
@@ -2588,13 +2660,22 @@ __global__ void __launch_bounds__(SOLVE_THREADS) k_solve_pgs(int begin, int end,
 		if (k < nF)
 			rows.fF[ri] = fFc[k];
 	}
-	vel[4 * int64_t(a)] = f4(l0, invMassA);
-	vel[4 * int64_t(a) + 1] = f4(a0, 0.0f);
+	vel.store(hi.x, f4(l0, invMassA), f4(a0, 0.0f));
 	if (dynB)
-	{
-		vel[4 * int64_t(b)] = f4(l1, invMassB);
-		vel[4 * int64_t(b) + 1] = f4(a1, 0.0f);
-	}
+		vel.store(hi.y, f4(l1, invMassB), f4(a1, 0.0f));
+}
+
+__global__ void __launch_bounds__(SOLVE_THREADS) k_solve_pgs(int begin, int end, int C, Rows rows,
+                                                              const float* rowsU, float4* vel, int doFriction,
+                                                              int velocityPass, uint32_t* broken)
+{
+	const int own = begin + blockIdx.x * SOLVE_THREADS + threadIdx.x;
+	const int o = min(own, end - 1);
+	PgsRow row;
+	loadPgsRow(o, C, rows, rowsU, doFriction != 0, velocityPass != 0, row);
+	if (own >= end)
+		return;
+	solvePgsRow(o, C, rows, row, VelPlain{vel, 0}, doFriction != 0, velocityPass != 0, broken);
 }
 
 // velocity changes after the position passes move the bodies (saveMotionVelocities,
@@ -2700,10 +2781,13 @@ __global__ void k_pgs_finalize(int n, float dt, float4* pos, float4* rot, float4
 }
 
 // integrateCoreStep (lowleveldynamics/src/DyTGSDynamics.cpp:1403-1476) of
-// body i whose velocity record is at v (scene-wide array or LDS)
-__device__ __forceinline__ void integrateBodyTGS(int i, float dt, float4* v, float4* svP, float4* svDQ,
+// body i
+template <class Vel>
+__device__ __forceinline__ void integrateBodyTGS(int i, float dt, const Vel& vel, float4* svP, float4* svDQ,
                                                  const float4* svI0, const float4* svI1)
 {
+	float4 v[4];
+	vel.load(i, v);
 	const f3 lv = mk(v[0]);
 	const f3 av = mk(v[1]);
 	const f3 delta = lv * dt;
@@ -2724,8 +2808,7 @@ __device__ __forceinline__ void integrateBodyTGS(int i, float dt, float4* v, flo
 		res.x += dq.x * q; res.y += dq.y * q; res.z += dq.z * q; res.w += dq.w * q;
 		svDQ[i] = f4(qnormalize(res));
 	}
-	v[3] = f4(mk(v[3]) + av * dt, 0.0f);
-	v[2] = f4(mk(v[2]) + delta, 0.0f);
+	vel.storeMoved(i, f4(mk(v[2]) + delta, 0.0f), f4(mk(v[3]) + av * dt, 0.0f));
 }
 
 __global__ void k_integrate(int n, float dt, float4* vel, float4* svP, float4* svDQ, const float4* svI0,
@@ -2734,7 +2817,7 @@ __global__ void k_integrate(int n, float dt, float4* vel, float4* svP, float4* s
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= n)
 		return;
-	integrateBodyTGS(i, dt, vel + 4 * int64_t(i), svP, svDQ, svI0, svI1);
+	integrateBodyTGS(i, dt, VelPlain{vel, 0}, svP, svDQ, svI0, svI1);
 }
 
 // The whole TGS iteration loop of independent worlds (the batched form).
@@ -2793,13 +2876,13 @@ __global__ void __launch_bounds__(SOLVE_WORLD_THREADS) k_solve_worlds(
 				if (e == s)
 					continue;
 				for (uint32_t o = s + tid; o < e; o += SOLVE_WORLD_THREADS)
-					solveContactRowTGS(int(o), C, rows, V, b0, minPen, muS, muD, invStepDt, biasScale, scale, brk);
+					solveContactRowTGS(int(o), C, rows, VelPlain{V, b0}, minPen, muS, muD, invStepDt, biasScale, scale, brk);
 				__syncthreads();
 			}
 			if (posIter)
 			{
 				for (int i = tid; i < nb; i += SOLVE_WORLD_THREADS)
-					integrateBodyTGS(b0 + i, stepDt, V + 4 * int64_t(i), svP, svDQ, svI0, svI1);
+					integrateBodyTGS(b0 + i, stepDt, VelPlain{V, b0}, svP, svDQ, svI0, svI1);
 				__syncthreads();
 			}
 		}
@@ -3269,13 +3352,11 @@ __global__ void k_joint_prep(int J, const int4* info, const float4* frame, const
 	          erp, lengthScale, head + JOINT_HEAD * int64_t(j), rows + JOINT_ROWS * int64_t(j));
 }
 
-__global__ void k_joint_solve(int begin, int end, const int4* info, const float4* head, float4* rows, float4* vel,
-                              const float4* svDQ, const float4* svI0, const float4* svI1, float elapsed, int conclude,
-                              const uint32_t* sleepFlags)
+template <class Vel>
+__device__ __forceinline__ void solveJointOf(int j, const int4* info, const float4* head, float4* rows, const Vel& vel,
+                                             const float4* svI0, const float4* svI1, float elapsed, bool conclude,
+                                             const uint32_t* sleepFlags)
 {
-	const int j = begin + blockIdx.x * blockDim.x + threadIdx.x;
-	if (j >= end)
-		return;
 	const int4 ji = info[j];
 	if (jointAsleep(ji, sleepFlags))
 		return;
@@ -3285,35 +3366,39 @@ __global__ void k_joint_solve(int begin, int end, const int4* info, const float4
 	q0.x = q0.y = q0.z = 0.0f; q0.w = 1.0f;
 	q1 = q0;
 	float w0 = 0.0f, w1 = 0.0f;
+	float4 v[4];
 	if (a >= 0)
 	{
-		const float4* v = vel + 4 * int64_t(a);
-		const float4 v0 = v[0];
-		l0 = mk(v0); w0 = v0.w; a0 = mk(v[1]); dl0 = mk(v[2]); da0 = mk(v[3]);
-		q0 = mkq(svDQ[a]);
+		vel.load(a, v);
+		l0 = mk(v[0]); w0 = v[0].w; a0 = mk(v[1]); dl0 = mk(v[2]); da0 = mk(v[3]);
+		q0 = mkq(vel.turn(a));
 	}
 	if (b >= 0)
 	{
-		const float4* v = vel + 4 * int64_t(b);
-		const float4 v0 = v[0];
-		l1 = mk(v0); w1 = v0.w; a1 = mk(v[1]); dl1 = mk(v[2]); da1 = mk(v[3]);
-		q1 = mkq(svDQ[b]);
+		vel.load(b, v);
+		l1 = mk(v[0]); w1 = v[0].w; a1 = mk(v[1]); dl1 = mk(v[2]); da1 = mk(v[3]);
+		q1 = mkq(vel.turn(b));
 	}
 	const m33 sI0 = bodySqrtInvI(a, svI0, svI1), sI1 = bodySqrtInvI(b, svI0, svI1);
 	const float4* h = head + JOINT_HEAD * int64_t(j);
 	solveJoint(__float_as_int(h[8].x), h, rows + JOINT_ROWS * int64_t(j), l0, a0, dl0, da0,
-	           q0, sI0, l1, a1, dl1, da1, q1, sI1, elapsed, conclude != 0);
+	           q0, sI0, l1, a1, dl1, da1, q1, sI1, elapsed, conclude);
 	if (a >= 0)
-	{
-		vel[4 * int64_t(a)] = f4(l0, w0);
-		vel[4 * int64_t(a) + 1] = f4(a0, 0.0f);
-	}
+		vel.store(a, f4(l0, w0), f4(a0, 0.0f));
 	if (b >= 0)
-	{
-		vel[4 * int64_t(b)] = f4(l1, w1);
-		vel[4 * int64_t(b) + 1] = f4(a1, 0.0f);
-	}
+		vel.store(b, f4(l1, w1), f4(a1, 0.0f));
 }
+
+__global__ void k_joint_solve(int begin, int end, const int4* info, const float4* head, float4* rows, float4* vel,
+                              const float4* svDQ, const float4* svI0, const float4* svI1, float elapsed, int conclude,
+                              const uint32_t* sleepFlags)
+{
+	const int j = begin + blockIdx.x * blockDim.x + threadIdx.x;
+	if (j >= end)
+		return;
+	solveJointOf(j, info, head, rows, VelTurn{{vel, 0}, svDQ}, svI0, svI1, elapsed, conclude != 0, sleepFlags);
+}
+
 
 // copyBackBodies (lowleveldynamics/src/DyTGSDynamics.cpp:1549-1580), with
 // the sleep check on the step's mean velocities (DyTGSDynamics.cpp:1561, 1577)
