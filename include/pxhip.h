@@ -296,13 +296,14 @@ int32_t pxh_scene_copy_contact_data(pxh_scene scene, void* data, uint32_t* nb_pa
 
 /* Launch shapes of the step. No counterpart in the reference, whose GPU
  * kernels have fixed shapes; results are the same bit for bit under every
- * setting. tuning[0] the TGS solve layout: PXH_SOLVE_LAYOUT_AUTO (the
+ * setting. tuning[0] the solve layout: PXH_SOLVE_LAYOUT_AUTO (the
  * per-world solve when every world has at most PXH_WORLD_SOLVE_MAX_BODIES
  * bodies, else one launch per colour and iteration), _COLORS or _WORLDS (one
  * persistent launch of every iteration of every world, each world in one
- * workgroup); tuning[1] workgroups of the per-world solve (0 = 4 per compute
- * unit); tuning[2] bodies per world whose velocity records the per-world
- * solve keeps in LDS (at most 1000, 64 B each; larger worlds work in HBM);
+ * workgroup); tuning[1] workgroups of the per-world solve (0 = as many as run
+ * at a time); tuning[2] bodies per world whose velocities the per-world solve
+ * keeps in LDS when the layout is _WORLDS (at most 1000, 32 B each; larger
+ * worlds work in HBM; layout auto keeps every world's);
  * tuning[3] autotuning: when positive, the next steps try every candidate
  * shape of the solve (the colour launches; where every world fits one
  * workgroup, the per-world solve at 8, 4, 2 and 1 workgroups per compute unit

@@ -246,15 +246,27 @@ void launch_solve(int begin, int end, int C, Rows rows, SolverBodies sb, float m
 // rows in (world, colour) order for the per-world solve
 void launch_color_keys_world(int C, const int* conA, const int* conB, int* conColor, ColorState cs,
                              const int* bodyWorld, uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st);
-int solve_world_threads();
-// every TGS iteration of every world in one launch of `grid` persistent
-// workgroups; queueHead: one device counter (zeroed by the launch);
-// segStart: nWorlds * CB + 1 row starts of (world, colour); worlds of at most
-// ldsBodies bodies keep their velocity records in LDS
-void launch_solve_worlds(int grid, int nWorlds, const int* worldOrder, uint32_t* queueHead, const int* bodyStart,
-                         const uint32_t* segStart, int CB, int C, Rows rows, SolverBodies sb, int posIters,
-                         int velIters, float stepDt, float muS, float muD, float invStepDt, float biasScale,
-                         float scale, uint32_t* broken, int ldsBodies, hipStream_t st, hipEvent_t evStart = nullptr,
+// every iteration of every world in one launch of `workgroups` persistent
+// workgroups (0: as many as run at a time), TGS or, with rowsU, PGS passes;
+// queueHead: one device counter (zeroed by the launch); segStart: nWorlds * CB + 1
+// row starts of (world, colour); worlds of at most ldsBodies bodies (at most
+// WORLD_LDS_BODIES) keep their velocities in LDS
+constexpr int WORLD_LDS_BODIES = 1024;
+struct WorldJoints
+{
+	int colors;          // joint colours (0: no joints)
+	const int* seg;      // per world, colors + 1 starts in order
+	const int* order;    // joints by (world, colour)
+	const int4* info;
+	const float4* head;
+	float4* rows;
+	const uint32_t* sleepFlags;
+};
+void launch_solve_worlds(int workgroups, int nWorlds, int maxWorldBodies, const int* worldOrder, uint32_t* queueHead,
+                         const int* bodyStart, const uint32_t* segStart, int CB, int C, Rows rows, const float* rowsU,
+                         SolverBodies sb, int posIters, int iters, float stepDt, float muS, float muD,
+                         float invStepDt, float biasScale, float scale, uint32_t* broken, int ldsBodies,
+                         const WorldJoints& joints, hipStream_t st, hipEvent_t evStart = nullptr,
                          hipEvent_t evStop = nullptr);
 // PGS: rows with the unbiased normal errors in rowsU; position passes
 // (velocityPass false) then velocity passes; SolverBodies p/dq hold the motion

@@ -2208,7 +2208,6 @@ PXH_D void prepBody(int o, int C, const int* order, const float4* ctN, const flo
 // took 5.9 us with the bodies first and an early exit, and takes 4.7 (the step
 // of a 20,011-body bin 1.43 -> 1.22 ms; 262,144 bodies 3.60 -> 3.49).
 constexpr int SOLVE_THREADS = 64;
-constexpr int SOLVE_WORLD_THREADS = 64;
 
 // Body velocity records: the scene's array, or a world's records
 // in LDS, whose first body is `base`).
@@ -2820,79 +2819,6 @@ __global__ void k_integrate(int n, float dt, float4* vel, float4* svP, float4* s
 	integrateBodyTGS(i, dt, VelPlain{vel, 0}, svP, svDQ, svI0, svI1);
 }
 
-// The whole TGS iteration loop of independent worlds (the batched form).
-// Persistent workgroups take worlds from a queue ordered by size (largest
-// first); a workgroup stages its world's velocity records in LDS (worlds of
-// at most ldsBodies bodies; larger ones work on the scene-wide array), then
-// for every position and velocity iteration solves the world's colours in
-// order, one barrier between colours, and after each position iteration
-// integrates the world's bodies, as the per-colour launches and k_integrate
-// do for all worlds at once. Rows are ordered by (world, colour):
-// segStart[w * CB + c] is the first row of colour c of world w. Every wave
-// leaves once the queue is empty. Same arithmetic in the same order as the
-// per-colour path (cf. solveWholeIslandTGS, gpusolver/src/CUDA/
-// solverMultiBlockTGS.cu:1686, which runs a small island in one block).
-__global__ void __launch_bounds__(SOLVE_WORLD_THREADS) k_solve_worlds(
-    int nWorlds, const int* worldOrder, uint32_t* queueHead, const int* bodyStart, const uint32_t* segStart, int CB,
-    int C, Rows rows, float4* vel, float4* svP, float4* svDQ, const float4* svI0, const float4* svI1, int posIters,
-    int velIters, float stepDt, float muS, float muD, float invStepDt, float biasScale, float scale, uint32_t* broken,
-    int ldsBodies)
-{
-	extern __shared__ float4 lds[];
-	__shared__ int sWorld;
-	const int tid = threadIdx.x;
-	for (;;)
-	{
-		if (tid == 0)
-		{
-			const uint32_t q = atomicAdd(queueHead, 1u);
-			sWorld = q < uint32_t(nWorlds) ? worldOrder[q] : -1;
-		}
-		__syncthreads();
-		const int w = sWorld;
-		__syncthreads();
-		if (w < 0)
-			return;
-		const int b0 = bodyStart[w], nb = bodyStart[w + 1] - b0;
-		const bool inLds = nb <= ldsBodies;
-		float4* V = inLds ? lds : vel + 4 * int64_t(b0);
-		if (inLds)
-			for (int i = tid; i < 4 * nb; i += SOLVE_WORLD_THREADS)
-				lds[i] = vel[4 * int64_t(b0) + i];
-		__syncthreads();
-		const uint32_t* seg = segStart + int64_t(w) * CB;
-		const uint32_t wEnd = seg[CB];
-		for (int it = 0; it < posIters + velIters; it++)
-		{
-			const bool posIter = it < posIters;
-			const float minPen = posIter ? -3.402823466e+38f : 0.0f;
-			uint32_t* brk = it == posIters + velIters - 1 ? broken : nullptr;
-			for (int c = 0; c < CB; c++)
-			{
-				const uint32_t s = seg[c];
-				if (s >= wEnd)
-					break;
-				const uint32_t e = seg[c + 1];
-				if (e == s)
-					continue;
-				for (uint32_t o = s + tid; o < e; o += SOLVE_WORLD_THREADS)
-					solveContactRowTGS(int(o), C, rows, VelPlain{V, b0}, minPen, muS, muD, invStepDt, biasScale, scale, brk);
-				__syncthreads();
-			}
-			if (posIter)
-			{
-				for (int i = tid; i < nb; i += SOLVE_WORLD_THREADS)
-					integrateBodyTGS(b0 + i, stepDt, VelPlain{V, b0}, svP, svDQ, svI0, svI1);
-				__syncthreads();
-			}
-		}
-		if (inLds)
-			for (int i = tid; i < 4 * nb; i += SOLVE_WORLD_THREADS)
-				vel[4 * int64_t(b0) + i] = lds[i];
-		__syncthreads();
-	}
-}
-
 // ---------------------------------------------------------------------------
 // joints (pxh_joint.h)
 // ---------------------------------------------------------------------------
@@ -3397,6 +3323,179 @@ __global__ void k_joint_solve(int begin, int end, const int4* info, const float4
 	if (j >= end)
 		return;
 	solveJointOf(j, info, head, rows, VelTurn{{vel, 0}, svDQ}, svI0, svI1, elapsed, conclude != 0, sleepFlags);
+}
+
+// A world's velocities in LDS, 32 bytes a body; the substeps' summed motion,
+// which only the integration writes, stays in the scene's array. Half the LDS of
+// whole records, so twice the worlds run at a time.
+struct VelWorld
+{
+	float4* lds;
+	float4* v;
+	const float4* dq;
+	int base;
+	PXH_D void load(int body, float4 (&r)[4]) const
+	{
+		const float4* p = lds + 2 * (body - base);
+		const float4* g = v + 4 * int64_t(body);
+		r[2] = g[2]; r[3] = g[3];
+		r[0] = p[0]; r[1] = p[1];
+	}
+	PXH_D void store(int body, float4 lin, float4 ang) const
+	{
+		float4* p = lds + 2 * (body - base);
+		p[0] = lin;
+		p[1] = ang;
+	}
+	PXH_D void storeMoved(int body, float4 lin, float4 ang) const
+	{
+		v[4 * int64_t(body) + 2] = lin;
+		v[4 * int64_t(body) + 3] = ang;
+	}
+	PXH_D float4 turn(int body) const { return dq[body]; }
+};
+
+// Every iteration of independent worlds (the batched form and small scenes).
+// Persistent workgroups take worlds from a queue
+// ordered by size (largest first); a workgroup keeps its world's velocities in
+// LDS (worlds of at most ldsBodies bodies; larger ones work on the scene's
+// array), then for every iteration solves the world's joints by colour and its
+// contacts by colour in order, one barrier between colours, and moves the bodies
+// (TGS) or keeps their motion (PGS), as the launches for all worlds at once do.
+// Rows are ordered by (world, colour): segStart[w * CB + c] is the first row of
+// colour c of world w. Every wave leaves once the queue is empty. Same
+// arithmetic in the same order as the per-colour path (cf. solveWholeIslandTGS,
+// gpusolver/src/CUDA/solverMultiBlockTGS.cu:1686, which runs a small island in
+// one block).
+//
+// Bound by the chain of colours: a row's data streams past while its bodies stay
+// in LDS, so the next colour's rows are loaded before the barrier (a thread
+// takes the same rows in every iteration, and their impulses are its own), and
+// the non-empty colours' starts are listed in LDS once. The prefetch holds about
+// 240 registers, two waves a SIMD; held to three it spills and takes 1,400 us
+// where this takes 770 (8,192 worlds; 957 without the prefetch at three). 301
+// worlds: 179 us against 247.
+template <int THREADS, bool PGS, bool JOINTS>
+__global__ void __launch_bounds__(THREADS, 2) k_solve_worlds(int nWorlds, const int* worldOrder, uint32_t* queueHead,
+                                                          const int* bodyStart, const uint32_t* segStart, int CB, int C,
+                                                          Rows rows, const float* rowsU, SolverBodies sb, int posIters,
+                                                          int iters, float stepDt, float muS, float muD,
+                                                          float invStepDt, float biasScale, float scale,
+                                                          uint32_t* broken, int ldsBodies, WorldJoints J)
+{
+	extern __shared__ float4 lds[];
+	uint32_t* list = reinterpret_cast<uint32_t*>(lds + 2 * ldsBodies);   // CB + 1
+	__shared__ int sWorld, sColors;
+	const int tid = threadIdx.x;
+	for (;;)
+	{
+		if (tid == 0)
+		{
+			const uint32_t q = atomicAdd(queueHead, 1u);
+			sWorld = q < uint32_t(nWorlds) ? worldOrder[q] : -1;
+		}
+		__syncthreads();
+		const int w = sWorld;
+		if (w < 0)
+			return;
+		const int b0 = bodyStart[w], nb = bodyStart[w + 1] - b0;
+		const bool inLds = nb <= ldsBodies;
+		if (inLds)
+			for (int i = tid; i < 2 * nb; i += THREADS)
+				lds[i] = sb.vel[4 * int64_t(b0 + (i >> 1)) + (i & 1)];
+		if (tid < 64)
+		{
+			const uint32_t* seg = segStart + int64_t(w) * CB;
+			int k = 0;
+			for (int c = tid; c - tid < CB; c += 64)
+			{
+				const uint32_t s = c < CB ? seg[c] : 0u, e = c < CB ? seg[c + 1] : 0u;
+				const uint64_t m = __ballot(s < e);
+				if (s < e)
+					list[k + __popcll(m & ((1ull << tid) - 1ull))] = s;
+				k += __popcll(m);
+			}
+			if (tid == 0)
+			{
+				list[k] = seg[CB];
+				sColors = k;
+			}
+		}
+		__syncthreads();
+		const int colors = sColors;
+		auto solve = [&](const auto& vel) {
+			typename std::conditional<PGS, PgsRow, TgsRow>::type row;
+			auto load = [&](int o, int it) {
+				if constexpr (PGS)
+					loadPgsRow(o, C, rows, rowsU, it >= posIters || posIters - it <= 3, it >= posIters, row);
+				else
+					loadTgsRow(o, C, rows, row);
+			};
+			if (colors > 0 && list[0] + tid < list[1])
+				load(int(list[0]) + tid, 0);
+			for (int it = 0; it < iters; it++)
+			{
+				const bool posIter = it < posIters;
+				uint32_t* brk = it == iters - 1 ? broken : nullptr;
+				if constexpr (JOINTS)
+					for (int c = 0; c < J.colors; c++)
+					{
+						const int* jseg = J.seg + int64_t(w) * (J.colors + 1);
+						const float elapsed = stepDt * float(min(it, posIters));
+						for (int k = jseg[c] + tid; k < jseg[c + 1]; k += THREADS)
+							solveJointOf(J.order[k], J.info, J.head, J.rows, vel, sb.i0, sb.i1, elapsed, it == posIters - 1,
+							             J.sleepFlags);
+						__syncthreads();
+					}
+				for (int c = 0; c < colors; c++)
+				{
+					const int e = int(list[c + 1]);
+					for (int o = int(list[c]) + tid; o < e;)
+					{
+						if constexpr (PGS)
+							solvePgsRow(o, C, rows, row, vel, !posIter || posIters - it <= 3, !posIter, brk);
+						else
+							solveTgsRow(o, C, rows, row, vel, posIter ? -3.402823466e+38f : 0.0f, muS, muD, invStepDt,
+							            biasScale, scale, brk);
+						o += THREADS;
+						if (o < e)
+							load(o, it);
+					}
+					const int nc = c + 1 < colors ? c + 1 : 0;
+					if (list[nc] + tid < list[nc + 1])
+						load(int(list[nc]) + tid, nc ? it : it + 1);
+					__syncthreads();
+				}
+				if constexpr (PGS)
+				{
+					if (it == posIters - 1)
+						for (int i = b0 + tid; i < b0 + nb; i += THREADS)
+						{
+							float4 v[4];
+							vel.load(i, v);
+							sb.p[i] = v[0];
+							sb.dq[i] = v[1];
+						}
+				}
+				else if (posIter)
+				{
+					for (int i = b0 + tid; i < b0 + nb; i += THREADS)
+						integrateBodyTGS(i, stepDt, vel, sb.p, sb.dq, sb.i0, sb.i1);
+					__syncthreads();
+				}
+			}
+		};
+		if (inLds)
+		{
+			solve(VelWorld{lds, sb.vel, sb.dq, b0});
+			__syncthreads();
+			for (int i = tid; i < 2 * nb; i += THREADS)
+				sb.vel[4 * int64_t(b0 + (i >> 1)) + (i & 1)] = lds[i];
+		}
+		else
+			solve(VelTurn{{sb.vel, 0}, sb.dq});
+		__syncthreads();
+	}
 }
 
 
@@ -4013,33 +4112,69 @@ void launch_color_keys_world(int C, const int* conA, const int* conB, int* conCo
 {
 	PXH_LAUNCH(k_color_keys_world, C, C, conA, conB, conColor, cs, bodyWorld, limit, keys, vals);
 }
-int solve_world_threads() { return SOLVE_WORLD_THREADS; }
 void launch_fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t st)
 {
 	PXH_LAUNCH(k_fill_u32, n, p, n, v);
 }
-void launch_solve_worlds(int grid, int nWorlds, const int* worldOrder, uint32_t* queueHead, const int* bodyStart,
-                         const uint32_t* segStart, int CB, int C, Rows rows, SolverBodies sb, int posIters,
-                         int velIters, float stepDt, float muS, float muD, float invStepDt, float biasScale,
-                         float scale, uint32_t* broken, int ldsBodies, hipStream_t st, hipEvent_t evStart,
-                         hipEvent_t evStop)
+template <int THREADS, bool PGS, bool JOINTS>
+static void solveWorlds(int grid, size_t shm, uint32_t* queueHead, hipStream_t st, hipEvent_t evStart,
+                        hipEvent_t evStop, int nWorlds, const int* worldOrder, const int* bodyStart,
+                        const uint32_t* segStart, int CB, int C, const Rows& rows, const float* rowsU,
+                        const SolverBodies& sb, int posIters, int iters, float stepDt, float muS, float muD,
+                        float invStepDt, float biasScale, float scale, uint32_t* broken, int ldsBodies,
+                        const WorldJoints& joints)
 {
-	if (nWorlds <= 0 || grid <= 0)
+	auto kernel = k_solve_worlds<THREADS, PGS, JOINTS>;
+	if (evStart)
+		hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(THREADS), shm, st, evStart, evStop, 0, nWorlds, worldOrder,
+		                      queueHead, bodyStart, segStart, CB, C, rows, rowsU, sb, posIters, iters, stepDt, muS, muD,
+		                      invStepDt, biasScale, scale, broken, ldsBodies, joints);
+	else
+		kernel<<<grid, THREADS, shm, st>>>(nWorlds, worldOrder, queueHead, bodyStart, segStart, CB, C, rows, rowsU, sb,
+		                                   posIters, iters, stepDt, muS, muD, invStepDt, biasScale, scale, broken,
+		                                   ldsBodies, joints);
+}
+void launch_solve_worlds(int workgroups, int nWorlds, int maxWorldBodies, const int* worldOrder, uint32_t* queueHead,
+                         const int* bodyStart, const uint32_t* segStart, int CB, int C, Rows rows, const float* rowsU,
+                         SolverBodies sb, int posIters, int iters, float stepDt, float muS, float muD,
+                         float invStepDt, float biasScale, float scale, uint32_t* broken, int ldsBodies,
+                         const WorldJoints& joints, hipStream_t st, hipEvent_t evStart, hipEvent_t evStop)
+{
+	if (nWorlds <= 0)
 		return;
+	int dev = 0, cus = 256;
+	(void)hipGetDevice(&dev);
+	(void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+	// One wave a world while the worlds fill the chip (their colours rarely have
+	// more than 64 rows), four where they do not: 301 worlds of up to 512 bodies
+	// step in 602 us with one and in 530 with four, 8,192 worlds in 2.26 and 2.77 ms.
+	const int threads = nWorlds < 4 * cus && maxWorldBodies > 64 ? 256 : 64;
+	ldsBodies = std::min(ldsBodies, WORLD_LDS_BODIES);
+	const size_t shm = sizeof(float4) * 2 * size_t(ldsBodies) + sizeof(uint32_t) * (size_t(CB) + 1);
+	// as many as run at a time: by LDS (160 KB a compute unit) and registers (8 waves)
+	const int perCu = std::max(1, std::min(int(163840 / (shm + 64)), 512 / threads));
+	const int grid = std::min(workgroups > 0 ? workgroups : perCu * cus, nWorlds);
 	// the queue starts at zero (a fill kernel, no memset packet)
 	k_fill_u32<<<1, 64, 0, st>>>(queueHead, 1, 0u);
-	const size_t shm = sizeof(float4) * 4 * size_t(ldsBodies);
-	if (evStart)
-		hipExtLaunchKernelGGL(k_solve_worlds, dim3(grid), dim3(SOLVE_WORLD_THREADS), shm, st, evStart, evStop, 0,
-		                      nWorlds, worldOrder, queueHead, bodyStart, segStart, CB, C, rows, sb.vel, sb.p, sb.dq,
-		                      sb.i0, sb.i1, posIters, velIters, stepDt, muS, muD, invStepDt, biasScale, scale, broken,
-		                      ldsBodies);
+	auto run = [&](auto t, auto pgs, auto j) {
+		solveWorlds<decltype(t)::value, decltype(pgs)::value, decltype(j)::value>(
+		    grid, shm, queueHead, st, evStart, evStop, nWorlds, worldOrder, bodyStart, segStart, CB, C, rows, rowsU, sb,
+		    posIters, iters, stepDt, muS, muD, invStepDt, biasScale, scale, broken, ldsBodies, joints);
+	};
+	auto kind = [&](auto t) {
+		if (rowsU)
+			run(t, std::true_type(), std::false_type());
+		else if (joints.colors > 0)
+			run(t, std::false_type(), std::true_type());
+		else
+			run(t, std::false_type(), std::false_type());
+	};
+	if (threads == 256)
+		kind(std::integral_constant<int, 256>());
 	else
-		k_solve_worlds<<<grid, SOLVE_WORLD_THREADS, shm, st>>>(nWorlds, worldOrder, queueHead, bodyStart, segStart, CB,
-		                                                       C, rows, sb.vel, sb.p, sb.dq, sb.i0, sb.i1, posIters,
-		                                                       velIters, stepDt, muS, muD, invStepDt, biasScale,
-		                                                       scale, broken, ldsBodies);
+		kind(std::integral_constant<int, 64>());
 }
+
 void launch_prep_pgs(int C, const int* order, const int* conA, const int* conB, const int* conSlot,
                      const float4* ctN, const float4* ctP, const float4* pos, const float4* rot, SolverBodies sb,
                      float invDt, float muS, float muD, float restDist, float fot, Rows rows, float* rowsU,

@@ -224,7 +224,7 @@ struct pxh_scene_t
 	DBuf<uint32_t> segStart, solveQueue;
 	bool lastWorldSolve = false;          // the last step used the per-world solve
 	// launch shapes (pxh_scene_set_tuning): solve layout, per-world solve
-	// workgroups (0: 4 per CU), bodies staged in LDS per world
+	// workgroups (0: as many as run at a time), bodies in LDS per world
 	int32_t tuning[4] = {PXH_SOLVE_LAYOUT_AUTO, 0, 512, 0};
 	// autotuning (tuning[3] steps per candidate): every candidate launch shape
 	// of the solve runs for that many real steps, its solve time taken from
@@ -255,6 +255,9 @@ struct pxh_scene_t
 	std::vector<float> hJF0, hJF1;
 	std::vector<float> hJP;   // 10 limit / drive parameters per joint
 	std::vector<int> jColorStart{0};
+	std::vector<int> hJOrder;   // joint of each device slot
+	bool jWorldsDirty = true;   // the per-world joint lists need a rebuild
+	DBuf<int> jWorldSeg, jWorldOrder;
 	int nJKeys = 0;
 	DBuf<int4> jInfo;
 	DBuf<float4> jFrame, jParam, jHead, jRows;
@@ -409,7 +412,7 @@ struct pxh_scene_t
 		f(prevRow); f(conRec); f(patchTable); f(bodyNext); f(bodyNeed); f(stepWords); f(gatherTmp); f(gatherIdx);
 		f(worldOrder); f(segStart); f(solveQueue); f(extLin); f(extAng); f(prevLin); f(prevAng);
 		f(evFound); f(evFoundScan); f(evMatched); f(evLost); f(evLostScan); f(evFoundKeys); f(evLostKeys);
-		f(jInfo); f(jFrame); f(jParam); f(jHead); f(jRows); f(jKeys); f(bpGroup);
+		f(jInfo); f(jFrame); f(jParam); f(jHead); f(jRows); f(jKeys); f(jWorldSeg); f(jWorldOrder); f(bpGroup);
 	}
 	// device bytes the scene holds (PxSimulationStatistics::gpuMemHeap)
 	int64_t deviceBytes()
@@ -638,6 +641,40 @@ int rebuild_topology(pxh_scene_t* s)
 	PXH_CHECK(hipMemcpy(s->bodyStart.p, s->hBodyStart.data(), s->hBodyStart.size() * sizeof(int),
 	                    hipMemcpyHostToDevice));
 	s->topologyDirty = false;
+	s->jWorldsDirty = true;
+	return PXH_OK;
+}
+
+// device joint slots by (world, colour) and each world's colour starts, for the
+// per-world solve
+int uploadWorldJoints(pxh_scene_t* s)
+{
+	const int J = int(s->hJOrder.size()), nC = int(s->jColorStart.size()) - 1, nW = worldCount(s);
+	std::vector<int> slots, world(size_t(J), 0), color(size_t(J), 0);
+	for (int c = 0; c < nC; c++)
+		for (int k = s->jColorStart[c]; k < s->jColorStart[c + 1]; k++)
+		{
+			const int i = s->hJOrder[k];
+			world[k] = s->hScene[s->hJA[i] >= 0 ? s->hJA[i] : s->hJB[i]];
+			color[k] = c;
+			slots.push_back(k);
+		}
+	std::stable_sort(slots.begin(), slots.end(), [&](int x, int y) { return world[x] < world[y]; });
+	std::vector<int> seg(size_t(nW) * (nC + 1) + 1, 0);
+	size_t at = 0;
+	for (int w = 0; w < nW; w++)
+		for (int c = 0; c <= nC; c++)
+		{
+			while (at < slots.size() && (world[slots[at]] < w || (world[slots[at]] == w && color[slots[at]] < c)))
+				at++;
+			seg[size_t(w) * (nC + 1) + c] = int(at);
+		}
+	PXH_CHECK(hipStreamSynchronize(s->stream));
+	if (int r = uploadVec(s->jWorldSeg, seg))
+		return r;
+	if (int r = uploadVec(s->jWorldOrder, slots))
+		return r;
+	s->jWorldsDirty = false;
 	return PXH_OK;
 }
 
@@ -1067,6 +1104,8 @@ int uploadJoints(pxh_scene_t* s)
 			keys.push_back((uint64_t(lo) << 32) | hi);
 		}
 	}
+	s->hJOrder = order;
+	s->jWorldsDirty = true;
 	std::sort(keys.begin(), keys.end());
 	keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
 	s->nJKeys = int(keys.size());
@@ -1629,7 +1668,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 			(void)hipGetDevice(&dev);
 			(void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
 			s->tuneCands.push_back(pxh_scene_t::TuneCand{{PXH_SOLVE_LAYOUT_COLORS, 0, s->tuning[2]}});
-			if (d.solver_type == PXH_SOLVER_TGS && s->maxWorldBodies <= PXH_WORLD_SOLVE_MAX_BODIES)
+			if (s->maxWorldBodies <= PXH_WORLD_SOLVE_MAX_BODIES)
 				for (int per : {8, 4, 2, 1})
 					for (int lds : {std::min(1000, std::max(s->maxWorldBodies, 1)), 0})
 						s->tuneCands.push_back(pxh_scene_t::TuneCand{{PXH_SOLVE_LAYOUT_WORLDS, per * cus, lds}});
@@ -1893,12 +1932,14 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		return fail(PXH_ERR_CAPACITY, "pxh_scene_simulate: too many planes in one world");
 	int nColors = 0;
 	std::vector<uint32_t> colorStart(1, 0);
-	// the per-world solve: TGS, and every world small enough for one workgroup
-	// (layout auto), or as the tuning asks
+	// the per-world solve: every world small enough for one workgroup (layout
+	// auto), or as the tuning asks
 	const int layout = s->tuning[0];
-	const bool worldSolve = d.solver_type == PXH_SOLVER_TGS && nWorlds > 0 && s->hJType.empty() &&
-	                        (layout == PXH_SOLVE_LAYOUT_WORLDS ||
-	                         (layout == PXH_SOLVE_LAYOUT_AUTO && s->maxWorldBodies <= PXH_WORLD_SOLVE_MAX_BODIES));
+	const bool worldSolve = nWorlds > 0 && (layout == PXH_SOLVE_LAYOUT_WORLDS ||
+	                                        (layout == PXH_SOLVE_LAYOUT_AUTO && s->maxWorldBodies <= PXH_WORLD_SOLVE_MAX_BODIES));
+	if (worldSolve && !s->hJType.empty() && s->jWorldsDirty)
+		if (int e = uploadWorldJoints(s))
+			return e;
 	s->lastWorldSolve = worldSolve;
 	int CB = 0;   // per-world solve: colour slots per world
 	if (worldSolve)
@@ -2066,7 +2107,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		PXH_CHECK(hipEventRecord(s->tuneEv[0], st));
 	s->statSolveLaunches = 0;
 	const int pgsPasses = P_ + std::max(V_, 1);
-	for (int it = 0; pgs && it < pgsPasses; it++)
+	for (int it = 0; pgs && !worldSolve && it < pgsPasses; it++)
 	{
 		const bool posIter = it < P_;
 		const bool doFriction = !posIter || P_ - it <= 3;
@@ -2083,23 +2124,21 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		if (it == P_ - 1)
 			pxh::launch_pgs_save_motion(n, sb, st);
 	}
-	if (!pgs && worldSolve)
+	if (worldSolve)
 	{
-		int grid = s->tuning[1];
-		if (grid <= 0)
-		{
-			int dev = 0, cus = 256;
-			(void)hipGetDevice(&dev);
-			(void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-			grid = 4 * cus;
-		}
-		grid = std::min(grid, nWorlds);
+		pxh::WorldJoints wj{};
+		if (nJ > 0)
+			wj = pxh::WorldJoints{int(s->jColorStart.size()) - 1, s->jWorldSeg.p, s->jWorldOrder.p, s->jInfo.p, s->jHead.p,
+			                      s->jRows.p, sleeping ? s->slFlags.p : nullptr};
+		// layout auto keeps every world's velocities in LDS
+		const int ldsBodies = layout == PXH_SOLVE_LAYOUT_AUTO ? std::max(s->maxWorldBodies, 1) : s->tuning[2];
 		hipEvent_t e0, e1;
 		s->profKernel(5, &e0, &e1);
 		s->statSolveLaunches++;
-		pxh::launch_solve_worlds(grid, nWorlds, s->worldOrder.p, s->solveQueue.p, s->bodyStart.p, s->segStart.p, CB,
-		                         C, rows, sb, P_, V_, stepDt, d.static_friction, d.dynamic_friction, invStepDt,
-		                         invStepDt * scale, scale, s->patchBroken[cur].p, s->tuning[2], st, e0, e1);
+		pxh::launch_solve_worlds(s->tuning[1], nWorlds, s->maxWorldBodies, s->worldOrder.p, s->solveQueue.p,
+		                         s->bodyStart.p, s->segStart.p, CB, C, rows, pgs ? s->rnU.p : nullptr, sb, P_,
+		                         pgs ? pgsPasses : P_ + V_, stepDt, d.static_friction, d.dynamic_friction, invStepDt,
+		                         invStepDt * scale, scale, s->patchBroken[cur].p, ldsBodies, wj, st, e0, e1);
 	}
 	for (int it = 0; !pgs && !worldSolve && it < P_ + V_; it++)
 	{
