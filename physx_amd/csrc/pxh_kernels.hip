@@ -944,6 +944,56 @@ PXH_D void storeContacts(int slot, const Contacts& c, int cnt, float4* ctN, floa
 			ctP[4 * int64_t(slot) + k] = make_float4(c.p[k].x, c.p[k].y, c.p[k].z, c.sep[k]);
 }
 
+// appends value to out where take, at the count *total (one atomic a block;
+// the order is left to chance, which nothing that reads the lists depends on)
+PXH_D void blockAppend(bool take, int value, int* out, uint32_t* total)
+{
+	__shared__ uint32_t waveCnt[16], blockBase;
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+	const uint64_t m = __ballot(take);
+	if (lane == 0)
+		waveCnt[w] = uint32_t(__popcll(m));
+	__syncthreads();
+	if (threadIdx.x == 0)
+	{
+		uint32_t sum = 0;
+		for (int i = 0; i < nw; i++)
+		{
+			const uint32_t c = waveCnt[i];
+			waveCnt[i] = sum;
+			sum += c;
+		}
+		blockBase = sum ? atomicAdd(total, sum) : 0u;
+	}
+	__syncthreads();
+	if (take)
+		out[blockBase + waveCnt[w] + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = value;
+	__syncthreads();
+}
+
+// Kernels whose items are long serial chains with branches of their own (hull
+// polygons, mesh triangles, joint rows) fill a wave only as far as the chip is
+// full: a wave of 64 such lanes runs every branch of every lane one after the
+// other, while most compute units idle. THIN_BLOCKS waves take `lanes` items
+// each at a time, one until there are more items than waves. 2,116 bodies on a
+// mesh: 584 us in 64-lane waves, 279 so; their sphere- and capsule-hull pairs
+// 209 and 89 us, the hull contacts 101 and 50.
+constexpr int THIN_BLOCKS = 4096;
+__host__ __device__ inline int thinLanes(uint32_t count)
+{
+	int l = 1;
+	while (l < 64 && uint32_t(l) * THIN_BLOCKS < count)
+		l *= 2;
+	return l;
+}
+// item of this lane for i = 0, 1, ...: false where it has none; loops end at the
+// same i for the whole wave
+#define PXH_THIN_LOOP(q, count)                                                                                    \
+	for (uint32_t lanes_ = uint32_t(thinLanes(count)), base_ = blockIdx.x * lanes_, q = base_ + threadIdx.x;       \
+	     base_ < uint32_t(count); base_ += gridDim.x * lanes_, q = base_ + threadIdx.x)                            \
+		if (threadIdx.x < lanes_ && q < uint32_t(count))
+static inline int thinGrid(int64_t most) { return int(std::min<int64_t>(std::max<int64_t>(most, 1), THIN_BLOCKS)); }
+
 // Body-body pairs; the shape order is the reference contact-method table's
 // (lower geometry type first), so body a of a sphere-box pair is the sphere.
 // Lanes past the pair count on the device (*dP) have no pair; pair p fills slot
@@ -1036,93 +1086,88 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_planes(int Q, int slotBase, c
 	storeContacts(slotBase + q, c, cnt, ctN, ctP);
 }
 
-// Sphere- and capsule-convex pairs: the class segments from *dConvex to *dP
-// hold the convex pairs; lane q takes pair *dConvex + q when its first shape
-// is round. For a box- or convex-convex pair it makes the bounding-sphere
-// test and lists the pair for k_np_convex_wave (list[1] counts, entries from
-// list[2 + cap]) or writes its empty slot.
-__global__ void k_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotBase, const uint2* pairs,
-                            const float4* pos, const float4* rot, const float4* geom, HullSet hs, float cd, float tol,
-                            float4* ctN, float4* ctP, uint32_t* list)
+// Convex pairs: the class segments from *dConvex to *dP hold them; lane q takes
+// pair *dConvex + q. Sphere- and capsule-convex pairs, and the box- and
+// convex-convex pairs whose bounding spheres come within the contact distance,
+// go to their lists, the others get their empty contact slot here. Two lists of
+// cap entries after two counts: 0 pairs to search (k_np_convex_wave and
+// k_np_convex_finish), 1 round pairs (k_np_round_convex).
+PXH_D uint32_t* cvxEntries(uint32_t* list, int cap, int which) { return list + 2 + int64_t(which) * cap; }
+PXH_D const uint32_t* cvxEntries(const uint32_t* list, int cap, int which) { return list + 2 + int64_t(which) * cap; }
+__global__ void __launch_bounds__(256) k_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotBase, const uint2* pairs,
+                            const float4* pos, const float4* geom, HullSet hs, float cd, float4* ctN, uint32_t* list)
 {
 	const int q = blockIdx.x * blockDim.x + threadIdx.x;
 	const uint32_t p = *dConvex + uint32_t(q);
 	const bool live = q < cap && p < *dP && p < uint32_t(cap);
-	uint2 ab = make_uint2(0u, 0u);
-	float4 g0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), g1 = g0;
-	int t0 = -1;
+	bool round = false, search = false;
 	if (live)
 	{
-		ab = pairs[p];
-		g0 = geom[ab.x];
-		g1 = geom[ab.y];
-		t0 = int(g0.w);
+		const uint2 ab = pairs[p];
+		const float4 g0 = geom[ab.x], g1 = geom[ab.y];
+		const int t0 = int(g0.w);
+		round = t0 == GEOM_SPHERE || t0 == GEOM_CAPSULE;
+		if (!round)
+		{
+			const f3 p0 = mk(pos[ab.x]), p1 = mk(pos[ab.y]);
+			const float r0 = t0 == GEOM_BOX ? sqrtf(g0.x * g0.x + g0.y * g0.y + g0.z * g0.z) : hs.be[int(g0.x)].w;
+			const float r1 = hs.be[int(g1.x)].w;
+			const f3 d = p1 - p0;
+			const float reach = r0 + r1 + cd;
+			search = dot(d, d) <= reach * reach;
+			if (!search)
+				ctN[slotBase + int(p)] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
+		}
 	}
-	const bool round = t0 == GEOM_SPHERE || t0 == GEOM_CAPSULE;
-	// Polytope pairs: those whose bounding spheres come within the contact
-	// distance go to the search list (one atomic per wave), the others get
-	// their empty contact slot here.
-	bool search = false;
-	if (live && !round)
+	blockAppend(search, int(p), reinterpret_cast<int*>(cvxEntries(list, cap, 0)), list);
+	blockAppend(round, int(p), reinterpret_cast<int*>(cvxEntries(list, cap, 1)), list + 1);
+}
+
+// sphere- and capsule-convex pairs of list 1
+__global__ void __launch_bounds__(64) k_np_round_convex(int cap, int slotBase, const uint2* pairs, const float4* pos,
+                                                        const float4* rot, const float4* geom, HullSet hs, float cd,
+                                                        float tol, float4* ctN, float4* ctP, const uint32_t* list)
+{
+	PXH_THIN_LOOP(q, min(list[1], uint32_t(cap)))
 	{
-		const f3 p0 = mk(pos[ab.x]), p1 = mk(pos[ab.y]);
-		const float r0 = t0 == GEOM_BOX ? sqrtf(g0.x * g0.x + g0.y * g0.y + g0.z * g0.z) : hs.be[int(g0.x)].w;
-		const float r1 = hs.be[int(g1.x)].w;
-		const f3 d = p1 - p0;
-		const float reach = r0 + r1 + cd;
-		search = dot(d, d) <= reach * reach;
-		if (!search)
-			ctN[slotBase + int(p)] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
+		const uint32_t p = cvxEntries(list, cap, 1)[q];
+		const uint2 ab = pairs[p];
+		const float4 g0 = geom[ab.x], g1 = geom[ab.y];
+		xf x1;
+		x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
+		Contacts c;
+		c.count = 0;
+		int cnt;
+		if (int(g0.w) == GEOM_SPHERE)
+			cnt = sphereConvex(g0.x, mk(pos[ab.x]), hullPoly(hs, int(g1.x)), x1, cd, c);
+		else
+		{
+			xf x0;
+			x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
+			cnt = capsulePoly(g0.x, g0.y, x0, hullPoly(hs, int(g1.x)), x1, cd, tol, c);
+		}
+		storeContacts(slotBase + int(p), c, cnt, ctN, ctP);
 	}
-	const uint64_t m = __ballot(search);
-	if (m)
-	{
-		const int lane = threadIdx.x & 63, lead = __ffsll((unsigned long long)m) - 1;
-		uint32_t at = 0u;
-		if (lane == lead)
-			at = atomicAdd(list + 1, uint32_t(__popcll(m)));
-		at = __shfl(at, lead);
-		if (search)
-			list[2 + cap + at + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = p;
-	}
-	if (!live || !round)
-		return;
-	xf x1;
-	x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
-	Contacts c;
-	c.count = 0;
-	int cnt;
-	if (t0 == GEOM_SPHERE)
-		cnt = sphereConvex(g0.x, mk(pos[ab.x]), hullPoly(hs, int(g1.x)), x1, cd, c);
-	else
-	{
-		xf x0;
-		x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
-		cnt = capsulePoly(g0.x, g0.y, x0, hullPoly(hs, int(g1.x)), x1, cd, tol, c);
-	}
-	storeContacts(slotBase + int(p), c, cnt, ctN, ctP);
 }
 
 // Box- and convex-convex pairs, separation phase: one wavefront per pair
-// (grid-stride over the convex segments) finds the closest features or the
-// minimum translation for each pair of the search list k_np_convex wrote
-// (list[1] entries from list[2 + cap]). A pair within the contact distance
-// stores (dist, n), cA, cB at wit[3p .. 3p+2] and is appended to the
-// touching list (list[0] entries from list[2]); any other pair gets its empty
-// contact slot here. Polytopes past the LDS limits are searched by lane 0
+// (grid-stride over the search list k_np_convex wrote) finds the closest
+// features or the minimum translation and stores (dist, n), cA, cB at
+// wit[3p .. 3p+2]; the contact phase looks at every searched pair's distance
+// (a list of the touching ones, an atomic on one word for each, cost 32 us of
+// 574 at 8,192 hulls). Polytopes past the LDS limits are searched by lane 0
 // alone.
 constexpr int CVX_WAVES = 4;
 __global__ void __launch_bounds__(64 * CVX_WAVES, 4)   // at least 4 waves per SIMD
-k_np_convex_wave(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotBase, const uint2* pairs,
-                 const float4* pos, const float4* rot, const float4* geom, HullSet hs, float cd, float4* wit,
-                 uint32_t* list, float4* ctN)
+k_np_convex_wave(int cap, const uint2* pairs, const float4* pos, const float4* rot, const float4* geom, HullSet hs,
+                 float cd, float4* wit, const uint32_t* list)
 {
 	__shared__ CvxLds lds[CVX_WAVES];
 	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-	const uint32_t n = min(list[1], uint32_t(cap));
+	const uint32_t n = min(list[0], uint32_t(cap));
 	for (uint32_t i = blockIdx.x * CVX_WAVES + w; i < n; i += gridDim.x * CVX_WAVES)
 	{
-		const uint32_t p = list[2 + cap + i];
+		const uint32_t p = cvxEntries(list, cap, 0)[i];
 		const uint2 ab = pairs[p];
 		const float4 g0 = geom[ab.x], g1 = geom[ab.y];
 		const int t0 = int(g0.w);
@@ -1144,76 +1189,72 @@ k_np_convex_wave(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotB
 		}
 		if (lane == 0)
 		{
+			wit[3 * int64_t(p)] = sep;
 			if (sep.x <= cd)
 			{
-				wit[3 * int64_t(p)] = sep;
 				wit[3 * int64_t(p) + 1] = f4(cA, 0.0f);
 				wit[3 * int64_t(p) + 2] = f4(cB, 0.0f);
-				list[2 + atomicAdd(list, 1u)] = p;
 			}
-			else
-				ctN[slotBase + int(p)] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
 		}
 	}
 }
 
-// Box- and convex-convex pairs, contact phase: one lane per listed (touching)
-// pair builds the contacts from the separation record (witness polygons,
-// clipping, reduction); the list order does not matter, pair p fills slot
-// slotBase + p.
-__global__ void k_np_convex_finish(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotBase,
-                                   const uint2* pairs, const float4* pos, const float4* rot, const float4* geom,
-                                   HullSet hs, float cd, float tol, const float4* wit, const uint32_t* list,
-                                   float4* ctN, float4* ctP)
+// Box- and convex-convex pairs, contact phase: one lane per searched pair
+// (witness polygons, clipping, reduction where it touches, else its empty slot);
+// the list order does not matter, pair p fills slot slotBase + p.
+__global__ void __launch_bounds__(64) k_np_convex_finish(int cap, int slotBase, const uint2* pairs, const float4* pos,
+                                                         const float4* rot, const float4* geom, HullSet hs, float cd,
+                                                         float tol, const float4* wit, const uint32_t* list,
+                                                         float4* ctN, float4* ctP)
 {
-	const int q = blockIdx.x * blockDim.x + threadIdx.x;
-	if (q >= cap || uint32_t(q) >= list[0])
-		return;
-	const uint32_t p = list[2 + q];
-	const uint2 ab = pairs[p];
-	const float4 g0 = geom[ab.x], g1 = geom[ab.y];
-	const int t0 = int(g0.w);
-	if (t0 == GEOM_SPHERE || t0 == GEOM_CAPSULE)
-		return;
-	const float4 sep = wit[3 * int64_t(p)];
-	Contacts c;
-	c.count = 0;
-	int cnt = 0;
-	if (sep.x <= cd)
+	PXH_THIN_LOOP(q, min(list[0], uint32_t(cap)))
 	{
-		xf x0, x1;
-		x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
-		x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
-		const Poly B = hullPoly(hs, int(g1.x));
-		const Poly A = t0 == GEOM_BOX ? boxPoly(mk(g0.x, g0.y, g0.z)) : hullPoly(hs, int(g0.x));
-		const mxf aToB = mxfOf(xinvmul(x1, x0));
-		cnt = convexContactsFrom(A, x0, B, x1, aToB, sep.x, mk(sep.y, sep.z, sep.w), mk(wit[3 * int64_t(p) + 1]),
-		                         mk(wit[3 * int64_t(p) + 2]), cd, tol, c);
+		const uint32_t p = cvxEntries(list, cap, 0)[q];
+		const uint2 ab = pairs[p];
+		const float4 g0 = geom[ab.x], g1 = geom[ab.y];
+		const int t0 = int(g0.w);
+		const float4 sep = wit[3 * int64_t(p)];
+		Contacts c;
+		c.count = 0;
+		int cnt = 0;
+		if (sep.x <= cd)
+		{
+			xf x0, x1;
+			x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
+			x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
+			const Poly B = hullPoly(hs, int(g1.x));
+			const Poly A = t0 == GEOM_BOX ? boxPoly(mk(g0.x, g0.y, g0.z)) : hullPoly(hs, int(g0.x));
+			const mxf aToB = mxfOf(xinvmul(x1, x0));
+			cnt = convexContactsFrom(A, x0, B, x1, aToB, sep.x, mk(sep.y, sep.z, sep.w), mk(wit[3 * int64_t(p) + 1]),
+			                         mk(wit[3 * int64_t(p) + 2]), cd, tol, c);
+		}
+		storeContacts(slotBase + int(p), c, cnt, ctN, ctP);
 	}
-	storeContacts(slotBase + int(p), c, cnt, ctN, ctP);
 }
 
 // Body-plane pairs of convex bodies (the others are left to k_np_planes); the
 // hull is constraint body a, so normals point from the plane to the hull.
-__global__ void k_np_planes_convex(int Q, int slotBase, const int* qBody, const int* qPlane, const float4* pos,
-                                   const float4* rot, const float4* geom, const float4* planes, HullSet hs, float cd,
-                                   float tol, float4* ctN, float4* ctP)
+__global__ void __launch_bounds__(64) k_np_planes_convex(int Q, int slotBase, const int* qBody, const int* qPlane,
+                                                         const float4* pos, const float4* rot, const float4* geom,
+                                                         const float4* planes, HullSet hs, float cd, float tol,
+                                                         float4* ctN, float4* ctP)
 {
-	const int q = blockIdx.x * blockDim.x + threadIdx.x;
-	if (q >= Q)
-		return;
-	const int i = qBody[q];
-	const float4 g = geom[i];
-	if (int(g.w) != GEOM_CONVEXMESH)
-		return;
-	const float4 pl = planes[qPlane[q]];
-	xf x;
-	x.p = mk(pos[i]); x.q = mkq(rot[i]);
-	Contacts c;
-	c.count = 0;
-	const int cnt = planeConvex(mk(pl), pl.w, hullPoly(hs, int(g.x)), x, cd, tol, c);
-	c.n = -c.n;
-	storeContacts(slotBase + q, c, cnt, ctN, ctP);
+	PXH_THIN_LOOP(q, Q)
+	{
+		const int i = qBody[q];
+		const float4 g = geom[i];
+		if (int(g.w) == GEOM_CONVEXMESH)
+		{
+			const float4 pl = planes[qPlane[q]];
+			xf x;
+			x.p = mk(pos[i]); x.q = mkq(rot[i]);
+			Contacts c;
+			c.count = 0;
+			const int cnt = planeConvex(mk(pl), pl.w, hullPoly(hs, int(g.x)), x, cd, tol, c);
+			c.n = -c.n;
+			storeContacts(slotBase + int(q), c, cnt, ctN, ctP);
+		}
+	}
 }
 
 // Contact data of the last step, one 128-byte record per constraint in
@@ -1474,33 +1515,6 @@ __global__ void k_color_pick(int m, const uint32_t* mDev, const int* list, int r
 			}
 		}
 	}
-}
-
-// appends value to out where take, at the count *total (one atomic a block;
-// the order is left to chance, which nothing that reads the lists depends on)
-PXH_D void blockAppend(bool take, int value, int* out, uint32_t* total)
-{
-	__shared__ uint32_t waveCnt[16], blockBase;
-	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-	const uint64_t m = __ballot(take);
-	if (lane == 0)
-		waveCnt[w] = uint32_t(__popcll(m));
-	__syncthreads();
-	if (threadIdx.x == 0)
-	{
-		uint32_t sum = 0;
-		for (int i = 0; i < nw; i++)
-		{
-			const uint32_t c = waveCnt[i];
-			waveCnt[i] = sum;
-			sum += c;
-		}
-		blockBase = sum ? atomicAdd(total, sum) : 0u;
-	}
-	__syncthreads();
-	if (take)
-		out[blockBase + waveCnt[w] + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = value;
-	__syncthreads();
 }
 
 // the constraints of the list that the rounds left uncoloured, as the next list
@@ -2831,14 +2845,11 @@ __global__ void k_integrate(int n, float dt, float4* vel, float4* svP, float4* s
 // patches of pxh_mesh.h into slots slotBase + k * MESH_MAXP + patch (deepest
 // first; empty slots count 0). More than MESH_MAX_TRIS candidates set
 // *overflow and leave the body without mesh contacts.
-__global__ void __launch_bounds__(64) k_np_mesh(int nMB, const int* meshBody, const int* world, const int4* worldMesh,
+PXH_D void meshContactsOf(int k, const int* meshBody, const int* world, const int4* worldMesh,
                                                 MeshSet M, const float4* pos, const float4* rot, const float4* geom,
                                                 HullSet hs, float cd, int slotBase, float4* ctN, float4* ctP,
                                                 uint32_t* overflow)
 {
-	const int k = blockIdx.x * blockDim.x + threadIdx.x;
-	if (k >= nMB)
-		return;
 	const int i = meshBody[k];
 	const int base = slotBase + k * MESH_MAXP;
 	for (int p = 0; p < MESH_MAXP; p++)
@@ -2938,6 +2949,15 @@ __global__ void __launch_bounds__(64) k_np_mesh(int nMB, const int* meshBody, co
 		for (int j = 0; j < cnt; j++)
 			ctP[4 * int64_t(base + a) + j] = f4(q.c[j].p, q.c[j].s);
 	}
+}
+
+__global__ void __launch_bounds__(64) k_np_mesh(int nMB, const int* meshBody, const int* world, const int4* worldMesh,
+                                                MeshSet M, const float4* pos, const float4* rot, const float4* geom,
+                                                HullSet hs, float cd, int slotBase, float4* ctN, float4* ctP,
+                                                uint32_t* overflow)
+{
+	PXH_THIN_LOOP(k, nMB)
+		meshContactsOf(int(k), meshBody, world, worldMesh, M, pos, rot, geom, hs, cd, slotBase, ctN, ctP, overflow);
 }
 
 // whether the bodies of a pair are joined: its (lower, higher) key is among
@@ -3251,14 +3271,11 @@ PXH_D bool jointAsleep(int4 ji, const uint32_t* sleepFlags)
 	       (ji.z < 0 || (sleepFlags[ji.z] & SLEEP_ASLEEP));
 }
 
-__global__ void k_joint_prep(int J, const int4* info, const float4* frame, const float4* param, const float4* pos,
+PXH_D void prepJointOf(int j, const int4* info, const float4* frame, const float4* param, const float4* pos,
                              const float4* rot, const float4* vel, const float4* rec, const float4* svI0,
                              const float4* svI1, float stepDt, float invStepDt, float invDt, float erp,
                              float lengthScale, float4* head, float4* rows, const uint32_t* sleepFlags)
 {
-	const int j = blockIdx.x * blockDim.x + threadIdx.x;
-	if (j >= J)
-		return;
 	const int4 ji = info[j];
 	if (jointAsleep(ji, sleepFlags))
 		return;
@@ -3276,6 +3293,18 @@ __global__ void k_joint_prep(int J, const int4* info, const float4* frame, const
 	prepJoint(ji.x, jp[0], jp[1], jp[2], bA, bB, jointFrame(frame + 4 * int64_t(j)),
 	          jointFrame(frame + 4 * int64_t(j) + 2), sI0, sI1, im0, im1, v0, w0, v1, w1, stepDt, invStepDt, invDt,
 	          erp, lengthScale, head + JOINT_HEAD * int64_t(j), rows + JOINT_ROWS * int64_t(j));
+}
+
+__global__ void __launch_bounds__(64) k_joint_prep(int J, const int4* info, const float4* frame, const float4* param,
+                                                   const float4* pos, const float4* rot, const float4* vel,
+                                                   const float4* rec, const float4* svI0, const float4* svI1,
+                                                   float stepDt, float invStepDt, float invDt, float erp,
+                                                   float lengthScale, float4* head, float4* rows,
+                                                   const uint32_t* sleepFlags)
+{
+	PXH_THIN_LOOP(j, J)
+		prepJointOf(int(j), info, frame, param, pos, rot, vel, rec, svI0, svI1, stepDt, invStepDt, invDt, erp,
+		            lengthScale, head, rows, sleepFlags);
 }
 
 template <class Vel>
@@ -3902,22 +3931,24 @@ void launch_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int 
                       const float4* pos, const float4* rot, const float4* geom, const HullSet& hs, float cd, float tol,
                       float4* wit, uint32_t* list, float4* ctN, float4* ctP, hipStream_t st)
 {
-	PXH_LAUNCH(k_np_convex, cap, cap, dP, dConvex, slotBase, pairs, pos, rot, geom, hs, cd, tol, ctN, ctP, list);
-	if (cap > 0)
-	{
-		// grid-stride: enough waves to fill the chip several times over
-		const int blocks = std::min((cap + CVX_WAVES - 1) / CVX_WAVES, 8192);
-		k_np_convex_wave<<<blocks, 64 * CVX_WAVES, 0, st>>>(cap, dP, dConvex, slotBase, pairs, pos, rot, geom, hs, cd,
-		                                                    wit, list, ctN);
-	}
-	PXH_LAUNCH(k_np_convex_finish, cap, cap, dP, dConvex, slotBase, pairs, pos, rot, geom, hs, cd, tol, wit, list, ctN,
-	           ctP);
+	if (cap <= 0)
+		return;
+	k_fill_u32<<<1, 64, 0, st>>>(list, 2, 0u);
+	PXH_LAUNCH(k_np_convex, cap, cap, dP, dConvex, slotBase, pairs, pos, geom, hs, cd, ctN, list);
+	// grid-stride: enough waves to fill the chip several times over
+	const int blocks = std::min((cap + CVX_WAVES - 1) / CVX_WAVES, 8192);
+	k_np_convex_wave<<<blocks, 64 * CVX_WAVES, 0, st>>>(cap, pairs, pos, rot, geom, hs, cd, wit, list);
+	k_np_round_convex<<<thinGrid(cap), 64, 0, st>>>(cap, slotBase, pairs, pos, rot, geom, hs, cd, tol, ctN, ctP, list);
+	k_np_convex_finish<<<thinGrid(cap), 64, 0, st>>>(cap, slotBase, pairs, pos, rot, geom, hs, cd, tol, wit, list, ctN,
+	                                                 ctP);
 }
 void launch_np_planes_convex(int Q, int slotBase, const int* qBody, const int* qPlane, const float4* pos,
                              const float4* rot, const float4* geom, const float4* planes, const HullSet& hs, float cd,
                              float tol, float4* ctN, float4* ctP, hipStream_t st)
 {
-	PXH_LAUNCH(k_np_planes_convex, Q, Q, slotBase, qBody, qPlane, pos, rot, geom, planes, hs, cd, tol, ctN, ctP);
+	if (Q > 0)
+		k_np_planes_convex<<<thinGrid(Q), 64, 0, st>>>(Q, slotBase, qBody, qPlane, pos, rot, geom, planes, hs, cd, tol,
+		                                               ctN, ctP);
 }
 void launch_np_planes(int Q, int slotBase, const int* qBody, const int* qPlane, const float4* pos, const float4* rot,
                       const float4* geom, const float4* planes, float cd, float4* ctN, float4* ctP, hipStream_t st)
@@ -3970,7 +4001,7 @@ void launch_np_mesh(int nMB, const int* meshBody, const int* world, const int4* 
                     int slotBase, float4* ctN, float4* ctP, uint32_t* overflow, hipStream_t st)
 {
 	if (nMB > 0)
-		k_np_mesh<<<nblk(nMB, 64), 64, 0, st>>>(nMB, meshBody, world, worldMesh, M, pos, rot, geom, hs, cd, slotBase,
+		k_np_mesh<<<thinGrid(nMB), 64, 0, st>>>(nMB, meshBody, world, worldMesh, M, pos, rot, geom, hs, cd, slotBase,
 		                                        ctN, ctP, overflow);
 }
 void launch_sleep_wake_bodies(int k, const int* bodies, SleepState ss, hipStream_t st)
@@ -3985,8 +4016,9 @@ void launch_joint_prep(int J, const int4* info, const float4* frame, const float
                        const float4* rot, SolverBodies sb, float stepDt, float invStepDt, float invDt, float erp,
                        float lengthScale, float4* head, float4* rows, const uint32_t* sleepFlags, hipStream_t st)
 {
-	PXH_LAUNCH(k_joint_prep, J, J, info, frame, param, pos, rot, sb.vel, sb.rec, sb.i0, sb.i1, stepDt, invStepDt,
-	           invDt, erp, lengthScale, head, rows, sleepFlags);
+	if (J > 0)
+		k_joint_prep<<<thinGrid(J), 64, 0, st>>>(J, info, frame, param, pos, rot, sb.vel, sb.rec, sb.i0, sb.i1, stepDt,
+		                                         invStepDt, invDt, erp, lengthScale, head, rows, sleepFlags);
 }
 void launch_joint_solve(int begin, int end, const int4* info, const float4* head, float4* rows, SolverBodies sb,
                         float elapsed, bool conclude, const uint32_t* sleepFlags, hipStream_t st)
