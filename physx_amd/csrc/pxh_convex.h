@@ -1110,7 +1110,7 @@ namespace pxh {
 // minimum in loop order wins), so the result is the same as the per-lane
 // path's.
 // ---------------------------------------------------------------------------
-constexpr int CVX_WAVE_V = 64, CVX_WAVE_P = 128, CVX_WAVE_E = 192;
+constexpr int CVX_WAVE_V = 64, CVX_WAVE_P = 128, CVX_WAVE_E = 192, CVX_ARCS = 32;
 
 struct CvxLds
 {
@@ -1118,11 +1118,22 @@ struct CvxLds
 	float4 vb[CVX_WAVE_V];   // B's vertices
 	float4 pa[CVX_WAVE_P];   // A's planes in B's frame
 	float4 pb[CVX_WAVE_P];   // B's planes
-	uint32_t polyA[CVX_WAVE_P], polyB[CVX_WAVE_P];
 	uint32_t ea[CVX_WAVE_E];
 	uint32_t eb[CVX_WAVE_E];
-	uint8_t vrA[2 * CVX_WAVE_E], vrB[2 * CVX_WAVE_E];   // a closed polytope has 2 vrefs per edge
-	uint8_t elA[CVX_WAVE_E], elB[CVX_WAVE_E];           // edges kept for the closest-feature search
+	union
+	{
+		struct   // closest features of separated polytopes
+		{
+			uint32_t polyA[CVX_WAVE_P], polyB[CVX_WAVE_P];
+			uint8_t vrA[2 * CVX_WAVE_E], vrB[2 * CVX_WAVE_E];   // a closed polytope has 2 vrefs per edge
+			uint8_t elA[CVX_WAVE_E], elB[CVX_WAVE_E];           // vertices and edges that may hold them
+		};
+		struct   // edge pairs of overlapping ones
+		{
+			float4 arc[3 * CVX_ARCS];   // arcs of some of B's edges: both (negated) normals and their cross product
+			uint32_t open[128];         // pairs whose arcs cross
+		};
+	};
 };
 
 PXH_D bool fitsWave(const Poly& A, const Poly& B)
@@ -1182,10 +1193,84 @@ struct FlatPair
 	}
 };
 
+// True only if A and B are farther apart than need: Gilbert's iteration for the
+// point of A - B nearest the origin (Gilbert 1966, "An iterative procedure for
+// computing the minimum of a quadratic form on a convex set"), each step's
+// support an axis that either shows the gap or moves v nearer. Eight lanes of a
+// wave share a pair and hold the same v; lane sub has every eighth vertex in
+// B's frame, the first 4 of each polytope in registers (a step reads no memory
+// below 33 vertices).
+constexpr int APART_LANES = 8, APART_ROUNDS = 8, APART_HELD = 4;
+
+// the smallest h of 8 lanes and, from its lane (the lowest among equals), p
+PXH_D void groupMin(float& h, f3& p)
+{
+	const int lane = __lane_id();
+	float m = h;
+	m = fminf(m, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(m), 0xB1, 0xF, 0xF, true)));    // quad 1 0 3 2
+	m = fminf(m, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(m), 0x4E, 0xF, 0xF, true)));    // quad 2 3 0 1
+	m = fminf(m, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(m), 0x141, 0xF, 0xF, true)));   // half-row mirror
+	const uint32_t mine = uint32_t(__ballot(h == m) >> (lane & 56)) & 0xFFu;
+	const int from = (lane & 56) + (mine ? __ffs(int(mine)) - 1 : 0);
+	p = mk(__shfl(p.x, from), __shfl(p.y, from), __shfl(p.z, from));
+	h = m;
+}
+
+PXH_D bool convexApart(const Poly& A, const mxf& aToB, const Poly& B, float need, int sub)
+{
+	f3 va[APART_HELD], vb[APART_HELD];
+#pragma unroll
+	for (int k = 0; k < APART_HELD; k++)
+	{
+		// past the last vertex: the first again
+		va[k] = mxtrans(aToB, A.vert(sub + APART_LANES * k < A.nv ? sub + APART_LANES * k : 0));
+		vb[k] = B.vert(sub + APART_LANES * k < B.nv ? sub + APART_LANES * k : 0);
+	}
+	f3 v = aToB.p;
+	for (int round = 0; round < APART_ROUNDS; round++)
+	{
+		const float l2 = dot(v, v);
+		if (!(l2 > need * need))
+			return false;
+		float ha = FLT_BIG, hb = FLT_BIG;
+		f3 pa = va[0], pb = vb[0];
+#pragma unroll
+		for (int k = 0; k < APART_HELD; k++)
+		{
+			const float h = dot(v, va[k]), g = -dot(v, vb[k]);
+			if (h < ha) { ha = h; pa = va[k]; }
+			if (g < hb) { hb = g; pb = vb[k]; }
+		}
+		for (int i = sub + APART_LANES * APART_HELD; i < A.nv; i += APART_LANES)
+		{
+			const f3 p = mxtrans(aToB, A.vert(i));
+			const float h = dot(v, p);
+			if (h < ha) { ha = h; pa = p; }
+		}
+		for (int i = sub + APART_LANES * APART_HELD; i < B.nv; i += APART_LANES)
+		{
+			const f3 p = B.vert(i);
+			const float h = -dot(v, p);
+			if (h < hb) { hb = h; pb = p; }
+		}
+		groupMin(ha, pa);
+		groupMin(hb, pb);
+		const float g = ha + hb;
+		if (g > 0.0f && g * g > need * need * l2)
+			return true;
+		if (!(l2 - g > 1e-3f * l2))
+			return false;   // v is nearest: the gap is |v|
+		const f3 d = pa - pb - v;
+		const float t = -dot(v, d) / dot(d, d);
+		v = v + d * fminf(fmaxf(t, 0.0f), 1.0f);
+	}
+	return false;
+}
+
 // The edges of each polytope whose bounding sphere comes within lim of the
 // other polytope's bounding box (both in B's frame, from the staged vertices),
 // listed in index order in L.elA / L.elB; every edge when lim is FLT_BIG.
-PXH_D void nearEdges(const Poly& A, const Poly& B, const CvxLds& L, int lane, float lim, int& nA, int& nB)
+PXH_D void nearEdges(const Poly& A, const Poly& B, CvxLds& L, int lane, float lim, int& nA, int& nB)
 {
 	const float BIG = FLT_BIG;
 	f3 aMin = mk(BIG, BIG, BIG), aMax = -aMin, bMin = aMin, bMax = aMax;
@@ -1210,7 +1295,6 @@ PXH_D void nearEdges(const Poly& A, const Poly& B, const CvxLds& L, int lane, fl
 		bMax = mk(fmaxf(bMax.x, __shfl_xor(bMax.x, off)), fmaxf(bMax.y, __shfl_xor(bMax.y, off)),
 		          fmaxf(bMax.z, __shfl_xor(bMax.z, off)));
 	}
-	CvxLds& W = const_cast<CvxLds&>(L);
 	nA = 0;
 	nB = 0;
 	for (int side = 0; side < 2; side++)
@@ -1237,7 +1321,7 @@ PXH_D void nearEdges(const Poly& A, const Poly& B, const CvxLds& L, int lane, fl
 			if (keep)
 			{
 				const int at = cnt + int(__popcll(m & ((1ull << lane) - 1ull)));
-				(side ? W.elB : W.elA)[at] = uint8_t(e);
+				(side ? L.elB : L.elA)[at] = uint8_t(e);
 			}
 			cnt += int(__popcll(m));
 		}
@@ -1248,15 +1332,17 @@ PXH_D void nearEdges(const Poly& A, const Poly& B, const CvxLds& L, int lane, fl
 
 // The face axes of polySeparation over the wave, from the staged vertices and
 // planes only: B's (order 0 | f << 8 | vertex), then A's (order 1 | ...). The
-// lane's least penetrating axis goes to best, bi; sep is set on every lane
-// when some axis shows no penetration. True when some axis separates the
-// polytopes by more than cd.
+// lane's least penetrating axis goes to best, bi and its most separating one
+// to gap, gi (kind << 24 | f); sep is set on every lane when some axis shows no
+// penetration. True when some axis separates the polytopes by more than cd.
 PXH_D bool faceAxesWave(const Poly& A, const Poly& B, float cd, const CvxLds& L, int lane, float& best, uint32_t& bi,
-                        bool& sep)
+                        bool& sep, float& gap, uint32_t& gi)
 {
 	const float BIG = FLT_BIG;
 	best = BIG;
 	bi = 0xFFFFFFFFu;
+	gap = 0.0f;
+	gi = 0;
 	bool far = false;
 	sep = false;
 	for (int f = lane; f < B.np; f += 64)
@@ -1272,6 +1358,11 @@ PXH_D bool faceAxesWave(const Poly& A, const Poly& B, float cd, const CvxLds& L,
 		}
 		far |= mn > cd;
 		sep |= mn > 0.0f;
+		if (mn > gap)
+		{
+			gap = mn;
+			gi = uint32_t(f);
+		}
 		if (!(mn > 0.0f) && -mn < best)
 		{
 			best = -mn;
@@ -1291,6 +1382,11 @@ PXH_D bool faceAxesWave(const Poly& A, const Poly& B, float cd, const CvxLds& L,
 		}
 		far |= mn > cd;
 		sep |= mn > 0.0f;
+		if (mn > gap)
+		{
+			gap = mn;
+			gi = (1u << 24) | uint32_t(f);
+		}
 		if (!(mn > 0.0f) && -mn < best)
 		{
 			best = -mn;
@@ -1301,12 +1397,69 @@ PXH_D bool faceAxesWave(const Poly& A, const Poly& B, float cd, const CvxLds& L,
 	return waveAny(far);
 }
 
+// The axis of edge pair k (ea * CVX_WAVE_E + eb), whose arcs cross: its overlap
+// goes to best, bi if it is smaller, or equal and the pair comes first
+PXH_D void edgeAxis(const CvxLds& L, int k, f3 bmean, float& best, uint32_t& bi, bool& sep)
+{
+	const int ea = k / CVX_WAVE_E, ebi = k - ea * CVX_WAVE_E;
+	const uint32_t e = L.ea[ea], g = L.eb[ebi];
+	const f3 a0 = ldsV(L.va, int(e & 0xFF)), a1 = ldsV(L.va, int((e >> 8) & 0xFF));
+	const f3 b0 = ldsV(L.vb, int(g & 0xFF)), b1 = ldsV(L.vb, int((g >> 8) & 0xFF));
+	f3 ax = cross(a1 - a0, b1 - b0);
+	const float l2 = dot(ax, ax);
+	if (l2 < 1e-12f)
+		return;
+	ax = ax * (1.0f / sqrtf(l2));
+	if (dot(ax, b0 - bmean) < 0.0f)
+		ax = -ax;
+	const float ov = dot(ax, b0) - dot(ax, a0);
+	const uint32_t code = (2u << 24) | uint32_t(k);
+	if (ov < 0.0f)
+		sep = true;
+	else if (ov < best || (ov == best && code < bi))
+	{
+		best = ov;
+		bi = code;
+	}
+}
+
+PXH_D float edgePairSq(const CvxLds& L, int ea, int eb, f3& c1, f3& c2)
+{
+	const uint32_t e = L.ea[ea], g = L.eb[eb];
+	return segClosestSq(ldsV(L.va, int(e & 0xFF)), ldsV(L.va, int((e >> 8) & 0xFF)), ldsV(L.vb, int(g & 0xFF)),
+	                    ldsV(L.vb, int((g >> 8) & 0xFF)), c1, c2);
+}
+
+// The entries i < n of the wave with keep(i), listed in index order
+template <class K> PXH_D int waveList(int n, int lane, uint8_t* out, K keep)
+{
+	int cnt = 0;
+	for (int base = 0; base < n; base += 64)
+	{
+		const int i = base + lane;
+		const bool k = i < n && keep(i);
+		const uint64_t m = __ballot(k);
+		if (k)
+			out[cnt + int(__popcll(m & ((1ull << lane) - 1ull)))] = uint8_t(i);
+		cnt += int(__popcll(m));
+	}
+	return cnt;
+}
+
+PXH_D float waveMin(float v)
+{
+	for (int off = 32; off >= 1; off >>= 1)
+		v = fminf(v, __shfl_xor(v, off));
+	return v;
+}
+
 // The rest of polySeparation over the wave (same results), after
 // faceAxesWave found no axis farther than cd; A, B in LDS as staged
-PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, const CvxLds& L, int lane, float best,
-                              uint32_t bi, bool sep, float& dist, f3& n, f3& cA, f3& cB)
+PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, CvxLds& L, int lane, float best,
+                              uint32_t bi, bool sep, float gap, uint32_t gi, float& dist, f3& n, f3& cA, f3& cB)
 {
 	const float BIG = FLT_BIG;
+	const bool slab = sep;   // some face axis separates
 	if (!sep)
 	{
 		f3 bmean = mk(0.0f, 0.0f, 0.0f);
@@ -1314,48 +1467,64 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, con
 			bmean = bmean + ldsV(L.vb, i);
 		bmean = bmean * (1.0f / float(B.nv));
 		// Edge pairs: each lane holds one of A's edges (its Gauss-map arc in
-		// registers) and walks B's edges, so B's edge data are read as LDS
-		// broadcasts. A block of R < 64 of A's edges gives each edge S = 64 / R
-		// lanes, which split B's edges between them. A lane visits its pairs in
-		// ascending index order, so with the lowest-index rule of waveArgMin
-		// the pair chosen is the first minimum of the flat order.
-		for (int base = 0; base < A.ne; base += 64)
+		// registers) and walks the arcs of B's edges, laid out CVX_ARCS at a time
+		// and read as LDS broadcasts. A block of R < 64 of A's edges gives each
+		// edge S = 64 / R lanes, which split B's edges between them. Few pairs'
+		// arcs cross (about one in 50 for hulls of 24 points), but one or two of
+		// every 64 do, and their axis costs three times the arc test: the crossing
+		// pairs are listed and measured 64 at a time.
+		int cnt = 0;
+		for (int b0 = 0; b0 < B.ne; b0 += CVX_ARCS)
 		{
-			const int R = min(64, A.ne - base), S = 64 / R, part = lane / R;
-			if (part >= S)
-				continue;
-			const int ea = base + lane - part * R;
-			const uint32_t e = L.ea[ea];
-			const f3 na = ldsV(L.pa, int((e >> 16) & 0xFF)), nb = ldsV(L.pa, int(e >> 24));
-			const f3 bxa = cross(nb, na);
-			for (int ebi = part; ebi < B.ne; ebi += S)
+			const int nb0 = min(CVX_ARCS, B.ne - b0);
+			if (lane < nb0)
 			{
-				const uint32_t g = L.eb[ebi];
+				const uint32_t g = L.eb[b0 + lane];
 				const f3 nc = -ldsV(L.pb, int((g >> 16) & 0xFF)), nd = -ldsV(L.pb, int(g >> 24));
 				const f3 dxc = cross(nd, nc);
-				const float cba = dot(nc, bxa), dba = dot(nd, bxa), adc = dot(na, dxc), bdc = dot(nb, dxc);
-				if (!(cba * dba < 0.0f && adc * bdc < 0.0f && cba * bdc > 0.0f))
-					continue;
-				const f3 a0 = ldsV(L.va, int(e & 0xFF)), a1 = ldsV(L.va, int((e >> 8) & 0xFF));
-				const f3 b0 = ldsV(L.vb, int(g & 0xFF)), b1 = ldsV(L.vb, int((g >> 8) & 0xFF));
-				f3 ax = cross(a1 - a0, b1 - b0);
-				const float l2 = dot(ax, ax);
-				if (l2 < 1e-12f)
-					continue;
-				ax = ax * (1.0f / sqrtf(l2));
-				if (dot(ax, b0 - bmean) < 0.0f)
-					ax = -ax;
-				const float ov = dot(ax, b0) - dot(ax, a0);
-				if (ov < 0.0f)
-					sep = true;
-				else if (ov < best)
+				L.arc[3 * lane] = f4(nc, dxc.x);
+				L.arc[3 * lane + 1] = f4(nd, dxc.y);
+				L.arc[3 * lane + 2].x = dxc.z;
+			}
+			waveSync();
+			for (int base = 0; base < A.ne; base += 64)
+			{
+				const int R = min(64, A.ne - base), S = 64 / R, part = lane / R;
+				const bool has = part < S;
+				const int ea = base + (has ? lane - part * R : 0);
+				const uint32_t e = L.ea[ea];
+				const f3 na = ldsV(L.pa, int((e >> 16) & 0xFF)), nb = ldsV(L.pa, int(e >> 24));
+				const f3 bxa = cross(nb, na);
+				for (int i0 = 0; i0 < nb0; i0 += S)
 				{
-					best = ov;
-					bi = (2u << 24) | uint32_t(ea * CVX_WAVE_E + ebi);
+					const int i = i0 + part;
+					bool arcs = has && i < nb0;
+					const int at = arcs ? 3 * i : 0;
+					const float4 c = L.arc[at], d = L.arc[at + 1];
+					const f3 nc = mk(c), nd = mk(d), dxc = mk(c.w, d.w, L.arc[at + 2].x);
+					const float cba = dot(nc, bxa), dba = dot(nd, bxa), adc = dot(na, dxc), bdc = dot(nb, dxc);
+					arcs = arcs && cba * dba < 0.0f && adc * bdc < 0.0f && cba * bdc > 0.0f;
+					const uint64_t m = __ballot(arcs);
+					if (m == 0ull)
+						continue;
+					if (arcs)
+						L.open[cnt + int(__popcll(m & ((1ull << lane) - 1ull)))] = uint32_t(ea * CVX_WAVE_E + b0 + i);
+					cnt += int(__popcll(m));
+					if (cnt >= 64)
+					{
+						cnt -= 64;
+						waveSync();
+						edgeAxis(L, int(L.open[cnt + lane]), bmean, best, bi, sep);
+						waveSync();
+					}
 				}
 			}
+			waveSync();
 		}
+		if (lane < cnt)
+			edgeAxis(L, int(L.open[lane]), bmean, best, bi, sep);
 		sep = waveAny(sep);
+		waveSync();
 	}
 	if (!sep)
 	{
@@ -1411,58 +1580,116 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, con
 		dist = -best;
 		return;
 	}
-	// separated: closest features (B faces x A vertices, A faces x B vertices,
-	// edge pairs), the first minimum in that order
+	// Separated: closest features (B faces x A vertices, A faces x B vertices,
+	// edge pairs), the first minimum in that order.
+	//
+	// The edges that meet at the closest two vertices hold a pair at squared
+	// distance U, so the minimum is no larger. Along the face axis that
+	// separates the polytopes most, A's heights less B's bound every distance
+	// from below: a vertex or an edge whose height alone is farther from the
+	// other polytope than lim = sqrt(U) plus a margin well above rounding holds
+	// no closest feature. What is left keeps its order and its indices, so the
+	// first minimum is unchanged.
+	int nA, nB;
+	float minA = 0.0f, maxB = 0.0f;
+	if (slab)
+	{
+		float g = -gap;
+		waveArgMin(g, gi);
+		const bool onA = (gi >> 24) != 0u;
+		const float4 pl = (onA ? L.pa : L.pb)[gi & 0xFFFFu];
+		const f3 sn = onA ? -mk(pl) : mk(pl);
+		const float sd = onA ? -pl.w : pl.w;
+		float ha = BIG, hb = -BIG;
+		if (lane < A.nv)
+			L.va[lane].w = ha = dot(sn, ldsV(L.va, lane)) + sd;
+		if (lane < B.nv)
+			L.vb[lane].w = hb = dot(sn, ldsV(L.vb, lane)) + sd;
+		minA = waveMin(ha);
+		maxB = -waveMin(-hb);
+	}
+	float near = BIG;
+	uint32_t ni = 0;
+	FlatPair fv(lane, B.nv);
+	for (int k = lane; k < A.nv * B.nv; k += 64, fv.next())
+	{
+		const f3 w = ldsV(L.va, fv.i) - ldsV(L.vb, fv.j);
+		const float s = dot(w, w);
+		if (s < near)
+		{
+			near = s;
+			ni = uint32_t(fv.i << 8 | fv.j);
+		}
+	}
+	waveArgMin(near, ni);
+	const uint32_t ia = ni >> 8, ib = ni & 0xFFu;
+	nA = waveList(A.ne, lane, L.elA, [&](int e) { return (L.ea[e] & 0xFF) == ia || ((L.ea[e] >> 8) & 0xFF) == ia; });
+	nB = waveList(B.ne, lane, L.elB, [&](int e) { return (L.eb[e] & 0xFF) == ib || ((L.eb[e] >> 8) & 0xFF) == ib; });
+	waveSync();
+	float U = BIG;
+	FlatPair fu(lane, nB);
+	for (int k = lane; k < nA * nB; k += 64, fu.next())
+	{
+		f3 c1, c2;
+		U = fminf(U, edgePairSq(L, L.elA[fu.i], L.elB[fu.j], c1, c2));
+	}
+	U = waveMin(U);
+	float lim = U < BIG ? sqrtf(U) + 1e-4f : BIG;
+	waveSync();
 	float d2 = BIG;
 	uint32_t di = 0xFFFFFFFFu;
-	FlatPair fb(lane, A.nv);
-	for (int k = lane; k < B.np * A.nv; k += 64, fb.next())
+	nA = waveList(A.nv, lane, L.elA, [&](int i) { return !(slab && L.va[i].w - maxB > lim); });
+	nB = waveList(B.nv, lane, L.elB, [&](int i) { return !(slab && minA - L.vb[i].w > lim); });
+	waveSync();
+	FlatPair fb(lane, nA);
+	for (int k = lane; k < B.np * nA; k += 64, fb.next())
 	{
-		const int f = fb.i, i = fb.j;
+		const int f = fb.i, i = L.elA[fb.j];
 		const float4 pl = L.pb[f];
-		const f3 bn = mk(pl.x, pl.y, pl.z), va = ldsV(L.va, i);
+		const f3 bn = mk(pl), va = ldsV(L.va, i);
 		const float h = dot(bn, va) + pl.w;
-		if (h < 0.0f || h * h >= d2)
+		if (h < 0.0f || h * h >= d2 || h * h > U)
 			continue;
 		if (!inPolygon(B, f, va - bn * h))
 			continue;
 		d2 = h * h;
-		di = uint32_t(k);
+		di = uint32_t(f * A.nv + i);
 	}
-	FlatPair fa(lane, B.nv);
-	for (int k = lane; k < A.np * B.nv; k += 64, fa.next())
+	FlatPair fa(lane, nB);
+	for (int k = lane; k < A.np * nB; k += 64, fa.next())
 	{
-		const int f = fa.i, i = fa.j;
+		const int f = fa.i, i = L.elB[fa.j];
 		const float4 pl = L.pa[f];
-		const f3 an = mk(pl.x, pl.y, pl.z), vb = ldsV(L.vb, i);
+		const f3 an = mk(pl), vb = ldsV(L.vb, i);
 		const float h = dot(an, vb) + pl.w;
-		if (h < 0.0f || h * h >= d2)
+		if (h < 0.0f || h * h >= d2 || h * h > U)
 			continue;
 		if (!inPolygon(A, f, mxtransinv(aToB, vb - an * h)))
 			continue;
 		d2 = h * h;
-		di = (1u << 24) | uint32_t(k);
+		di = (1u << 24) | uint32_t(f * B.nv + i);
 	}
-	// Edge pairs. The face-vertex pairs bound the squared distance by U; an
-	// edge whose bounding sphere lies farther than sqrt(U) (plus a margin well
-	// above rounding) from the other polytope's bounding box cannot be part of
-	// a pair that reaches U, so only the remaining edges are paired. Pair
-	// indices keep their unpruned order, so the first minimum is unchanged.
-	float U = d2;
-	for (int off = 32; off >= 1; off >>= 1)
-		U = fminf(U, __shfl_xor(U, off));
-	const float lim = U < BIG ? sqrtf(U) + 1e-4f : BIG;
-	int nA = 0, nB = 0;
-	nearEdges(A, B, L, lane, lim, nA, nB);
+	U = waveMin(fminf(U, d2));
+	lim = U < BIG ? sqrtf(U) + 1e-4f : BIG;
 	waveSync();
+	if (slab)
+	{
+		nA = waveList(A.ne, lane, L.elA, [&](int e) {
+			return !(fminf(L.va[L.ea[e] & 0xFF].w, L.va[(L.ea[e] >> 8) & 0xFF].w) - maxB > lim);
+		});
+		nB = waveList(B.ne, lane, L.elB, [&](int e) {
+			return !(minA - fmaxf(L.vb[L.eb[e] & 0xFF].w, L.vb[(L.eb[e] >> 8) & 0xFF].w) > lim);
+		});
+		waveSync();
+	}
+	else
+		nearEdges(A, B, L, lane, lim, nA, nB);
 	FlatPair fe(lane, nB);
 	for (int k = lane; k < nA * nB; k += 64, fe.next())
 	{
 		const int ea = L.elA[fe.i], ebi = L.elB[fe.j];
-		const uint32_t e = L.ea[ea], g = L.eb[ebi];
 		f3 c1, c2;
-		const float s = segClosestSq(ldsV(L.va, int(e & 0xFF)), ldsV(L.va, int((e >> 8) & 0xFF)),
-		                             ldsV(L.vb, int(g & 0xFF)), ldsV(L.vb, int((g >> 8) & 0xFF)), c1, c2);
+		const float s = edgePairSq(L, ea, ebi, c1, c2);
 		if (s < d2)
 		{
 			d2 = s;
@@ -1495,9 +1722,7 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, con
 	else
 	{
 		const int ea = int(k) / B.ne, ebi = int(k) - ea * B.ne;
-		const uint32_t e = L.ea[ea], g = L.eb[ebi];
-		segClosestSq(ldsV(L.va, int(e & 0xFF)), ldsV(L.va, int((e >> 8) & 0xFF)), ldsV(L.vb, int(g & 0xFF)),
-		             ldsV(L.vb, int((g >> 8) & 0xFF)), cA, cB);
+		edgePairSq(L, ea, ebi, cA, cB);
 	}
 	dist = sqrtf(d2);
 	n = (cA - cB) * (1.0f / dist);
@@ -1524,7 +1749,9 @@ PXH_D void convexSeparationWave(const Poly& A, const xf& x0, const Poly& B, cons
 	float best;
 	uint32_t bi;
 	bool sepd;
-	if (faceAxesWave(A, B, cd, L, lane, best, bi, sepd))
+	float gap;
+	uint32_t gi;
+	if (faceAxesWave(A, B, cd, L, lane, best, bi, sepd, gap, gi))
 	{
 		// farther apart than the contact distance
 		sep = make_float4(2.0f * cd + 1.0f, 1.0f, 0.0f, 0.0f);
@@ -1567,7 +1794,7 @@ PXH_D void convexSeparationWave(const Poly& A, const xf& x0, const Poly& B, cons
 	waveSync();
 	float dist = 0.0f;
 	f3 n = mk(1.0f, 0.0f, 0.0f), cA = mk(0.0f, 0.0f, 0.0f), cB = cA;
-	polySeparationWave(Al, aToB, Bl, L, lane, best, bi, sepd, dist, n, cA, cB);
+	polySeparationWave(Al, aToB, Bl, L, lane, best, bi, sepd, gap, gi, dist, n, cA, cB);
 	waveSync();   // the staged data stay in use until every lane is done
 	sep.x = dist;
 	sep.y = n.x; sep.z = n.y; sep.w = n.z;

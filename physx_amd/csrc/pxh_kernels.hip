@@ -954,16 +954,19 @@ PXH_D void blockAppend(bool take, int value, int* out, uint32_t* total)
 	if (lane == 0)
 		waveCnt[w] = uint32_t(__popcll(m));
 	__syncthreads();
-	if (threadIdx.x == 0)
+	if (threadIdx.x < 64)
 	{
-		uint32_t sum = 0;
-		for (int i = 0; i < nw; i++)
+		const uint32_t c = lane < nw ? waveCnt[lane] : 0u;
+		uint32_t sum = c;
+		for (int off = 1; off < 16; off <<= 1)
 		{
-			const uint32_t c = waveCnt[i];
-			waveCnt[i] = sum;
-			sum += c;
+			const uint32_t o = __shfl_up(sum, off);
+			sum += lane >= off ? o : 0u;
 		}
-		blockBase = sum ? atomicAdd(total, sum) : 0u;
+		if (lane < nw)
+			waveCnt[lane] = sum - c;
+		if (lane == nw - 1)
+			blockBase = sum ? atomicAdd(total, sum) : 0u;
 	}
 	__syncthreads();
 	if (take)
@@ -1086,41 +1089,61 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_planes(int Q, int slotBase, c
 	storeContacts(slotBase + q, c, cnt, ctN, ctP);
 }
 
-// Convex pairs: the class segments from *dConvex to *dP hold them; lane q takes
-// pair *dConvex + q. Sphere- and capsule-convex pairs, and the box- and
-// convex-convex pairs whose bounding spheres come within the contact distance,
-// go to their lists, the others get their empty contact slot here. Two lists of
-// cap entries after two counts: 0 pairs to search (k_np_convex_wave and
-// k_np_convex_finish), 1 round pairs (k_np_round_convex).
+// Convex pairs: the class segments from *dConvex to *dP hold them. Sphere- and
+// capsule-convex pairs, and the box- and convex-convex pairs whose bounding
+// spheres come within the contact distance and that a few support steps don't
+// show to be farther apart, go to their lists, the others get their empty
+// contact slot here. Two lists of cap entries after two counts: 0 pairs to
+// search (k_np_convex_wave and k_np_convex_finish), 1 round pairs
+// (k_np_round_convex). Three of four pairs of a rubble pile don't touch; the
+// steps take 8 lanes of a pair where the search takes a wave: of 8,192 hulls'
+// 89,000 pairs, 7 us without and 39 with them, for 386 and 276 us of search.
 PXH_D uint32_t* cvxEntries(uint32_t* list, int cap, int which) { return list + 2 + int64_t(which) * cap; }
 PXH_D const uint32_t* cvxEntries(const uint32_t* list, int cap, int which) { return list + 2 + int64_t(which) * cap; }
-__global__ void __launch_bounds__(256) k_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int slotBase, const uint2* pairs,
-                            const float4* pos, const float4* geom, HullSet hs, float cd, float4* ctN, uint32_t* list)
+constexpr int APART_BLOCK = 1024;
+__global__ void __launch_bounds__(APART_BLOCK) k_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex,
+                            int slotBase, const uint2* pairs, const float4* pos, const float4* rot, const float4* geom,
+                            HullSet hs, float cd, float4* ctN, uint32_t* list)
 {
-	const int q = blockIdx.x * blockDim.x + threadIdx.x;
-	const uint32_t p = *dConvex + uint32_t(q);
-	const bool live = q < cap && p < *dP && p < uint32_t(cap);
-	bool round = false, search = false;
-	if (live)
+	constexpr uint32_t PAIRS = APART_BLOCK / APART_LANES;
+	const uint32_t end = min(*dP, uint32_t(cap));
+	const int sub = threadIdx.x % APART_LANES;
+	for (uint32_t p0 = *dConvex + blockIdx.x * PAIRS; p0 < end; p0 += gridDim.x * PAIRS)
 	{
-		const uint2 ab = pairs[p];
-		const float4 g0 = geom[ab.x], g1 = geom[ab.y];
-		const int t0 = int(g0.w);
-		round = t0 == GEOM_SPHERE || t0 == GEOM_CAPSULE;
-		if (!round)
+		const uint32_t p = p0 + threadIdx.x / APART_LANES;
+		bool round = false, search = false;
+		if (p < end)
 		{
-			const f3 p0 = mk(pos[ab.x]), p1 = mk(pos[ab.y]);
-			const float r0 = t0 == GEOM_BOX ? sqrtf(g0.x * g0.x + g0.y * g0.y + g0.z * g0.z) : hs.be[int(g0.x)].w;
-			const float r1 = hs.be[int(g1.x)].w;
-			const f3 d = p1 - p0;
-			const float reach = r0 + r1 + cd;
-			search = dot(d, d) <= reach * reach;
-			if (!search)
-				ctN[slotBase + int(p)] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
+			const uint2 ab = pairs[p];
+			const float4 g0 = geom[ab.x], g1 = geom[ab.y];
+			const int t0 = int(g0.w);
+			round = t0 == GEOM_SPHERE || t0 == GEOM_CAPSULE;
+			if (!round)
+			{
+				xf x0, x1;
+				x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
+				x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
+				const float r0 = t0 == GEOM_BOX ? sqrtf(g0.x * g0.x + g0.y * g0.y + g0.z * g0.z) : hs.be[int(g0.x)].w;
+				const float r1 = hs.be[int(g1.x)].w;
+				const f3 d = x1.p - x0.p;
+				const float reach = r0 + r1 + cd;
+				search = dot(d, d) <= reach * reach;
+				if (search)
+				{
+					// what the search would round away is left to it
+					const float need = cd + 1e-5f * reach;
+					const Poly B = hullPoly(hs, int(g1.x));
+					const mxf aToB = mxfOf(xinvmul(x1, x0));
+					const Poly A = t0 == GEOM_BOX ? boxPoly(mk(g0.x, g0.y, g0.z)) : hullPoly(hs, int(g0.x));
+					search = !convexApart(A, aToB, B, need, sub);
+				}
+				if (!search && sub == 0)
+					ctN[slotBase + int(p)] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
+			}
 		}
+		blockAppend(search && sub == 0, int(p), reinterpret_cast<int*>(cvxEntries(list, cap, 0)), list);
+		blockAppend(round && sub == 0, int(p), reinterpret_cast<int*>(cvxEntries(list, cap, 1)), list + 1);
 	}
-	blockAppend(search, int(p), reinterpret_cast<int*>(cvxEntries(list, cap, 0)), list);
-	blockAppend(round, int(p), reinterpret_cast<int*>(cvxEntries(list, cap, 1)), list + 1);
 }
 
 // sphere- and capsule-convex pairs of list 1
@@ -1153,7 +1176,11 @@ __global__ void __launch_bounds__(64) k_np_round_convex(int cap, int slotBase, c
 // Box- and convex-convex pairs, separation phase: one wavefront per pair
 // (grid-stride over the search list k_np_convex wrote) finds the closest
 // features or the minimum translation and stores (dist, n), cA, cB at
-// wit[3p .. 3p+2]; the contact phase looks at every searched pair's distance
+// wit[3p .. 3p+2]; bound by vector instructions (half of its time at 386 us),
+// so what it saves are pairs, edges and lanes without a result: 542 us at 8,192
+// hulls of 24 points before crossing arcs were listed and closest features
+// bounded, 386 after, 276 with k_np_convex's steps, 261 with B's arcs laid out.
+// The contact phase looks at every searched pair's distance
 // (a list of the touching ones, an atomic on one word for each, cost 32 us of
 // 574 at 8,192 hulls). Polytopes past the LDS limits are searched by lane 0
 // alone.
@@ -3934,7 +3961,8 @@ void launch_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int 
 	if (cap <= 0)
 		return;
 	k_fill_u32<<<1, 64, 0, st>>>(list, 2, 0u);
-	PXH_LAUNCH(k_np_convex, cap, cap, dP, dConvex, slotBase, pairs, pos, geom, hs, cd, ctN, list);
+	k_np_convex<<<std::min((cap + APART_BLOCK / APART_LANES - 1) / (APART_BLOCK / APART_LANES), 1024), APART_BLOCK, 0, st>>>(
+		cap, dP, dConvex, slotBase, pairs, pos, rot, geom, hs, cd, ctN, list);
 	// grid-stride: enough waves to fill the chip several times over
 	const int blocks = std::min((cap + CVX_WAVES - 1) / CVX_WAVES, 8192);
 	k_np_convex_wave<<<blocks, 64 * CVX_WAVES, 0, st>>>(cap, pairs, pos, rot, geom, hs, cd, wit, list);
