@@ -348,11 +348,11 @@ void launch_sleep_islands(int n, int Q, int cap, const uint32_t* dP, const uint2
                           SleepState ss, hipStream_t st);
 // body-mesh contacts of the nMB bodies of meshBody (worlds with a mesh;
 // worldMesh[w] = first tree node, node count, or -1) into slots
-// slotBase + k * MESH_MAXP + patch; *overflow set when a body meets more than
-// MESH_MAX_TRIS triangles
+// slotBase + k * MESH_MAXP + patch. state holds 2 + nMB words: set when a body meets
+// more than MESH_MAX_TRIS triangles; bodies left to the lane form, their count first
 void launch_np_mesh(int nMB, const int* meshBody, const int* world, const int4* worldMesh, const MeshSet& M,
                     const float4* pos, const float4* rot, const float4* geom, const HullSet& hs, float cd,
-                    int slotBase, float4* ctN, float4* ctP, uint32_t* overflow, hipStream_t st);
+                    int slotBase, float4* ctN, float4* ctP, uint32_t* state, hipStream_t st);
 // PxRigidDynamic::wakeUp of k bodies (device indices)
 void launch_sleep_wake_bodies(int k, const int* bodies, SleepState ss, hipStream_t st);
 // sleep state readback: wake counter and asleep flag per body

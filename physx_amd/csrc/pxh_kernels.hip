@@ -979,8 +979,8 @@ PXH_D void blockAppend(bool take, int value, int* out, uint32_t* total)
 // full: a wave of 64 such lanes runs every branch of every lane one after the
 // other, while most compute units idle. THIN_BLOCKS waves take `lanes` items
 // each at a time, one until there are more items than waves. 2,116 bodies on a
-// mesh: 584 us in 64-lane waves, 279 so; their sphere- and capsule-hull pairs
-// 209 and 89 us, the hull contacts 101 and 50.
+// mesh: their sphere- and capsule-hull pairs 209 us in 64-lane waves and 89 so,
+// the hull contacts 101 and 50.
 constexpr int THIN_BLOCKS = 4096;
 __host__ __device__ inline int thinLanes(uint32_t count)
 {
@@ -2978,13 +2978,105 @@ PXH_D void meshContactsOf(int k, const int* meshBody, const int* world, const in
 	}
 }
 
-__global__ void __launch_bounds__(64) k_np_mesh(int nMB, const int* meshBody, const int* world, const int4* worldMesh,
-                                                MeshSet M, const float4* pos, const float4* rot, const float4* geom,
-                                                HullSet hs, float cd, int slotBase, float4* ctN, float4* ctP,
-                                                uint32_t* overflow)
+// The same over a wave per body (pxh_mesh.h): every body but those a wave can't
+// hold, which go to rest (a count, then their k).
+__global__ void __launch_bounds__(64) k_np_mesh_wave(int nMB, const int* meshBody, const int* world,
+                                                     const int4* worldMesh, MeshSet M, const float4* pos,
+                                                     const float4* rot, const float4* geom, HullSet hs, float cd,
+                                                     int slotBase, float4* ctN, float4* ctP, uint32_t* overflow,
+                                                     uint32_t* rest)
 {
-	PXH_THIN_LOOP(k, nMB)
-		meshContactsOf(int(k), meshBody, world, worldMesh, M, pos, rot, geom, hs, cd, slotBase, ctN, ctP, overflow);
+	__shared__ MeshLds L;
+	const int lane = threadIdx.x;
+	for (int k = blockIdx.x; k < nMB; k += gridDim.x)
+	{
+		const int i = meshBody[k];
+		const int base = slotBase + k * MESH_MAXP;
+		const int4 wm = worldMesh[world[i]];
+		int nc = 0;
+		if (wm.x >= 0)
+		{
+			f3 mn, mx;
+			shapeBounds(i, pos, rot, geom, hs, mn, mx);
+			nc = meshCandidates(M, wm.x, wm.y, mn - mk(cd, cd, cd), mx + mk(cd, cd, cd), L, lane);
+		}
+		if (nc > MESH_MAX_TRIS)
+		{
+			if (lane == 0)
+				atomicOr(overflow, 1u);
+			nc = 0;
+		}
+		MeshWave P;
+		P.init(lane);
+		int type = GEOM_SPHERE;
+		bool done = true;
+		if (nc > 0)
+		{
+			const float4 g = geom[i];
+			type = int(g.w);
+			xf x;
+			x.p = mk(pos[i]);
+			x.q = mkq(rot[i]);
+			if (type == GEOM_SPHERE || type == GEOM_CAPSULE)
+			{
+				const f3 tmp = qrot(x.q, mk(1.0f, 0.0f, 0.0f)) * g.y;
+				done = nc <= 64;
+				if (done && type == GEOM_SPHERE)
+					meshRoundWave<false>(M, L.idx, nc, x.p, x.p, x.p, g.x, cd, lane, P);
+				else if (done)
+					meshRoundWave<true>(M, L.idx, nc, x.p + tmp, x.p - tmp, x.p, g.x, cd, lane, P);
+			}
+			else
+				done = meshPolyWave(M, nc, type == GEOM_CONVEXMESH ? hullPoly(hs, int(g.x)) : boxPoly(mk(g.x, g.y, g.z)),
+				                    x, cd, L, lane, P);
+		}
+		if (done)
+		{
+			// patches by their least separation, the first among equals
+			int rank = 0;
+			for (int j = 0; j < P.np; j++)
+			{
+				const float v = laneOf(P.maxPen, j * (MESH_PC + 1));
+				rank += v < P.maxPen || (v == P.maxPen && j < P.patch);
+			}
+			const int keep = P.np < MESH_MAXP ? P.np : MESH_MAXP;
+			for (int a = 0; a < MESH_MAXP; a++)
+			{
+				const uint64_t m = __ballot(a < keep && P.patch < P.np && rank == a);
+				if (m == 0ull)
+				{
+					if (lane == 0)
+						ctN[base + a].w = __int_as_float(0);
+					continue;
+				}
+				const int l0 = firstLane(m);
+				int cnt = P.reduce4(l0, laneOf(P.count, l0)), from = l0;
+				if (type == GEOM_SPHERE)
+				{
+					for (int j = 1; j < cnt; j++)
+						if (laneOf(P.s, from) > laneOf(P.s, l0 + j)) from = l0 + j;
+					cnt = 1;
+				}
+				if (lane == l0)
+					ctN[base + a] = f4(P.n, __int_as_float(cnt));
+				if (lane >= from && lane < from + cnt)
+					ctP[4 * int64_t(base + a) + lane - from] = f4(P.p, P.s);
+			}
+		}
+		else if (lane == 0)
+			rest[1 + atomicAdd(rest, 1u)] = uint32_t(k);
+		waveSync();
+	}
+}
+
+__global__ void __launch_bounds__(64) k_np_mesh_rest(const uint32_t* rest, const int* meshBody, const int* world,
+                                                     const int4* worldMesh, MeshSet M, const float4* pos,
+                                                     const float4* rot, const float4* geom, HullSet hs, float cd,
+                                                     int slotBase, float4* ctN, float4* ctP, uint32_t* overflow)
+{
+	PXH_THIN_LOOP(q, rest[0])
+		meshContactsOf(int(rest[1 + q]), meshBody, world, worldMesh, M, pos, rot, geom, hs, cd, slotBase, ctN, ctP,
+		               overflow);
 }
 
 // whether the bodies of a pair are joined: its (lower, higher) key is among
@@ -4026,11 +4118,16 @@ void launch_sleep_islands(int n, int Q, int cap, const uint32_t* dP, const uint2
 }
 void launch_np_mesh(int nMB, const int* meshBody, const int* world, const int4* worldMesh, const MeshSet& M,
                     const float4* pos, const float4* rot, const float4* geom, const HullSet& hs, float cd,
-                    int slotBase, float4* ctN, float4* ctP, uint32_t* overflow, hipStream_t st)
+                    int slotBase, float4* ctN, float4* ctP, uint32_t* state, hipStream_t st)
 {
-	if (nMB > 0)
-		k_np_mesh<<<thinGrid(nMB), 64, 0, st>>>(nMB, meshBody, world, worldMesh, M, pos, rot, geom, hs, cd, slotBase,
-		                                        ctN, ctP, overflow);
+	if (nMB <= 0)
+		return;
+	uint32_t* rest = state + 1;
+	k_fill_u32<<<1, 64, 0, st>>>(state, 2, 0u);
+	k_np_mesh_wave<<<std::min(nMB, 8192), 64, 0, st>>>(nMB, meshBody, world, worldMesh, M, pos, rot, geom, hs, cd,
+	                                                   slotBase, ctN, ctP, state, rest);
+	k_np_mesh_rest<<<thinGrid(nMB), 64, 0, st>>>(rest, meshBody, world, worldMesh, M, pos, rot, geom, hs, cd, slotBase,
+	                                             ctN, ctP, state);
 }
 void launch_sleep_wake_bodies(int k, const int* bodies, SleepState ss, hipStream_t st)
 {

@@ -1788,8 +1788,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		s->profEnd(pk);
 		if (nMB > 0)
 		{
-			PXH_CHECK(s->meshOverflow.ensure(1));
-			pxh::launch_fill_u32(s->meshOverflow.p, 1, 0u, st);
+			PXH_CHECK(s->meshOverflow.ensure(2 + size_t(nMB)));
 			pxh::launch_np_mesh(nMB, s->meshBody.p, s->scene.p, s->worldMesh.p, s->meshSet(), s->pos.p, s->rot.p,
 			                    s->geom.p, s->hullSet(), cd, pairEnd, s->ctN.p, s->ctP.p, s->meshOverflow.p, st);
 		}
