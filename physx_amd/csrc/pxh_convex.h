@@ -373,7 +373,7 @@ PXH_D float triArea2(f3 a, f3 b, f3 c)
 }
 
 // Gu::contains (geomutils/src/pcm/GuPCMContactGenUtil.cpp:35-103) for an n-gon
-PXH_D bool polyContainsN(const f3* verts, int nv, f3 p, f3 mn, f3 mx)
+template <class V> PXH_D bool polyContainsN(const V* verts, int nv, f3 p, f3 mn, f3 mx)
 {
 	if ((mn.x > p.x || p.x > mx.x) || (mn.y > p.y || p.y > mx.y))
 		return false;
@@ -399,223 +399,6 @@ PXH_D bool polyContainsN(const f3* verts, int nv, f3 p, f3 mn, f3 mx)
 		}
 	}
 	return inter > 0;
-}
-
-// generatedContacts (geomutils/src/pcm/GuPCMContactGenBoxConvex.cpp:331-530):
-// reference polygon `ref` of P0, incident polygon `inc` of P1, t0To1 maps
-// P0's frame to P1's. Points keep la on P1 (P1's frame), lb on P0's
-// reference plane (P0's frame), ln the reference normal (P0's frame).
-PXH_D void generatedContacts(const Poly& P0, const Poly& P1, int ref, int inc, const mxf& t0To1, PC* mc, int& nc,
-                             float cd)
-{
-	const float feps = 1.1920928955078125e-7f;
-	const f3 n = normalize(P0.pn(ref));
-	const m33 rot = rotFromZ(n);
-	const int nr = P0.pcount(ref), ni = P1.pcount(inc);
-	f3 p0[HULL_MAX_POLY_VERTS], p1[HULL_MAX_POLY_VERTS];
-	float t1[HULL_MAX_POLY_VERTS];
-	bool pen1[HULL_MAX_POLY_VERTS];
-	const f3 sPoint = P1.vert(P1.pvert(inc, 0));
-	f3 rMin = mk(FLT_BIG, FLT_BIG, FLT_BIG), rMax = -rMin;
-	for (int i = 0; i < nr; i++)
-	{
-		p0[i] = mmul(rot, P0.vert(P0.pvert(ref, i)));
-		rMin = mk(fminf(rMin.x, p0[i].x), fminf(rMin.y, p0[i].y), fminf(rMin.z, p0[i].z));
-		rMax = mk(fmaxf(rMax.x, p0[i].x), fmaxf(rMax.y, p0[i].y), fmaxf(rMax.z, p0[i].z));
-	}
-	rMin = rMin - mk(feps, feps, feps);
-	rMax = rMax + mk(feps, feps, feps);
-	const float d = p0[0].z, rd = d + cd;
-	f3 iMin = mk(FLT_BIG, FLT_BIG, FLT_BIG), iMax = -iMin;
-	int inside = 0;
-	for (int i = 0; i < ni; i++)
-	{
-		const f3 vert1 = P1.vert(P1.pvert(inc, i));
-		const f3 a = mxtransinv(t0To1, vert1);
-		f3 q = mmul(rot, a);
-		const float z = q.z;
-		t1[i] = z - d;
-		q.z = d;
-		p1[i] = q;
-		iMin = mk(fminf(iMin.x, q.x), fminf(iMin.y, q.y), fminf(iMin.z, q.z));
-		iMax = mk(fmaxf(iMax.x, q.x), fmaxf(iMax.y, q.y), fmaxf(iMax.z, q.z));
-		pen1[i] = rd > z;
-		if (pen1[i] && polyContainsN(p0, nr, q, rMin, rMax))
-		{
-			inside++;
-			if (nc == HULL_MAX_CONTACTS)
-				return;
-			PC& c = mc[nc++];
-			c.la = vert1;
-			c.lb = mtmul(rot, q);
-			c.ln = n;
-			c.pen = t1[i];
-		}
-	}
-	if (inside == ni)
-		return;
-	inside = 0;
-	iMin = iMin - mk(feps, feps, feps);
-	iMax = iMax + mk(feps, feps, feps);
-	const f3 incN = normalize(P1.pn(inc));
-	const f3 nIn1 = mmul(t0To1.r, n);
-	for (int i = 0; i < nr; i++)
-	{
-		if (!polyContainsN(p1, ni, p0[i], iMin, iMax))
-			continue;
-		const f3 vert0 = mtmul(rot, p0[i]);
-		const f3 a = mxtrans(t0To1, vert0);
-		const float t = dot(incN, sPoint - a) / dot(incN, nIn1);
-		if (t > cd)
-			continue;
-		inside++;
-		if (nc == HULL_MAX_CONTACTS)
-			return;
-		PC& c = mc[nc++];
-		c.la = nIn1 * t + a;
-		c.lb = vert0;
-		c.ln = n;
-		c.pen = t;
-	}
-	if (inside == nr)
-		return;
-	for (int iS = 0, iE = ni - 1; iS < ni; iE = iS++)
-	{
-		if (!pen1[iS] && !pen1[iE])
-			continue;
-		const f3 ipA = p1[iS], ipB = p1[iE];
-		const f3 ipAO = mk(ipA.x, ipA.y, t1[iS] + d), ipBO = mk(ipB.x, ipB.y, t1[iE] + d);
-		const float iMnx = fminf(ipA.x, ipB.x), iMny = fminf(ipA.y, ipB.y);
-		const float iMxx = fmaxf(ipA.x, ipB.x), iMxy = fmaxf(ipA.y, ipB.y);
-		for (int rS = 0, rE = nr - 1; rS < nr; rE = rS++)
-		{
-			const f3 rpA = p0[rS], rpB = p0[rE];
-			const float rMnx = fminf(rpA.x, rpB.x), rMny = fminf(rpA.y, rpB.y);
-			const float rMxx = fmaxf(rpA.x, rpB.x), rMxy = fmaxf(rpA.y, rpB.y);
-			if (iMnx > rMxx || iMny > rMxy || rMnx > iMxx || rMny > iMxy)
-				continue;
-			const float a1 = triArea2(rpA, rpB, ipA), a2 = triArea2(rpA, rpB, ipB);
-			if (!(0.0f > a1 * a2))
-				continue;
-			const float a3 = triArea2(ipA, ipB, rpA), a4 = triArea2(ipA, ipB, rpB);
-			if (!(0.0f > a3 * a4))
-				continue;
-			const float t = a1 / (a2 - a1);
-			const f3 pBB = ipAO - (ipBO - ipAO) * t;
-			const f3 pAA = mk(pBB.x, pBB.y, d);
-			const float pen = pBB.z - pAA.z;
-			if (pen > cd)
-				continue;
-			if (nc == HULL_MAX_CONTACTS)
-				return;
-			PC& c = mc[nc++];
-			c.la = mxtrans(t0To1, mtmul(rot, pBB));
-			c.lb = mtmul(rot, pAA);
-			c.ln = n;
-			c.pen = pen;
-		}
-	}
-}
-
-// reduction to four (PersistentContactManifold::addBatchManifoldContacts,
-// geomutils/src/pcm/GuPersistentContactManifold.cpp:805-830)
-PXH_D int batchReduce(PC* mc, int nc, float tol)
-{
-	if (nc <= 4)
-		return nc;
-	int ch[4];
-	reduceBatchT<HULL_MAX_CONTACTS>(mc, nc, tol, ch);
-	PC out[4];
-	for (int i = 0; i < 4; i++)
-		out[i] = mc[ch[i]];
-	for (int i = 0; i < 4; i++)
-		mc[i] = out[i];
-	return 4;
-}
-
-// manifold -> contacts: points on shape1 in the world, the summed normal,
-// points within the contact distance (PersistentContactManifold::
-// addManifoldContactsToContactBuffer / getWorldNormal,
-// geomutils/src/pcm/GuPersistentContactManifold.cpp:739-762, GuPersistentContactManifold.h:405-416)
-PXH_D int manifoldOut(const PC* m, int n, const xf& x1, float cd, Contacts& o)
-{
-	if (n == 0)
-		return 0;
-	f3 s = m[0].ln;
-	for (int i = 1; i < n; i++)
-		s = s + m[i].ln;
-	o.n = normalize(qrot(x1.q, s));
-	int k = 0;
-	for (int i = 0; i < n && k < 4; i++)
-		if (cd >= m[i].pen)
-		{
-			o.p[k] = xtrans(x1, m[i].lb);
-			o.sep[k] = m[i].pen;
-			k++;
-		}
-	o.count = k;
-	return k;
-}
-
-// Contacts of a box- or convex-convex pair from its separation (dist, n from
-// B towards A, closest points or minimum-translation witnesses cA, cB in B's
-// frame): witness polygons, clipping and reduction to four.
-PXH_D int convexContactsFrom(const Poly& A, const xf& x0, const Poly& B, const xf& x1, const mxf& aToB, float dist,
-                             f3 n, f3 cA, f3 cB, float cd, float tol, Contacts& o)
-{
-	if (dist > cd)
-		return 0;
-	const float lo = tol * 1e-2f, hi = tol * 5e-2f;
-	const float tA = fminf(fmaxf(A.margin, lo), hi), tB = fminf(fmaxf(B.margin, lo), hi);
-	const f3 negN = -n;
-	const f3 nIn0 = mtmul(aToB.r, n);
-	const int f1 = witnessPolygon(B, negN, cB, tB);
-	const int f0 = witnessPolygon(A, nIn0, mxtransinv(aToB, cA), tA);
-	const f3 refN = normalize(B.pn(f1)), incN = normalize(A.pn(f0));
-	PC mc[HULL_MAX_CONTACTS];
-	int nc = 0;
-	if (fabsf(dot(refN, negN)) >= fabsf(dot(incN, nIn0)))
-	{
-		const mxf bToA = mxfOf(xinvmul(x0, x1));
-		generatedContacts(B, A, f1, f0, bToA, mc, nc, cd);
-	}
-	else
-	{
-		generatedContacts(A, B, f0, f1, aToB, mc, nc, cd);
-		const f3 nn = -mmul(aToB.r, incN);
-		for (int i = 0; i < nc; i++)
-		{
-			const f3 t = mc[i].lb;
-			mc[i].lb = mc[i].la;
-			mc[i].la = t;
-			mc[i].ln = nn;
-		}
-	}
-	if (nc == 0)
-	{
-		// the closest-feature / minimum-translation point stays the only point
-		mc[0].la = mxtransinv(aToB, cA);
-		mc[0].lb = cB;
-		mc[0].ln = n;
-		mc[0].pen = dist;
-		nc = 1;
-	}
-	else
-		nc = batchReduce(mc, nc, tol);
-	return manifoldOut(mc, nc, x1, cd, o);
-}
-
-// Gu::pcmContactConvexConvex / pcmContactBoxConvex on a fresh manifold
-// (geomutils/src/pcm/GuPCMContactConvexConvex.cpp:111-276, GuPCMContactBoxConvex.cpp;
-// Gu::generateFullContactManifold and Gu::addGJKEPAContacts,
-// GuPCMContactGenBoxConvex.cpp:532-720). A is shape0, B is shape1.
-PXH_D int convexConvex(const Poly& A, const xf& x0, const Poly& B, const xf& x1, float cd, float tol, Contacts& o)
-{
-	const mxf aToB = mxfOf(xinvmul(x1, x0));
-	float dist = 0.0f;
-	f3 n = mk(1.0f, 0.0f, 0.0f), cA = mk(0.0f, 0.0f, 0.0f), cB = cA;
-	polySeparation(A, aToB, B, cd, dist, n, cA, cB);
-	return convexContactsFrom(A, x0, B, x1, aToB, dist, n, cA, cB, cd, tol, o);
 }
 
 // Gu::pcmContactSphereConvex on a fresh manifold
@@ -997,105 +780,6 @@ PXH_D int capsulePoly(float r, float hh, const xf& x0, const Poly& B, const xf& 
 			pushContact(o, xtrans(x0, c.la) - wn * r, sep);
 	}
 	return o.count;
-}
-
-// Gu::pcmContactPlaneConvex on a fresh manifold
-// (geomutils/src/pcm/GuPCMContactPlaneConvex.cpp:36-227): the face most
-// opposed to the plane normal, or the better face of the edge whose summed
-// face normals are most opposed to it (5e-4 bias towards edges); the chosen
-// face's vertices below the contact distance, taken once more when an edge
-// was chosen (the reference passes over the same face twice); reduced to
-// four. Normal from the hull towards the plane.
-PXH_D int planeConvex(f3 pn, float pd, const Poly& B, const xf& tb, float cd, float tol, Contacts& o)
-{
-	const f3 n = normalize(qrotinv(tb.q, pn));
-	const f3 nn = -n;
-	float minProj = FLT_BIG;
-	int face = 0;
-	for (int i = 0; i < B.np; i++)
-	{
-		const float proj = dot(n, B.pn(i));
-		if (minProj > proj) { minProj = proj; face = i; }
-	}
-	int edgeSel = -1;
-	minProj = minProj - 5e-4f;
-	float maxDpSq = minProj * minProj;
-	for (int e = 0; e < B.ne; e++)
-	{
-		const uint32_t g = B.edge(e);
-		const f3 en = B.pn(int((g >> 16) & 0xFF)) + B.pn(int(g >> 24));
-		const float enMagSq = dot(en, en);
-		const float dp = dot(en, nn);
-		const float sqDp = dp * dp;
-		if (dp >= 0.0f && sqDp > maxDpSq * enMagSq)
-		{
-			maxDpSq = sqDp / enMagSq;
-			edgeSel = e;
-		}
-	}
-	int passes = 1;
-	if (edgeSel >= 0)
-	{
-		const uint32_t g = B.edge(edgeSel);
-		const int f0 = int((g >> 16) & 0xFF), f1 = int(g >> 24);
-		face = dot(B.pn(f0), nn) > dot(B.pn(f1), nn) ? f0 : f1;
-		passes = 2;
-	}
-	PC mc[HULL_MAX_CONTACTS];
-	int nc = 0;
-	float deepest = FLT_BIG;
-	int dv = 0;
-	for (int i = 0; i < B.nv; i++)
-	{
-		const float s = dot(pn, xtrans(tb, B.vert(i))) + pd;
-		if (s < deepest) { deepest = s; dv = i; }
-	}
-	bool deepestTaken = false;
-	const int cnt = B.pcount(face);
-	for (int pass = 0; pass < passes; pass++)
-		for (int k = 0; k < cnt; k++)
-		{
-			const int vi = B.pvert(face, k);
-			const f3 lv = B.vert(vi);
-			const f3 pw = xtrans(tb, lv);
-			const float s = dot(pn, pw) + pd;
-			if (cd > s && nc < HULL_MAX_CONTACTS)
-			{
-				mc[nc].la = lv;
-				mc[nc].lb = pw - pn * s;
-				mc[nc].ln = pn;
-				mc[nc].pen = s;
-				nc++;
-				deepestTaken |= vi == dv;
-			}
-		}
-	// Deliberate deviation: when the chosen face does not hold the hull's
-	// deepest vertex (an irregular hull can rest on a vertex that the face most
-	// opposed to the plane does not contain), that vertex joins the batch. The
-	// reference scene's persistent manifold keeps such a vertex from earlier
-	// steps; a step that generates contacts afresh has to add it.
-	if (!deepestTaken && cd > deepest && nc < HULL_MAX_CONTACTS)
-	{
-		const f3 lv = B.vert(dv);
-		const f3 pw = xtrans(tb, lv);
-		mc[nc].la = lv;
-		mc[nc].lb = pw - pn * deepest;
-		mc[nc].ln = pn;
-		mc[nc].pen = deepest;
-		nc++;
-	}
-	nc = batchReduce(mc, nc, tol);
-	o.n = -pn;
-	int k = 0;
-	for (int i = 0; i < nc; i++)
-		if (cd >= mc[i].pen)
-		{
-			o.p[k] = mc[i].lb;
-			o.sep[k] = mc[i].pen;
-			k++;
-		}
-	o.count = k;
-	return k;
 }
 
 }  // namespace pxh
@@ -1800,6 +1484,451 @@ PXH_D void convexSeparationWave(const Poly& A, const xf& x0, const Poly& B, cons
 	sep.y = n.x; sep.z = n.y; sep.w = n.z;
 	wA = cA;
 	wB = cB;
+}
+
+// ---------------------------------------------------------------------------
+// Contacts of a pair over a wave. In one lane the polygons, the points and the
+// reduction's candidates lie in scratch memory and every face, vertex and edge
+// waits for the one before: 107 us for the pairs of 8,192 hulls that touch, 65
+// for their plane pairs (16-lane waves). Here the wave scans the faces, takes a
+// vertex or an edge pair a lane and keeps the points in the order of the lane
+// form, so the choices are the same.
+// ---------------------------------------------------------------------------
+struct ContactLds
+{
+	float4 p0[HULL_MAX_POLY_VERTS], p1[HULL_MAX_POLY_VERTS];   // the polygons in the reference polygon's frame
+	float4 pts[HULL_MAX_CONTACTS];                             // point, separation
+};
+
+PXH_D int laneOf(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+PXH_D float laneOf(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
+PXH_D f3 laneOf(f3 v, int l) { return mk(laneOf(v.x, l), laneOf(v.y, l), laneOf(v.z, l)); }
+PXH_D float4 laneOf(float4 v, int l)
+{
+	return make_float4(laneOf(v.x, l), laneOf(v.y, l), laneOf(v.z, l), laneOf(v.w, l));
+}
+
+PXH_D int laneRank(uint64_t m, int lane) { return int(__popcll(m & ((1ull << lane) - 1ull))); }
+
+// witnessPolygon
+PXH_D int witnessPolygonWave(const Poly& P, f3 normal, f3 closest, float tolerance, int lane)
+{
+	const float eps = -tolerance;
+	float minDist = FLT_BIG, least = FLT_BIG;   // least: minus the largest distance
+	uint32_t first = 0u, maxIdx = 0xFFFFFFFFu;
+	if (lane > 0)
+		first = 0xFFFFFFFFu;
+	for (int i = lane; i < P.np; i += 64)
+	{
+		const float dist = dot(P.pn(i), closest) + P.pd(i);
+		const float pdi = dist >= eps ? fabsf(dist) : FLT_BIG;
+		if (minDist > pdi) { minDist = pdi; first = uint32_t(i); }
+		if (-dist < least) { least = -dist; maxIdx = uint32_t(i); }
+	}
+	waveArgMin(minDist, first);
+	if (minDist == FLT_BIG)
+	{
+		waveArgMin(least, maxIdx);
+		return maxIdx == 0xFFFFFFFFu ? 0 : int(maxIdx);
+	}
+	const float firstProj = dot(normalize(P.pn(int(first))), normal);
+	float bestProj = firstProj;
+	uint32_t idx = 0xFFFFFFFFu;
+	for (int i = lane; i < P.np; i += 64)
+	{
+		const f3 pn = P.pn(i);
+		const float di = dot(pn, closest) + P.pd(i);
+		const float pdi = di >= eps ? fabsf(di) : FLT_BIG;
+		if ((tolerance > (pdi - minDist)) && (int(first) != i))
+		{
+			const float proj = dot(normalize(pn), normal);
+			if (bestProj > proj) { idx = uint32_t(i); bestProj = proj; }
+		}
+	}
+	waveArgMin(bestProj, idx);
+	return idx == 0xFFFFFFFFu ? int(first) : int(idx);
+}
+
+// the bounds of the lanes' points that have one, widened
+PXH_D void waveBounds(bool has, f3 p, f3& mn, f3& mx)
+{
+	const float feps = 1.1920928955078125e-7f;
+	mn = has ? p : mk(FLT_BIG, FLT_BIG, FLT_BIG);
+	mx = has ? p : -mk(FLT_BIG, FLT_BIG, FLT_BIG);
+	for (int off = HULL_MAX_POLY_VERTS / 2; off >= 1; off >>= 1)
+	{
+		mn.x = fminf(mn.x, __shfl_xor(mn.x, off));
+		mn.y = fminf(mn.y, __shfl_xor(mn.y, off));
+		mx.x = fmaxf(mx.x, __shfl_xor(mx.x, off));
+		mx.y = fmaxf(mx.y, __shfl_xor(mx.y, off));
+	}
+	mn = laneOf(mn, 0) - mk(feps, feps, feps);
+	mx = laneOf(mx, 0) + mk(feps, feps, feps);
+}
+
+// generatedContacts (geomutils/src/pcm/GuPCMContactGenBoxConvex.cpp:331-530) into
+// L.pts: reference polygon `ref` of P0, incident polygon `inc` of P1, t0To1 maps
+// P0's frame to P1's; the points on P1 (its frame, onP1) or on P0's reference
+// plane (its frame), first the incident vertices inside, then the reference ones,
+// then the edge crossings; their number
+PXH_D int generatedContactsWave(const Poly& P0, const Poly& P1, int ref, int inc, const mxf& t0To1, float cd, bool onP1,
+                                ContactLds& L, int lane)
+{
+	const f3 n = normalize(P0.pn(ref));
+	const m33 rot = rotFromZ(n);
+	const int nr = P0.pcount(ref), ni = P1.pcount(inc);
+	const bool isRef = lane < nr, isInc = lane < ni;
+	f3 q0 = mk(0.0f, 0.0f, 0.0f), q1 = q0, vert1 = q0, mn, mx;
+	if (isRef)
+	{
+		q0 = mmul(rot, P0.vert(P0.pvert(ref, lane)));
+		L.p0[lane] = f4(q0, 0.0f);
+	}
+	const float d = laneOf(q0.z, 0), rd = d + cd;
+	float t1 = 0.0f;
+	bool pen = false;
+	if (isInc)
+	{
+		vert1 = P1.vert(P1.pvert(inc, lane));
+		q1 = mmul(rot, mxtransinv(t0To1, vert1));
+		const float z = q1.z;
+		t1 = z - d;
+		q1.z = d;
+		L.p1[lane] = f4(q1, t1);
+		pen = rd > z;
+	}
+	const uint64_t pens = __ballot(pen);
+	const f3 sPoint = laneOf(vert1, 0);
+	waveSync();
+	waveBounds(isRef, q0, mn, mx);
+	bool in = pen && polyContainsN(L.p0, nr, q1, mn, mx);
+	uint64_t m = __ballot(in);
+	if (in)
+		L.pts[laneRank(m, lane)] = f4(onP1 ? vert1 : mtmul(rot, q1), t1);
+	int nc = int(__popcll(m));
+	if (nc == ni)
+		return nc;
+	waveBounds(isInc, q1, mn, mx);
+	const f3 incN = normalize(P1.pn(inc));
+	const f3 nIn1 = mmul(t0To1.r, n);
+	in = isRef && polyContainsN(L.p1, ni, q0, mn, mx);
+	f3 vert0 = q0, a = q0;
+	float t = 0.0f;
+	if (in)
+	{
+		vert0 = mtmul(rot, q0);
+		a = mxtrans(t0To1, vert0);
+		t = dot(incN, sPoint - a) / dot(incN, nIn1);
+		in = !(t > cd);
+	}
+	m = __ballot(in);
+	if (in)
+		L.pts[nc + laneRank(m, lane)] = f4(onP1 ? nIn1 * t + a : vert0, t);
+	const int inside = int(__popcll(m));
+	nc += inside;
+	if (inside == nr)
+		return nc;
+	FlatPair fp(lane, nr);
+	for (int k = lane; __any(k < ni * nr); k += 64, fp.next())
+	{
+		bool hit = k < ni * nr;
+		f3 pt = q0;
+		float sep = 0.0f;
+		if (hit)
+		{
+			const int iS = fp.i, rS = fp.j, iE = iS == 0 ? ni - 1 : iS - 1, rE = rS == 0 ? nr - 1 : rS - 1;
+			const float4 sA = L.p1[iS], sB = L.p1[iE];
+			const f3 ipA = mk(sA), ipB = mk(sB), rpA = mk(L.p0[rS]), rpB = mk(L.p0[rE]);
+			const float a1 = triArea2(rpA, rpB, ipA), a2 = triArea2(rpA, rpB, ipB);
+			const float a3 = triArea2(ipA, ipB, rpA), a4 = triArea2(ipA, ipB, rpB);
+			hit = (((pens >> iS) | (pens >> iE)) & 1ull) != 0ull &&
+			      !(fminf(ipA.x, ipB.x) > fmaxf(rpA.x, rpB.x) || fminf(ipA.y, ipB.y) > fmaxf(rpA.y, rpB.y) ||
+			        fminf(rpA.x, rpB.x) > fmaxf(ipA.x, ipB.x) || fminf(rpA.y, rpB.y) > fmaxf(ipA.y, ipB.y)) &&
+			      0.0f > a1 * a2 && 0.0f > a3 * a4;
+			if (hit)
+			{
+				const f3 ipAO = mk(ipA.x, ipA.y, sA.w + d), ipBO = mk(ipB.x, ipB.y, sB.w + d);
+				const float u = a1 / (a2 - a1);
+				const f3 pBB = ipAO - (ipBO - ipAO) * u;
+				const f3 pAA = mk(pBB.x, pBB.y, d);
+				sep = pBB.z - pAA.z;
+				hit = !(sep > cd);
+				pt = onP1 ? mxtrans(t0To1, mtmul(rot, pBB)) : mtmul(rot, pAA);
+			}
+		}
+		m = __ballot(hit);
+		const int to = nc + laneRank(m, lane);
+		if (hit && to < HULL_MAX_CONTACTS)
+			L.pts[to] = f4(pt, sep);
+		nc += int(__popcll(m));
+		if (nc >= HULL_MAX_CONTACTS)
+			return HULL_MAX_CONTACTS;
+	}
+	return nc;
+}
+
+// Reduction to four (PersistentContactManifold::addBatchManifoldContacts,
+// geomutils/src/pcm/GuPersistentContactManifold.cpp:805-830) of the points in LDS
+// (their common normal cn0): their number, and in lane i the i-th
+PXH_D int batchReduceWave(const float4* pts, int n, f3 cn0, float tol, int lane, float4& out)
+{
+	float4 c = pts[lane < n ? lane : 0];
+	out = c;
+	if (n <= 4)
+		return n;
+	int nc = n;
+	// lane i holds candidate i; one that is taken leaves its place to the last
+	auto drop = [&](int ci) {
+		nc--;
+		const float4 last = laneOf(c, nc);
+		if (lane == ci)
+			c = last;
+	};
+	float maxPen = laneOf(c.w, 0), minPen = maxPen;
+	int ci = 0;
+	for (int i = 1; i < n; i++)
+	{
+		const float pen = laneOf(c.w, i);
+		minPen = fmaxf(minPen, pen);
+		if (maxPen > pen) { maxPen = pen; ci = i; }
+	}
+	float4 ch[4];
+	ch[0] = laneOf(c, ci);
+	const f3 b0 = mk(ch[0]);
+	drop(ci);
+	f3 v = mk(c) - b0;
+	float h = dot(v, v);
+	float maxDist = laneOf(h, 0);
+	ci = 0;
+	for (int i = 1; i < nc; i++)
+	{
+		const float d = laneOf(h, i);
+		if (d > maxDist) { maxDist = d; ci = i; }
+	}
+	ch[1] = laneOf(c, ci);
+	drop(ci);
+	f3 nrm = cross(mk(ch[1]) - b0, cn0);
+	const float sq = dot(nrm, nrm);
+	if (sq > 0.0f) { const float len = sqrtf(sq); nrm = mk(nrm.x / len, nrm.y / len, nrm.z / len); } else nrm = cn0;
+	v = mk(c) - b0;
+	h = dot(v, nrm);
+	maxDist = -FLT_BIG;
+	float minDist = FLT_BIG;
+	ci = 0;
+	int ci1 = 0;
+	for (int i = 0; i < nc; i++)
+	{
+		const float d = laneOf(h, i);
+		if (d > maxDist) { maxDist = d; ci = i; }
+		if (minDist > d) { minDist = d; ci1 = i; }
+	}
+	ch[2] = laneOf(c, ci);
+	ch[3] = laneOf(c, ci1);
+	drop(ci);
+	if (nc == ci1)
+		ci1 = ci;
+	if (minDist * maxDist > 0.0f)
+	{
+		v = mk(c) - b0;
+		h = dot(v, nrm);
+		maxDist = -FLT_BIG;
+		for (int i = 0; i < nc; i++)
+		{
+			const float d = laneOf(h, i);
+			if (d > maxDist) { maxDist = d; ci1 = i; }
+		}
+		if (maxDist > -FLT_BIG)
+			ch[3] = laneOf(c, ci1);
+	}
+	drop(ci1);
+	const float eps = tol * 0.02f;
+	if (eps > maxPen && minPen > eps)
+	{
+#pragma unroll
+		for (int i = 0; i < 4; i++)
+		{
+			float pen = ch[i].w;
+			if (pen > eps)
+			{
+				int cidx = -1;
+				for (int j = 0; j < nc; j++)
+				{
+					const float pen1 = laneOf(c.w, j);
+					if (pen > pen1 && eps > pen1) { pen = pen1; cidx = j; }
+				}
+				if (cidx >= 0)
+				{
+					const float4 orig = ch[i];
+					ch[i] = laneOf(c, cidx);
+					if (lane == cidx)
+						c = orig;
+				}
+			}
+		}
+	}
+	out = lane == 0 ? ch[0] : lane == 1 ? ch[1] : lane == 2 ? ch[2] : ch[3];
+	return 4;
+}
+
+// Contacts of a box- or convex-convex pair no farther apart than cd, from its
+// separation (dist, n from B towards A, closest points or minimum-translation
+// witnesses cA, cB in B's frame), into contact slot `slot`: witness polygons,
+// clipping and reduction to four, as Gu::pcmContactConvexConvex /
+// pcmContactBoxConvex on a fresh manifold
+// (geomutils/src/pcm/GuPCMContactConvexConvex.cpp:111-276, GuPCMContactBoxConvex.cpp;
+// Gu::generateFullContactManifold and Gu::addGJKEPAContacts,
+// GuPCMContactGenBoxConvex.cpp:532-720); points on shape1 in the world and the
+// summed normal (PersistentContactManifold::addManifoldContactsToContactBuffer /
+// getWorldNormal, GuPersistentContactManifold.cpp:739-762,
+// GuPersistentContactManifold.h:405-416)
+PXH_D void convexContactsWave(const Poly& A, const xf& x0, const Poly& B, const xf& x1, float dist, f3 n, f3 cA, f3 cB,
+                              float cd, float tol, ContactLds& L, int lane, int64_t slot, float4* ctN, float4* ctP)
+{
+	const mxf aToB = mxfOf(xinvmul(x1, x0));
+	const float lo = tol * 1e-2f, hi = tol * 5e-2f;
+	const float tA = fminf(fmaxf(A.margin, lo), hi), tB = fminf(fmaxf(B.margin, lo), hi);
+	const f3 negN = -n;
+	const f3 nIn0 = mtmul(aToB.r, n);
+	const int f1 = witnessPolygonWave(B, negN, cB, tB, lane);
+	const int f0 = witnessPolygonWave(A, nIn0, mxtransinv(aToB, cA), tA, lane);
+	const f3 refN = normalize(B.pn(f1)), incN = normalize(A.pn(f0));
+	f3 ln;
+	int nc;
+	if (fabsf(dot(refN, negN)) >= fabsf(dot(incN, nIn0)))
+	{
+		const mxf bToA = mxfOf(xinvmul(x0, x1));
+		nc = generatedContactsWave(B, A, f1, f0, bToA, cd, false, L, lane);
+		ln = refN;
+	}
+	else
+	{
+		nc = generatedContactsWave(A, B, f0, f1, aToB, cd, true, L, lane);
+		ln = -mmul(aToB.r, incN);
+	}
+	waveSync();
+	float4 pt = f4(cB, dist);
+	if (nc == 0)
+	{
+		// the closest-feature / minimum-translation point stays the only point
+		ln = n;
+		nc = 1;
+	}
+	else
+		nc = batchReduceWave(L.pts, nc, ln, tol, lane, pt);
+	f3 s = ln;
+	for (int i = 1; i < nc; i++)
+		s = s + ln;
+	const bool keep = lane < nc && cd >= pt.w;
+	const uint64_t m = __ballot(keep);
+	if (keep)
+		ctP[4 * slot + laneRank(m, lane)] = f4(xtrans(x1, mk(pt)), pt.w);
+	if (lane == 0)
+		ctN[slot] = f4(normalize(qrot(x1.q, s)), __int_as_float(int(__popcll(m))));
+	waveSync();
+}
+
+// Gu::pcmContactPlaneConvex on a fresh manifold
+// (geomutils/src/pcm/GuPCMContactPlaneConvex.cpp:36-227) into contact slot `slot`,
+// the normal from the plane to the hull: the face most opposed to the plane
+// normal, or the better face of the edge whose summed face normals are most
+// opposed to it (5e-4 bias towards edges); the chosen face's vertices below the
+// contact distance, taken once more when an edge was chosen (the reference
+// passes over the same face twice); reduced to four.
+// Deliberate deviation: when the chosen face does not hold the hull's deepest
+// vertex (an irregular hull can rest on a vertex that the face most opposed to
+// the plane does not contain), that vertex joins the batch. The reference scene's
+// persistent manifold keeps such a vertex from earlier steps; a step that
+// generates contacts afresh has to add it.
+PXH_D void planeConvexWave(f3 pn, float pd, const Poly& B, const xf& tb, float cd, float tol, ContactLds& L, int lane,
+                           int64_t slot, float4* ctN, float4* ctP)
+{
+	const f3 n = normalize(qrotinv(tb.q, pn));
+	const f3 nn = -n;
+	float minProj = FLT_BIG;
+	uint32_t faceIdx = lane == 0 ? 0u : 0xFFFFFFFFu;
+	for (int i = lane; i < B.np; i += 64)
+	{
+		const float proj = dot(n, B.pn(i));
+		if (minProj > proj) { minProj = proj; faceIdx = uint32_t(i); }
+	}
+	waveArgMin(minProj, faceIdx);
+	int face = faceIdx == 0xFFFFFFFFu ? 0 : int(faceIdx);
+	int edgeSel = -1;
+	minProj = minProj - 5e-4f;
+	float maxDpSq = minProj * minProj;
+	for (int base = 0; base < B.ne; base += 64)
+	{
+		// the next edge of the block that beats the best so far, until none does
+		const bool has = base + lane < B.ne;
+		const uint32_t g = B.edge(has ? base + lane : 0);
+		const f3 en = B.pn(int((g >> 16) & 0xFF)) + B.pn(int(g >> 24));
+		const float enMagSq = dot(en, en);
+		const float dp = dot(en, nn);
+		const float sqDp = dp * dp;
+		int from = 0;
+		while (from < 64)
+		{
+			const uint64_t m = __ballot(has && lane >= from && dp >= 0.0f && sqDp > maxDpSq * enMagSq);
+			if (m == 0ull)
+				break;
+			const int l = __ffsll((unsigned long long)m) - 1;
+			maxDpSq = laneOf(sqDp / enMagSq, l);
+			edgeSel = base + l;
+			from = l + 1;
+		}
+	}
+	int passes = 1;
+	if (edgeSel >= 0)
+	{
+		const uint32_t g = B.edge(edgeSel);
+		const int f0 = int((g >> 16) & 0xFF), f1 = int(g >> 24);
+		face = dot(B.pn(f0), nn) > dot(B.pn(f1), nn) ? f0 : f1;
+		passes = 2;
+	}
+	float deepest = FLT_BIG;
+	uint32_t dv = lane == 0 ? 0u : 0xFFFFFFFFu;
+	for (int i = lane; i < B.nv; i += 64)
+	{
+		const float s = dot(pn, xtrans(tb, B.vert(i))) + pd;
+		if (s < deepest) { deepest = s; dv = uint32_t(i); }
+	}
+	waveArgMin(deepest, dv);
+	if (dv == 0xFFFFFFFFu)
+		dv = 0u;
+	const int cnt = B.pcount(face);
+	bool below = lane < passes * cnt, isDeepest = false;
+	f3 pw = pn;
+	float s = 0.0f;
+	if (below)
+	{
+		const int vi = B.pvert(face, lane < cnt ? lane : lane - cnt);
+		pw = xtrans(tb, B.vert(vi));
+		s = dot(pn, pw) + pd;
+		below = cd > s;
+		isDeepest = vi == int(dv);
+	}
+	const uint64_t m = __ballot(below);
+	if (below)
+		L.pts[laneRank(m, lane)] = f4(pw - pn * s, s);
+	int nc = int(__popcll(m));
+	if (!__any(below && isDeepest) && cd > deepest && nc < HULL_MAX_CONTACTS)
+	{
+		const f3 dw = xtrans(tb, B.vert(int(dv)));
+		if (lane == 0)
+			L.pts[nc] = f4(dw - pn * deepest, deepest);
+		nc++;
+	}
+	waveSync();
+	float4 pt = f4(pn, 0.0f);
+	if (nc > 0)
+		nc = batchReduceWave(L.pts, nc, pn, tol, lane, pt);
+	const bool keep = lane < nc && cd >= pt.w;
+	const uint64_t k = __ballot(keep);
+	if (keep)
+		ctP[4 * slot + laneRank(k, lane)] = pt;
+	if (lane == 0)
+		ctN[slot] = f4(pn, __int_as_float(int(__popcll(k))));
+	waveSync();
 }
 
 }  // namespace pxh

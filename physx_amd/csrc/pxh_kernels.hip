@@ -1226,60 +1226,80 @@ k_np_convex_wave(int cap, const uint2* pairs, const float4* pos, const float4* r
 	}
 }
 
-// Box- and convex-convex pairs, contact phase: one lane per searched pair
-// (witness polygons, clipping, reduction where it touches, else its empty slot);
-// the list order does not matter, pair p fills slot slotBase + p.
+// Box- and convex-convex pairs, contact phase: a wave per touching pair of the
+// search list (witness polygons, clipping, reduction); the others get their empty
+// slot. Waves take thinLanes pairs at a time. The list order does not matter, pair
+// p fills slot slotBase + p.
 __global__ void __launch_bounds__(64) k_np_convex_finish(int cap, int slotBase, const uint2* pairs, const float4* pos,
                                                          const float4* rot, const float4* geom, HullSet hs, float cd,
                                                          float tol, const float4* wit, const uint32_t* list,
                                                          float4* ctN, float4* ctP)
 {
-	PXH_THIN_LOOP(q, min(list[0], uint32_t(cap)))
+	__shared__ ContactLds L;
+	const int lane = threadIdx.x;
+	const uint32_t count = min(list[0], uint32_t(cap)), lanes = uint32_t(thinLanes(count));
+	for (uint32_t base = blockIdx.x * lanes; base < count; base += gridDim.x * lanes)
 	{
-		const uint32_t p = cvxEntries(list, cap, 0)[q];
-		const uint2 ab = pairs[p];
-		const float4 g0 = geom[ab.x], g1 = geom[ab.y];
-		const int t0 = int(g0.w);
-		const float4 sep = wit[3 * int64_t(p)];
-		Contacts c;
-		c.count = 0;
-		int cnt = 0;
-		if (sep.x <= cd)
+		const bool live = uint32_t(lane) < lanes && base + lane < count;
+		const int p = live ? int(cvxEntries(list, cap, 0)[base + lane]) : 0;
+		const bool touch = live && wit[3 * int64_t(p)].x <= cd;
+		if (live && !touch)
+			ctN[slotBase + p] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
+		for (uint64_t m = __ballot(touch); m != 0ull; m &= m - 1ull)
 		{
+			const int pp = laneOf(p, __ffsll((unsigned long long)m) - 1);
+			const uint2 ab = pairs[pp];
+			const float4 g0 = geom[ab.x], g1 = geom[ab.y], sep = wit[3 * int64_t(pp)];
 			xf x0, x1;
 			x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
 			x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
 			const Poly B = hullPoly(hs, int(g1.x));
-			const Poly A = t0 == GEOM_BOX ? boxPoly(mk(g0.x, g0.y, g0.z)) : hullPoly(hs, int(g0.x));
-			const mxf aToB = mxfOf(xinvmul(x1, x0));
-			cnt = convexContactsFrom(A, x0, B, x1, aToB, sep.x, mk(sep.y, sep.z, sep.w), mk(wit[3 * int64_t(p) + 1]),
-			                         mk(wit[3 * int64_t(p) + 2]), cd, tol, c);
+			const Poly A = int(g0.w) == GEOM_BOX ? boxPoly(mk(g0.x, g0.y, g0.z)) : hullPoly(hs, int(g0.x));
+			convexContactsWave(A, x0, B, x1, sep.x, mk(sep.y, sep.z, sep.w), mk(wit[3 * int64_t(pp) + 1]),
+			                   mk(wit[3 * int64_t(pp) + 2]), cd, tol, L, lane, int64_t(slotBase) + pp, ctN, ctP);
 		}
-		storeContacts(slotBase + int(p), c, cnt, ctN, ctP);
 	}
 }
 
-// Body-plane pairs of convex bodies (the others are left to k_np_planes); the
-// hull is constraint body a, so normals point from the plane to the hull.
+// Body-plane pairs of convex bodies (the others are left to k_np_planes), a wave
+// per hull that its bounding sphere does not keep off the plane; the hull is
+// constraint body a, so normals point from the plane to the hull.
 __global__ void __launch_bounds__(64) k_np_planes_convex(int Q, int slotBase, const int* qBody, const int* qPlane,
                                                          const float4* pos, const float4* rot, const float4* geom,
                                                          const float4* planes, HullSet hs, float cd, float tol,
                                                          float4* ctN, float4* ctP)
 {
-	PXH_THIN_LOOP(q, Q)
+	__shared__ ContactLds L;
+	const int lane = threadIdx.x, lanes = thinLanes(uint32_t(Q));
+	for (int base = blockIdx.x * lanes; base < Q; base += gridDim.x * lanes)
 	{
-		const int i = qBody[q];
-		const float4 g = geom[i];
-		if (int(g.w) == GEOM_CONVEXMESH)
+		const int q = base + lane;
+		bool near = false;
+		if (lane < lanes && q < Q)
 		{
-			const float4 pl = planes[qPlane[q]];
+			const int i = qBody[q];
+			const float4 g = geom[i];
+			if (int(g.w) == GEOM_CONVEXMESH)
+			{
+				const float4 pl = planes[qPlane[q]];
+				const f3 x = mk(pos[i]);
+				const float r = hs.be[int(g.x)].w;
+				// the margin is well above the rounding of a vertex's own distance
+				const float slack = 1e-5f * (fabsf(x.x) + fabsf(x.y) + fabsf(x.z) + fabsf(pl.w) + r);
+				near = !(dot(mk(pl), x) + pl.w > r * sqrtf(dot(mk(pl), mk(pl))) + cd + slack);
+				if (!near)
+					ctN[slotBase + q] = f4(mk(pl), __int_as_float(0));
+			}
+		}
+		for (uint64_t m = __ballot(near); m != 0ull; m &= m - 1ull)
+		{
+			const int qq = base + __ffsll((unsigned long long)m) - 1;
+			const int i = qBody[qq];
+			const float4 pl = planes[qPlane[qq]];
 			xf x;
 			x.p = mk(pos[i]); x.q = mkq(rot[i]);
-			Contacts c;
-			c.count = 0;
-			const int cnt = planeConvex(mk(pl), pl.w, hullPoly(hs, int(g.x)), x, cd, tol, c);
-			c.n = -c.n;
-			storeContacts(slotBase + int(q), c, cnt, ctN, ctP);
+			planeConvexWave(mk(pl), pl.w, hullPoly(hs, int(geom[i].x)), x, cd, tol, L, lane, int64_t(slotBase) + qq, ctN,
+			                ctP);
 		}
 	}
 }

@@ -508,9 +508,6 @@ struct MeshLds
 	float4 pts[MESH_ROUND * (MESH_CLIP + 1)], tmp[MESH_ROUND * (MESH_CLIP + 1)];
 };
 
-PXH_D int laneOf(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
-PXH_D float laneOf(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
-PXH_D f3 laneOf(f3 v, int l) { return mk(laneOf(v.x, l), laneOf(v.y, l), laneOf(v.z, l)); }
 PXH_D int firstLane(uint64_t m) { return __ffsll((unsigned long long)m) - 1; }
 
 // MPatches over the wave: lane 9 k + j holds point j of patch k, the 9 lanes of a

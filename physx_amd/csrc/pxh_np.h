@@ -532,91 +532,7 @@ PXH_D void calcContacts(float exIn, float eyIn, const f3 (&pts)[4], f3 incN, flo
 
 // PersistentContactManifold::reduceBatchContacts
 // (geomutils/src/pcm/GuPersistentContactManifold.cpp:1008-1172)
-template <int MAXN>
-PXH_D void reduceBatchT(const PC* m, int n, float tol, int* ch)
-{
-	int cand[MAXN];
-	float maxPen = m[0].pen, minPen = maxPen;
-	int index = 0, ci = 0;
-	cand[0] = 0;
-	int nc = n;
-	for (int i = 1; i < n; i++)
-	{
-		cand[i] = i;
-		const float pen = m[i].pen;
-		minPen = fmaxf(minPen, pen);
-		if (maxPen > pen) { maxPen = pen; index = i; ci = i; }
-	}
-	ch[0] = index;
-	nc--; cand[ci] = cand[nc];
-	f3 v = m[cand[0]].lb - m[ch[0]].lb;
-	float maxDist = dot(v, v);
-	index = cand[0]; ci = 0;
-	for (int i = 1; i < nc; i++)
-	{
-		v = m[cand[i]].lb - m[ch[0]].lb;
-		const float d = dot(v, v);
-		if (d > maxDist) { maxDist = d; index = cand[i]; ci = i; }
-	}
-	ch[1] = index;
-	nc--; cand[ci] = cand[nc];
-	v = m[ch[1]].lb - m[ch[0]].lb;
-	const f3 cn0 = m[ch[0]].ln;
-	f3 nrm = cross(v, cn0);
-	const float sq = dot(nrm, nrm);
-	if (sq > 0.0f) { const float L = sqrtf(sq); nrm = mk(nrm.x / L, nrm.y / L, nrm.z / L); } else nrm = cn0;
-	maxDist = -FLT_BIG; index = cand[0]; ci = 0;
-	float minDist = FLT_BIG;
-	int index1 = cand[0], ci1 = 0;
-	for (int i = 0; i < nc; i++)
-	{
-		v = m[cand[i]].lb - m[ch[0]].lb;
-		const float d = dot(v, nrm);
-		if (d > maxDist) { maxDist = d; index = cand[i]; ci = i; }
-		if (minDist > d) { minDist = d; index1 = cand[i]; ci1 = i; }
-	}
-	ch[2] = index;
-	nc--; cand[ci] = cand[nc];
-	if (nc == ci1)
-		ci1 = ci;
-	if (minDist * maxDist > 0.0f)
-	{
-		maxDist = -FLT_BIG;
-		for (int i = 0; i < nc; i++)
-		{
-			v = m[cand[i]].lb - m[ch[0]].lb;
-			const float d = dot(v, nrm);
-			if (d > maxDist) { maxDist = d; index1 = cand[i]; ci1 = i; }
-		}
-	}
-	ch[3] = index1;
-	nc--; cand[ci1] = cand[nc];
-	const float eps = tol * 0.02f;
-	if (eps > maxPen && minPen > eps)
-	{
-		for (int i = 0; i < 4; i++)
-		{
-			float pen = m[ch[i]].pen;
-			if (pen > eps)
-			{
-				int cidx = -1;
-				for (int j = 0; j < nc; j++)
-				{
-					const float pen1 = m[cand[j]].pen;
-					if (pen > pen1 && eps > pen1) { pen = pen1; cidx = j; }
-				}
-				if (cidx >= 0)
-				{
-					const int orig = ch[i];
-					ch[i] = cand[cidx];
-					cand[cidx] = orig;
-				}
-			}
-		}
-	}
-}
-
-// reduceBatchT on a lane's points in LDS (their common normal cn0): the
+// of a lane's points in LDS (their common normal cn0): the
 // candidate list is sixteen 4-bit indices in one 64-bit word and the four
 // choices stay in registers, so nothing is indexed in scratch. Same choices in
 // the same order.
