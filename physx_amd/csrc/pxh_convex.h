@@ -303,6 +303,11 @@ PXH_D void polySeparation(const Poly& A, const mxf& aToB, const Poly& B, float c
 	n = (cA - cB) * (1.0f / dist);
 }
 
+PXH_D void waveArgMin(float& v, uint32_t& idx);
+PXH_D float waveMin(float v);
+PXH_D f3 laneOf(f3 v, int l);
+PXH_D int witnessPolygonWave(const Poly& P, f3 normal, f3 closest, float tolerance, int lane);
+
 // Gu::getWitnessPolygonIndex (geomutils/src/pcm/GuPCMContactGenUtil.cpp:201-271);
 // the per-polygon distances are evaluated again in the second pass
 PXH_D int witnessPolygon(const Poly& P, f3 normal, f3 closest, float tolerance)
@@ -403,43 +408,52 @@ template <class V> PXH_D bool polyContainsN(const V* verts, int nv, f3 p, f3 mn,
 
 // Gu::pcmContactSphereConvex on a fresh manifold
 // (geomutils/src/pcm/GuPCMContactSphereConvex.cpp:110-246)
-PXH_D int sphereConvex(float r, f3 p0, const Poly& B, const xf& x1, float cd, Contacts& o)
+// (over the wave: the lanes share the faces and edges, the first minimum in
+// their order wins)
+PXH_D int sphereConvexWave(float r, f3 p0, const Poly& B, const xf& x1, float cd, int lane, Contacts& o)
 {
 	const f3 c = xtransinv(x1, p0);
-	float hmax = -FLT_BIG;
-	int fm = 0;
-	for (int f = 0; f < B.np; f++)
+	float least = FLT_BIG;   // minus the largest height
+	uint32_t fm = 0xFFFFFFFFu;
+	for (int f = lane; f < B.np; f += 64)
 	{
 		const float h = dot(B.pn(f), c) + B.pd(f);
-		if (h > hmax) { hmax = h; fm = f; }
+		if (-h < least) { least = -h; fm = uint32_t(f); }
 	}
+	waveArgMin(least, fm);
+	const float hmax = -least;
 	f3 n;
 	float pen;
 	if (hmax <= 0.0f)
 	{
-		n = B.pn(fm);
+		n = B.pn(fm == 0xFFFFFFFFu ? 0 : int(fm));
 		pen = hmax - r;
 	}
 	else
 	{
 		float d2 = FLT_BIG;
+		uint32_t at = 0xFFFFFFFFu;
 		f3 q = c;
-		for (int f = 0; f < B.np; f++)
+		for (int f = lane; f < B.np; f += 64)
 		{
 			const f3 bn = B.pn(f);
 			const float h = dot(bn, c) + B.pd(f);
 			if (h < 0.0f || h * h >= d2)
 				continue;
 			const f3 pq = c - bn * h;
-			if (inPolygon(B, f, pq)) { d2 = h * h; q = pq; }
+			if (inPolygon(B, f, pq)) { d2 = h * h; q = pq; at = uint32_t(f); }
 		}
-		for (int e = 0; e < B.ne; e++)
+		for (int e = lane; e < B.ne; e += 64)
 		{
 			const uint32_t g = B.edge(e);
 			f3 c1, c2;
 			const float s = segClosestSq(c, c, B.vert(int(g & 0xFF)), B.vert(int((g >> 8) & 0xFF)), c1, c2);
-			if (s < d2) { d2 = s; q = c2; }
+			if (s < d2) { d2 = s; q = c2; at = uint32_t(B.np + e); }
 		}
+		const uint32_t mine = at;
+		waveArgMin(d2, at);
+		const uint64_t m = __ballot(mine == at && at != 0xFFFFFFFFu);
+		q = m ? laneOf(q, __ffsll((unsigned long long)m) - 1) : c;
 		const float dist = sqrtf(d2);
 		if (dist > r + cd)
 			return 0;
@@ -554,6 +568,105 @@ PXH_D float segPoly(const Poly& B, f3 p, f3 q, f3& n, f3& cA, f3& cB)
 	return -best;
 }
 
+// segPoly over the wave: the lanes share B's faces and edges, the first minimum
+// in their order wins
+PXH_D float segPolyWave(const Poly& B, f3 p, f3 q, int lane, f3& n, f3& cA, f3& cB)
+{
+	const f3 d = q - p;
+	float t0 = 0.0f, t1 = 1.0f;
+	bool out = false;
+	for (int f = lane; f < B.np; f += 64)
+	{
+		const f3 fn = B.pn(f);
+		const float hp = dot(fn, p) + B.pd(f), dn = dot(fn, d);
+		if (dn == 0.0f)
+			out |= hp > 0.0f;
+		else if (dn < 0.0f)
+			t0 = fmaxf(t0, -hp / dn);
+		else
+			t1 = fminf(t1, -hp / dn);
+	}
+	t0 = -waveMin(-t0);
+	t1 = waveMin(t1);
+	float best = FLT_BIG;
+	uint32_t at = 0xFFFFFFFFu;
+	cA = p;
+	cB = p;
+	if (__any(out) || t0 > t1)
+	{
+		for (int k = lane; k < 2 * B.np; k += 64)
+		{
+			const int f = k < B.np ? k : k - B.np;
+			const f3 c = k < B.np ? p : q;
+			const f3 fn = B.pn(f);
+			const float h = dot(fn, c) + B.pd(f);
+			if (h < 0.0f || h * h >= best)
+				continue;
+			const f3 pc = c - fn * h;
+			if (inPolygon(B, f, pc)) { best = h * h; cA = c; cB = pc; at = uint32_t(k); }
+		}
+		for (int e = lane; e < B.ne; e += 64)
+		{
+			const uint32_t ed = B.edge(e);
+			f3 c1, c2;
+			const float s = segClosestSq(p, q, B.vert(ed & 0xFF), B.vert((ed >> 8) & 0xFF), c1, c2);
+			if (s < best) { best = s; cA = c1; cB = c2; at = uint32_t(2 * B.np + e); }
+		}
+		const uint32_t mine = at;
+		waveArgMin(best, at);
+		const uint64_t m = __ballot(mine == at && at != 0xFFFFFFFFu);
+		const int l = m ? __ffsll((unsigned long long)m) - 1 : 0;
+		cA = m ? laneOf(cA, l) : p;
+		cB = m ? laneOf(cB, l) : p;
+		const float dist = sqrtf(best);
+		n = (cA - cB) * (1.0f / dist);
+		return dist;
+	}
+	f3 axis = mk(1.0f, 0.0f, 0.0f);
+	for (int f = lane; f < B.np; f += 64)
+	{
+		const f3 fn = B.pn(f);
+		const float depth = -B.pd(f) - fminf(dot(fn, p), dot(fn, q));
+		if (depth < best) { best = depth; axis = fn; at = uint32_t(f); }
+	}
+	for (int e = lane; e < B.ne; e += 64)
+	{
+		const uint32_t ed = B.edge(e);
+		const f3 a = B.vert(ed & 0xFF), b = B.vert((ed >> 8) & 0xFF);
+		f3 c = cross(d, b - a);
+		const float l2 = dot(c, c);
+		if (!(l2 > 1e-12f))
+			continue;
+		c = c * (1.0f / sqrtf(l2));
+		float mnB = FLT_BIG, mxB = -FLT_BIG;
+		for (int i = 0; i < B.nv; i++)
+		{
+			const float s = dot(c, B.vert(i));
+			mnB = fminf(mnB, s);
+			mxB = fmaxf(mxB, s);
+		}
+		const float sp = dot(c, p), sq = dot(c, q);
+		const float dp = mxB - fminf(sp, sq), dm = fmaxf(sp, sq) - mnB;
+		if (dp < best) { best = dp; axis = c; at = uint32_t(B.np + e); }
+		if (dm < best) { best = dm; axis = -c; at = uint32_t(B.np + e); }
+	}
+	const uint32_t mine = at;
+	waveArgMin(best, at);
+	const uint64_t m = __ballot(mine == at && at != 0xFFFFFFFFu);
+	axis = m ? laneOf(axis, __ffsll((unsigned long long)m) - 1) : mk(1.0f, 0.0f, 0.0f);
+	n = axis;
+	if (at != 0xFFFFFFFFu && at >= uint32_t(B.np))
+	{
+		const uint32_t ed = B.edge(int(at) - B.np);
+		f3 c2;
+		segClosestSq(p, q, B.vert(ed & 0xFF), B.vert((ed >> 8) & 0xFF), cA, c2);
+	}
+	else
+		cA = dot(axis, q) < dot(axis, p) ? q : p;
+	cB = cA + axis * best;
+	return -best;
+}
+
 constexpr int CAPSULE_MAX_CONTACTS = HULL_MAX_POLY_VERTS + 2;
 
 // generatedCapsuleBoxFaceContacts (geomutils/src/pcm/GuPCMContactGenSphereCapsule.cpp:221-284):
@@ -598,19 +711,17 @@ PXH_D void capsuleFaceContacts(const Poly& B, int f, f3 p0, f3 p1, f3 n, float i
 
 // intersectRayPolyhedron (GuPCMContactGenSphereCapsule.cpp:98-141): the entry
 // parameter of the ray a + t dir, t >= 0, into B
-PXH_D bool rayPolyhedron(const Poly& B, f3 a, f3 dir, float& tEnter)
+PXH_D bool rayPolyhedronWave(const Poly& B, f3 a, f3 dir, int lane, float& tEnter)
 {
 	float tFirst = 0.0f, tLast = FLT_BIG;
-	for (int k = 0; k < B.np; k++)
+	bool out = false;
+	for (int k = lane; k < B.np; k += 64)
 	{
 		const f3 fn = B.pn(k);
 		const float den = dot(fn, dir);
 		const float dist = dot(fn, a) + B.pd(k);
 		if (1e-7f > fabsf(den))
-		{
-			if (dist > 0.0f)
-				return false;
-		}
+			out |= dist > 0.0f;
 		else
 		{
 			const float t = -(dist / den);
@@ -619,23 +730,23 @@ PXH_D bool rayPolyhedron(const Poly& B, f3 a, f3 dir, float& tEnter)
 			if (!(0.0f > den) && tLast > t)
 				tLast = t;
 		}
-		if (tFirst > tLast)
-			return false;
 	}
+	tFirst = -waveMin(-tFirst);
+	tLast = waveMin(tLast);
 	tEnter = tFirst;
-	return true;
+	return !(__any(out) || tFirst > tLast);
 }
 
 // generatedFaceContacts (GuPCMContactGenSphereCapsule.cpp:286-310): each
 // endpoint's ray along -n into the hull, entered within radius + contact
 // distance
-PXH_D void capsuleRayContacts(const Poly& B, f3 p0, f3 p1, f3 n, float infl, const mxf& aToB, PC* mc, int& nc)
+PXH_D void capsuleRayContacts(const Poly& B, f3 p0, f3 p1, f3 n, float infl, const mxf& aToB, int lane, PC* mc, int& nc)
 {
 	for (int k = 0; k < 2; k++)
 	{
 		const f3 e = k ? p1 : p0;
 		float tE;
-		if (rayPolyhedron(B, e, -n, tE) && infl >= tE)
+		if (rayPolyhedronWave(B, e, -n, lane, tE) && infl >= tE)
 		{
 			mc[nc].la = mxtransinv(aToB, e);
 			mc[nc].lb = (-n) * tE + e;
@@ -728,21 +839,24 @@ PXH_D void reduceBatch2(const PC* m, int n, int& i0, int& i1)
 // polytope; box: endpoint contacts on the witness polygon, convex: endpoint
 // rays into the hull; fewer than two: edge contacts on the witness polygon;
 // none: the closest-point contact; reduced to two. Points on the capsule's
-// surface, separation less the radius, normal from the polytope.
-PXH_D int capsulePoly(float r, float hh, const xf& x0, const Poly& B, const xf& x1, float cd, float tol, Contacts& o)
+// surface, separation less the radius, normal from the polytope. BOX: one pair a
+// lane; else a hull and one pair over the wave, every lane with the same points.
+template <bool BOX>
+PXH_D int capsulePoly(float r, float hh, const xf& x0, const Poly& B, const xf& x1, float cd, float tol, int lane,
+                      Contacts& o)
 {
 	const mxf aToB = mxfOf(xinvmul(x1, x0));
 	const f3 ext = mmul(aToB.r, mk(hh, 0.0f, 0.0f));
 	const f3 p0 = aToB.p + ext, p1 = aToB.p - ext;
 	f3 n, cA, cB;
-	const float dist = segPoly(B, p0, p1, n, cA, cB);
+	const float dist = BOX ? segPoly(B, p0, p1, n, cA, cB) : segPolyWave(B, p0, p1, lane, n, cA, cB);
 	if (dist > r + cd)
 		return 0;
 	const float infl = r + cd;
 	const float wtol = fminf(fmaxf(B.margin, tol * 1e-2f), tol * 5e-2f);
 	PC mc[CAPSULE_MAX_CONTACTS];
 	int nc = 0;
-	if (B.box)
+	if constexpr (BOX)
 	{
 		const int f = witnessPolygon(B, -n, cB, wtol);
 		capsuleFaceContacts(B, f, p0, p1, n, infl, aToB, mc, nc);
@@ -751,9 +865,9 @@ PXH_D int capsulePoly(float r, float hh, const xf& x0, const Poly& B, const xf& 
 	}
 	else
 	{
-		capsuleRayContacts(B, p0, p1, n, infl, aToB, mc, nc);
+		capsuleRayContacts(B, p0, p1, n, infl, aToB, lane, mc, nc);
 		if (nc < 2)
-			capsuleEEContacts(B, witnessPolygon(B, -n, cB, wtol), p0, p1, n, infl, aToB, mc, nc);
+			capsuleEEContacts(B, witnessPolygonWave(B, -n, cB, wtol, lane), p0, p1, n, infl, aToB, mc, nc);
 	}
 	int i0 = 0, i1 = 1;
 	if (nc == 0)

@@ -974,13 +974,11 @@ PXH_D void blockAppend(bool take, int value, int* out, uint32_t* total)
 	__syncthreads();
 }
 
-// Kernels whose items are long serial chains with branches of their own (hull
-// polygons, mesh triangles, joint rows) fill a wave only as far as the chip is
+// Kernels whose items are long serial chains with branches of their own (joint
+// rows, a wave's pairs one after the other) fill a wave only as far as the chip is
 // full: a wave of 64 such lanes runs every branch of every lane one after the
 // other, while most compute units idle. THIN_BLOCKS waves take `lanes` items
-// each at a time, one until there are more items than waves. 2,116 bodies on a
-// mesh: their sphere- and capsule-hull pairs 209 us in 64-lane waves and 89 so,
-// the hull contacts 101 and 50.
+// each at a time, one until there are more items than waves.
 constexpr int THIN_BLOCKS = 4096;
 __host__ __device__ inline int thinLanes(uint32_t count)
 {
@@ -1045,7 +1043,7 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_pairs(int cap, const uint32_t
 			else if (t1 == GEOM_CAPSULE)
 				cnt = capsuleCapsule(g0.x, g0.y, x0, g1.x, g1.y, x1, cd, c);
 			else if (t0 == GEOM_CAPSULE)
-				cnt = capsulePoly(g0.x, g0.y, x0, boxPoly(mk(g1.x, g1.y, g1.z)), x1, cd, tol, c);
+				cnt = capsulePoly<true>(g0.x, g0.y, x0, boxPoly(mk(g1.x, g1.y, g1.z)), x1, cd, tol, 0, c);
 			else
 				cnt = boxBoxFace(mk(g0.x, g0.y, g0.z), x0, mk(g1.x, g1.y, g1.z), x1, cd, tol, points + threadIdx.x, c);
 		}
@@ -1097,10 +1095,10 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_planes(int Q, int slotBase, c
 // search (k_np_convex_wave and k_np_convex_finish), 1 round pairs
 // (k_np_round_convex). Three of four pairs of a rubble pile don't touch; the
 // steps take 8 lanes of a pair where the search takes a wave: of 8,192 hulls'
-// 89,000 pairs, 7 us without and 39 with them, for 386 and 276 us of search.
+// 89,000 pairs, 7 us without and 37 with them, for 386 and 276 us of search.
 PXH_D uint32_t* cvxEntries(uint32_t* list, int cap, int which) { return list + 2 + int64_t(which) * cap; }
 PXH_D const uint32_t* cvxEntries(const uint32_t* list, int cap, int which) { return list + 2 + int64_t(which) * cap; }
-constexpr int APART_BLOCK = 1024;
+constexpr int APART_BLOCK = 512;
 __global__ void __launch_bounds__(APART_BLOCK) k_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex,
                             int slotBase, const uint2* pairs, const float4* pos, const float4* rot, const float4* geom,
                             HullSet hs, float cd, float4* ctN, uint32_t* list)
@@ -1146,30 +1144,47 @@ __global__ void __launch_bounds__(APART_BLOCK) k_np_convex(int cap, const uint32
 	}
 }
 
-// sphere- and capsule-convex pairs of list 1
+// sphere- and capsule-convex pairs of list 1, a wave per pair that its bounding
+// spheres do not settle; waves take thinLanes pairs at a time. A lane's chain over
+// a hull's faces and edges bound them: the pairs of 2,116 mixed bodies on a terrain took
+// 86 us in a lane each, 13 over the wave.
 __global__ void __launch_bounds__(64) k_np_round_convex(int cap, int slotBase, const uint2* pairs, const float4* pos,
                                                         const float4* rot, const float4* geom, HullSet hs, float cd,
                                                         float tol, float4* ctN, float4* ctP, const uint32_t* list)
 {
-	PXH_THIN_LOOP(q, min(list[1], uint32_t(cap)))
+	const int lane = threadIdx.x;
+	const uint32_t count = min(list[1], uint32_t(cap)), lanes = uint32_t(thinLanes(count));
+	for (uint32_t base = blockIdx.x * lanes; base < count; base += gridDim.x * lanes)
 	{
-		const uint32_t p = cvxEntries(list, cap, 1)[q];
-		const uint2 ab = pairs[p];
-		const float4 g0 = geom[ab.x], g1 = geom[ab.y];
-		xf x1;
-		x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
-		Contacts c;
-		c.count = 0;
-		int cnt;
-		if (int(g0.w) == GEOM_SPHERE)
-			cnt = sphereConvex(g0.x, mk(pos[ab.x]), hullPoly(hs, int(g1.x)), x1, cd, c);
-		else
+		const bool live = uint32_t(lane) < lanes && base + lane < count;
+		const int p = live ? int(cvxEntries(list, cap, 1)[base + lane]) : 0;
+		bool near = false;
+		if (live)
 		{
-			xf x0;
-			x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
-			cnt = capsulePoly(g0.x, g0.y, x0, hullPoly(hs, int(g1.x)), x1, cd, tol, c);
+			const uint2 ab = pairs[p];
+			const float4 g0 = geom[ab.x];
+			const f3 d = mk(pos[ab.y]) - mk(pos[ab.x]);
+			const float reach = (g0.x + (int(g0.w) == GEOM_CAPSULE ? g0.y : 0.0f) + hs.be[int(geom[ab.y].x)].w + cd) * 1.00001f;
+			near = !(dot(d, d) > reach * reach);
+			if (!near)
+				ctN[slotBase + p] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
 		}
-		storeContacts(slotBase + int(p), c, cnt, ctN, ctP);
+		for (uint64_t m = __ballot(near); m != 0ull; m &= m - 1ull)
+		{
+			const int pp = laneOf(p, __ffsll((unsigned long long)m) - 1);
+			const uint2 ab = pairs[pp];
+			const float4 g0 = geom[ab.x], g1 = geom[ab.y];
+			xf x0, x1;
+			x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
+			x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
+			const Poly B = hullPoly(hs, int(g1.x));
+			Contacts c;
+			c.count = 0;
+			const int cnt = int(g0.w) == GEOM_SPHERE ? sphereConvexWave(g0.x, x0.p, B, x1, cd, lane, c)
+			                                         : capsulePoly<false>(g0.x, g0.y, x0, B, x1, cd, tol, lane, c);
+			if (lane == 0)
+				storeContacts(slotBase + pp, c, cnt, ctN, ctP);
+		}
 	}
 }
 
@@ -3897,7 +3912,7 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_immediate(int n, const int* t
 		cnt = planeCapsule(pn, -dot(pn, x0.p), g1[0], g1[1], x1, cd, c);
 	}
 	else if (t0 == GEOM_CAPSULE && t1 == GEOM_BOX)
-		cnt = capsulePoly(g0[0], g0[1], x0, boxPoly(mk(g1[0], g1[1], g1[2])), x1, cd, tol, c);
+		cnt = capsulePoly<true>(g0[0], g0[1], x0, boxPoly(mk(g1[0], g1[1], g1[2])), x1, cd, tol, 0, c);
 	boxBoxEdgeWave(cnt == BOXBOX_EDGE, mk(g0[0], g0[1], g0[2]), x0, mk(g1[0], g1[1], g1[2]), x1, cd, c, cnt);
 	if (own >= n)
 		return;
@@ -4073,7 +4088,7 @@ void launch_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int 
 	if (cap <= 0)
 		return;
 	k_fill_u32<<<1, 64, 0, st>>>(list, 2, 0u);
-	k_np_convex<<<std::min((cap + APART_BLOCK / APART_LANES - 1) / (APART_BLOCK / APART_LANES), 1024), APART_BLOCK, 0, st>>>(
+	k_np_convex<<<std::min((cap + APART_BLOCK / APART_LANES - 1) / (APART_BLOCK / APART_LANES), 2048), APART_BLOCK, 0, st>>>(
 		cap, dP, dConvex, slotBase, pairs, pos, rot, geom, hs, cd, ctN, list);
 	// grid-stride: enough waves to fill the chip several times over
 	const int blocks = std::min((cap + CVX_WAVES - 1) / CVX_WAVES, 8192);

@@ -32,3 +32,23 @@ def test_convex_search_matches_oracle(cuda, n_points, pitch):
     n = _compare_contacts(g, o)
     print(n_points, pitch, g.stats()["bp_pairs"], "pairs,", n, "with contacts", flush=True)
     assert 40 < n < g.stats()["bp_pairs"]
+
+
+@pytest.mark.parametrize("n_points,pitch", [(4, 0.5), (16, 0.7), (40, 0.65), (90, 0.7)])
+def test_round_convex_matches_oracle(cuda, n_points, pitch):
+    """Spheres and capsules among hulls, apart, touching and inside."""
+    sc = S.convex_layers(n_bodies=216, per_side=6, pitch=pitch, n_points=n_points, seed=n_points)
+    i = np.arange(sc.n)
+    ball, cap = i % 3 == 1, i % 3 == 2
+    rng = np.random.default_rng(n_points)
+    sc.shape_type[ball], sc.shape_type[cap] = S.SPHERE, S.CAPSULE
+    sc.dims[ball, 0] = rng.uniform(0.1, 0.35, int(ball.sum()))
+    sc.dims[cap, 0] = rng.uniform(0.05, 0.2, int(cap.sum()))
+    sc.dims[cap, 1] = rng.uniform(0.05, 0.4, int(cap.sum()))
+    g = P.Scene(sc, position_iterations=4, velocity_iterations=1)
+    o = L.OracleWorld(sc, pos_iters=4, vel_iters=1)
+    g.step(DT)
+    o.step(DT)
+    n = _compare_contacts(g, o)
+    print(n_points, pitch, g.stats()["bp_pairs"], "pairs,", n, "with contacts", flush=True)
+    assert 40 < n < g.stats()["bp_pairs"]
