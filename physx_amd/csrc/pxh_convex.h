@@ -36,6 +36,7 @@ struct Poly
 	bool box;
 	f3 h;
 	float margin;
+	float slack;   // how far polygon vertices lie below their planes
 
 	PXH_D f3 vert(int i) const
 	{
@@ -80,6 +81,7 @@ PXH_D Poly hullPoly(const HullSet& hs, int id)
 	p.box = false;
 	p.h = mk(0.0f, 0.0f, 0.0f);
 	p.margin = hs.bc[id].w;
+	p.slack = __int_as_float(b.w);
 	return p;
 }
 
@@ -94,6 +96,7 @@ PXH_D Poly boxPoly(f3 h)
 	p.box = true;
 	p.h = h;
 	p.margin = fminf(h.x, fminf(h.y, h.z)) * 0.15f;
+	p.slack = 0.0f;
 	return p;
 }
 
@@ -1385,9 +1388,9 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, Cvx
 	// distance U, so the minimum is no larger. Along the face axis that
 	// separates the polytopes most, A's heights less B's bound every distance
 	// from below: a vertex or an edge whose height alone is farther from the
-	// other polytope than lim = sqrt(U) plus a margin well above rounding holds
-	// no closest feature. What is left keeps its order and its indices, so the
-	// first minimum is unchanged.
+	// other polytope than lim = sqrt(U) plus a margin well above rounding, and
+	// above what planes lie off their polygons' vertices, holds no closest feature.
+	// What is left keeps its order and its indices, so the first minimum is unchanged.
 	int nA, nB;
 	float minA = 0.0f, maxB = 0.0f;
 	if (slab)
@@ -1432,7 +1435,8 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, Cvx
 		U = fminf(U, edgePairSq(L, L.elA[fu.i], L.elB[fu.j], c1, c2));
 	}
 	U = waveMin(U);
-	float lim = U < BIG ? sqrtf(U) + 1e-4f : BIG;
+	const float margin = 1e-4f + A.slack + B.slack;
+	float lim = U < BIG ? sqrtf(U) + margin : BIG;
 	waveSync();
 	float d2 = BIG;
 	uint32_t di = 0xFFFFFFFFu;
@@ -1468,7 +1472,7 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, Cvx
 		di = (1u << 24) | uint32_t(f * B.nv + i);
 	}
 	U = waveMin(fminf(U, d2));
-	lim = U < BIG ? sqrtf(U) + 1e-4f : BIG;
+	lim = U < BIG ? sqrtf(U) + margin : BIG;
 	waveSync();
 	if (slab)
 	{

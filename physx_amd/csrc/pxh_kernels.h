@@ -21,7 +21,7 @@ struct HullSet
 	const uint8_t* vr;       // polygon vertex loops (hull-local vertex indices)
 	const uint32_t* edge;    // v0 | v1 << 8 | face left << 16 | face right << 24
 	const int4* info;        // vertex first, vertex count, polygon first, polygon count
-	const int4* info2;       // vref first, edge first, edge count, 0
+	const int4* info2;       // vref first, edge first, edge count, slack of the planes (float bits)
 	const float4* bc;        // local bounds centre, GJK margin
 	const float4* be;        // local bounds extents, radius about the shape origin
 };

@@ -1128,12 +1128,12 @@ __global__ void __launch_bounds__(APART_BLOCK) k_np_convex(int cap, const uint32
 				search = dot(d, d) <= reach * reach;
 				if (search)
 				{
-					// what the search would round away is left to it
-					const float need = cd + 1e-5f * reach;
 					const Poly B = hullPoly(hs, int(g1.x));
 					const mxf aToB = mxfOf(xinvmul(x1, x0));
 					const Poly A = t0 == GEOM_BOX ? boxPoly(mk(g0.x, g0.y, g0.z)) : hullPoly(hs, int(g0.x));
-					search = !convexApart(A, aToB, B, need, sub);
+					// pairs within rounding, or within what planes lie off their
+					// polygons' vertices (which the search also measures to), stay
+					search = !convexApart(A, aToB, B, cd + 1e-5f * reach + 4.0f * (A.slack + B.slack), sub);
 				}
 				if (!search && sub == 0)
 					ctN[slotBase + int(p)] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
@@ -1164,7 +1164,9 @@ __global__ void __launch_bounds__(64) k_np_round_convex(int cap, int slotBase, c
 			const uint2 ab = pairs[p];
 			const float4 g0 = geom[ab.x];
 			const f3 d = mk(pos[ab.y]) - mk(pos[ab.x]);
-			const float reach = (g0.x + (int(g0.w) == GEOM_CAPSULE ? g0.y : 0.0f) + hs.be[int(geom[ab.y].x)].w + cd) * 1.00001f;
+			const int hull = int(geom[ab.y].x);
+			const float core = g0.x + (int(g0.w) == GEOM_CAPSULE ? g0.y : 0.0f);
+			const float reach = (core + hs.be[hull].w + cd + 4.0f * __int_as_float(hs.info2[hull].w)) * 1.00001f;
 			near = !(dot(d, d) > reach * reach);
 			if (!near)
 				ctN[slotBase + p] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));

@@ -705,7 +705,19 @@ int appendHull(pxh_scene_t* s, const pxh::Hull& h)
 			return fail(PXH_ERR_UNSUPPORTED, "convex mesh: polygon with more than 16 vertices");
 	const int nv = int(h.verts.size() / 3), np = int(h.polys.size()), ne = int(h.edgeVerts.size() / 2);
 	s->hHullInfo.push_back(make_int4(int(s->hHullV.size()), nv, int(s->hHullP.size()), np));
-	s->hHullInfo2.push_back(make_int4(int(s->hHullVR.size()), int(s->hHullEdge.size()), ne, 0));
+	// how far a polygon's vertices lie below its plane (faces merged within a few
+	// degrees, or a cooked hull's own planes): plane distances are short of the
+	// vertices' distances by no more
+	float slack = 0.0f;
+	for (const pxh::HullPolygon& hp : h.polys)
+		for (int k = 0; k < int(hp.count); k++)
+		{
+			const float* v = &h.verts[3 * size_t(h.vref[size_t(hp.first) + size_t(k)])];
+			slack = std::max(slack, -(hp.plane[0] * v[0] + hp.plane[1] * v[1] + hp.plane[2] * v[2] + hp.plane[3]));
+		}
+	int slackBits;
+	std::memcpy(&slackBits, &slack, sizeof(slackBits));
+	s->hHullInfo2.push_back(make_int4(int(s->hHullVR.size()), int(s->hHullEdge.size()), ne, slackBits));
 	for (int i = 0; i < nv; i++)
 		s->hHullV.push_back(make_float4(h.verts[3 * i], h.verts[3 * i + 1], h.verts[3 * i + 2], 0.0f));
 	for (const pxh::HullPolygon& hp : h.polys)
