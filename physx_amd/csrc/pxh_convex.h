@@ -906,10 +906,9 @@ namespace pxh {
 // ---------------------------------------------------------------------------
 // One wavefront per convex pair: the 64 lanes split the face-axis, edge-pair
 // and closest-feature searches of polySeparation over the pair's vertices,
-// planes and edges staged in LDS; lane 0 then picks the witness polygons,
-// clips and reduces. Every search keeps polySeparation's order (the first
-// minimum in loop order wins), so the result is the same as the per-lane
-// path's.
+// planes and edges staged in LDS. Every search keeps polySeparation's order
+// (the first minimum in loop order wins), so the result is the same as the
+// per-lane path's.
 // ---------------------------------------------------------------------------
 constexpr int CVX_WAVE_V = 64, CVX_WAVE_P = 128, CVX_WAVE_E = 192, CVX_ARCS = 32;
 

@@ -2903,7 +2903,7 @@ __global__ void k_integrate(int n, float dt, float4* vel, float4* svP, float4* s
 // jointed bodies do not collide (PxConstraintFlag::eCOLLISION_ENABLED is off
 // by default, physx/include/PxConstraint.h): their pair slots lose their
 // contacts before the constraint list is built
-// Body-mesh narrowphase, one lane per body of a world with a mesh (k-th of
+// Body-mesh narrowphase of one body of a world with a mesh in a lane (k-th of
 // meshBody): candidate triangles through the mesh's tree (depth-first nodes,
 // each with the index after its subtree), taken in triangle order, then the
 // patches of pxh_mesh.h into slots slotBase + k * MESH_MAXP + patch (deepest

@@ -1,4 +1,5 @@
-// Contacts of one body against a static triangle mesh, one lane per body.
+// Contacts of one body against a static triangle mesh: a wave per body, a lane
+// where a wave can't hold it.
 //
 // A restatement of the reference's PCM mesh contact generation
 // (geomutils/src/pcm/GuPCMContactSphereMesh.cpp:160-501,

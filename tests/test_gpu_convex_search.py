@@ -52,3 +52,44 @@ def test_round_convex_matches_oracle(cuda, n_points, pitch):
     n = _compare_contacts(g, o)
     print(n_points, pitch, g.stats()["bp_pairs"], "pairs,", n, "with contacts", flush=True)
     assert 40 < n < g.stats()["bp_pairs"]
+
+
+def test_pairs_about_the_contact_distance_match_oracle(cuda):
+    """1,000 pairs of hulls whose vertices are, along the line of their centres, a
+    little less, as much or a little more than the contact distance apart:
+    whichever the separation search keeps or drops, the support steps, bounding
+    spheres and feature bounds before it decide alike. Odd pairs are a hull and a
+    capsule."""
+    n = 2000
+    sc = S.convex_layers(n_bodies=n, per_side=40, n_points=24, seed=21)
+    off = np.concatenate([[0], np.cumsum(sc.hull_counts)])
+    rng = np.random.default_rng(5)
+    cd = 0.04   # two contact offsets
+
+    def turned(i):
+        pts = P.cook_convex(sc.hull_points[off[i]:off[i + 1]])["verts"].astype(np.float64)
+        q, x = sc.pose[i, 3:6].astype(np.float64), float(sc.pose[i, 6])
+        return pts + 2.0 * np.cross(q, np.cross(q, pts) + x * pts)
+
+    for k in range(0, n, 2):
+        a, b = k, k + 1
+        va = turned(a)
+        if k % 4 == 2:
+            sc.shape_type[b] = S.CAPSULE
+            sc.dims[b] = (0.2, 0.3, 0.0, 0.0)
+            reach = 0.5
+            sc.pose[b, 3:7] = (0.0, 0.0, 0.0, 1.0)
+        else:
+            reach = -turned(b)[:, 0].min()
+        x = (k // 2) % 32 * 8.0
+        y, z = (k // 64) % 32 * 8.0, 0.0
+        sc.pose[a, :3] = (x, y, z)
+        sc.pose[b, :3] = (x + va[:, 0].max() + reach + cd + rng.uniform(-3e-3, 2e-3), y, z)
+    sc.planes, sc.plane_scene = np.zeros((0, 4), np.float32), np.zeros(0, np.int32)
+    sc.lin_vel[:], sc.ang_vel[:] = 0.0, 0.0
+    g = P.Scene(sc, position_iterations=4, velocity_iterations=1)
+    o = L.OracleWorld(sc, pos_iters=4, vel_iters=1)
+    g.step(DT)
+    o.step(DT)
+    assert _compare_contacts(g, o) > 0
+    print(g.stats()["bp_pairs"], "pairs,", g.stats()["constraints"], "with contacts", flush=True)
