@@ -309,7 +309,7 @@ PXH_D void polySeparation(const Poly& A, const mxf& aToB, const Poly& B, float c
 PXH_D void waveArgMin(float& v, uint32_t& idx);
 PXH_D float waveMin(float v);
 PXH_D f3 laneOf(f3 v, int l);
-PXH_D int witnessPolygonWave(const Poly& P, f3 normal, f3 closest, float tolerance, int lane);
+template <int LANES> PXH_D int witnessPolygonLanes(const Poly& P, f3 normal, f3 closest, float tolerance, int lane);
 
 // Gu::getWitnessPolygonIndex (geomutils/src/pcm/GuPCMContactGenUtil.cpp:201-271);
 // the per-polygon distances are evaluated again in the second pass
@@ -870,7 +870,7 @@ PXH_D int capsulePoly(float r, float hh, const xf& x0, const Poly& B, const xf& 
 	{
 		capsuleRayContacts(B, p0, p1, n, infl, aToB, lane, mc, nc);
 		if (nc < 2)
-			capsuleEEContacts(B, witnessPolygonWave(B, -n, cB, wtol, lane), p0, p1, n, infl, aToB, mc, nc);
+			capsuleEEContacts(B, witnessPolygonLanes<64>(B, -n, cB, wtol, lane), p0, p1, n, infl, aToB, mc, nc);
 	}
 	int i0 = 0, i1 = 1;
 	if (nc == 0)
@@ -1604,12 +1604,12 @@ PXH_D void convexSeparationWave(const Poly& A, const xf& x0, const Poly& B, cons
 }
 
 // ---------------------------------------------------------------------------
-// Contacts of a pair over a wave. In one lane the polygons, the points and the
-// reduction's candidates lie in scratch memory and every face, vertex and edge
-// waits for the one before: 107 us for the pairs of 8,192 hulls that touch, 65
-// for their plane pairs (16-lane waves). Here the wave scans the faces, takes a
-// vertex or an edge pair a lane and keeps the points in the order of the lane
-// form, so the choices are the same.
+// Contacts of a pair over 16 lanes, or of a hull and a plane over a wave. In one
+// lane the polygons, the points and the reduction's candidates lie in scratch
+// memory and every face, vertex and edge waits for the one before. Here the lanes
+// share the faces, take a vertex or an edge pair each and keep the points in the
+// order of the one-lane form, so the choices are the same. 8,192 hulls: pairs 107
+// us in lanes, 43 so (90 with a wave each); plane pairs 65 and 20.
 // ---------------------------------------------------------------------------
 struct ContactLds
 {
@@ -1627,31 +1627,61 @@ PXH_D float4 laneOf(float4 v, int l)
 
 PXH_D int laneRank(uint64_t m, int lane) { return int(__popcll(m & ((1ull << lane) - 1ull))); }
 
-// witnessPolygon
-PXH_D int witnessPolygonWave(const Poly& P, f3 normal, f3 closest, float tolerance, int lane)
+// Groups of 16 lanes, as many as a polygon may have vertices: lane i of a group is
+// gl = i; the lanes of a group always take the same way
+constexpr int GROUP = 16;
+static_assert(HULL_MAX_POLY_VERTS <= GROUP, "a polygon's vertices take a lane each");
+PXH_D uint32_t groupBallot(bool b) { return uint32_t(__ballot(b) >> (__lane_id() & 48)) & 0xFFFFu; }
+PXH_D float groupLane(float v, int i) { return __shfl(v, i, GROUP); }
+PXH_D f3 groupLane(f3 v, int i) { return mk(groupLane(v.x, i), groupLane(v.y, i), groupLane(v.z, i)); }
+PXH_D int groupRank(uint32_t m, int gl) { return __popc(m & ((1u << gl) - 1u)); }
+PXH_D void groupArgMin(float& v, uint32_t& idx)
+{
+	for (int off = GROUP / 2; off >= 1; off >>= 1)
+	{
+		const float ov = __shfl_xor(v, off);
+		const uint32_t oi = __shfl_xor(idx, off);
+		if (ov < v || (ov == v && oi < idx))
+		{
+			v = ov;
+			idx = oi;
+		}
+	}
+}
+
+template <int LANES> PXH_D void lanesArgMin(float& v, uint32_t& idx)
+{
+	if constexpr (LANES == 64)
+		waveArgMin(v, idx);
+	else
+		groupArgMin(v, idx);
+}
+
+// witnessPolygon over LANES lanes (64 or a group)
+template <int LANES> PXH_D int witnessPolygonLanes(const Poly& P, f3 normal, f3 closest, float tolerance, int lane)
 {
 	const float eps = -tolerance;
 	float minDist = FLT_BIG, least = FLT_BIG;   // least: minus the largest distance
 	uint32_t first = 0u, maxIdx = 0xFFFFFFFFu;
 	if (lane > 0)
 		first = 0xFFFFFFFFu;
-	for (int i = lane; i < P.np; i += 64)
+	for (int i = lane; i < P.np; i += LANES)
 	{
 		const float dist = dot(P.pn(i), closest) + P.pd(i);
 		const float pdi = dist >= eps ? fabsf(dist) : FLT_BIG;
 		if (minDist > pdi) { minDist = pdi; first = uint32_t(i); }
 		if (-dist < least) { least = -dist; maxIdx = uint32_t(i); }
 	}
-	waveArgMin(minDist, first);
+	lanesArgMin<LANES>(minDist, first);
 	if (minDist == FLT_BIG)
 	{
-		waveArgMin(least, maxIdx);
+		lanesArgMin<LANES>(least, maxIdx);
 		return maxIdx == 0xFFFFFFFFu ? 0 : int(maxIdx);
 	}
 	const float firstProj = dot(normalize(P.pn(int(first))), normal);
 	float bestProj = firstProj;
 	uint32_t idx = 0xFFFFFFFFu;
-	for (int i = lane; i < P.np; i += 64)
+	for (int i = lane; i < P.np; i += LANES)
 	{
 		const f3 pn = P.pn(i);
 		const float di = dot(pn, closest) + P.pd(i);
@@ -1662,25 +1692,25 @@ PXH_D int witnessPolygonWave(const Poly& P, f3 normal, f3 closest, float toleran
 			if (bestProj > proj) { idx = uint32_t(i); bestProj = proj; }
 		}
 	}
-	waveArgMin(bestProj, idx);
+	lanesArgMin<LANES>(bestProj, idx);
 	return idx == 0xFFFFFFFFu ? int(first) : int(idx);
 }
 
-// the bounds of the lanes' points that have one, widened
-PXH_D void waveBounds(bool has, f3 p, f3& mn, f3& mx)
+// the bounds of a group's points, widened
+PXH_D void groupBounds(bool has, f3 p, f3& mn, f3& mx)
 {
 	const float feps = 1.1920928955078125e-7f;
 	mn = has ? p : mk(FLT_BIG, FLT_BIG, FLT_BIG);
 	mx = has ? p : -mk(FLT_BIG, FLT_BIG, FLT_BIG);
-	for (int off = HULL_MAX_POLY_VERTS / 2; off >= 1; off >>= 1)
+	for (int off = GROUP / 2; off >= 1; off >>= 1)
 	{
 		mn.x = fminf(mn.x, __shfl_xor(mn.x, off));
 		mn.y = fminf(mn.y, __shfl_xor(mn.y, off));
 		mx.x = fmaxf(mx.x, __shfl_xor(mx.x, off));
 		mx.y = fmaxf(mx.y, __shfl_xor(mx.y, off));
 	}
-	mn = laneOf(mn, 0) - mk(feps, feps, feps);
-	mx = laneOf(mx, 0) + mk(feps, feps, feps);
+	mn = mn - mk(feps, feps, feps);
+	mx = mx + mk(feps, feps, feps);
 }
 
 // generatedContacts (geomutils/src/pcm/GuPCMContactGenBoxConvex.cpp:331-530) into
@@ -1688,44 +1718,44 @@ PXH_D void waveBounds(bool has, f3 p, f3& mn, f3& mx)
 // P0's frame to P1's; the points on P1 (its frame, onP1) or on P0's reference
 // plane (its frame), first the incident vertices inside, then the reference ones,
 // then the edge crossings; their number
-PXH_D int generatedContactsWave(const Poly& P0, const Poly& P1, int ref, int inc, const mxf& t0To1, float cd, bool onP1,
-                                ContactLds& L, int lane)
+PXH_D int generatedContactsGroup(const Poly& P0, const Poly& P1, int ref, int inc, const mxf& t0To1, float cd, bool onP1,
+                                ContactLds& L, int gl)
 {
 	const f3 n = normalize(P0.pn(ref));
 	const m33 rot = rotFromZ(n);
 	const int nr = P0.pcount(ref), ni = P1.pcount(inc);
-	const bool isRef = lane < nr, isInc = lane < ni;
+	const bool isRef = gl < nr, isInc = gl < ni;
 	f3 q0 = mk(0.0f, 0.0f, 0.0f), q1 = q0, vert1 = q0, mn, mx;
 	if (isRef)
 	{
-		q0 = mmul(rot, P0.vert(P0.pvert(ref, lane)));
-		L.p0[lane] = f4(q0, 0.0f);
+		q0 = mmul(rot, P0.vert(P0.pvert(ref, gl)));
+		L.p0[gl] = f4(q0, 0.0f);
 	}
-	const float d = laneOf(q0.z, 0), rd = d + cd;
+	const float d = groupLane(q0.z, 0), rd = d + cd;
 	float t1 = 0.0f;
 	bool pen = false;
 	if (isInc)
 	{
-		vert1 = P1.vert(P1.pvert(inc, lane));
+		vert1 = P1.vert(P1.pvert(inc, gl));
 		q1 = mmul(rot, mxtransinv(t0To1, vert1));
 		const float z = q1.z;
 		t1 = z - d;
 		q1.z = d;
-		L.p1[lane] = f4(q1, t1);
+		L.p1[gl] = f4(q1, t1);
 		pen = rd > z;
 	}
-	const uint64_t pens = __ballot(pen);
-	const f3 sPoint = laneOf(vert1, 0);
+	const uint32_t pens = groupBallot(pen);
+	const f3 sPoint = groupLane(vert1, 0);
 	waveSync();
-	waveBounds(isRef, q0, mn, mx);
+	groupBounds(isRef, q0, mn, mx);
 	bool in = pen && polyContainsN(L.p0, nr, q1, mn, mx);
-	uint64_t m = __ballot(in);
+	uint32_t m = groupBallot(in);
 	if (in)
-		L.pts[laneRank(m, lane)] = f4(onP1 ? vert1 : mtmul(rot, q1), t1);
-	int nc = int(__popcll(m));
+		L.pts[groupRank(m, gl)] = f4(onP1 ? vert1 : mtmul(rot, q1), t1);
+	int nc = __popc(m);
 	if (nc == ni)
 		return nc;
-	waveBounds(isInc, q1, mn, mx);
+	groupBounds(isInc, q1, mn, mx);
 	const f3 incN = normalize(P1.pn(inc));
 	const f3 nIn1 = mmul(t0To1.r, n);
 	in = isRef && polyContainsN(L.p1, ni, q0, mn, mx);
@@ -1738,27 +1768,27 @@ PXH_D int generatedContactsWave(const Poly& P0, const Poly& P1, int ref, int inc
 		t = dot(incN, sPoint - a) / dot(incN, nIn1);
 		in = !(t > cd);
 	}
-	m = __ballot(in);
+	m = groupBallot(in);
 	if (in)
-		L.pts[nc + laneRank(m, lane)] = f4(onP1 ? nIn1 * t + a : vert0, t);
-	const int inside = int(__popcll(m));
+		L.pts[nc + groupRank(m, gl)] = f4(onP1 ? nIn1 * t + a : vert0, t);
+	const int inside = __popc(m);
 	nc += inside;
 	if (inside == nr)
 		return nc;
-	FlatPair fp(lane, nr);
-	for (int k = lane; __any(k < ni * nr); k += 64, fp.next())
+	for (int k0 = 0; k0 < ni * nr; k0 += GROUP)
 	{
+		const int k = k0 + gl;
 		bool hit = k < ni * nr;
 		f3 pt = q0;
 		float sep = 0.0f;
 		if (hit)
 		{
-			const int iS = fp.i, rS = fp.j, iE = iS == 0 ? ni - 1 : iS - 1, rE = rS == 0 ? nr - 1 : rS - 1;
+			const int iS = k / nr, rS = k - iS * nr, iE = iS == 0 ? ni - 1 : iS - 1, rE = rS == 0 ? nr - 1 : rS - 1;
 			const float4 sA = L.p1[iS], sB = L.p1[iE];
 			const f3 ipA = mk(sA), ipB = mk(sB), rpA = mk(L.p0[rS]), rpB = mk(L.p0[rE]);
 			const float a1 = triArea2(rpA, rpB, ipA), a2 = triArea2(rpA, rpB, ipB);
 			const float a3 = triArea2(ipA, ipB, rpA), a4 = triArea2(ipA, ipB, rpB);
-			hit = (((pens >> iS) | (pens >> iE)) & 1ull) != 0ull &&
+			hit = (((pens >> iS) | (pens >> iE)) & 1u) != 0u &&
 			      !(fminf(ipA.x, ipB.x) > fmaxf(rpA.x, rpB.x) || fminf(ipA.y, ipB.y) > fmaxf(rpA.y, rpB.y) ||
 			        fminf(rpA.x, rpB.x) > fmaxf(ipA.x, ipB.x) || fminf(rpA.y, rpB.y) > fmaxf(ipA.y, ipB.y)) &&
 			      0.0f > a1 * a2 && 0.0f > a3 * a4;
@@ -1773,11 +1803,11 @@ PXH_D int generatedContactsWave(const Poly& P0, const Poly& P1, int ref, int inc
 				pt = onP1 ? mxtrans(t0To1, mtmul(rot, pBB)) : mtmul(rot, pAA);
 			}
 		}
-		m = __ballot(hit);
-		const int to = nc + laneRank(m, lane);
+		m = groupBallot(hit);
+		const int to = nc + groupRank(m, gl);
 		if (hit && to < HULL_MAX_CONTACTS)
 			L.pts[to] = f4(pt, sep);
-		nc += int(__popcll(m));
+		nc += __popc(m);
 		if (nc >= HULL_MAX_CONTACTS)
 			return HULL_MAX_CONTACTS;
 	}
@@ -1785,77 +1815,67 @@ PXH_D int generatedContactsWave(const Poly& P0, const Poly& P1, int ref, int inc
 }
 
 // Reduction to four (PersistentContactManifold::addBatchManifoldContacts,
-// geomutils/src/pcm/GuPersistentContactManifold.cpp:805-830) of the points in LDS
-// (their common normal cn0): their number, and in lane i the i-th
-PXH_D int batchReduceWave(const float4* pts, int n, f3 cn0, float tol, int lane, float4& out)
+// geomutils/src/pcm/GuPersistentContactManifold.cpp:805-830, reduceBatchContacts
+// :1008-1172) of the group's points in LDS (their common normal cn0): their
+// number, and in lane i the i-th. The points are the candidate list: one that is
+// taken leaves its place to the last.
+PXH_D int batchReduceGroup(float4* pts, int n, f3 cn0, float tol, int gl, float4& out)
 {
-	float4 c = pts[lane < n ? lane : 0];
-	out = c;
+	out = pts[gl < n ? gl : 0];
 	if (n <= 4)
 		return n;
 	int nc = n;
-	// lane i holds candidate i; one that is taken leaves its place to the last
 	auto drop = [&](int ci) {
 		nc--;
-		const float4 last = laneOf(c, nc);
-		if (lane == ci)
-			c = last;
+		const float4 last = pts[nc];
+		waveSync();
+		if (gl == 0)
+			pts[ci] = last;
+		waveSync();
 	};
-	float maxPen = laneOf(c.w, 0), minPen = maxPen;
-	int ci = 0;
-	for (int i = 1; i < n; i++)
-	{
-		const float pen = laneOf(c.w, i);
-		minPen = fmaxf(minPen, pen);
-		if (maxPen > pen) { maxPen = pen; ci = i; }
-	}
+	// the first candidate of the least value, -1 if none is below FLT_BIG
+	auto least = [&](auto value, float& v) {
+		v = FLT_BIG;
+		uint32_t idx = 0xFFFFFFFFu;
+		for (int i = gl; i < nc; i += GROUP)
+		{
+			const float x = value(pts[i]);
+			if (x < v) { v = x; idx = uint32_t(i); }
+		}
+		groupArgMin(v, idx);
+		return int(idx);
+	};
+	float maxPen, minPen, maxDist, minDist;
+	int ci = max(least([](float4 c) { return c.w; }, maxPen), 0);
+	least([](float4 c) { return -c.w; }, minPen);
+	minPen = -minPen;
 	float4 ch[4];
-	ch[0] = laneOf(c, ci);
+	ch[0] = pts[ci];
 	const f3 b0 = mk(ch[0]);
 	drop(ci);
-	f3 v = mk(c) - b0;
-	float h = dot(v, v);
-	float maxDist = laneOf(h, 0);
-	ci = 0;
-	for (int i = 1; i < nc; i++)
-	{
-		const float d = laneOf(h, i);
-		if (d > maxDist) { maxDist = d; ci = i; }
-	}
-	ch[1] = laneOf(c, ci);
+	ci = max(least([&](float4 c) { const f3 v = mk(c) - b0; return -dot(v, v); }, maxDist), 0);
+	ch[1] = pts[ci];
 	drop(ci);
 	f3 nrm = cross(mk(ch[1]) - b0, cn0);
 	const float sq = dot(nrm, nrm);
 	if (sq > 0.0f) { const float len = sqrtf(sq); nrm = mk(nrm.x / len, nrm.y / len, nrm.z / len); } else nrm = cn0;
-	v = mk(c) - b0;
-	h = dot(v, nrm);
-	maxDist = -FLT_BIG;
-	float minDist = FLT_BIG;
-	ci = 0;
-	int ci1 = 0;
-	for (int i = 0; i < nc; i++)
-	{
-		const float d = laneOf(h, i);
-		if (d > maxDist) { maxDist = d; ci = i; }
-		if (minDist > d) { minDist = d; ci1 = i; }
-	}
-	ch[2] = laneOf(c, ci);
-	ch[3] = laneOf(c, ci1);
+	auto height = [&](float4 c) { return dot(mk(c) - b0, nrm); };
+	ci = max(least([&](float4 c) { return -height(c); }, maxDist), 0);
+	maxDist = -maxDist;
+	int ci1 = max(least(height, minDist), 0);
+	ch[2] = pts[ci];
+	ch[3] = pts[ci1];
 	drop(ci);
 	if (nc == ci1)
 		ci1 = ci;
 	if (minDist * maxDist > 0.0f)
 	{
-		v = mk(c) - b0;
-		h = dot(v, nrm);
-		maxDist = -FLT_BIG;
-		for (int i = 0; i < nc; i++)
+		const int far = least([&](float4 c) { return -height(c); }, maxDist);
+		if (far >= 0)
 		{
-			const float d = laneOf(h, i);
-			if (d > maxDist) { maxDist = d; ci1 = i; }
+			ci1 = far;
+			ch[3] = pts[far];
 		}
-		if (maxDist > -FLT_BIG)
-			ch[3] = laneOf(c, ci1);
 	}
 	drop(ci1);
 	const float eps = tol * 0.02f;
@@ -1864,26 +1884,24 @@ PXH_D int batchReduceWave(const float4* pts, int n, f3 cn0, float tol, int lane,
 #pragma unroll
 		for (int i = 0; i < 4; i++)
 		{
-			float pen = ch[i].w;
+			const float pen = ch[i].w;
 			if (pen > eps)
 			{
-				int cidx = -1;
-				for (int j = 0; j < nc; j++)
-				{
-					const float pen1 = laneOf(c.w, j);
-					if (pen > pen1 && eps > pen1) { pen = pen1; cidx = j; }
-				}
-				if (cidx >= 0)
+				float v;
+				const int c = least([&](float4 q) { return pen > q.w && eps > q.w ? q.w : FLT_BIG; }, v);
+				if (c >= 0)
 				{
 					const float4 orig = ch[i];
-					ch[i] = laneOf(c, cidx);
-					if (lane == cidx)
-						c = orig;
+					ch[i] = pts[c];
+					waveSync();
+					if (gl == 0)
+						pts[c] = orig;
+					waveSync();
 				}
 			}
 		}
 	}
-	out = lane == 0 ? ch[0] : lane == 1 ? ch[1] : lane == 2 ? ch[2] : ch[3];
+	out = gl == 0 ? ch[0] : gl == 1 ? ch[1] : gl == 2 ? ch[2] : ch[3];
 	return 4;
 }
 
@@ -1898,28 +1916,28 @@ PXH_D int batchReduceWave(const float4* pts, int n, f3 cn0, float tol, int lane,
 // summed normal (PersistentContactManifold::addManifoldContactsToContactBuffer /
 // getWorldNormal, GuPersistentContactManifold.cpp:739-762,
 // GuPersistentContactManifold.h:405-416)
-PXH_D void convexContactsWave(const Poly& A, const xf& x0, const Poly& B, const xf& x1, float dist, f3 n, f3 cA, f3 cB,
-                              float cd, float tol, ContactLds& L, int lane, int64_t slot, float4* ctN, float4* ctP)
+PXH_D void convexContactsGroup(const Poly& A, const xf& x0, const Poly& B, const xf& x1, float dist, f3 n, f3 cA, f3 cB,
+                              float cd, float tol, ContactLds& L, int gl, int64_t slot, float4* ctN, float4* ctP)
 {
 	const mxf aToB = mxfOf(xinvmul(x1, x0));
 	const float lo = tol * 1e-2f, hi = tol * 5e-2f;
 	const float tA = fminf(fmaxf(A.margin, lo), hi), tB = fminf(fmaxf(B.margin, lo), hi);
 	const f3 negN = -n;
 	const f3 nIn0 = mtmul(aToB.r, n);
-	const int f1 = witnessPolygonWave(B, negN, cB, tB, lane);
-	const int f0 = witnessPolygonWave(A, nIn0, mxtransinv(aToB, cA), tA, lane);
+	const int f1 = witnessPolygonLanes<GROUP>(B, negN, cB, tB, gl);
+	const int f0 = witnessPolygonLanes<GROUP>(A, nIn0, mxtransinv(aToB, cA), tA, gl);
 	const f3 refN = normalize(B.pn(f1)), incN = normalize(A.pn(f0));
 	f3 ln;
 	int nc;
 	if (fabsf(dot(refN, negN)) >= fabsf(dot(incN, nIn0)))
 	{
 		const mxf bToA = mxfOf(xinvmul(x0, x1));
-		nc = generatedContactsWave(B, A, f1, f0, bToA, cd, false, L, lane);
+		nc = generatedContactsGroup(B, A, f1, f0, bToA, cd, false, L, gl);
 		ln = refN;
 	}
 	else
 	{
-		nc = generatedContactsWave(A, B, f0, f1, aToB, cd, true, L, lane);
+		nc = generatedContactsGroup(A, B, f0, f1, aToB, cd, true, L, gl);
 		ln = -mmul(aToB.r, incN);
 	}
 	waveSync();
@@ -1931,16 +1949,16 @@ PXH_D void convexContactsWave(const Poly& A, const xf& x0, const Poly& B, const 
 		nc = 1;
 	}
 	else
-		nc = batchReduceWave(L.pts, nc, ln, tol, lane, pt);
+		nc = batchReduceGroup(L.pts, nc, ln, tol, gl, pt);
 	f3 s = ln;
 	for (int i = 1; i < nc; i++)
 		s = s + ln;
-	const bool keep = lane < nc && cd >= pt.w;
-	const uint64_t m = __ballot(keep);
+	const bool keep = gl < nc && cd >= pt.w;
+	const uint32_t m = groupBallot(keep);
 	if (keep)
-		ctP[4 * slot + laneRank(m, lane)] = f4(xtrans(x1, mk(pt)), pt.w);
-	if (lane == 0)
-		ctN[slot] = f4(normalize(qrot(x1.q, s)), __int_as_float(int(__popcll(m))));
+		ctP[4 * slot + groupRank(m, gl)] = f4(xtrans(x1, mk(pt)), pt.w);
+	if (gl == 0)
+		ctN[slot] = f4(normalize(qrot(x1.q, s)), __int_as_float(int(__popc(m))));
 	waveSync();
 }
 
@@ -2038,7 +2056,7 @@ PXH_D void planeConvexWave(f3 pn, float pd, const Poly& B, const xf& tb, float c
 	waveSync();
 	float4 pt = f4(pn, 0.0f);
 	if (nc > 0)
-		nc = batchReduceWave(L.pts, nc, pn, tol, lane, pt);
+		nc = batchReduceGroup(L.pts, nc, pn, tol, lane & (GROUP - 1), pt);
 	const bool keep = lane < nc && cd >= pt.w;
 	const uint64_t k = __ballot(keep);
 	if (keep)

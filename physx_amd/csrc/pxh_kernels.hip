@@ -1243,38 +1243,39 @@ k_np_convex_wave(int cap, const uint2* pairs, const float4* pos, const float4* r
 	}
 }
 
-// Box- and convex-convex pairs, contact phase: a wave per touching pair of the
+// Box- and convex-convex pairs, contact phase: 16 lanes per touching pair of the
 // search list (witness polygons, clipping, reduction); the others get their empty
-// slot. Waves take thinLanes pairs at a time. The list order does not matter, pair
-// p fills slot slotBase + p.
+// slot. The list order does not matter, pair p fills slot slotBase + p. Bound by a
+// pair's chain of dependent loads and steps: for 20,600 touching pairs of 8,192
+// hulls 107 us in a lane each, 90 in a wave each, 43 so (a terrain's few pairs
+// 42, 13 and 19: a wave that takes one group only still needs 18).
 __global__ void __launch_bounds__(64) k_np_convex_finish(int cap, int slotBase, const uint2* pairs, const float4* pos,
                                                          const float4* rot, const float4* geom, HullSet hs, float cd,
                                                          float tol, const float4* wit, const uint32_t* list,
                                                          float4* ctN, float4* ctP)
 {
-	__shared__ ContactLds L;
-	const int lane = threadIdx.x;
-	const uint32_t count = min(list[0], uint32_t(cap)), lanes = uint32_t(thinLanes(count));
-	for (uint32_t base = blockIdx.x * lanes; base < count; base += gridDim.x * lanes)
+	__shared__ ContactLds lds[64 / GROUP];
+	const int gl = threadIdx.x % GROUP, group = threadIdx.x / GROUP;
+	const uint32_t count = min(list[0], uint32_t(cap));
+	for (uint32_t q = blockIdx.x * (64 / GROUP) + group; q < count; q += gridDim.x * (64 / GROUP))
 	{
-		const bool live = uint32_t(lane) < lanes && base + lane < count;
-		const int p = live ? int(cvxEntries(list, cap, 0)[base + lane]) : 0;
-		const bool touch = live && wit[3 * int64_t(p)].x <= cd;
-		if (live && !touch)
-			ctN[slotBase + p] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
-		for (uint64_t m = __ballot(touch); m != 0ull; m &= m - 1ull)
+		const int p = int(cvxEntries(list, cap, 0)[q]);
+		const float4 sep = wit[3 * int64_t(p)];
+		if (!(sep.x <= cd))
 		{
-			const int pp = laneOf(p, __ffsll((unsigned long long)m) - 1);
-			const uint2 ab = pairs[pp];
-			const float4 g0 = geom[ab.x], g1 = geom[ab.y], sep = wit[3 * int64_t(pp)];
-			xf x0, x1;
-			x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
-			x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
-			const Poly B = hullPoly(hs, int(g1.x));
-			const Poly A = int(g0.w) == GEOM_BOX ? boxPoly(mk(g0.x, g0.y, g0.z)) : hullPoly(hs, int(g0.x));
-			convexContactsWave(A, x0, B, x1, sep.x, mk(sep.y, sep.z, sep.w), mk(wit[3 * int64_t(pp) + 1]),
-			                   mk(wit[3 * int64_t(pp) + 2]), cd, tol, L, lane, int64_t(slotBase) + pp, ctN, ctP);
+			if (gl == 0)
+				ctN[slotBase + p] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(0));
+			continue;
 		}
+		const uint2 ab = pairs[p];
+		const float4 g0 = geom[ab.x], g1 = geom[ab.y];
+		xf x0, x1;
+		x0.p = mk(pos[ab.x]); x0.q = mkq(rot[ab.x]);
+		x1.p = mk(pos[ab.y]); x1.q = mkq(rot[ab.y]);
+		const Poly B = hullPoly(hs, int(g1.x));
+		const Poly A = int(g0.w) == GEOM_BOX ? boxPoly(mk(g0.x, g0.y, g0.z)) : hullPoly(hs, int(g0.x));
+		convexContactsGroup(A, x0, B, x1, sep.x, mk(sep.y, sep.z, sep.w), mk(wit[3 * int64_t(p) + 1]),
+		                    mk(wit[3 * int64_t(p) + 2]), cd, tol, lds[group], gl, int64_t(slotBase) + p, ctN, ctP);
 	}
 }
 
@@ -4096,7 +4097,7 @@ void launch_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int 
 	const int blocks = std::min((cap + CVX_WAVES - 1) / CVX_WAVES, 8192);
 	k_np_convex_wave<<<blocks, 64 * CVX_WAVES, 0, st>>>(cap, pairs, pos, rot, geom, hs, cd, wit, list);
 	k_np_round_convex<<<thinGrid(cap), 64, 0, st>>>(cap, slotBase, pairs, pos, rot, geom, hs, cd, tol, ctN, ctP, list);
-	k_np_convex_finish<<<thinGrid(cap), 64, 0, st>>>(cap, slotBase, pairs, pos, rot, geom, hs, cd, tol, wit, list, ctN,
+	k_np_convex_finish<<<std::min((cap * GROUP + 63) / 64, 16384), 64, 0, st>>>(cap, slotBase, pairs, pos, rot, geom, hs, cd, tol, wit, list, ctN,
 	                                                 ctP);
 }
 void launch_np_planes_convex(int Q, int slotBase, const int* qBody, const int* qPlane, const float4* pos,
