@@ -3655,6 +3655,7 @@ __global__ void __launch_bounds__(THREADS, 2) k_solve_worlds(int nWorlds, const 
 				if constexpr (PGS)
 				{
 					if (it == posIters - 1)
+					{
 						for (int i = b0 + tid; i < b0 + nb; i += THREADS)
 						{
 							float4 v[4];
@@ -3662,6 +3663,8 @@ __global__ void __launch_bounds__(THREADS, 2) k_solve_worlds(int nWorlds, const 
 							sb.p[i] = v[0];
 							sb.dq[i] = v[1];
 						}
+						__syncthreads();   // the velocity passes change what is saved here
+					}
 				}
 				else if (posIter)
 				{

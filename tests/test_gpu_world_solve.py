@@ -75,3 +75,24 @@ def test_worlds_added_after_joints(cuda):
         scenes.append(s)
     for x, y in zip(scenes[1].bodies(), scenes[0].bodies()):
         np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("lds", [None, 0])
+@pytest.mark.parametrize("bodies", [65, 257, 500, 1023, 1024])
+def test_pgs_motion_of_large_worlds(cuda, bodies, lds):
+    """PGS worlds with several bodies a thread, the last wave of them partly
+    idle: the motion saved after the position passes is that of the position
+    passes, before any velocity pass changes it."""
+    sc = S.batched_piles(n_scenes=4, nmin=bodies, nmax=bodies, seed=bodies)
+    kw = dict(position_iterations=4, velocity_iterations=2, solver_type=P.PXH_SOLVER_PGS)
+    a, b = P.Scene(sc, **kw), P.Scene(sc, **kw)
+    a.set_tuning(layout=P.PXH_SOLVE_LAYOUT_COLORS)
+    if lds is not None:
+        b.set_tuning(layout=P.PXH_SOLVE_LAYOUT_WORLDS, lds_bodies=lds)
+    for _ in range(40):
+        a.step(DT)
+        b.step(DT)
+    assert b.stats()["solve_launches"] == 1 < a.stats()["solve_launches"]
+    assert a.stats()["constraints"] > bodies
+    for x, y, name in zip(b.bodies(), a.bodies(), ("pose", "linear velocity", "angular velocity")):
+        np.testing.assert_array_equal(x, y, err_msg=name)
