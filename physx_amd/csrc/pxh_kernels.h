@@ -215,9 +215,9 @@ void launch_color_rounds(int m, const uint32_t* mDev, const int* list, int first
                          const int* conA, const int* conB, const uint64_t* conKey, int* conColor, uint64_t* best,
                          ColorState cs, int* out, uint32_t* left, uint32_t* ran, bool oneBlock, hipStream_t st);
 void launch_fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t st);
-// body-plane colours, then the (colour, index) sort keys
-void launch_color_keys(int C, const int* conA, const int* conB, int* conColor, ColorState cs, uint32_t limit,
-                       uint64_t* keys, uint32_t* vals, hipStream_t st);
+// body-plane and body-mesh colours (nPlanes planes in all), then the (colour, index) sort keys
+void launch_color_keys(int C, const int* conA, const int* conB, int nPlanes, int* conColor, ColorState cs,
+                       uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st);
 void launch_patch_table(int m, const uint64_t* keys, ulonglong2* table, uint32_t mask, hipStream_t st);
 // finds each constraint's row of the previous step; body-body constraints keep
 // their previous colour, the others go to list (count in cs.words[STEP_OPEN])
@@ -244,7 +244,7 @@ void launch_solve(int begin, int end, int C, Rows rows, SolverBodies sb, float m
                   float invStepDt, float biasScale, float scale, uint32_t* broken, hipStream_t st,
                   hipEvent_t evStart = nullptr, hipEvent_t evStop = nullptr);
 // rows in (world, colour) order for the per-world solve
-void launch_color_keys_world(int C, const int* conA, const int* conB, int* conColor, ColorState cs,
+void launch_color_keys_world(int C, const int* conA, const int* conB, int nPlanes, int* conColor, ColorState cs,
                              const int* bodyWorld, uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st);
 // every iteration of every world in one launch of `workgroups` persistent
 // workgroups (0: as many as run at a time), TGS or, with rowsU, PGS passes;

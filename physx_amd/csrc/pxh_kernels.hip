@@ -1722,21 +1722,39 @@ __global__ void k_color_mask(int C, const int* conA, const int* conB, const int*
 		atomicOr(&cs.mask[b], 1ull << col);
 }
 
-// Body-plane constraints go after every colour of their body's body-body
-// constraints, one colour each in constraint order (the reference places
-// static constraints at maxSolverNormalProgress + k:
+// Body-plane and body-mesh constraints go after every colour of their body's
+// body-body constraints, one colour each in constraint order (the reference
+// places static constraints at maxSolverNormalProgress + k:
 // lowleveldynamics/src/DyConstraintPartition.cpp:168-179, 604-616). The last
-// colour of a body is the top bit of its mask, or past 63 its `next`. A body's
-// body-plane constraints are consecutive in the constraint list (slots are
-// body-major); k counts the ones before c.
-PXH_D int constraintColor(int c, const int* conA, const int* conB, const ColorState& cs, int* conColor)
+// colour of a body is the top bit of its mask, or past 63 its `next`. k counts the
+// body's static constraints before c: its plane constraints lead the list beside
+// each other (slots are body-major, the bodies ascending), its mesh patches end it,
+// also beside each other, with the body pairs between; where a world has planes
+// and a mesh, a patch finds its body's plane constraints by bisection.
+PXH_D int constraintColor(int c, const int* conA, const int* conB, int nPlanes, const ColorState& cs, int* conColor)
 {
+	auto plane = [&](int e) { return conB[e] < 0 && -1 - conB[e] < nPlanes; };
 	if (conB[c] >= 0)
 		return conColor[c];
 	const int a = conA[c];
+	const bool patch = !plane(c);
 	int k = 0;
-	for (int e = c - 1; e >= 0 && conA[e] == a && conB[e] < 0; e--)
+	for (int e = c - 1; e >= 0 && conA[e] == a && conB[e] < 0 && plane(e) != patch; e--)
 		k++;
+	if (patch && nPlanes > 0)
+	{
+		int lo = 0, hi = c;
+		while (lo < hi)
+		{
+			const int m = (lo + hi) >> 1;
+			if (plane(m) && conA[m] < a)
+				lo = m + 1;
+			else
+				hi = m;
+		}
+		for (; lo < c && plane(lo) && conA[lo] == a; lo++)
+			k++;
+	}
 	const unsigned long long m = cs.mask[a];
 	const int next = max(int(cs.next[a]), m ? 64 - __clzll((long long)m) : 0);
 	conColor[c] = next + k;
@@ -1825,13 +1843,13 @@ __global__ void __launch_bounds__(256) k_con_prev(int C, const int* conA, const 
 // colour-ordered constraint list by a stable radix sort of (colour, index)
 // A constraint not coloured yet (-1, when the rounds have not finished) sorts
 // to colour `limit`, past every real colour.
-__global__ void k_color_keys(int C, const int* conA, const int* conB, int* conColor, ColorState cs, uint32_t limit,
-                             uint64_t* keys, uint32_t* vals)
+__global__ void k_color_keys(int C, const int* conA, const int* conB, int nPlanes, int* conColor, ColorState cs,
+                             uint32_t limit, uint64_t* keys, uint32_t* vals)
 {
 	const int c = blockIdx.x * blockDim.x + threadIdx.x;
 	if (c < C)
 	{
-		const int col = constraintColor(c, conA, conB, cs, conColor);
+		const int col = constraintColor(c, conA, conB, nPlanes, cs, conColor);
 		const uint32_t k = col < 0 ? limit : min(uint32_t(col), limit);
 		keys[c] = (uint64_t(k) << 32) | uint32_t(c);
 		vals[c] = uint32_t(c);
@@ -1839,16 +1857,16 @@ __global__ void k_color_keys(int C, const int* conA, const int* conB, int* conCo
 }
 // rows ordered by (world, colour): key world * CB + colour, CB = limit + 1; the
 // largest colour in the step's words (one atomic a block)
-__global__ void __launch_bounds__(256) k_color_keys_world(int C, const int* conA, const int* conB, int* conColor,
-                                                          ColorState cs, const int* bodyWorld, uint32_t limit,
-                                                          uint64_t* keys, uint32_t* vals)
+__global__ void __launch_bounds__(256) k_color_keys_world(int C, const int* conA, const int* conB, int nPlanes,
+                                                          int* conColor, ColorState cs, const int* bodyWorld,
+                                                          uint32_t limit, uint64_t* keys, uint32_t* vals)
 {
 	__shared__ int red[4];
 	const int c = blockIdx.x * blockDim.x + threadIdx.x;
 	int top = 0;
 	if (c < C)
 	{
-		const int col = constraintColor(c, conA, conB, cs, conColor);
+		const int col = constraintColor(c, conA, conB, nPlanes, cs, conColor);
 		const uint32_t k = col < 0 ? limit : min(uint32_t(col), limit);
 		const uint64_t w = uint64_t(bodyWorld[conA[c]]);
 		keys[c] = ((w * (limit + 1) + k) << 32) | uint32_t(c);
@@ -4265,10 +4283,10 @@ void launch_con_prev(int C, const int* conA, const int* conB, const int* conSlot
 {
 	PXH_LAUNCH(k_con_prev, C, C, conA, conB, conSlot, io, conColor, cs, list);
 }
-void launch_color_keys(int C, const int* conA, const int* conB, int* conColor, ColorState cs, uint32_t limit,
-                       uint64_t* keys, uint32_t* vals, hipStream_t st)
+void launch_color_keys(int C, const int* conA, const int* conB, int nPlanes, int* conColor, ColorState cs,
+                       uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st)
 {
-	PXH_LAUNCH(k_color_keys, C, C, conA, conB, conColor, cs, limit, keys, vals);
+	PXH_LAUNCH(k_color_keys, C, C, conA, conB, nPlanes, conColor, cs, limit, keys, vals);
 }
 void launch_preintegrate(int n, const float4* pos, const float4* rot, const float4* lin, const float4* ang,
                          const float4* invI, float3 gdt, float linDampDt, float angDampDt, float maxLinSq,
@@ -4305,10 +4323,10 @@ void launch_solve(int begin, int end, int C, Rows rows, SolverBodies sb, float m
 		k_solve<<<grid, block, 0, st>>>(begin, end, C, rows, sb.vel, minPen, muS, muD, invStepDt, biasScale, scale,
 		                                broken);
 }
-void launch_color_keys_world(int C, const int* conA, const int* conB, int* conColor, ColorState cs,
+void launch_color_keys_world(int C, const int* conA, const int* conB, int nPlanes, int* conColor, ColorState cs,
                              const int* bodyWorld, uint32_t limit, uint64_t* keys, uint32_t* vals, hipStream_t st)
 {
-	PXH_LAUNCH(k_color_keys_world, C, C, conA, conB, conColor, cs, bodyWorld, limit, keys, vals);
+	PXH_LAUNCH(k_color_keys_world, C, C, conA, conB, nPlanes, conColor, cs, bodyWorld, limit, keys, vals);
 }
 void launch_fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t st)
 {

@@ -682,8 +682,8 @@ int uploadWorldJoints(pxh_scene_t* s)
 // before them the pair and constraint counts) in [0, kHostColorSlots), the
 // step's counters (u64) at kHostCounterSlot, its device words at kHostWordSlot
 constexpr size_t kHostCountsBytes = 65536;
-constexpr int kHostColorSlots = 15000;
-constexpr int kHostCounterSlot = 15000;
+constexpr int kHostColorSlots = 15004;
+constexpr int kHostCounterSlot = 15008;
 constexpr int kHostWordSlot = 15016;
 
 // b[i] = b[idx[i]] for i < n, through a scratch buffer that stays with the scene
@@ -1938,7 +1938,9 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	}
 	int rounds = 0;
 	const int kMaxRounds = 960;
-	if (64 + kMaxRounds + s->maxPlanes + 2 > kHostColorSlots)
+	// colours of a body's static constraints, past its body-body ones
+	const int staticColors = s->maxPlanes + (s->nMeshBodies > 0 ? pxh::MESH_MAXP : 0);
+	if (64 + kMaxRounds + staticColors + 2 > kHostColorSlots)
 		return fail(PXH_ERR_CAPACITY, "pxh_scene_simulate: too many planes in one world");
 	int nColors = 0;
 	std::vector<uint32_t> colorStart(1, 0);
@@ -1973,9 +1975,9 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		                         s->stepWords.p + pxh::STEP_RAN, oneBlock, st);
 		rounds += batch;
 		// row order: stable radix sort of (colour, index), colours staying below
-		// 64 + rounds + planes per world; for the per-world solve of (world,
+		// 64 + rounds + planes and mesh patches; for the per-world solve of (world,
 		// colour, index), the row starts of every (world, colour) from the keys
-		const int colorBound = 64 + rounds + s->maxPlanes + 1;
+		const int colorBound = 64 + rounds + staticColors + 1;
 		uint64_t slots = uint64_t(colorBound) + 1;
 		if (worldSolve)
 		{
@@ -1991,11 +1993,11 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		uint32_t* va = alt ? s->vals.p : reinterpret_cast<uint32_t*>(s->order.p);
 		uint32_t* vb = alt ? reinterpret_cast<uint32_t*>(s->order.p) : s->vals2.p;
 		if (worldSolve)
-			pxh::launch_color_keys_world(C, s->conA.p, s->conB.p, s->conColor.p, colors, s->scene.p,
+			pxh::launch_color_keys_world(C, s->conA.p, s->conB.p, s->m, s->conColor.p, colors, s->scene.p,
 			                             uint32_t(colorBound), s->keys.p, va, st);
 		else
-			pxh::launch_color_keys(C, s->conA.p, s->conB.p, s->conColor.p, colors, uint32_t(colorBound), s->keys.p, va,
-			                       st);
+			pxh::launch_color_keys(C, s->conA.p, s->conB.p, s->m, s->conColor.p, colors, uint32_t(colorBound), s->keys.p,
+			                       va, st);
 		pxh::launch_radix_sort(s->keys.p, va, s->keys2.p, vb, C, 0, bits, s->hist.p, st, alt);
 		const uint64_t* ck = alt ? s->keys2.p : s->keys.p;
 		pxh::launch_row_start(C, ck, worldSolve ? s->segStart.p : s->hostCounts,
