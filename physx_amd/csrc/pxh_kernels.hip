@@ -13,6 +13,7 @@
 //   solve (solverMultiBlockTGS.cu solveBlockUnified)        k_solve
 //   integration (integrationTGS.cu)                         k_integrate, k_finalize
 #include "pxh_kernels.h"
+#include "pxh_launch.h"
 #include <hip/hip_ext.h>
 #include "pxh_np.h"
 #include "pxh_convex.h"
@@ -4112,14 +4113,14 @@ void launch_np_convex(int cap, const uint32_t* dP, const uint32_t* dConvex, int 
 	if (cap <= 0)
 		return;
 	k_fill_u32<<<1, 64, 0, st>>>(list, 2, 0u);
-	k_np_convex<<<std::min((cap + APART_BLOCK / APART_LANES - 1) / (APART_BLOCK / APART_LANES), 2048), APART_BLOCK, 0, st>>>(
-		cap, dP, dConvex, slotBase, pairs, pos, rot, geom, hs, cd, ctN, list);
 	// grid-stride: enough waves to fill the chip several times over
-	const int blocks = std::min((cap + CVX_WAVES - 1) / CVX_WAVES, 8192);
-	k_np_convex_wave<<<blocks, 64 * CVX_WAVES, 0, st>>>(cap, pairs, pos, rot, geom, hs, cd, wit, list);
+	k_np_convex<<<strideBlocks(cap, APART_BLOCK / APART_LANES, 2048), APART_BLOCK, 0, st>>>(
+	    cap, dP, dConvex, slotBase, pairs, pos, rot, geom, hs, cd, ctN, list);
+	k_np_convex_wave<<<strideBlocks(cap, CVX_WAVES, 8192), 64 * CVX_WAVES, 0, st>>>(cap, pairs, pos, rot, geom, hs, cd,
+	                                                                              wit, list);
 	k_np_round_convex<<<thinGrid(cap), 64, 0, st>>>(cap, slotBase, pairs, pos, rot, geom, hs, cd, tol, ctN, ctP, list);
-	k_np_convex_finish<<<std::min((cap * GROUP + 63) / 64, 16384), 64, 0, st>>>(cap, slotBase, pairs, pos, rot, geom, hs, cd, tol, wit, list, ctN,
-	                                                 ctP);
+	k_np_convex_finish<<<strideBlocks(cap, 64 / GROUP, 16384), 64, 0, st>>>(cap, slotBase, pairs, pos, rot, geom, hs, cd,
+	                                                                      tol, wit, list, ctN, ctP);
 }
 void launch_np_planes_convex(int Q, int slotBase, const int* qBody, const int* qPlane, const float4* pos,
                              const float4* rot, const float4* geom, const float4* planes, const HullSet& hs, float cd,
