@@ -1387,8 +1387,10 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, Cvx
 	// distance U, so the minimum is no larger. Along the face axis that
 	// separates the polytopes most, A's heights less B's bound every distance
 	// from below: a vertex or an edge whose height alone is farther from the
-	// other polytope than lim = sqrt(U) plus a margin well above rounding, and
-	// above what planes lie off their polygons' vertices, holds no closest feature.
+	// other polytope than lim = sqrt(U) plus a margin holds no closest feature. The
+	// margin is above what planes lie off their polygons' vertices and well above
+	// rounding: a height or a distance is off by a few units in the last place (6e-8
+	// each) of the largest coordinate, the margin is 1e-5 of it.
 	// What is left keeps its order and its indices, so the first minimum is unchanged.
 	int nA, nB;
 	float minA = 0.0f, maxB = 0.0f;
@@ -1434,7 +1436,9 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, Cvx
 		U = fminf(U, edgePairSq(L, L.elA[fu.i], L.elB[fu.j], c1, c2));
 	}
 	U = waveMin(U);
-	const float margin = 1e-4f + A.slack + B.slack;
+	const f3 pA = lane < A.nv ? ldsV(L.va, lane) : mk(0.0f, 0.0f, 0.0f), pB = lane < B.nv ? ldsV(L.vb, lane) : pA;
+	const float extent = -waveMin(-fmaxf(fabsf(pA.x) + fabsf(pA.y) + fabsf(pA.z), fabsf(pB.x) + fabsf(pB.y) + fabsf(pB.z)));
+	const float margin = 1e-4f + 1e-5f * extent + A.slack + B.slack;
 	float lim = U < BIG ? sqrtf(U) + margin : BIG;
 	waveSync();
 	float d2 = BIG;

@@ -93,3 +93,55 @@ def test_pairs_about_the_contact_distance_match_oracle(cuda):
     o.step(DT)
     assert _compare_contacts(g, o) > 0
     print(g.stats()["bp_pairs"], "pairs,", g.stats()["constraints"], "with contacts", flush=True)
+
+
+@pytest.mark.parametrize("scale", [0.01, 1.0, 100.0, 1e4, 1e5])
+def test_parallel_faces_at_scale_match_oracle(cuda, monkeypatch, scale):
+    """400 pairs of bricks with facing faces parallel and less than the contact
+    distance apart, lengths in units from 100 m to 10 um: every vertex and
+    edge of the facing faces lies at the distance itself, so a feature bound that
+    is tighter than the rounding of a height drops them. The tolerances scale with
+    the lengths; the rounding of coordinates of 1.5 lengths is 1e-7 of them."""
+    pairs = 400
+    rng = np.random.default_rng(17)
+    half = rng.uniform(0.2, 0.6, (2 * pairs, 3)) * scale
+    corner = np.array([[x, y, z] for x in (-1, 1) for y in (-1, 1) for z in (-1, 1)], np.float64)
+    pts = (half[:, None, :] * corner).astype(np.float32)
+    q = rng.normal(size=(pairs, 4))
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    cd = 0.04 * scale
+    d = np.zeros((pairs, 3))
+    d[:, 0] = half[::2, 0] + half[1::2, 0] + rng.uniform(0.05, 0.95, pairs) * cd
+    d[:, 1:] = rng.uniform(-0.15, 0.15, (pairs, 2)) * scale
+    qv, w = q[:, :3], q[:, 3:]
+    t = 2.0 * np.cross(qv, d)
+    at = d + w * t + np.cross(qv, t)
+    n = 2 * pairs
+    pose = np.zeros((n, 7), np.float32)
+    pose[1::2, :3] = at
+    pose[::2, 3:] = q
+    # the second brick turned about the line between the faces
+    a = rng.uniform(0.0, np.pi, (pairs, 1))
+    sx, cx = np.sin(a), np.cos(a)
+    x, y, z_, w_ = (q[:, k:k + 1] for k in range(4))
+    pose[1::2, 3:] = np.concatenate([x * cx + w_ * sx, y * cx + z_ * sx, z_ * cx - y * sx, w_ * cx - x * sx], 1)
+    dims = np.zeros((n, 4), np.float32)
+    dims[:, 0] = np.arange(n)
+    m, inn = S.mass_props(np.full(n, S.BOX, np.int32), np.concatenate([half, half[:, :1]], 1), 1000.0 / scale**3)
+    z = np.zeros((n, 3), np.float32)
+    sc = S.Scene(np.full(n, S.CONVEX, np.int32), dims, pose, z, z.copy(), m, inn,
+                 np.repeat(np.arange(pairs, dtype=np.int32), 2), np.zeros((0, 4), np.float32), np.zeros(0, np.int32),
+                 pairs, "bricks", {}, pts.reshape(-1, 3), np.full(n, 8, np.int32))
+    desc = L.default_desc
+
+    def scaled(*a):
+        c = desc(*a)
+        c.contact_offset, c.tolerance_length = 0.02 * scale, scale
+        return c
+
+    monkeypatch.setattr(L, "default_desc", scaled)
+    g = P.Scene(sc, position_iterations=4, velocity_iterations=1, contact_offset=0.02 * scale, tolerance_length=scale)
+    o = L.OracleWorld(sc, pos_iters=4, vel_iters=1)
+    g.step(DT)
+    o.step(DT)
+    assert _compare_contacts(g, o, tol_p=1e-4 * scale) == pairs
