@@ -100,8 +100,9 @@ def test_parallel_faces_at_scale_match_oracle(cuda, monkeypatch, scale):
     """400 pairs of bricks with facing faces parallel and less than the contact
     distance apart, lengths in units from 100 m to 10 um: every vertex and
     edge of the facing faces lies at the distance itself, so a feature bound that
-    is tighter than the rounding of a height drops them. The tolerances scale with
-    the lengths; the rounding of coordinates of 1.5 lengths is 1e-7 of them."""
+    is tighter than the rounding of a height drops them (with a margin of 1e-4
+    at every size 6 pairs lost their contact at 1e4 and 1 at 1e5). The tolerances
+    scale with the lengths; the rounding of coordinates of 1.5 lengths is 1e-7 of them."""
     pairs = 400
     rng = np.random.default_rng(17)
     half = rng.uniform(0.2, 0.6, (2 * pairs, 3)) * scale
