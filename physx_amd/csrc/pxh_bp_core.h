@@ -72,7 +72,8 @@ int broadphase(Ctx* s, int classes, int n, int nWorlds, int maxWorldBodies, cons
 {
 	PXH_CHECK(s->gridF.ensure(nWorlds));
 	PXH_CHECK(s->gridI.ensure(nWorlds));
-	PXH_CHECK(s->scanTmp.ensure(scan_tmp_size(std::max<int64_t>(int64_t(classes) * n + 1, 256 * 1024)) + 1024));
+	PXH_CHECK(s->scanTmp.ensure(
+	    std::max(scan_tmp_size(std::max<int64_t>(int64_t(classes) * n + 1, 256 * 1024)), radix_tmp_size(n)) + 1024));
 	PXH_CHECK(s->gridAcc.ensure(size_t(5) * nWorlds));
 	PXH_CHECK(s->keys.ensure(n));
 	PXH_CHECK(s->keys2.ensure(n));
@@ -83,8 +84,8 @@ int broadphase(Ctx* s, int classes, int n, int nWorlds, int maxWorldBodies, cons
 	const int nblocks = (n + radix_tile() - 1) / radix_tile();
 	PXH_CHECK(s->hist.ensure(size_t(256) * std::max(nblocks, 1)));
 	bool alt = false;
-	launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, n, 32, bitsFor(totalRows - 1u), s->hist.p, st,
-	                  alt);
+	launch_radix_sort(s->keys.p, s->vals.p, s->keys2.p, s->vals2.p, n, 32, bitsFor(totalRows - 1u), s->hist.p,
+	                  s->scanTmp.p, st, alt);
 	s->sortedKeys = alt ? s->keys2.p : s->keys.p;
 	const uint32_t* sv = alt ? s->vals2.p : s->vals.p;
 
@@ -168,10 +169,12 @@ int bp_update(Ctx* bp, const float* bounds, const uint32_t* groups, const float*
 	launch_pair_keys(P, bp->pairs.p, ids, bp->pkCur.p, bp->vals.p, st);
 	const int nblocks = (P + radix_tile() - 1) / radix_tile();
 	PXH_CHECK(bp->hist.ensure(size_t(256) * std::max(nblocks, 1)));
-	PXH_CHECK(bp->scanTmp.ensure(scan_tmp_size(std::max<int64_t>(P + 1, int64_t(bp->nCur) + 1)) + 1024));
+	PXH_CHECK(bp->scanTmp.ensure(
+	    std::max(scan_tmp_size(std::max<int64_t>(int64_t(P) + 1, int64_t(bp->nCur) + 1)), radix_tmp_size(P)) + 1024));
 	bool alt = false;
 	const int bits = bitsFor(uint64_t(ids ? std::max<uint32_t>(idBound, 1u) : uint32_t(std::max(n, 1))) - 1);
-	launch_radix_sort(bp->pkCur.p, bp->vals.p, bp->pkTmp.p, bp->vals2.p, P, bits, bits, bp->hist.p, st, alt);
+	launch_radix_sort(bp->pkCur.p, bp->vals.p, bp->pkTmp.p, bp->vals2.p, P, bits, bits, bp->hist.p, bp->scanTmp.p, st,
+	                  alt);
 	if (alt)
 		std::swap(bp->pkCur, bp->pkTmp);
 	bp->nCur = P;

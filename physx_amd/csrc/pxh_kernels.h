@@ -141,12 +141,14 @@ constexpr int COLOR_SHORT_LIST = 2048;
 
 int64_t scan_tmp_size(int64_t n);
 void launch_scan(uint32_t* data, int64_t n, uint32_t* tmp, hipStream_t st);
-// keys per radix-sort workgroup (its histogram holds 256 counts per workgroup)
+// keys per radix-sort workgroup (its histogram holds 256 counts per workgroup);
+// words of scan scratch a sort of n keys needs
 int radix_tile();
+int64_t radix_tmp_size(int n);
 // stable sort by the key's high word, below 2^highBits, then by the low
 // lowBits bits of its low word (0: the low word is not compared)
 void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t* vals2, int n, int lowBits,
-                       int highBits, uint32_t* hist, hipStream_t st, bool& resultInAlt);
+                       int highBits, uint32_t* hist, uint32_t* scanTmp, hipStream_t st, bool& resultInAlt);
 // whether a sort of n keys of `bits` bits leaves its result in keys2 / vals2
 bool radix_result_in_alt(int n, int bits);
 
@@ -197,9 +199,9 @@ void launch_copy_contacts(int C, int maxPairs, const int* order, const int* conA
 // constraint list of the touching slots: slots [0, Q) are body-plane pairs, body
 // pairs follow up to the device count *dP; conPKey: world-relative pair identity
 // (world tag 16 | local a 24 | local b or 0x800000 | plane 24). flags: S entries,
-// tileSums: one per con_tile() slots; hostCounts (host memory) receives *dP, the constraint
+// tileSums: con_tmp_size(S) entries; hostCounts (host memory) receives *dP, the constraint
 // count and *overflow (0 when null)
-int con_tile();
+int64_t con_tmp_size(int64_t slots);
 void launch_con_build(int S, int Q, int pairEnd, const uint32_t* dP, const float4* ctN, uint32_t* flags,
                       uint32_t* tileSums, const uint2* pairs, const int* qBody, const int* qPlane, const int* meshBody,
                       int nPlanes, const int* local, const int* planeLocal, const int* world, const int* worldTag,

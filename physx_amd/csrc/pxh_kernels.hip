@@ -70,9 +70,11 @@ PXH_D uint32_t blockExclScan(uint32_t v, uint32_t* sh, uint32_t& total)
 // tile adds up the sums before it and scans its own elements; an array of one
 // tile needs the second launch alone. Bound by launches and their latency at
 // the step's sizes: 11 us on average at 262k bodies, where three launches and a
-// second pass over the data took 13. A tile of 4,096 keeps the sums to add up
-// below 1,500 for the largest arrays here (six pair classes of a million
-// bodies).
+// second pass over the data took 13. Adding up grows with the square of the
+// tiles, so past SUMS_DIRECT of them the sums are scanned first (adding up and
+// scanning: 4,096 tiles 42 / 44 us, 8,192 tiles 90 / 71, 32,768 tiles 715 / 378; the
+// constraint list's 1,024-slot tiles: 4,096 25 / 26 us, 8,192 49 / 41, 65,536 940 / 324).
+constexpr int SUMS_DIRECT = 4096;
 constexpr int SCAN_THREADS = 256, SCAN_ITEMS = 16, SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
 
 // sum over the block; every thread gets it (sh: 8 entries)
@@ -107,7 +109,26 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_sums(const uint32_t* data
 		sums[blockIdx.x] = v;
 }
 
+// what the tiles before this one hold: the tile's entry of scanned sums, or their
+// sum, added up here (sh: 8 entries; its barriers also publish LDS)
+template <bool SCANNED> PXH_D uint32_t tilesBefore(const uint32_t* sums, uint32_t* sh)
+{
+	if constexpr (SCANNED)
+	{
+		__syncthreads();
+		return sums[blockIdx.x];
+	}
+	else
+	{
+		uint32_t before = 0;
+		for (int t = threadIdx.x; t < int(blockIdx.x); t += int(blockDim.x))
+			before += sums[t];
+		return blockSum(before, sh);
+	}
+}
+
 // in-place exclusive scan of each tile, offset by the sums of the tiles before it
+template <bool SCANNED>
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(uint32_t* data, int64_t n, const uint32_t* sums)
 {
 	__shared__ uint32_t sh[33];
@@ -120,10 +141,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(uint32_t* data, int
 		const int i = k * SCAN_THREADS + threadIdx.x;
 		tile[at(i)] = base + i < n ? data[base + i] : 0u;
 	}
-	uint32_t before = 0;
-	for (int t = threadIdx.x; t < int(blockIdx.x); t += SCAN_THREADS)
-		before += sums[t];
-	before = blockSum(before, sh);   // its barriers also publish the tile
+	const uint32_t before = tilesBefore<SCANNED>(sums, sh);
 	uint32_t loc[SCAN_ITEMS];
 	uint32_t sum = 0;
 #pragma unroll
@@ -158,16 +176,20 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(uint32_t* data, int
 // them cost no pass.
 //
 // Up to RS_SMALL keys: one launch, one workgroup keeps the keys in registers
-// through every pass. More: two launches a pass, the digit counts of 4,096-key
-// tiles and the scatter, in which each tile adds up the counts of the tiles
-// before it itself (a 262,144-key sort has 64 tiles), so no scan runs between.
+// through every pass. Up to RS_DIRECT tiles of 4,096: two launches a pass, the
+// digit counts of the tiles and the scatter, in which each tile adds up the counts
+// of all tiles itself, so no scan runs between. Past that, since the adding up
+// grows with the square of the tiles, the counts are laid out digit by digit and
+// scanned between the two.
 // A key's rank in its wave comes from eight ballots (the lanes with its digit).
-// Bound by launches and latency. 262,144 broadphase keys (51 bits, seven
-// passes): 107 us, where a count, a scan of three launches and a bit-by-bit
-// split a pass took 219; 4,096 keys (six passes): 30 us in one launch against
-// 117 in thirty; a million keys: 18 us a scatter against 22.
+// Bound by launches and latency. 262,144 broadphase keys (51 bits, seven passes):
+// 92 us back to back, where a count, a scan of three launches and a bit-by-bit split
+// a pass took 219 in the step. One workgroup against tiles: 4,096 keys 34 / 67 us,
+// 8,192 keys 59 / 76 (of 16 bits 19 / 22). Adding up against scanning: 256 tiles
+// 128 / 155 us, 512 tiles 225 / 198, 4,096 tiles 5.3 / 1.1 ms.
 constexpr int RS_THREADS = 1024, RS_ITEMS = 4, RS_TILE = RS_THREADS * RS_ITEMS;
 constexpr int RS_SMALL_THREADS = 1024, RS_SMALL_ITEMS = 8, RS_SMALL = RS_SMALL_THREADS * RS_SMALL_ITEMS;
+constexpr int RS_DIRECT = 384;
 int radix_tile() { return RS_TILE; }
 
 PXH_D uint32_t rsDigit(uint64_t key, int lowBits, int shift)
@@ -190,8 +212,15 @@ PXH_D uint64_t rsPeers(uint32_t d, bool valid)
 	return m;
 }
 
+// where the counts of digit d of tile b lie: tile by tile, or digit by digit for a scan
+template <bool SCANNED> PXH_D int64_t rsCount(int d, int b, int nblocks)
+{
+	return SCANNED ? int64_t(d) * nblocks + b : int64_t(b) * 256 + d;
+}
+
+template <bool SCANNED>
 __global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const uint64_t* keys, int n, int lowBits, int shift,
-                                                        uint32_t* hist)
+                                                        uint32_t* hist, int nblocks)
 {
 	__shared__ uint32_t cnt[256];
 	if (threadIdx.x < 256)
@@ -207,9 +236,10 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const uint64_t* keys, in
 	}
 	__syncthreads();
 	if (threadIdx.x < 256)
-		hist[int64_t(blockIdx.x) * 256 + threadIdx.x] = cnt[threadIdx.x];
+		hist[rsCount<SCANNED>(threadIdx.x, blockIdx.x, nblocks)] = cnt[threadIdx.x];
 }
 
+template <bool SCANNED>
 __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const uint64_t* kin, const uint32_t* vin, uint64_t* kout,
                                                            uint32_t* vout, int n, int lowBits, int shift,
                                                            const uint32_t* hist, int nblocks)
@@ -237,13 +267,14 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const uint64_t* kin, 
 		cnt[w][i] = 0u;
 	// this digit's count over all tiles and over the tiles before this one,
 	// every PARTS-th tile to each part of the block
+	if constexpr (!SCANNED)
 	{
 		const int d = threadIdx.x & 255, p = threadIdx.x >> 8;
 		uint32_t all = 0, before = 0;
 #pragma unroll 8
 		for (int b = p; b < nblocks; b += PARTS)
 		{
-			const uint32_t c = hist[int64_t(b) * 256 + d];
+			const uint32_t c = hist[rsCount<false>(d, b, nblocks)];
 			all += c;
 			before += b < int(blockIdx.x) ? c : 0u;
 		}
@@ -280,16 +311,21 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const uint64_t* kin, 
 				cnt[i][d] = own;
 				own += c;
 			}
-#pragma unroll
-			for (int p = 0; p < PARTS; p++)
+			if constexpr (SCANNED)
+				before = hist[rsCount<true>(d, blockIdx.x, nblocks)];
+			else
 			{
-				total += part[p][0][d];
-				before += part[p][1][d];
+#pragma unroll
+				for (int p = 0; p < PARTS; p++)
+				{
+					total += part[p][0][d];
+					before += part[p][1][d];
+				}
 			}
 		}
 		uint32_t sum;
 		const uint32_t local = blockExclScan(own, sh, sum);
-		const uint32_t pre = blockExclScan(total, sh, sum);
+		const uint32_t pre = SCANNED ? 0u : blockExclScan(total, sh, sum);
 		if (threadIdx.x < 256)
 		{
 			start[d] = local;
@@ -1368,7 +1404,6 @@ PXH_D bool liveSlot(int s, int Q, int pairEnd, const uint32_t* dP)
 // than the scan's: a thread that built up to sixteen constraints one after the
 // other took 20 us at 20,011 bodies)
 constexpr int CON_THREADS = 256, CON_ITEMS = 4, CON_TILE = CON_THREADS * CON_ITEMS;
-int con_tile() { return CON_TILE; }
 __global__ void __launch_bounds__(CON_THREADS) k_touch_flags(int S, int Q, int pairEnd, const uint32_t* dP,
                                                              const float4* ctN, uint32_t* flags, uint32_t* sums)
 {
@@ -1442,6 +1477,7 @@ PXH_D void buildConstraint(int s, int c, int Q, int pairEnd, const uint2* pairs,
 	conColor[c] = b >= 0 ? -1 : -2;  // -2: body-plane, placed after the body-body rounds
 }
 
+template <bool SCANNED>
 __global__ void __launch_bounds__(CON_THREADS) k_con_build(
     int S, int Q, int pairEnd, const uint32_t* dP, const uint32_t* flags, const uint32_t* sums, const uint2* pairs,
     const int* qBody, const int* qPlane, const int* meshBody, int nPlanes, const int* local, const int* planeLocal,
@@ -1451,10 +1487,7 @@ __global__ void __launch_bounds__(CON_THREADS) k_con_build(
 	__shared__ uint32_t sh[33];
 	__shared__ uint32_t waveSum[CON_ITEMS][CON_THREADS / 64];
 	const int base = blockIdx.x * CON_TILE;
-	uint32_t before = 0;
-	for (int t = threadIdx.x; t < int(blockIdx.x); t += CON_THREADS)
-		before += sums[t];
-	before = blockSum(before, sh);
+	const uint32_t before = tilesBefore<SCANNED>(sums, sh);
 	// slot k * CON_THREADS + thread of the tile: its place among the wave's flags
 	// of row k, then the waves before it
 	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -3966,15 +3999,31 @@ void launch_scan(uint32_t* data, int64_t n, uint32_t* tmp, hipStream_t st)
 	const int nb = nblk(n, SCAN_TILE);
 	if (nb > 1)
 		k_scan_sums<<<nb, SCAN_THREADS, 0, st>>>(data, n, tmp);
-	k_scan_tiles<<<nb, SCAN_THREADS, 0, st>>>(data, n, tmp);
+	if (nb > SUMS_DIRECT)
+	{
+		launch_scan(tmp, nb, tmp + nb, st);
+		k_scan_tiles<true><<<nb, SCAN_THREADS, 0, st>>>(data, n, tmp);
+	}
+	else
+		k_scan_tiles<false><<<nb, SCAN_THREADS, 0, st>>>(data, n, tmp);
 }
 
-int64_t scan_tmp_size(int64_t n) { return (std::max<int64_t>(n, 0) + SCAN_TILE - 1) / SCAN_TILE + 1; }
+int64_t scan_tmp_size(int64_t n)
+{
+	const int64_t nb = (std::max<int64_t>(n, 0) + SCAN_TILE - 1) / SCAN_TILE;
+	return nb + 1 + (nb > SUMS_DIRECT ? scan_tmp_size(nb) : 0);
+}
+int64_t con_tmp_size(int64_t slots)
+{
+	const int64_t nb = slots / CON_TILE + 1;
+	return nb + scan_tmp_size(nb);
+}
 
+int64_t radix_tmp_size(int n) { return scan_tmp_size(int64_t(256) * nblk(n, RS_TILE)); }
 bool radix_result_in_alt(int n, int bits) { return n > RS_SMALL && ((bits + 7) / 8) % 2 == 1; }
 
 void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t* vals2, int n, int lowBits,
-                       int highBits, uint32_t* hist, hipStream_t st, bool& resultInAlt)
+                       int highBits, uint32_t* hist, uint32_t* scanTmp, hipStream_t st, bool& resultInAlt)
 {
 	resultInAlt = false;
 	const int bits = lowBits + highBits;
@@ -3999,8 +4048,17 @@ void launch_radix_sort(uint64_t* keys, uint32_t* vals, uint64_t* keys2, uint32_t
 	uint32_t* vb = vals2;
 	for (int shift = 0; shift < bits; shift += 8)
 	{
-		k_rs_hist<<<nb, RS_THREADS, 0, st>>>(ka, n, lowBits, shift, hist);
-		k_rs_scatter<<<nb, RS_THREADS, 0, st>>>(ka, va, kb, vb, n, lowBits, shift, hist, nb);
+		if (nb > RS_DIRECT)
+		{
+			k_rs_hist<true><<<nb, RS_THREADS, 0, st>>>(ka, n, lowBits, shift, hist, nb);
+			launch_scan(hist, int64_t(256) * nb, scanTmp, st);
+			k_rs_scatter<true><<<nb, RS_THREADS, 0, st>>>(ka, va, kb, vb, n, lowBits, shift, hist, nb);
+		}
+		else
+		{
+			k_rs_hist<false><<<nb, RS_THREADS, 0, st>>>(ka, n, lowBits, shift, hist, nb);
+			k_rs_scatter<false><<<nb, RS_THREADS, 0, st>>>(ka, va, kb, vb, n, lowBits, shift, hist, nb);
+		}
 		uint64_t* tk = ka; ka = kb; kb = tk;
 		uint32_t* tv = va; va = vb; vb = tv;
 		resultInAlt = !resultInAlt;
@@ -4015,9 +4073,9 @@ void launch_bounds(int n, const float4* pos, const float4* rot, const float4* ge
 {
 	PXH_LAUNCH(k_bounds, n, n, pos, rot, geom, hs, co, bmin, bmax, cs);
 }
-// Worlds of up to 8,192 bodies take a workgroup each (4,096 bodies in one world:
-// 7 us against 11 in four launches); a larger world takes the launches over
-// all bodies, whose blocks spread over the chip.
+// Worlds of up to 8,192 bodies take a workgroup each (in one world, against four
+// launches: 4,096 bodies 6.4 / 10.4 us, 8,192 8.7 / 10.6, 12,288 11.4 / 10.7); a
+// larger world takes the launches over all bodies, whose blocks spread over the chip.
 constexpr int WORLD_GRID_MAX = 8192;
 void launch_scene_grid(int n, int nScenes, int maxWorldBodies, const int* bodyStart, const int* scene,
                        const float4* bmin, const float4* bmax, uint32_t* acc, float4* gridF, int2* gridI,
@@ -4221,9 +4279,13 @@ void launch_con_build(int S, int Q, int pairEnd, const uint32_t* dP, const float
 {
 	const int nb = std::max(nblk(S, CON_TILE), 1);
 	k_touch_flags<<<nb, CON_THREADS, 0, st>>>(S, Q, pairEnd, dP, ctN, flags, scanTmp);
-	k_con_build<<<nb, CON_THREADS, 0, st>>>(S, Q, pairEnd, dP, flags, scanTmp, pairs, qBody, qPlane, meshBody, nPlanes,
-	                                         local, planeLocal, world, worldTag, overflow, conA, conB, conSlot, conKey,
-	                                         conPKey, conColor, hostCounts);
+	const bool scanned = nb > SUMS_DIRECT;
+	if (scanned)
+		launch_scan(scanTmp, nb, scanTmp + nb, st);
+	auto kernel = scanned ? k_con_build<true> : k_con_build<false>;
+	kernel<<<nb, CON_THREADS, 0, st>>>(S, Q, pairEnd, dP, flags, scanTmp, pairs, qBody, qPlane, meshBody, nPlanes, local,
+	                                   planeLocal, world, worldTag, overflow, conA, conB, conSlot, conKey, conPKey,
+	                                   conColor, hostCounts);
 }
 
 __global__ void k_gather4(int n, const int* idx, const uint32_t* in, uint32_t* out)

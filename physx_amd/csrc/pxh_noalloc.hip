@@ -87,7 +87,7 @@ size_t carve(unsigned char* base, NoAllocBP& c)
 	k.take(c.keys, N); k.take(c.keys2, N);
 	k.take(c.vals, NP); k.take(c.vals2, NP);
 	k.take(c.hist, 256 * tiles);
-	k.take(c.scanTmp, size_t(pxh::scan_tmp_size(int64_t(scanN))) + 1024);
+	k.take(c.scanTmp, size_t(std::max(pxh::scan_tmp_size(int64_t(scanN)), pxh::radix_tmp_size(int(NP)))) + 1024);
 	k.take(c.counts, std::max(size_t(pxh::PAIR_CLASSES) * N + 1, P + 1));
 	k.take(c.flags, P + 1); k.take(c.flags2, P + 1); k.take(c.rows, P + 1);
 	k.take(c.pkPrev, P); k.take(c.pkCur, P); k.take(c.pkTmp, P);

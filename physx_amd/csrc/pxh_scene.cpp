@@ -1828,7 +1828,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 			                          int(s->hJType.size()), s->jInfo.p, s->lin.p, s->ang.p, ss, st);
 		}
 		PXH_CHECK(s->flags.ensure(size_t(S) + 1));
-		PXH_CHECK(s->scanTmp.ensure(size_t(S) / size_t(pxh::con_tile()) + 1));
+		PXH_CHECK(s->scanTmp.ensure(size_t(pxh::con_tmp_size(S))));
 		const size_t Sc = std::max(S, 1);
 		PXH_CHECK(s->conA.ensure(Sc));
 		PXH_CHECK(s->conB.ensure(Sc));
@@ -1935,6 +1935,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 	{
 		const int nb = (C + pxh::radix_tile() - 1) / pxh::radix_tile();
 		PXH_CHECK(s->hist.ensure(size_t(256) * std::max(nb, 1)));
+		PXH_CHECK(s->scanTmp.ensure(size_t(pxh::radix_tmp_size(C))));
 	}
 	int rounds = 0;
 	const int kMaxRounds = 960;
@@ -1998,7 +1999,7 @@ int32_t pxh_scene_simulate(pxh_scene s, float dt)
 		else
 			pxh::launch_color_keys(C, s->conA.p, s->conB.p, s->m, s->conColor.p, colors, uint32_t(colorBound), s->keys.p,
 			                       va, st);
-		pxh::launch_radix_sort(s->keys.p, va, s->keys2.p, vb, C, 0, bits, s->hist.p, st, alt);
+		pxh::launch_radix_sort(s->keys.p, va, s->keys2.p, vb, C, 0, bits, s->hist.p, s->scanTmp.p, st, alt);
 		const uint64_t* ck = alt ? s->keys2.p : s->keys.p;
 		pxh::launch_row_start(C, ck, worldSolve ? s->segStart.p : s->hostCounts,
 		                      worldSolve ? uint32_t(slots) : uint32_t(colorBound), st, s->stepWords.p,

@@ -8,6 +8,7 @@ import pytest
 
 import oracle_libs as L
 import physx_amd as P
+from physx_amd import scenes as S
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +55,46 @@ def test_broadphase_one_row(cuda, n):
     prev = np.zeros(0, np.int64)
     for k in range(2):
         prev = _check(bp, _boxes(n, 4.0, n + k, line=True), prev, cuda)
+
+
+@pytest.mark.parametrize("n", [384 * 4096, 384 * 4096 + 1, 17_000_000])
+def test_broadphase_many_tiles(cuda, n):
+    """The last size whose sort tiles add up each other's counts, the first whose
+    counts are scanned, and one whose pair counts take a scan of scanned sums (more
+    than 4,096 tiles of 4,096): boxes in a shuffled order along rows, each one
+    overlapping the next of its row and no other."""
+    import torch
+    row = 4096
+    g = torch.Generator(device="cuda").manual_seed(n)
+    place = torch.randperm(n, generator=g, device="cuda")   # box -> place
+    x, y = (place % row).float(), (place // row).float() * 2.0
+    z = torch.zeros_like(x)
+    bounds = torch.stack([x - 0.6, y - 0.5, z - 0.5, x + 0.6, y + 0.5, z + 0.5], 1).contiguous()
+    torch.cuda.synchronize()   # the update reads the bounds on its own stream
+    bp = P.BroadPhase()
+    bp.update(bounds)
+    created, deleted = bp.fetch_results()
+    box = torch.empty_like(place)
+    box[place] = torch.arange(n, device="cuda")
+    k = torch.arange(n - 1, device="cuda")
+    k = k[k % row != row - 1]
+    a, b = torch.minimum(box[k], box[k + 1]), torch.maximum(box[k], box[k + 1])
+    want = torch.sort(a * (1 << 32) + b).values
+    got = torch.from_numpy(created.astype(np.int64)).cuda()
+    assert len(deleted) == 0
+    assert torch.equal(got[:, 0] * (1 << 32) + got[:, 1], want)
+    bp.close()
+
+
+@pytest.mark.parametrize("per_body", [1, 800, 1000])
+def test_constraint_list_many_tiles(cuda, per_body):
+    """more contact slots than 4,096 tiles of 1,024 (from the room for pairs asked
+    for): the same bits as with the least room"""
+    sc = S.batched_piles(n_scenes=1, nmin=5000, nmax=5000, seed=5)
+    a, b = P.Scene(sc), P.Scene(sc, max_pairs_per_body=per_body)
+    for _ in range(12):
+        a.step(1.0 / 60.0)
+        b.step(1.0 / 60.0)
+    assert a.stats()["constraints"] == b.stats()["constraints"] > 0
+    for u, v in zip(a.bodies(), b.bodies()):
+        np.testing.assert_array_equal(u, v)
