@@ -1046,7 +1046,7 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_pairs(int cap, const uint32_t
                                                          const float4* rot, const float4* geom, float cd, float tol,
                                                          float4* ctN, float4* ctP)
 {
-	__shared__ float4 points[BOX_MAX_POINTS * NP_THREADS];
+	__shared__ float4 points[3 * BOX_MAX_POINTS * NP_THREADS / 4];
 	const int p = blockIdx.x * NP_THREADS + threadIdx.x;
 	const bool live = p < cap && uint32_t(p) < *dConvex && uint32_t(p) < *dP;
 	if (!__any(live))
@@ -1082,7 +1082,7 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_pairs(int cap, const uint32_t
 			else if (t0 == GEOM_CAPSULE)
 				cnt = capsulePoly<true>(g0.x, g0.y, x0, boxPoly(mk(g1.x, g1.y, g1.z)), x1, cd, tol, 0, c);
 			else
-				cnt = boxBoxFace(mk(g0.x, g0.y, g0.z), x0, mk(g1.x, g1.y, g1.z), x1, cd, tol, points + threadIdx.x, c);
+				cnt = boxBoxFace(mk(g0.x, g0.y, g0.z), x0, mk(g1.x, g1.y, g1.z), x1, cd, tol, BoxPoints{reinterpret_cast<float*>(points) + threadIdx.x}, c);
 		}
 	}
 	boxBoxEdgeWave(cnt == BOXBOX_EDGE, mk(g0.x, g0.y, g0.z), x0, mk(g1.x, g1.y, g1.z), x1, cd, c, cnt);
@@ -3929,7 +3929,7 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_immediate(int n, const int* t
                                                              const float* pose1, float cd, float tol, float* out,
                                                              int* counts)
 {
-	__shared__ float4 points[BOX_MAX_POINTS * NP_THREADS];
+	__shared__ float4 points[3 * BOX_MAX_POINTS * NP_THREADS / 4];
 	// lanes past the last pair repeat it (they help the wave's box searches) and store nothing
 	const int own = blockIdx.x * NP_THREADS + threadIdx.x;
 	const int k = min(own, n - 1);
@@ -3959,7 +3959,7 @@ __global__ void __launch_bounds__(NP_THREADS) k_np_immediate(int n, const int* t
 		cnt = planeBox(pn, -dot(pn, x0.p), mk(g1[0], g1[1], g1[2]), x1, cd, points + threadIdx.x, c);
 	}
 	else if (t0 == GEOM_BOX && t1 == GEOM_BOX)
-		cnt = boxBoxFace(mk(g0[0], g0[1], g0[2]), x0, mk(g1[0], g1[1], g1[2]), x1, cd, tol, points + threadIdx.x, c);
+		cnt = boxBoxFace(mk(g0[0], g0[1], g0[2]), x0, mk(g1[0], g1[1], g1[2]), x1, cd, tol, BoxPoints{reinterpret_cast<float*>(points) + threadIdx.x}, c);
 	else if (t0 == GEOM_SPHERE && t1 == GEOM_CAPSULE)
 		cnt = sphereCapsule(g0[0], x0.p, g1[0], g1[1], x1, cd, c);
 	else if (t0 == GEOM_CAPSULE && t1 == GEOM_CAPSULE)

@@ -461,16 +461,35 @@ PXH_D bool polyContains(const f3 (&verts)[4], f3 p, f3 mn, f3 mx)
 	return inter > 0;
 }
 
-// Manifold points of one lane in LDS (x, y, z, penetration), 64 lanes side by
-// side: entry k at m[64 * k], so a wave's accesses are free of bank conflicts
-// whatever each lane's k. In private arrays these dynamically indexed points
-// went through scratch memory.
-constexpr int BOX_MAX_POINTS = 16;
+// Manifold points of one lane in LDS, 64 lanes side by side, so a wave's accesses
+// are free of bank conflicts whatever each lane's k. In private arrays these
+// dynamically indexed points went through scratch memory. A point is its position
+// in the reference face's plane and its penetration (minus its height), transformed
+// where it is read: 9 KB a wave, so as many waves run as the registers allow (16 a
+// compute unit). With 16 places of transformed points, 16 KB and 10 waves, a million
+// box pairs took 160 us and capsule-box pairs, which share the kernel, 205 (172 with
+// everything in scratch); now 132 and 165.
+//
+// Twelve places are enough: with a < 4 incident vertices inside the reference face
+// (all four end the search), those a, at most four reference corners, and for each
+// of the 4 - a other vertices at most one point on each of its two edges:
+// a + 4 + 2 (4 - a) = 12 - a.
+constexpr int BOX_MAX_POINTS = 12;
+struct BoxPoints
+{
+	float* m;
+	PXH_D void put(int k, float x, float y, float pen) const
+	{
+		m[192 * k] = x; m[192 * k + 64] = y; m[192 * k + 128] = pen;
+	}
+	PXH_D f3 at(int k) const { return mk(m[192 * k], m[192 * k + 64], m[192 * k + 128]); }
+	PXH_D float pen(int k) const { return m[192 * k + 128]; }
+};
 
 // calculateContacts (:170-330): up to 16 manifold points in reference-face
 // space. A point is kept as its position q on the incident face alone: its
 // partner on the reference face is (q.x, q.y, 0) and its penetration -q.z.
-PXH_D void calcContacts(float exIn, float eyIn, const f3 (&pts)[4], f3 incN, float4* m, int& nc, float cd)
+PXH_D void calcContacts(float exIn, float eyIn, const f3 (&pts)[4], f3 incN, const BoxPoints& m, int& nc, float cd)
 {
 	const float ex = exIn * 1.0001f, ey = eyIn * 1.0001f;
 	bool pen[4], area[4];
@@ -484,7 +503,7 @@ PXH_D void calcContacts(float exIn, float eyIn, const f3 (&pts)[4], f3 incN, flo
 		pen[i] = cd > z;
 		area[i] = pen[i] && ex >= fabsf(pts[i].x) && ey >= fabsf(pts[i].y);
 		if (area[i])
-			m[64 * nc++] = f4(pts[i], z);
+			m.put(nc++, pts[i].x, pts[i].y, z);
 	}
 	if (nc == 4)
 		return;
@@ -497,7 +516,7 @@ PXH_D void calcContacts(float exIn, float eyIn, const f3 (&pts)[4], f3 incN, flo
 		{
 			const float t = dot(incN, pts[0] - q0) / denom;
 			if (cd > -t)
-				m[64 * nc++] = make_float4(q0.x, q0.y, t, -t);
+				m.put(nc++, q0.x, q0.y, -t);
 		}
 	}
 	const f3 ext = mk(ex, ey, FLT_BIG);
@@ -519,12 +538,12 @@ PXH_D void calcContacts(float exIn, float eyIn, const f3 (&pts)[4], f3 incN, flo
 			if (!c0)
 			{
 				const f3 ip = d * tmin + p0;
-				m[64 * nc++] = f4(ip, -ip.z);
+				m.put(nc++, ip.x, ip.y, -ip.z);
 			}
 			if (!c1)
 			{
 				const f3 ip = d * tmax + p0;
-				m[64 * nc++] = f4(ip, -ip.z);
+				m.put(nc++, ip.x, ip.y, -ip.z);
 			}
 		}
 	}
@@ -536,35 +555,35 @@ PXH_D void calcContacts(float exIn, float eyIn, const f3 (&pts)[4], f3 incN, flo
 // candidate list is sixteen 4-bit indices in one 64-bit word and the four
 // choices stay in registers, so nothing is indexed in scratch. Same choices in
 // the same order.
-PXH_D void reduceBatchLds(const float4* m, int n, f3 cn0, float tol, int (&ch)[4])
+template <class Pos> PXH_D void reduceBatchLds(const BoxPoints& m, Pos pos, int n, f3 cn0, float tol, int (&ch)[4])
 {
 	uint64_t cand = 0xFEDCBA9876543210ull;
 	auto at = [&](int i) { return int(cand >> (4 * i)) & 15; };
 	auto put = [&](int i, int v) { cand = (cand & ~(15ull << (4 * i))) | (uint64_t(v) << (4 * i)); };
-	float maxPen = m[0].w, minPen = maxPen;
+	float maxPen = m.pen(0), minPen = maxPen;
 	int index = 0, ci = 0;
 	int nc = n;
 	for (int i = 1; i < n; i++)
 	{
-		const float pen = m[64 * i].w;
+		const float pen = m.pen(i);
 		minPen = fmaxf(minPen, pen);
 		if (maxPen > pen) { maxPen = pen; index = i; ci = i; }
 	}
 	ch[0] = index;
-	const f3 b0 = mk(m[64 * index]);
+	const f3 b0 = pos(index);
 	nc--; put(ci, at(nc));
-	f3 v = mk(m[64 * at(0)]) - b0;
+	f3 v = pos(at(0)) - b0;
 	float maxDist = dot(v, v);
 	index = at(0); ci = 0;
 	for (int i = 1; i < nc; i++)
 	{
-		v = mk(m[64 * at(i)]) - b0;
+		v = pos(at(i)) - b0;
 		const float d = dot(v, v);
 		if (d > maxDist) { maxDist = d; index = at(i); ci = i; }
 	}
 	ch[1] = index;
 	nc--; put(ci, at(nc));
-	v = mk(m[64 * index]) - b0;
+	v = pos(index) - b0;
 	f3 nrm = cross(v, cn0);
 	const float sq = dot(nrm, nrm);
 	if (sq > 0.0f) { const float L = sqrtf(sq); nrm = mk(nrm.x / L, nrm.y / L, nrm.z / L); } else nrm = cn0;
@@ -573,7 +592,7 @@ PXH_D void reduceBatchLds(const float4* m, int n, f3 cn0, float tol, int (&ch)[4
 	int index1 = at(0), ci1 = 0;
 	for (int i = 0; i < nc; i++)
 	{
-		v = mk(m[64 * at(i)]) - b0;
+		v = pos(at(i)) - b0;
 		const float d = dot(v, nrm);
 		if (d > maxDist) { maxDist = d; index = at(i); ci = i; }
 		if (minDist > d) { minDist = d; index1 = at(i); ci1 = i; }
@@ -587,7 +606,7 @@ PXH_D void reduceBatchLds(const float4* m, int n, f3 cn0, float tol, int (&ch)[4
 		maxDist = -FLT_BIG;
 		for (int i = 0; i < nc; i++)
 		{
-			v = mk(m[64 * at(i)]) - b0;
+			v = pos(at(i)) - b0;
 			const float d = dot(v, nrm);
 			if (d > maxDist) { maxDist = d; index1 = at(i); ci1 = i; }
 		}
@@ -600,13 +619,13 @@ PXH_D void reduceBatchLds(const float4* m, int n, f3 cn0, float tol, int (&ch)[4
 #pragma unroll
 		for (int i = 0; i < 4; i++)
 		{
-			float pen = m[64 * ch[i]].w;
+			float pen = m.pen(ch[i]);
 			if (pen > eps)
 			{
 				int cidx = -1;
 				for (int j = 0; j < nc; j++)
 				{
-					const float pen1 = m[64 * at(j)].w;
+					const float pen1 = m.pen(at(j));
 					if (pen > pen1 && eps > pen1) { pen = pen1; cidx = j; }
 				}
 				if (cidx >= 0)
@@ -857,7 +876,7 @@ PXH_D void boxBoxEdgeWave(bool need, f3 e0_, const xf& x0_, f3 e1_, const xf& x1
 // up to the clipping; a pair that it leaves without a point returns
 // BOXBOX_EDGE and is finished by boxBoxEdgeWave. m: the lane's points in LDS.
 constexpr int BOXBOX_EDGE = -2;
-PXH_D int boxBoxFace(f3 e0, const xf& x0, f3 e1, const xf& x1, float cd, float tol, float4* m, Contacts& o)
+PXH_D int boxBoxFace(f3 e0, const xf& x0, f3 e1, const xf& x1, float cd, float tol, const BoxPoints& m, Contacts& o)
 {
 	mxf t0, t1;
 	boxFrames(x0, x1, t0, t1);
@@ -971,14 +990,13 @@ PXH_D int boxBoxFace(f3 e0, const xf& x0, f3 e1, const xf& x1, float cd, float t
 	// the output only needs the box1-side point (lb before the swap is on the
 	// incident box, so after a swap the box1 point is la)
 	int idx[4] = {0, 1, 2, 3};
-	for (int i = 0; i < nc; i++)
-	{
-		const float4 q = m[64 * i];
-		m[64 * i] = f4(mxtrans(newTo1, mk(q.x, q.y, flip ? 0.0f : q.z)), q.w);
-	}
+	auto pos = [&](int i) {
+		const f3 q = m.at(i);
+		return mxtrans(newTo1, mk(q.x, q.y, flip ? 0.0f : -q.z));
+	};
 	if (nc > 4)
 	{
-		reduceBatchLds(m, nc, lnB, tol, idx);
+		reduceBatchLds(m, pos, nc, lnB, tol, idx);
 		nc = 4;
 	}
 	o.n = normalize(mmul(t1.r, lnB));
@@ -988,9 +1006,8 @@ PXH_D int boxBoxFace(f3 e0, const xf& x0, f3 e1, const xf& x1, float cd, float t
 	{
 		if (i >= nc)
 			break;
-		const float4 q = m[64 * idx[i]];
-		o.p[i] = mxtrans(t1, mk(q));
-		o.sep[i] = q.w;
+		o.p[i] = mxtrans(t1, pos(idx[i]));
+		o.sep[i] = m.pen(idx[i]);
 	}
 	return nc;
 }
