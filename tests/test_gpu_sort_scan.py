@@ -98,3 +98,20 @@ def test_constraint_list_many_tiles(cuda, per_body):
     assert a.stats()["constraints"] == b.stats()["constraints"] > 0
     for u, v in zip(a.bodies(), b.bodies()):
         np.testing.assert_array_equal(u, v)
+
+
+@pytest.mark.parametrize("n", [2, 65, 700, 3000])
+@pytest.mark.parametrize("extent", [(60.0, 0.0, 0.0), (20.0, 50.0, 0.0), (20.0, 0.0, 50.0), (10.0, 50.0, 50.0)])
+def test_broadphase_few_rows(cuda, n, extent):
+    """One box so wide that the grid has one, two or four rows: of a body's nine
+    lanes in the sweep one, two or four have candidates, and only lanes before
+    another one count theirs again to place them."""
+    rng = np.random.default_rng(n)
+    bp = P.BroadPhase()
+    prev = np.zeros(0, np.int64)
+    for _ in range(2):
+        c = rng.uniform(0.0, 1.0, (n, 3)) * extent
+        h = rng.uniform(0.1, 0.6, (n, 3))
+        h[n // 2] = 20.0
+        prev = _check(bp, np.concatenate([c - h, c + h], 1).astype(np.float32), prev, cuda)
+    assert len(prev) > 0
