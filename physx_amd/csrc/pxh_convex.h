@@ -37,6 +37,7 @@ struct Poly
 	f3 h;
 	float margin;
 	float slack;   // how far polygon vertices lie below their planes
+	float radius;  // of the vertices about the origin
 
 	PXH_D f3 vert(int i) const
 	{
@@ -82,6 +83,7 @@ PXH_D Poly hullPoly(const HullSet& hs, int id)
 	p.h = mk(0.0f, 0.0f, 0.0f);
 	p.margin = hs.bc[id].w;
 	p.slack = __int_as_float(b.w);
+	p.radius = hs.be[id].w;
 	return p;
 }
 
@@ -97,6 +99,7 @@ PXH_D Poly boxPoly(f3 h)
 	p.h = h;
 	p.margin = fminf(h.x, fminf(h.y, h.z)) * 0.15f;
 	p.slack = 0.0f;
+	p.radius = sqrtf(dot(h, h));
 	return p;
 }
 
@@ -1390,7 +1393,7 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, Cvx
 	// other polytope than lim = sqrt(U) plus a margin holds no closest feature. The
 	// margin is above what planes lie off their polygons' vertices and well above
 	// rounding: a height or a distance is off by a few units in the last place (6e-8
-	// each) of the largest coordinate, the margin is 1e-5 of it.
+	// each) of the largest coordinate, the margin is 1e-5 of what bounds that.
 	// What is left keeps its order and its indices, so the first minimum is unchanged.
 	int nA, nB;
 	float minA = 0.0f, maxB = 0.0f;
@@ -1436,8 +1439,7 @@ PXH_D void polySeparationWave(const Poly& A, const mxf& aToB, const Poly& B, Cvx
 		U = fminf(U, edgePairSq(L, L.elA[fu.i], L.elB[fu.j], c1, c2));
 	}
 	U = waveMin(U);
-	const f3 pA = lane < A.nv ? ldsV(L.va, lane) : mk(0.0f, 0.0f, 0.0f), pB = lane < B.nv ? ldsV(L.vb, lane) : pA;
-	const float extent = -waveMin(-fmaxf(fabsf(pA.x) + fabsf(pA.y) + fabsf(pA.z), fabsf(pB.x) + fabsf(pB.y) + fabsf(pB.z)));
+	const float extent = fabsf(aToB.p.x) + fabsf(aToB.p.y) + fabsf(aToB.p.z) + A.radius + B.radius;
 	const float margin = 1e-4f + 1e-5f * extent + A.slack + B.slack;
 	float lim = U < BIG ? sqrtf(U) + margin : BIG;
 	waveSync();
