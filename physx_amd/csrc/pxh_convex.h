@@ -1,5 +1,9 @@
-// Convex contact generation on the device, one pair per lane: convex mesh
-// (and the box seen as a polytope) against convex mesh, sphere and plane.
+// Convex contact generation on the device: convex mesh (and the box seen as a
+// polytope) against convex mesh, sphere, capsule and plane. The support steps that
+// drop pairs take eight lanes a pair (convexApart), the separation search a wave
+// (convexSeparationWave; one lane for hulls past its LDS, polySeparation), the
+// contacts of hull pairs 16 lanes (convexContactsGroup), those of spheres, capsules
+// and planes against a hull a wave, capsules against a box a lane (capsulePoly).
 // Each generator follows the reference's PCM contact generation on a fresh
 // manifold, so a pair gives the contacts of PxGenerateContacts with an empty
 // PxCache: the separation is the exact closest-feature distance or minimum

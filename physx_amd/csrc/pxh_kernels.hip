@@ -1049,11 +1049,11 @@ static inline int thinGrid(int64_t most) { return int(std::min<int64_t>(std::max
 // Body-body pairs; the shape order is the reference contact-method table's
 // (lower geometry type first), so body a of a sphere-box pair is the sphere.
 // Lanes past the pair count on the device (*dP) have no pair; pair p fills slot
-// slotBase + p. One wave per workgroup: its box manifolds take 16 KB of LDS, and
+// slotBase + p. One wave per workgroup: its box manifolds take 9 KB of LDS, and
 // the box pairs that clipping leaves without a point share the wave
 // (boxBoxEdgeWave), so no lane leaves before that. Bound by the longest lane of a
 // wave: with that search in one lane and the manifolds in scratch memory the
-// settled 262k sphere/box bin took 513 us, a 4,096-box pile 202 us; now 165 and 26.
+// settled 262k sphere/box bin took 513 us, a 4,096-box pile 202 us; now 136 and 28.
 constexpr int NP_THREADS = 64;
 __global__ void __launch_bounds__(NP_THREADS) k_np_pairs(int cap, const uint32_t* dP, const uint32_t* dConvex,
                                                          int slotBase, const uint2* pairs, const float4* pos,
@@ -2530,16 +2530,6 @@ __device__ __forceinline__ void solveTgsRow(int o, int C, const Rows& rows, TgsR
 	vel.store(hi.x, f4(l0, invMassA), f4(a0, 0.0f));
 	if (dynB)
 		vel.store(hi.y, f4(l1, invMassB), f4(a1, 0.0f));
-}
-
-template <class Vel>
-__device__ __forceinline__ void solveContactRowTGS(int o, int C, const Rows& rows, const Vel& vel, float minPen,
-                                                   float muS, float muD, float invStepDt, float biasScale,
-                                                   float scale, uint32_t* broken)
-{
-	TgsRow row;
-	loadTgsRow(o, C, rows, row);
-	solveTgsRow(o, C, rows, row, vel, minPen, muS, muD, invStepDt, biasScale, scale, broken);
 }
 
 __global__ void __launch_bounds__(SOLVE_THREADS) k_solve(int begin, int end, int C, Rows rows, float4* vel,
