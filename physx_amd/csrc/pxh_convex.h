@@ -578,6 +578,28 @@ PXH_D float segPoly(const Poly& B, f3 p, f3 q, f3& n, f3& cA, f3& cB)
 	return -best;
 }
 
+// whether some of B's planes keep the segment p, q outside, in one lane; the test
+// that segPoly, segPolyWave and (p = q) sphereConvexWave take a contact inside by
+PXH_D bool planesKeepOut(const Poly& B, f3 p, f3 q)
+{
+	const f3 d = q - p;
+	float t0 = 0.0f, t1 = 1.0f;
+	bool out = false;
+	for (int f = 0; f < B.np && !out; f++)
+	{
+		const f3 fn = B.pn(f);
+		const float hp = dot(fn, p) + B.pd(f), dn = dot(fn, d);
+		if (dn == 0.0f)
+			out = hp > 0.0f;
+		else if (dn < 0.0f)
+			t0 = fmaxf(t0, -hp / dn);
+		else
+			t1 = fminf(t1, -hp / dn);
+		out |= t0 > t1;
+	}
+	return out;
+}
+
 // segPoly over the wave: the lanes share B's faces and edges, the first minimum
 // in their order wins
 PXH_D float segPolyWave(const Poly& B, f3 p, f3 q, int lane, f3& n, f3& cA, f3& cB)

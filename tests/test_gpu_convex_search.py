@@ -146,3 +146,61 @@ def test_parallel_faces_at_scale_match_oracle(cuda, monkeypatch, scale):
     g.step(DT)
     o.step(DT)
     assert _compare_contacts(g, o, tol_p=1e-4 * scale) == pairs
+
+
+@pytest.mark.parametrize("capsules", [False, True])
+def test_round_shapes_inside_planes_past_the_vertices(cuda, monkeypatch, capsules):
+    """Merged faces of thin blades have planes that meet well outside the hull's
+    vertices, farther from its origin than any of them. A small sphere or capsule
+    there is inside every plane and has its contact, though the bounding spheres are
+    apart."""
+    from scipy.spatial import HalfspaceIntersection
+    r, cd = 0.001, 0.002
+    hulls, at = [], []
+    # blades (about one in a thousand) that have such a place within their vertices'
+    # box, where the broadphase reports the pair, and past their bounding sphere by
+    # more than four times what the planes lie off the vertices
+    for points, seed in [(10, 3345), (10, 3851), (10, 3949), (10, 3979), (12, 1244), (12, 1611), (12, 2076),
+                         (12, 2468), (12, 3143), (12, 3180), (12, 3979)]:
+        v = np.random.default_rng(seed).normal(size=(points, 3))
+        v = (v / np.linalg.norm(v, axis=1, keepdims=True) * [0.8, 0.5, 0.015]).astype(np.float32)
+        h = P.cook_convex(v)
+        pl = np.asarray(h["planes"], np.float64).reshape(-1, 4)
+        w = np.asarray(h["verts"], np.float64).reshape(-1, 3)
+        face = np.repeat(np.arange(len(pl)), h["poly_counts"])
+        slack = -((w[h["vrefs"]] * pl[face, :3]).sum(1) + pl[face, 3]).min()
+        c = HalfspaceIntersection(pl, w.mean(0)).intersections * (1.0 - 1e-3)
+        far = np.linalg.norm(c, axis=1) > np.linalg.norm(w, axis=1).max() + r + cd + 4.0 * slack + 1e-4
+        box = ((c > w.min(0) - r) & (c < w.max(0) + r)).all(1)
+        c = c[far & box]
+        hulls += [np.concatenate([v, np.repeat(v[:1], 12 - points, 0)])] * len(c)
+        at += list(c)
+    n = 2 * len(at)
+    t = np.full(n, S.CONVEX, np.int32)
+    dims = np.zeros((n, 4), np.float32)
+    dims[::2, 0] = np.arange(len(at))
+    t[1::2] = S.CAPSULE if capsules else S.SPHERE
+    dims[1::2, 0] = r
+    if capsules:
+        dims[1::2, 1] = 1e-4
+    pose = np.zeros((n, 7), np.float32)
+    pose[:, 6] = 1.0
+    pose[1::2, :3] = at
+    m, inn = S.mass_props(np.full(n, S.BOX, np.int32), np.full((n, 4), 0.3, np.float32), 1000.0)
+    z = np.zeros((n, 3), np.float32)
+    sc = S.Scene(t, dims, pose, z, z.copy(), m, inn, np.repeat(np.arange(len(at), dtype=np.int32), 2),
+                 np.zeros((0, 4), np.float32), np.zeros(0, np.int32), len(at), "blades", {}, np.concatenate(hulls),
+                 np.full(len(at), 12, np.int32))
+    desc = L.default_desc
+
+    def small(*a):
+        d = desc(*a)
+        d.contact_offset = cd / 2
+        return d
+
+    monkeypatch.setattr(L, "default_desc", small)
+    g = P.Scene(sc, position_iterations=4, velocity_iterations=1, contact_offset=cd / 2)
+    o = L.OracleWorld(sc, pos_iters=4, vel_iters=1)
+    g.step(DT)
+    o.step(DT)
+    assert _compare_contacts(g, o) >= 11
